@@ -1,6 +1,6 @@
 // Batched launcher: an arbitrary source set packed into lane groups, several
 // traversal contexts in flight on their own HIP streams, each level a
-// captured hipGraph of three kernels (expand, inspect, direction decision):
+// captured hipGraph of two kernels (expand; inspect and direction decision):
 // the direction is decided on the device, so the host only polls once per
 // burst of levels.
 #include <hip/hip_runtime.h>
@@ -202,7 +202,19 @@ InspectArgs dd_inspect_args(const ibfs_batch_s *b, const Ctx &c) {
   a.vpt = b->cfg.inspect_vpt;
   a.nw = b->cfg.wg_size / 64;
   a.hsplit = HubSplit{b->hc.deg, b->hc.tie, b->hc.cut};
+  a.spread = ctl_spread(c.ctl, b->R);
+  a.decide = split_hubs(b->g, b->hc, b->cfg) == 0;
   return a;
+}
+
+// Inspection of the plan's level and the decision of the next one (the
+// inspector's last workgroup decides unless split levels are on).
+hipError_t inspect_decide(const ibfs_batch_s *b, const Ctx &c) {
+  const InspectArgs a = dd_inspect_args(b, c);
+  const hipError_t e = launch_inspect(b->W, a, c.st);
+  if (e != hipSuccess || a.decide) return e;
+  return launch_plan_decide(c.d_plan, c.ctl, b->R, c.hs, b->W, split_hubs(b->g, b->hc, b->cfg),
+                            c.st);
 }
 
 int alloc_ctx(ibfs_batch_s *b, Ctx &c) {
@@ -216,7 +228,7 @@ int alloc_ctx(ibfs_batch_s *b, Ctx &c) {
     if (err == hipSuccess) err = hipHostMalloc(p, bytes ? bytes : 1, hipHostMallocDefault);
   };
   A((void **)&c.ring, (size_t)b->R * slot_bytes);
-  A((void **)&c.ctl, sizeof(LevelCtl) * (size_t)b->R);
+  A((void **)&c.ctl, ctl_ring_bytes(b->R));
   for (int i = 0; i < 6; ++i)
     if (i != Q_TD_L) A((void **)&c.q.q[i], sizeof(int32_t) * (size_t)Vq);
   A((void **)&c.q.chunks, sizeof(int2) * ((size_t)Vq + (size_t)(b->g->E >> b->chunk_shift) + 2));
@@ -267,10 +279,7 @@ int alloc_ctx(ibfs_batch_s *b, Ctx &c) {
       e1 = launch_expand_dd(b->W, b->g->d_beg, b->g->d_adj, b->g->d_tadj, c.ring, c.flags, b->R,
                             Vt, c.ctl, c.d_plan, c.hs, c.q, b->chunk_shift,
                             HubSplit{b->hc.deg, b->hc.tie, b->hc.cut}, c.tl, b->grid, c.st);
-      e2 = launch_inspect(b->W, dd_inspect_args(b, c), c.st);
-      if (e2 == hipSuccess)
-        e2 = launch_plan_decide(c.d_plan, c.ctl, b->R, c.hs, b->W,
-                                split_hubs(b->g, b->hc, b->cfg), c.st);
+      e2 = inspect_decide(b, c);
     }
     hipGraph_t &gr = pass == 0 ? c.graph : c.graph_burst;
     hipError_t e3 = hipStreamEndCapture(c.st, &gr);
@@ -343,10 +352,9 @@ int start_group(ibfs_batch_s *b, Ctx &c, const int32_t *src, int64_t g0, int k, 
   HIP_TRY(hipMemcpyAsync(c.d_setup, c.h_setup, c.setup_bytes, hipMemcpyHostToDevice, c.st));
   HIP_TRY(launch_zero3_u64(slot(b, c, 0), b->g->Vt * W, reinterpret_cast<u64 *>(c.flags),
                            (b->g->Vt + 7) / 8, reinterpret_cast<u64 *>(c.ctl),
-                           (int64_t)b->R * CTL_WORDS, c.st));
+                           (int64_t)(ctl_ring_bytes(b->R) / 8), c.st));
   HIP_TRY(launch_init_sources(W, c.d_src, k, 0, slot(b, c, 0), c.flags, c.st));
-  HIP_TRY(launch_inspect(W, dd_inspect_args(b, c), c.st));
-  HIP_TRY(launch_plan_decide(c.d_plan, c.ctl, b->R, c.hs, W, split_hubs(b->g, b->hc, b->cfg), c.st));
+  HIP_TRY(inspect_decide(b, c));
   c.g0 = g0;
   c.k = k;
   c.base = 0;
@@ -395,9 +403,7 @@ int launch_burst(ibfs_batch_s *b, Ctx &c, ibfs_stats *stats) {
                                c.tl, b->grid, c.st));
       HIP_TRY(launch_admit_dd(b->W, c.d_al, c.d_plan, c.ring, b->R, b->g->Vt, c.ctl, c.flags,
                               c.st));
-      HIP_TRY(launch_inspect(b->W, dd_inspect_args(b, c), c.st));
-      HIP_TRY(launch_plan_decide(c.d_plan, c.ctl, b->R, c.hs, b->W,
-                                 split_hubs(b->g, b->hc, b->cfg), c.st));
+      HIP_TRY(inspect_decide(b, c));
     } else {
       HIP_TRY(hipGraphLaunch(c.exec, c.st));
     }

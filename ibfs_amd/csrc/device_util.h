@@ -59,16 +59,41 @@ __device__ __forceinline__ bool differs(const u64 (&x)[W], const u64 (&y)[W]) {
   return d;
 }
 
+// Wave reductions through DPP moves (row shifts, then row broadcasts: lane 63
+// holds the result, read back as a scalar).  A lane that is not active
+// contributes nothing, but lane 63 must be: call them with the whole wave.  A
+// shuffle-based reduction goes through the LDS pipe twice per step and value.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ u64 dpp_or_zero(u64 x) {
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)x, CTRL, ROWS, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), CTRL, ROWS, 0xf, false);
+  return (u64)lo | ((u64)hi << 32);
+}
+
+__device__ __forceinline__ u64 lane63(u64 x) {
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)x, 63);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(x >> 32), 63);
+  return (u64)lo | ((u64)hi << 32);
+}
+
 __device__ __forceinline__ u64 wave_or(u64 x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x |= __shfl_xor(x, o, 64);
-  return x;
+  x |= dpp_or_zero<0x111, 0xf>(x);  // row_shr:1
+  x |= dpp_or_zero<0x112, 0xf>(x);  // row_shr:2
+  x |= dpp_or_zero<0x114, 0xf>(x);  // row_shr:4
+  x |= dpp_or_zero<0x118, 0xf>(x);  // row_shr:8
+  x |= dpp_or_zero<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x |= dpp_or_zero<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  return lane63(x);
 }
 
 __device__ __forceinline__ u64 wave_sum(u64 x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;
+  x += dpp_or_zero<0x111, 0xf>(x);
+  x += dpp_or_zero<0x112, 0xf>(x);
+  x += dpp_or_zero<0x114, 0xf>(x);
+  x += dpp_or_zero<0x118, 0xf>(x);
+  x += dpp_or_zero<0x142, 0xa>(x);
+  x += dpp_or_zero<0x143, 0xc>(x);
+  return lane63(x);
 }
 
 __device__ __forceinline__ unsigned wave_incl_scan(unsigned x, int lane) {

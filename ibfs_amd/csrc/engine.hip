@@ -36,7 +36,7 @@ struct ibfs_engine_s {
   u64 *ring = nullptr;
   LevelCtl *d_ctl = nullptr;
   LevelCtl *h_ctl = nullptr;  // pinned
-  CtlPost *post = nullptr;    // coherent pinned: control blocks posted by k_post_ctl
+  CtlPost *post = nullptr;    // coherent pinned: control blocks posted by the inspector
   u64 post_seq = 0;
   Queues q{};
   u64 *d_masks = nullptr;     // [0,W) lanes_all, [W,2W) sel, [2W, 2W+(R+1)W) level masks
@@ -124,12 +124,6 @@ hipError_t elapsed_ms(float *ms, hipEvent_t a, hipEvent_t b) {
     if (q != hipSuccess) return q;
   }
   return hipEventElapsedTime(ms, a, b);
-}
-
-int post_and_wait(ibfs_engine_s *e, const LevelCtl *d) {
-  const u64 seq = ++e->post_seq;
-  HIP_TRY(launch_post_ctl(d, e->post, seq, e->st));
-  return wait_post(e, seq);
 }
 
 hipEvent_t next_event(ibfs_engine_s *e) {
@@ -240,7 +234,8 @@ int decide(const ibfs_engine_s *e, int L, const LevelCtl &c, int dir_prev, u64 n
 }
 
 // Host-driven inspector arguments (the pass also refreshes the hub cache
-// from cur for the next bottom-up level).
+// from cur for the next bottom-up level); it posts its control block with the
+// next tag (wait_post).
 InspectArgs inspect_args(ibfs_engine_s *e, const u64 *prev, const u64 *cur, u64 *next,
                          const u64 *lam_prev, LevelCtl *ctl, LevelCtl *ctl_zero, int full_diff) {
   InspectArgs a{};
@@ -264,6 +259,9 @@ InspectArgs inspect_args(ibfs_engine_s *e, const u64 *prev, const u64 *cur, u64 
   a.vpt = e->cfg.inspect_vpt;
   a.nw = e->cfg.wg_size / 64;
   a.hsplit = HubSplit{e->hc.deg, e->hc.tie, e->hc.cut};
+  a.spread = ctl_spread(e->d_ctl, e->R);
+  a.post = e->post;
+  a.post_tag = ++e->post_seq;
   return a;
 }
 
@@ -324,7 +322,7 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
 
   // level 0: S_0 = source bits; inspection builds the level-1 queues
   HIP_TRY(launch_zero3_u64(slot(e, 0), Vt * W, reinterpret_cast<u64 *>(e->flags), (Vt + 7) / 8,
-                           reinterpret_cast<u64 *>(e->d_ctl), (int64_t)e->R * CTL_WORDS, e->st));
+                           reinterpret_cast<u64 *>(e->d_ctl), (int64_t)(ctl_ring_bytes(e->R) / 8), e->st));
   HIP_TRY(launch_init_sources(W, e->d_src, k, 0, slot(e, 0), e->flags, e->st));
   hipEvent_t ti0 = nullptr, ti1 = nullptr;
   if (timing) { ti0 = next_event(e); HIP_TRY(hipEventRecord(ti0, e->st)); }
@@ -333,7 +331,7 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
                          e->st));
   if (timing) { ti1 = next_event(e); HIP_TRY(hipEventRecord(ti1, e->st)); }
   {
-    const int rc = post_and_wait(e, &e->d_ctl[0]);
+    const int rc = wait_post(e, e->post_seq);
     if (rc) return rc;
   }
   auto record = [&](int L, int dir, const LevelCtl &c, float exp_ms, float insp_ms) {
@@ -452,14 +450,12 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
                                            (dir == 1 || tdf) ? 0 : 1),
                            e->st));
     if (timing) { y1 = next_event(e); HIP_TRY(hipEventRecord(y1, e->st)); }
-    const u64 seq = ++e->post_seq;
-    HIP_TRY(launch_post_ctl(&e->d_ctl[L % e->R], e->post, seq, e->st));
     {
       const int rc = settle();  // level L-1, while level L runs
       if (rc) return rc;
     }
     {
-      const int rc = wait_post(e, seq);
+      const int rc = wait_post(e, e->post_seq);
       if (rc) return rc;
     }
     if (stats) stats->n_inspect_launches++;
@@ -936,7 +932,7 @@ int ibfs_engine_create(ibfs_graph_t g, const ibfs_config *cfg_in, ibfs_engine_t 
     if (err == hipSuccess) err = hipHostMalloc(p, bytes ? bytes : 1, hipHostMallocDefault);
   };
   A((void **)&e->ring, (size_t)R * slot_bytes);
-  A((void **)&e->d_ctl, sizeof(LevelCtl) * (size_t)R);
+  A((void **)&e->d_ctl, ctl_ring_bytes(R));
   H((void **)&e->h_ctl, sizeof(LevelCtl));
   if (err == hipSuccess) err = hipHostMalloc((void **)&e->post, sizeof(CtlPost), hipHostMallocCoherent);
   if (err == hipSuccess) std::memset(e->post, 0, sizeof(CtlPost));

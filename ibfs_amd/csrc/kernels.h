@@ -35,10 +35,33 @@ constexpr int64_t CTL_WORDS = sizeof(LevelCtl) / 8;
 // as one little-endian 64-bit counter)
 static_assert(offsetof(LevelCtl, q) % 8 == 0, "LevelCtl queue pairs");
 
+// The inspector's workgroups add their counters into CTL_COPIES copies, one
+// cache line each (workgroup b into copy b % CTL_COPIES); the last workgroup
+// to finish (ticket) folds them into the level's control block and leaves
+// copies and ticket zero for the next pass.  Device atomics on one line
+// serialise at about 3.6 ns: 512 workgroups adding 8 counters each to one
+// block of counters would spend 15 us of a pass there.
+constexpr int CTL_COPIES = 16;
+struct alignas(128) CtlSpread {
+  u64 v[CTL_COPIES][16];  // n_changed .. m_front_nh (6), then the lanes that gained (MAX_W)
+  unsigned ticket;
+};
+static_assert(6 + MAX_W <= 16 && CTL_COPIES * 16 <= 256, "CtlSpread layout");
+// A ring of R control blocks is allocated with its CtlSpread behind it and
+// both start a traversal at zero.
+constexpr size_t ctl_ring_bytes(int R) {
+  return ((sizeof(LevelCtl) * (size_t)R + 127) & ~(size_t)127) + sizeof(CtlSpread);
+}
+inline CtlSpread *ctl_spread(LevelCtl *ring, int R) {
+  return reinterpret_cast<CtlSpread *>(reinterpret_cast<char *>(ring) + ctl_ring_bytes(R) -
+                                       sizeof(CtlSpread));
+}
+
 enum { Q_TD_S = 0, Q_TD_M = 1, Q_TD_L = 2, Q_BU_S = 3, Q_BU_M = 4, Q_BU_L = 5 };
 
-// Device-resident plan of a device-driven traversal: k_plan_decide writes the
-// next level's direction here after each inspection, the expander reads it.
+// Device-resident plan of a device-driven traversal: the inspector's last
+// workgroup (k_plan_decide with split levels) writes the next level's
+// direction here, the expander reads it.
 struct Plan {
   int level;            // level to expand next (== level being inspected)
   int dir;              // direction of `level`: 0 top-down, 1 bottom-up, 2 hybrid, 3 split,
@@ -180,6 +203,14 @@ struct Queues {
   int2 *chunks;   // (vertex, chunk index) of top-down large vertices
 };
 
+// A control block posted to coherent pinned host memory: the block's words,
+// then `tag` once they have arrived, so a host that reads the tag with an
+// acquire load sees the block without a copy command or an event.
+struct CtlPost {
+  LevelCtl c;
+  u64 tag;
+};
+
 // Arguments of one inspector pass.  Host-driven: prev/cur/next/lam_prev/ctl
 // given explicitly and plan == nullptr.  Device-driven: plan != nullptr and
 // the level, snapshot slots and control blocks are derived from plan->level.
@@ -213,6 +244,10 @@ struct InspectArgs {
   int full_diff;
   int nw;               // waves per workgroup: 4, 8 or 16 (0: 8)
   HubSplit hsplit;      // frontier degrees outside the pulled hubs are counted separately
+  CtlSpread *spread;    // the pass's counters before they are folded into ctl
+  int decide;           // plan mode: the last workgroup also decides the next level
+  CtlPost *post;        // host-driven (or null): the control block is posted here
+  u64 post_tag;
 };
 
 // The launchers report hipGetLastError() after their launches; a HIP call
@@ -225,14 +260,6 @@ hipError_t launch_fill_u64(u64 *p, int64_t n, u64 value, hipStream_t st);
 // zeros in [p0, p0+n0), [p1, p1+n1) and [p2, p2+n2) (u64 words), one launch
 hipError_t launch_zero3_u64(u64 *p0, int64_t n0, u64 *p1, int64_t n1, u64 *p2, int64_t n2,
                             hipStream_t st);
-// A control block posted to coherent pinned host memory: the block's words,
-// then `tag` with a system-scope release, so a host that reads the tag with
-// an acquire load sees the block without a copy command or an event.
-struct CtlPost {
-  LevelCtl c;
-  u64 tag;
-};
-hipError_t launch_post_ctl(const LevelCtl *src, CtlPost *dst, u64 tag, hipStream_t st);
 hipError_t launch_fill_i32(int32_t *p, int64_t n, int32_t value, hipStream_t st);
 // S0[src[i]] |= bit lane0+i, i < k (src in traversal ids; -1 entries skipped).
 hipError_t launch_init_sources(int W, const int32_t *src, int k, int lane0, u64 *S0,
@@ -275,7 +302,8 @@ hipError_t launch_expand_dd(int W, const int64_t *beg, const int32_t *adj, const
 hipError_t launch_tail_patch(int W, TailLog tl, int64_t n, int T, const int32_t *vid,
                              const LaneOut *lanes, const u64 *sel, int k_lanes, u64 *sum_out,
                              hipStream_t st);
-// Device-driven direction decision for plan->level + 1; a bottom-up choice
+// Device-driven direction decision for plan->level + 1 as a launch of its
+// own, for split levels only (InspectArgs::decide otherwise): a bottom-up choice
 // becomes a split level when some active lanes hold fewer than
 // plan->split_cov % of the top `hubs` hubs in the hub cache hs (W words per
 // hub).

@@ -26,18 +26,6 @@ __global__ void k_zero3_u64(u64 *p0, int64_t n0, u64 *p1, int64_t n1, u64 *p2, i
   }
 }
 
-// One wave: thread t < CTL_WORDS copies word t of the block (vector stores),
-// makes it visible system-wide, and after the barrier thread 0 releases the tag.
-__global__ void k_post_ctl(const LevelCtl *src, CtlPost *dst, u64 tag) {
-  const int t = threadIdx.x;
-  if (t < (int)CTL_WORDS) {
-    reinterpret_cast<u64 *>(&dst->c)[t] = atomic_read(reinterpret_cast<const u64 *>(src) + t);
-    __threadfence_system();
-  }
-  __syncthreads();
-  if (t == 0) __hip_atomic_store(&dst->tag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 __global__ void k_fill_i32(int32_t *p, int64_t n, int32_t value) {
   for (int64_t i = (int64_t)blockIdx.x * BS + threadIdx.x; i < n; i += (int64_t)gridDim.x * BS)
     p[i] = value;
@@ -99,31 +87,27 @@ __global__ void k_admit_dd(const AdmitList *al, const Plan *plan, u64 *ring, int
   }
 }
 
-// Direction of level L+1 from the counters of level L (same rule as the
-// host-driven driver): fixed switch level, or alpha/beta; or the entry into
-// and the progress of the sparse tail (Plan::tail_div).
-__device__ void plan_decide(Plan *p, const LevelCtl *c, int L) {
-  if (p->tail_start) {
-    // sparse tail level L: the records it appended are the next frontier;
-    // none ends the traversal, an overflowing log ends it for a dense rerun
-    const u64 cnt = atomic_read(&p->tail_count);
-    if (cnt > p->tail_cap || cnt == p->tail_hi) {
-      p->done = 1;
-      p->last = L - 1;
-      return;
-    }
-    p->tail_lo = p->tail_hi;
-    p->tail_hi = cnt;
-    p->dirlog[(L + 1) & 255] = 4;
-    p->level = L + 1;
+// Progress of the sparse tail, and the direction of level L+1 from the
+// counters of level L (same rule as the host-driven driver): fixed switch
+// level, or alpha/beta; or the entry into the sparse tail (Plan::tail_div).
+__device__ void plan_tail(Plan *p, int L) {
+  // sparse tail level L: the records it appended are the next frontier; none
+  // ends the traversal, an overflowing log ends it for a dense rerun
+  const u64 cnt = atomic_read(&p->tail_count);
+  if (cnt > p->tail_cap || cnt == p->tail_hi) {
+    p->done = 1;
+    p->last = L - 1;
     return;
   }
-  const u64 nch = atomic_read(&c->n_changed);
-  const u64 nf = atomic_read(&c->n_front);
-  const u64 mf = atomic_read(&c->m_front);
-  const u64 mc = atomic_read(&c->m_cand);
-  const u64 nc = atomic_read(&c->n_cand);
-  const u64 mfn = atomic_read(&c->m_front_nh);
+  p->tail_lo = p->tail_hi;
+  p->tail_hi = cnt;
+  p->dirlog[(L + 1) & 255] = 4;
+  p->level = L + 1;
+}
+
+__device__ void plan_decide(Plan *p, const LevelCtl &c, int L) {
+  const u64 nch = c.n_changed, nf = c.n_front, mf = c.m_front;
+  const u64 mc = c.m_cand, nc = c.n_cand, mfn = c.m_front_nh;
   if (nch == 0 && L >= p->hold) {
     p->done = 1;
     // level 0 always ends a window: lanes whose source is isolated change
@@ -180,7 +164,7 @@ __device__ void plan_decide(Plan *p, const LevelCtl *c, int L) {
 // atomics serialize, so their number per level is what this layout keeps
 // small.  Entries go to ballot prefix positions, ascending vertex order
 // within a tile.  Device-driven mode: the level and its slots come from the
-// plan; k_plan_decide then picks the next direction.
+// plan, and the last workgroup picks the next direction.
 __device__ __forceinline__ unsigned lanes_below(u64 m) {
   return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
@@ -191,6 +175,9 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
   __shared__ unsigned wsum[2][NW][6];   // per-wave class totals, double-buffered by tile parity
   __shared__ unsigned wbase[2][NW][6];  // per-wave queue bases
   __shared__ u64 red[NW][6 + W];
+  __shared__ u64 fold[CTL_COPIES][16];
+  __shared__ LevelCtl fin;
+  __shared__ int last_s;
 
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const u64 *prev = a.prev, *cur = a.cur;
@@ -199,8 +186,12 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
   LevelCtl *ctl = a.ctl, *ctl_zero = a.ctl_zero;
   int full = a.full_diff;
   if (a.plan) {
-    if (a.plan->done || a.plan->tail_start) return;  // sparse tail levels skip the pass
+    if (a.plan->done) return;
     const int L = a.plan->level;
+    if (a.plan->tail_start) {  // sparse tail levels skip the pass
+      if (a.decide && blockIdx.x == 0 && t == 0) plan_tail(a.plan, L);
+      return;
+    }
     full = (L == 0 || !(a.plan->dir == 1 || (a.plan->dir == 0 && a.plan->td_flag)));
     const int64_t slot = a.V * W;
     prev = L > 0 ? a.ring + (int64_t)((L - 1) % a.R) * slot : nullptr;
@@ -226,7 +217,8 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
     load_word<W>(cur + (int64_t)a.hubs[i] * W, x);
     store_word<W>(a.hs + i * W, x);
   }
-  u64 n_changed = 0, n_front = 0, m_front = 0, n_cand = 0, m_cand = 0, m_front_nh = 0;
+  unsigned n_changed = 0, n_front = 0, n_cand = 0;  // of the wave
+  u64 m_front = 0, m_cand = 0, m_front_nh = 0;      // of the lane
   const HubSplit hsp = a.hsplit;
   const int64_t V = a.V;
   const int sml = a.sml, lrg = a.lrg, cs = a.chunk_shift;
@@ -292,9 +284,7 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
         store_word<W>(next + v * W, n);
         const int dg = dgv[i];
         if (ch) {
-          ++n_changed;
           if (dg > 0) {
-            ++n_front;
             m_front += (u64)dg;
             if (!is_hub(hsp, v, dg)) m_front_nh += (u64)dg;
             tc = degree_class(dg, sml, lrg);
@@ -302,19 +292,24 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
           }
         }
         if (dg > 0 && !cover) {
-          ++n_cand;
           m_cand += (u64)dg;
           bc = degree_class(dg, sml, lrg);
         }
       }
       code[i] = (uint8_t)(tc | (bc << 2));
+      n_changed += (unsigned)__popcll(__ballot(ch));
       tot[Q_TD_S] += (unsigned)__popcll(__ballot(tc == 1));
       tot[Q_TD_M] += (unsigned)__popcll(__ballot(tc == 2));
-      if (__ballot(tc == 3)) tot[Q_TD_L] += (unsigned)wave_sum((u64)nck);
+      if (const u64 m3 = __ballot(tc == 3)) {
+        n_front += (unsigned)__popcll(m3);
+        tot[Q_TD_L] += (unsigned)wave_sum((u64)nck);
+      }
       tot[Q_BU_S] += (unsigned)__popcll(__ballot(bc == 1));
       tot[Q_BU_M] += (unsigned)__popcll(__ballot(bc == 2));
       tot[Q_BU_L] += (unsigned)__popcll(__ballot(bc == 3));
     }
+    n_front += tot[Q_TD_S] + tot[Q_TD_M];
+    n_cand += tot[Q_BU_S] + tot[Q_BU_M] + tot[Q_BU_L];
     if (lane == 0) {
 #pragma unroll
       for (int k = 0; k < 6; ++k) wsum[par][wv][k] = tot[k];
@@ -373,34 +368,73 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
     }
   }
 
-  // workgroup reduction of the level counters, one atomic each
-  u64 vals[6 + W] = {n_changed, n_front, m_front, n_cand, m_cand, m_front_nh};
+  // The level's counters: waves, then the workgroup, then one atomic each
+  // into the workgroup's copy.
+  u64 vals[6 + W] = {n_changed, n_front, 0, n_cand, 0, 0};
+  if (n_front) {
+    vals[2] = wave_sum(m_front);
+    vals[5] = wave_sum(m_front_nh);
+  }
+  if (n_cand) vals[4] = wave_sum(m_cand);
 #pragma unroll
-  for (int w = 0; w < W; ++w) vals[6 + w] = lamacc[w];
-#pragma unroll
-  for (int i = 0; i < 6; ++i) vals[i] = wave_sum(vals[i]);
-#pragma unroll
-  for (int w = 0; w < W; ++w) vals[6 + w] = wave_or(vals[6 + w]);
+  for (int w = 0; w < W; ++w) vals[6 + w] = n_changed ? wave_or(lamacc[w]) : 0;
   if (lane == 0) {
 #pragma unroll
     for (int i = 0; i < 6 + W; ++i) red[wv][i] = vals[i];
   }
   __syncthreads();
-  if (t < 6) {  // n_changed .. m_front_nh are consecutive
+  CtlSpread *sp = a.spread;
+  if (t < 6 + W) {
     u64 s = 0;
-    for (int w = 0; w < NW; ++w) s += red[w][t];
-    if (s) atomicAdd(&(&ctl->n_changed)[t], s);
-  } else if (t < 6 + W) {
-    u64 s = 0;
-    for (int w = 0; w < NW; ++w) s |= red[w][t];
-    if (s) atomicOr(&ctl->lam[t - 6], s);
+    for (int w = 0; w < NW; ++w) s = t < 6 ? s + red[w][t] : s | red[w][t];
+    u64 *d = &sp->v[blockIdx.x % CTL_COPIES][t];
+    if (s && t < 6) atomicAdd(d, s);
+    else if (s) atomicOr(d, s);
   }
+  // Measured against one set of counters and a launch of its own that posted
+  // or decided: 512 x 512 grid, 128 lanes, 35.1 -> 31.0 us per level; R-MAT
+  // s18 closeness 310 -> 291 ms; R-MAT s22, 8 groups of 128, 15.0 -> 14.6 ms.
+  // The last workgroup to take a ticket folds the copies.  What it reads was
+  // written by device atomics alone, and each workgroup has waited for the
+  // completion of its own before its ticket: no cache is written back or
+  // invalidated in the middle of the pass, as an agent-scope fence would do
+  // on this multi-XCD part.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (t == 0) last_s = atomicAdd(&sp->ticket, 1u) == gridDim.x - 1;
+  __syncthreads();
+  if (!last_s) return;
+  if (t < CTL_COPIES * 16) {
+    u64 *d = &sp->v[t >> 4][t & 15];
+    fold[t >> 4][t & 15] = atomic_read(d);
+    __hip_atomic_store(d, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (t == 0) __hip_atomic_store(&sp->ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (t < (int)CTL_WORDS) reinterpret_cast<u64 *>(&fin)[t] = 0;
+  __syncthreads();
+  if (t < 6 + W) {
+    u64 s = 0;
+    for (int c = 0; c < CTL_COPIES; ++c) s = t < 6 ? s + fold[c][t] : s | fold[c][t];
+    if (t < 6) (&ctl->n_changed)[t] = (&fin.n_changed)[t] = s;
+    else ctl->lam[t - 6] = fin.lam[t - 6] = s;
+  } else if (t >= 32 && t < 35) {
+    reinterpret_cast<u64 *>(fin.q)[t - 32] = atomic_read(reinterpret_cast<const u64 *>(ctl->q) + t - 32);
+  }
+  __syncthreads();
+  if (a.post) {  // one wave: the block's words arrive at the host before the tag
+    if (t < (int)CTL_WORDS)
+      __hip_atomic_store(&reinterpret_cast<u64 *>(&a.post->c)[t], reinterpret_cast<u64 *>(&fin)[t],
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (t == 0)
+      __hip_atomic_store(&a.post->tag, a.post_tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (a.plan && a.decide && t == 0) plan_decide(a.plan, fin, a.plan->level);
 }
 
-// Device-driven decision after the inspection of plan->level.  A separate
-// launch instead of a last-workgroup election inside the inspector: on this
-// multi-XCD part each workgroup's agent-scope fence would write back and
-// invalidate its L2 in the middle of the pass.
+// Device-driven decision after the inspection of plan->level, as a launch of
+// its own: the split rule reads hub-cache words that other workgroups of the
+// inspector stored, which they see only past a kernel boundary.
 // Thread 0 applies the direction rule.  A bottom-up choice with split_cov > 0
 // then samples 64 of the top `hubs` hubs in the hub cache hs (S_L words, W per
 // hub; wave w takes word w): an active lane set in at least split_cov % of
@@ -417,7 +451,8 @@ __global__ __launch_bounds__(512) void k_plan_decide(Plan *plan, const LevelCtl 
   __syncthreads();  // every wave has read the plan before thread 0 changes it
   if (done) return;
   if (t == 0) {
-    plan_decide(plan, ctl_ring + L % R, L);
+    if (plan->tail_start) plan_tail(plan, L);
+    else plan_decide(plan, ctl_ring[L % R], L);
     dir_s = plan->done ? -1 : plan->dir;
   }
   __syncthreads();
@@ -1272,8 +1307,9 @@ static void inspect_w(const InspectArgs &a, hipStream_t st) {
   else inspect_nw<W, 8>(a, st);
 }
 
+// A graph without an edge (V == 0) still runs one workgroup: the pass also
+// posts the control block and decides the next level.
 hipError_t launch_inspect(int W, const InspectArgs &a, hipStream_t st) {
-  if (a.V <= 0) return hipSuccess;
   IBFS_DISPATCH_W(W, inspect_w<WW>(a, st));
   return hipGetLastError();
 }
@@ -1333,12 +1369,6 @@ hipError_t launch_expand_hy(int W, const int64_t *beg, const int32_t *adj, const
   const Gather gs{prev, hs};
   IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_hy<WW>, g, blk, 0, st, beg, adj, tadj, gs, cur,
                                         ctl_prev, q, chunk_shift, hsplit));
-  return hipGetLastError();
-}
-
-hipError_t launch_post_ctl(const LevelCtl *src, CtlPost *dst, u64 tag, hipStream_t st) {
-  static_assert(CTL_WORDS <= 64, "one wave posts the control block");
-  hipLaunchKernelGGL(k_post_ctl, dim3(1), dim3(64), 0, st, src, dst, tag);
   return hipGetLastError();
 }
 

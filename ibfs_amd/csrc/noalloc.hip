@@ -37,7 +37,7 @@ constexpr size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 constexpr size_t OFF_RING = 0;
 constexpr size_t SZ_RING = size_t(NA_R) * NA_VT * NA_W * sizeof(u64);
 constexpr size_t OFF_CTL = OFF_RING + up256(SZ_RING);
-constexpr size_t SZ_CTL = size_t(NA_R) * sizeof(LevelCtl);
+constexpr size_t SZ_CTL = ctl_ring_bytes(NA_R);
 constexpr size_t OFF_Q = OFF_CTL + up256(SZ_CTL);
 constexpr size_t SZ_Q1 = up256(size_t(NA_VT) * sizeof(int32_t));
 constexpr size_t OFF_CHUNKS = OFF_Q + 5 * SZ_Q1;
@@ -192,7 +192,7 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   // the previous call's contents stay in the array: clear what starts at zero
   NA_TRY(launch_fill_u64(ring, Vt * W, 0ull, st));  // slot 0
   NA_TRY(launch_fill_u64(reinterpret_cast<u64 *>(flags), (Vt + 7) / 8, 0ull, st));
-  NA_TRY(launch_fill_u64(reinterpret_cast<u64 *>(ctl), (int64_t)R * CTL_WORDS, 0ull, st));
+  NA_TRY(launch_fill_u64(reinterpret_cast<u64 *>(ctl), (int64_t)(ctl_ring_bytes(R) / 8), 0ull, st));
   NA_TRY(launch_fill_u64(count, 1, 0ull, st));
   SourceList sl{};
   for (int i = 0; i < k; ++i) sl.src[i] = src[i];
@@ -226,8 +226,9 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   a.vpt = cfg.inspect_vpt;
   a.nw = cfg.wg_size / 64;
   a.hsplit = hsp;
+  a.spread = ctl_spread(ctl, R);
+  a.decide = 1;
   NA_TRY(launch_inspect(W, a, st));
-  NA_TRY(launch_plan_decide(plan, ctl, R, hs, W, 0, st));
 
   const EmitSpace sp{g->d_cid, V, Vt, g->d_deg};
   const int vec4 = (V % 4 == 0) && ((uintptr_t)dout % 16 == 0);
@@ -244,7 +245,6 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
       NA_TRY(launch_expand_dd(W, g->d_beg, g->d_adj, g->d_tadj, ring, flags, R, Vt, ctl, plan, hs,
                               q, cs, hsp, TailLog{}, grid, st));
       NA_TRY(launch_inspect(W, a, st));
-      NA_TRY(launch_plan_decide(plan, ctl, R, hs, W, 0, st));
     }
     if (int rc = wait_null_stream()) return rc;
     PlanHead ph{};

@@ -243,7 +243,18 @@ InspectArgs plan_args(const ibfs_server_s *s, const SCtx &c) {
   a.vpt = s->cfg.inspect_vpt;
   a.nw = s->cfg.wg_size / 64;
   a.hsplit = HubSplit{s->hc.deg, s->hc.tie, s->hc.cut};
+  a.spread = ctl_spread(c.ctl, s->R);
+  a.decide = split_hubs(s->g, s->hc, s->cfg) == 0;
   return a;
+}
+
+// Inspection of the plan's level at width W and the decision of the next one
+// (the inspector's last workgroup decides unless split levels are on).
+hipError_t inspect_decide(const ibfs_server_s *s, const SCtx &c, int W) {
+  const InspectArgs a = plan_args(s, c);
+  const hipError_t e = launch_inspect(W, a, c.st);
+  if (e != hipSuccess || a.decide) return e;
+  return launch_plan_decide(c.d_plan, c.ctl, s->R, c.hs, W, split_hubs(s->g, s->hc, s->cfg), c.st);
 }
 
 int alloc_ctx(ibfs_server_s *s, SCtx &c) {
@@ -256,7 +267,7 @@ int alloc_ctx(ibfs_server_s *s, SCtx &c) {
     if (err == hipSuccess) err = hipHostMalloc(p, bytes ? bytes : 1, hipHostMallocDefault);
   };
   A((void **)&c.ring, (size_t)s->R * (size_t)V * (size_t)s->W * sizeof(u64));
-  A((void **)&c.ctl, sizeof(LevelCtl) * (size_t)s->R);
+  A((void **)&c.ctl, ctl_ring_bytes(s->R));
   H((void **)&c.h_ctl, sizeof(LevelCtl));
   for (int i = 0; i < 6; ++i)
     if (i != Q_TD_L) A((void **)&c.q.q[i], sizeof(int32_t) * (size_t)V);
@@ -299,10 +310,7 @@ int alloc_ctx(ibfs_server_s *s, SCtx &c) {
                               s->g->Vt, c.ctl, c.d_plan, c.hs, c.q, s->chunk_shift,
                               HubSplit{s->hc.deg, s->hc.tie, s->hc.cut}, TailLog{}, s->grid,
                               c.st);
-        e2 = launch_inspect(Wc, plan_args(s, c), c.st);
-        if (e2 == hipSuccess)
-          e2 = launch_plan_decide(c.d_plan, c.ctl, s->R, c.hs, Wc,
-                                  split_hubs(s->g, s->hc, s->cfg), c.st);
+        e2 = inspect_decide(s, c, Wc);
       }
       hipGraph_t &gr = pass == 0 ? c.graph[i] : c.graph_burst[i];
       hipError_t e3 = hipStreamEndCapture(c.st, &gr);
@@ -403,6 +411,7 @@ int inspect_level(ibfs_server_s *s, SCtx &c, int L, const u64 *filter, const u64
   a.vpt = s->cfg.inspect_vpt;
   a.nw = s->cfg.wg_size / 64;
   a.hsplit = HubSplit{s->hc.deg, s->hc.tie, s->hc.cut};
+  a.spread = ctl_spread(c.ctl, s->R);
   a.full_diff = full_diff;
   HIP_CHK(launch_inspect(W, a, c.st));
   HIP_CHK(hipMemcpyAsync(c.h_ctl, c.ctl + L % s->R, sizeof(LevelCtl), hipMemcpyDeviceToHost, c.st));
@@ -424,7 +433,7 @@ int start_ctx(ibfs_server_s *s, SCtx &c) {
   // S_0, the changed flags and the control blocks zeroed in one launch
   HIP_CHK(launch_zero3_u64(slot(s, c, 0), s->g->Vt * W, reinterpret_cast<u64 *>(c.flags),
                            (s->g->Vt + 7) / 8, reinterpret_cast<u64 *>(c.ctl),
-                           (int64_t)s->R * CTL_WORDS, c.st));
+                           (int64_t)(ctl_ring_bytes(s->R) / 8), c.st));
   std::vector<u64> A(W, 0), keep(W, ~0ull), nand(W, ~0ull);
   int n = 0;
   int rc = admit(s, c, 0, A.data(), &n);
@@ -652,9 +661,7 @@ int cohort_burst(ibfs_server_s *s, SCtx &c, bool locked) {
                                s->g->Vt, c.ctl, c.d_plan, c.hs, c.q, s->chunk_shift, hsp,
                                TailLog{}, s->grid, c.st));
       HIP_CHK(launch_admit_dd(c.W, c.d_al, c.d_plan, c.ring, s->R, s->g->Vt, c.ctl, c.flags, c.st));
-      HIP_CHK(launch_inspect(c.W, plan_args(s, c), c.st));
-      HIP_CHK(launch_plan_decide(c.d_plan, c.ctl, s->R, c.hs, c.W,
-                                 split_hubs(s->g, s->hc, s->cfg), c.st));
+      HIP_CHK(inspect_decide(s, c, c.W));
     } else {
       HIP_CHK(hipGraphLaunch(x, c.st));
     }
@@ -713,7 +720,7 @@ int start_cohort(ibfs_server_s *s, SCtx &c) {
   // S_0, the changed flags and the control blocks zeroed in one launch
   HIP_CHK(launch_zero3_u64(slot(s, c, 0), s->g->Vt * W, reinterpret_cast<u64 *>(c.flags),
                            (s->g->Vt + 7) / 8, reinterpret_cast<u64 *>(c.ctl),
-                           (int64_t)s->R * CTL_WORDS, c.st));
+                           (int64_t)(ctl_ring_bytes(s->R) / 8), c.st));
   // the cohort's first sources take lanes 0, 1, ...; with phase offsets a
   // lane whose source's two-hop size says it runs ahead of the others starts
   // at a later level (admitted then through the admission list)
@@ -766,8 +773,7 @@ int start_cohort(ibfs_server_s *s, SCtx &c) {
   plan_init(c.h_plan, s->cfg, s->hc.rho_q10, (u64)s->g->V);
   c.h_plan->hold = c.a_max;
   HIP_CHK(hipMemcpyAsync(c.d_plan, c.h_plan, sizeof(Plan), hipMemcpyHostToDevice, c.st));
-  HIP_CHK(launch_inspect(W, plan_args(s, c), c.st));
-  HIP_CHK(launch_plan_decide(c.d_plan, c.ctl, s->R, c.hs, W, split_hubs(s->g, s->hc, s->cfg), c.st));
+  HIP_CHK(inspect_decide(s, c, W));
   c.coh = 1;
   c.dlevel = 1;
   c.last_admit = 0;

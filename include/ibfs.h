@@ -306,7 +306,7 @@ int ibfs_engine_level_log(ibfs_engine_t e, ibfs_level_info *out, int32_t cap,
  * array and its previous contents (what must start at zero is cleared by
  * each call); the library serialises calls within a process, and two
  * processes have separate copies of the array. */
-#define IBFS_NOALLOC_SCRATCH_BYTES 43324928
+#define IBFS_NOALLOC_SCRATCH_BYTES 43327232
 int ibfs_traversal_noalloc(ibfs_graph_t g, const ibfs_config *cfg,
                            const int32_t *src, int32_t k, int32_t *depth_out,
                            int64_t *traversed_edges);
