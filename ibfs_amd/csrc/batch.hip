@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "common.h"
+#include "graph_dev.h"
 #include "host_copy.h"
 #include "kernels.h"
 
@@ -134,7 +135,7 @@ void release_ctx(Ctx &c) {
   c.graph = c.graph_burst = nullptr;
   dfree(c.ring);
   dfree(c.ctl);
-  for (int i = 0; i < 6; ++i) dfree(c.q.q[i]);
+  for (int i = 0; i < NQ; ++i) dfree(c.q.q[i]);
   dfree(c.q.chunks);
   dfree(c.hs);
   dfree(c.flags);
@@ -190,6 +191,7 @@ InspectArgs dd_inspect_args(const ibfs_batch_s *b, const Ctx &c) {
   a.sml = b->cfg.sml_shed;
   a.lrg = b->cfg.lrg_shed;
   a.chunk_shift = b->chunk_shift;
+  a.chunk_extra = (unsigned)(b->g->E >> b->chunk_shift) + 1;
   a.hubs = b->g->d_hubs;
   a.H = b->g->H;
   a.hs = c.hs;
@@ -201,7 +203,7 @@ InspectArgs dd_inspect_args(const ibfs_batch_s *b, const Ctx &c) {
   a.flags = c.flags;
   a.vpt = b->cfg.inspect_vpt;
   a.nw = b->cfg.wg_size / 64;
-  a.hsplit = HubSplit{b->hc.deg, b->hc.tie, b->hc.cut};
+  a.hsplit = hub_split(b->hc);
   a.spread = ctl_spread(c.ctl, b->R);
   a.decide = split_hubs(b->g, b->hc, b->cfg) == 0;
   return a;
@@ -229,9 +231,9 @@ int alloc_ctx(ibfs_batch_s *b, Ctx &c) {
   };
   A((void **)&c.ring, (size_t)b->R * slot_bytes);
   A((void **)&c.ctl, ctl_ring_bytes(b->R));
-  for (int i = 0; i < 6; ++i)
-    if (i != Q_TD_L) A((void **)&c.q.q[i], sizeof(int32_t) * (size_t)Vq);
-  A((void **)&c.q.chunks, sizeof(int2) * ((size_t)Vq + (size_t)(b->g->E >> b->chunk_shift) + 2));
+  for (int i = 0; i < NQ; ++i)
+    if (i != Q_TD_L) A((void **)&c.q.q[i], sizeof(int32_t) * queue_entries((size_t)Vq));
+  A((void **)&c.q.chunks, sizeof(int2) * chunk_entries((size_t)Vq, (size_t)b->g->E, b->chunk_shift));
   A((void **)&c.hs, sizeof(u64) * (size_t)b->W * (size_t)std::max<int64_t>(b->g->H, 1));
   A((void **)&c.flags, sizeof(u64) * (size_t)((Vq + 7) / 8));
   {  // set-up block: masks, sources, lane table, plan (256-byte aligned parts)
@@ -276,9 +278,8 @@ int alloc_ctx(ibfs_batch_s *b, Ctx &c) {
     HIP_TRY(hipStreamBeginCapture(c.st, hipStreamCaptureModeThreadLocal));
     hipError_t e1 = hipSuccess, e2 = hipSuccess;
     for (int r = 0; r < reps && e1 == hipSuccess && e2 == hipSuccess; ++r) {
-      e1 = launch_expand_dd(b->W, b->g->d_beg, b->g->d_adj, b->g->d_tadj, c.ring, c.flags, b->R,
-                            Vt, c.ctl, c.d_plan, c.hs, c.q, b->chunk_shift,
-                            HubSplit{b->hc.deg, b->hc.tie, b->hc.cut}, c.tl, b->grid, c.st);
+      e1 = launch_expand_dd(b->W, graph_dev(b->g, b->cfg, b->hc), c.ring, c.flags, b->R, c.ctl,
+                            c.d_plan, c.hs, c.q, c.tl, b->grid, c.st);
       e2 = inspect_decide(b, c);
     }
     hipGraph_t &gr = pass == 0 ? c.graph : c.graph_burst;
@@ -397,10 +398,8 @@ int launch_burst(ibfs_batch_s *b, Ctx &c, ibfs_stats *stats) {
       c.h_al->level = c.level;
       c.h_al->n = n;
       HIP_TRY(hipMemcpyAsync(c.d_al, c.h_al, sizeof(AdmitList), hipMemcpyHostToDevice, c.st));
-      const HubSplit hsp{b->hc.deg, b->hc.tie, b->hc.cut};
-      HIP_TRY(launch_expand_dd(b->W, b->g->d_beg, b->g->d_adj, b->g->d_tadj, c.ring, c.flags,
-                               b->R, b->g->Vt, c.ctl, c.d_plan, c.hs, c.q, b->chunk_shift, hsp,
-                               c.tl, b->grid, c.st));
+      HIP_TRY(launch_expand_dd(b->W, graph_dev(b->g, b->cfg, b->hc), c.ring, c.flags, b->R, c.ctl,
+                               c.d_plan, c.hs, c.q, c.tl, b->grid, c.st));
       HIP_TRY(launch_admit_dd(b->W, c.d_al, c.d_plan, c.ring, b->R, b->g->Vt, c.ctl, c.flags,
                               c.st));
       HIP_TRY(inspect_decide(b, c));

@@ -121,6 +121,7 @@ struct ibfs_graph_s {
   int64_t *d_beg = nullptr;   // Vt+1, traversal ids
   int32_t *d_adj = nullptr;   // adjacency in input order (top-down, GroupBy)
   int32_t *d_tadj = nullptr;  // traversal adjacency: by descending degree, hubs encoded
+  int32_t *d_head = nullptr;  // 2 x Vt x 4: the first 8 entries of each traversal-adjacency list
   int32_t *d_deg = nullptr;   // Vt
   int32_t *d_hubs = nullptr;  // the H highest-degree vertices
   int32_t *d_cid = nullptr;   // V: original id -> traversal id or -1

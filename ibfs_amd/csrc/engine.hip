@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "common.h"
+#include "graph_dev.h"
 #include "host_copy.h"
 #include "kernels.h"
 
@@ -187,7 +188,7 @@ void engine_release(ibfs_engine_s *e) {
   dfree(e->d_ctl);
   hfree(e->h_ctl);
   hfree(e->post);
-  for (int i = 0; i < 6; ++i) dfree(e->q.q[i]);
+  for (int i = 0; i < NQ; ++i) dfree(e->q.q[i]);
   dfree(e->q.chunks);
   dfree(e->d_masks);
   hfree(e->h_masks);
@@ -237,8 +238,10 @@ int decide(const ibfs_engine_s *e, int L, const LevelCtl &c, int dir_prev, u64 n
 // from cur for the next bottom-up level); it posts its control block with the
 // next tag (wait_post).
 InspectArgs inspect_args(ibfs_engine_s *e, const u64 *prev, const u64 *cur, u64 *next,
-                         const u64 *lam_prev, LevelCtl *ctl, LevelCtl *ctl_zero, int full_diff) {
+                         const u64 *lam_prev, LevelCtl *ctl, LevelCtl *ctl_zero, int full_diff,
+                         int queue_bu) {
   InspectArgs a{};
+  a.queue_bu = queue_bu;
   a.full_diff = full_diff;
   a.prev = prev;
   a.cur = cur;
@@ -252,13 +255,14 @@ InspectArgs inspect_args(ibfs_engine_s *e, const u64 *prev, const u64 *cur, u64 
   a.sml = e->cfg.sml_shed;
   a.lrg = e->cfg.lrg_shed;
   a.chunk_shift = e->chunk_shift;
+  a.chunk_extra = (unsigned)(e->g->E >> e->chunk_shift) + 1;
   a.hubs = e->g->d_hubs;
   a.H = e->g->H;
   a.hs = e->hs;
   a.flags = e->flags;
   a.vpt = e->cfg.inspect_vpt;
   a.nw = e->cfg.wg_size / 64;
-  a.hsplit = HubSplit{e->hc.deg, e->hc.tie, e->hc.cut};
+  a.hsplit = hub_split(e->hc);
   a.spread = ctl_spread(e->d_ctl, e->R);
   a.post = e->post;
   a.post_tag = ++e->post_seq;
@@ -293,6 +297,7 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
   e->W = 1;
   while (e->W * 64 < k && e->W < e->Wmax) e->W *= 2;
   const int W = e->W;
+  const GraphDev gd = graph_dev(g, e->cfg, e->hc);
   e->ev_used = 0;
   e->emit_ev.clear();
   e->log.clear();
@@ -327,7 +332,7 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
   hipEvent_t ti0 = nullptr, ti1 = nullptr;
   if (timing) { ti0 = next_event(e); HIP_TRY(hipEventRecord(ti0, e->st)); }
   HIP_TRY(launch_inspect(W, inspect_args(e, nullptr, slot(e, 0), slot(e, 1), e->d_masks,
-                                         &e->d_ctl[0], &e->d_ctl[1 % e->R], 1),
+                                         &e->d_ctl[0], &e->d_ctl[1 % e->R], 1, 0),
                          e->st));
   if (timing) { ti1 = next_event(e); HIP_TRY(hipEventRecord(ti1, e->st)); }
   {
@@ -345,7 +350,7 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
     li.m_unvisited = (int64_t)c.m_cand;
     for (int i = 0; i < 3; ++i) {
       li.q_td[i] = c.q[i];
-      li.q_bu[i] = c.q[3 + i];
+      li.q_bu[i] = c.cls[i];
     }
     li.expand_ms = exp_ms;
     li.inspect_ms = insp_ms;
@@ -407,18 +412,17 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
     const int dir = decide(e, L, c, dir_prev, nf_prev);
     const bool tdf = dir == 0 && flag_top_down(c.m_front, (u64)g->V);
     // lam of level L-1 is the first member of its control block
-    const u64 *lamp = reinterpret_cast<const u64 *>(e->d_ctl + (L - 1) % e->R);
+    const LevelCtl *cp = e->d_ctl + (L - 1) % e->R;
+    const u64 *lamp = cp->lam;
     hipEvent_t x0 = nullptr, x1 = nullptr, y1 = nullptr;
     if (timing) { x0 = next_event(e); HIP_TRY(hipEventRecord(x0, e->st)); }
     if (dir == 0) {
-      HIP_TRY(launch_expand_td(W, g->d_beg, g->d_adj, slot(e, L - 1), slot(e, L), lamp, e->q,
-                               c.q[Q_TD_S], c.q[Q_TD_M], c.q[Q_TD_L], e->chunk_shift,
-                               tdf ? e->flags : nullptr, e->st));
+      HIP_TRY(launch_expand_td(W, gd, slot(e, L - 1), slot(e, L), cp, e->q, c.q[Q_TD_S],
+                               c.q[Q_TD_M], c.q[Q_TD_L], tdf ? e->flags : nullptr, e->st));
       if (stats) stats->n_td_launches++;
     } else if (dir == 2) {
-      HIP_TRY(launch_expand_hy(W, g->d_beg, g->d_adj, g->d_tadj, slot(e, L - 1), e->hs,
-                               slot(e, L), &e->d_ctl[(L - 1) % e->R], e->q, e->chunk_shift,
-                               HubSplit{e->hc.deg, e->hc.tie, e->hc.cut}, e->hy_grid, e->st));
+      HIP_TRY(launch_expand_hy(W, gd, slot(e, L - 1), e->hs, slot(e, L),
+                               cp, e->q, e->hy_grid, e->st));
       if (stats) stats->n_hy_launches++;
     } else {
       if (e->cfg.work_model) {  // instrumentation: exact early-termination prefixes
@@ -429,9 +433,8 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
                                hipMemcpyDeviceToHost, e->st));
         if (timing) HIP_TRY(hipEventRecord(x0, e->st));
       }
-      HIP_TRY(launch_expand_bu(W, g->d_beg, g->d_tadj, slot(e, L - 1), e->hs, slot(e, L),
-                               e->flags, lamp, e->q, c.q[Q_BU_S], c.q[Q_BU_M], c.q[Q_BU_L],
-                               e->st));
+      HIP_TRY(launch_expand_bu(W, gd, slot(e, L - 1), e->hs, slot(e, L), e->flags, cp, e->q,
+                               c.bu_queued ? (int64_t)c.q[Q_BU] : Vt, (int)c.bu_queued, e->st));
       if (stats) stats->n_bu_launches++;
     }
     if (timing) { x1 = next_event(e); HIP_TRY(hipEventRecord(x1, e->st)); }
@@ -447,7 +450,8 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
     }
     HIP_TRY(launch_inspect(W, inspect_args(e, slot(e, L - 1), slot(e, L), slot(e, L + 1), lamp,
                                            &e->d_ctl[L % e->R], &e->d_ctl[(L + 1) % e->R],
-                                           (dir == 1 || tdf) ? 0 : 1),
+                                           (dir == 1 || tdf) ? 0 : 1,
+                                           candidates_queued(L, c.n_cand, (u64)Vt)),
                            e->st));
     if (timing) { y1 = next_event(e); HIP_TRY(hipEventRecord(y1, e->st)); }
     {
@@ -769,7 +773,9 @@ int ibfs_graph_create_ex(const int64_t *beg, int64_t V, const int32_t *adj, int6
   const size_t vtb = sizeof(int32_t) * (size_t)std::max<int64_t>(Vt, 1);
   hipError_t err = hipMalloc((void **)&g->d_beg, sizeof(int64_t) * (size_t)(Vt + 1));
   if (err == hipSuccess) err = hipMalloc((void **)&g->d_adj, eb);
-  if (err == hipSuccess) err = hipMalloc((void **)&g->d_tadj, eb);
+  // bottom-up reads four entries at a time, so up to three past the last list
+  if (err == hipSuccess) err = hipMalloc((void **)&g->d_tadj, eb + 4 * sizeof(int32_t));
+  if (err == hipSuccess) err = hipMalloc((void **)&g->d_head, sizeof(int4) * 2 * (size_t)std::max<int64_t>(Vt, 1));
   if (err == hipSuccess) err = hipMalloc((void **)&g->d_deg, vtb);
   if (err == hipSuccess) err = hipMalloc((void **)&g->d_hubs, sizeof(int32_t) * (size_t)std::max<int64_t>(H, 1));
   if (err == hipSuccess) err = hipMalloc((void **)&g->d_cid, sizeof(int32_t) * (size_t)V);
@@ -777,6 +783,7 @@ int ibfs_graph_create_ex(const int64_t *beg, int64_t V, const int32_t *adj, int6
   if (err == hipSuccess) err = hipMemcpy(g->d_beg, tbeg.data(), sizeof(int64_t) * (size_t)(Vt + 1), hipMemcpyHostToDevice);
   if (err == hipSuccess && E > 0) err = hipMemcpy(g->d_adj, xadj.data(), sizeof(int32_t) * (size_t)E, hipMemcpyHostToDevice);
   if (err == hipSuccess && E > 0) err = hipMemcpy(g->d_tadj, tadj.data(), sizeof(int32_t) * (size_t)E, hipMemcpyHostToDevice);
+  if (err == hipSuccess) err = launch_build_head(g->d_beg, g->d_tadj, Vt, reinterpret_cast<int4 *>(g->d_head), nullptr);
   if (err == hipSuccess && Vt > 0) err = hipMemcpy(g->d_deg, tdeg.data(), sizeof(int32_t) * (size_t)Vt, hipMemcpyHostToDevice);
   if (err == hipSuccess && H > 0) err = hipMemcpy(g->d_hubs, order.data(), sizeof(int32_t) * (size_t)H, hipMemcpyHostToDevice);
   if (err == hipSuccess) err = hipMemcpy(g->d_cid, cid.data(), sizeof(int32_t) * (size_t)V, hipMemcpyHostToDevice);
@@ -791,6 +798,7 @@ int ibfs_graph_create_ex(const int64_t *beg, int64_t V, const int32_t *adj, int6
     dfree(g->d_beg);
     dfree(g->d_adj);
     dfree(g->d_tadj);
+    dfree(g->d_head);
     dfree(g->d_deg);
     dfree(g->d_hubs);
     dfree(g->d_cid);
@@ -845,6 +853,7 @@ int ibfs_graph_destroy(ibfs_graph_t g) {
   dfree(g->d_beg);
   dfree(g->d_adj);
   dfree(g->d_tadj);
+  dfree(g->d_head);
   dfree(g->d_deg);
   dfree(g->d_hubs);
   dfree(g->d_cid);
@@ -936,10 +945,9 @@ int ibfs_engine_create(ibfs_graph_t g, const ibfs_config *cfg_in, ibfs_engine_t 
   H((void **)&e->h_ctl, sizeof(LevelCtl));
   if (err == hipSuccess) err = hipHostMalloc((void **)&e->post, sizeof(CtlPost), hipHostMallocCoherent);
   if (err == hipSuccess) std::memset(e->post, 0, sizeof(CtlPost));
-  for (int i = 0; i < 6; ++i)
-    if (i != Q_TD_L) A((void **)&e->q.q[i], sizeof(int32_t) * (size_t)Vt);
-  const size_t nchunks = (size_t)Vt + (size_t)(g->E >> e->chunk_shift) + 2;
-  A((void **)&e->q.chunks, sizeof(int2) * nchunks);
+  for (int i = 0; i < NQ; ++i)
+    if (i != Q_TD_L) A((void **)&e->q.q[i], sizeof(int32_t) * queue_entries((size_t)Vt));
+  A((void **)&e->q.chunks, sizeof(int2) * chunk_entries((size_t)Vt, (size_t)g->E, e->chunk_shift));
   A((void **)&e->d_masks, sizeof(u64) * masks_words(e));
   H((void **)&e->h_masks, sizeof(u64) * masks_words(e));
   A((void **)&e->d_src, sizeof(int32_t) * (size_t)e->K);

@@ -14,6 +14,8 @@ typedef unsigned long long u64;
 
 constexpr int MAX_W = 8;               // status words per vertex: up to 512 lanes
 constexpr int MAX_LANES = 64 * MAX_W;
+constexpr int QSEG = 8;              // segments of each queue
+constexpr int MAX_TILE = 8192;       // vertices of the inspector's largest tile
 
 // Per-level control block, written by the inspector of level L with device
 // atomics and read by the expanders of level L+1, the direction decision and
@@ -26,27 +28,45 @@ struct alignas(64) LevelCtl {
   u64 n_cand;          // bottom-up candidates for L+1
   u64 m_cand;          // sum of their degrees
   u64 m_front_nh;      // sum of the degrees of frontier vertices that are not hubs
-  unsigned int q[6];   // queue lengths: td sml, td mid, td lrg chunks, bu sml, bu mid, bu lrg
-  unsigned int pad[14];
+  unsigned int q[4];   // queue lengths: td sml, td mid, td lrg chunks, bu candidates (if queued)
+  unsigned int cls[3]; // bottom-up candidates per degree class: sml, mid, lrg
+  unsigned int bu_queued;  // 1: q[Q_BU] candidates are in the queue; 0: no queue, scan every vertex
+  // Queue entry i of class c is at segment s (pre[c][s] <= i, the last such s),
+  // position s * cap + i - pre[c][s], cap = chunkcap for td lrg, else segcap.
+  unsigned int segcap, chunkcap;
+  unsigned int pad[10];
+  unsigned int pre[4][QSEG];
 };
-static_assert(sizeof(LevelCtl) == 192, "LevelCtl layout");
+static_assert(sizeof(LevelCtl) == 320, "LevelCtl layout");
 constexpr int64_t CTL_WORDS = sizeof(LevelCtl) / 8;
-// the inspector reserves queue ranges two classes at a time (q[2j], q[2j+1]
-// as one little-endian 64-bit counter)
-static_assert(offsetof(LevelCtl, q) % 8 == 0, "LevelCtl queue pairs");
+// Entries a queue array needs for V vertices, and the chunk array for E
+// adjacency entries in chunks of 2^shift: tile k of the inspector fills
+// segment k % QSEG, so a segment holds at most its share of the tiles (and the
+// chunks of those vertices).
+constexpr size_t queue_entries(size_t V) { return V + (size_t)QSEG * MAX_TILE; }
+constexpr size_t chunk_entries(size_t V, size_t E, int shift) {
+  return queue_entries(V) + (size_t)QSEG * ((E >> shift) + 1);
+}
 
 // The inspector's workgroups add their counters into CTL_COPIES copies, one
-// cache line each (workgroup b into copy b % CTL_COPIES); the last workgroup
-// to finish (ticket) folds them into the level's control block and leaves
-// copies and ticket zero for the next pass.  Device atomics on one line
-// serialise at about 3.6 ns: 512 workgroups adding 8 counters each to one
-// block of counters would spend 15 us of a pass there.
+// cache line each (workgroup b into copy b % CTL_COPIES), and take a ticket of
+// that copy; the last of a copy takes one of `top`, and the last of those
+// folds the copies into the level's control block and leaves everything zero
+// for the next pass.  The tiles reserve queue ranges in the counters of their
+// segment, two queues at a time (little-endian 64-bit pairs).  Device atomics
+// on one line serialise, at about 3.6 ns each and 11 ns where the old value is
+// returned: 512 workgroups adding 8 counters each to one block would spend
+// 15 us of a pass there, and taking tickets of one counter 6 us.
 constexpr int CTL_COPIES = 16;
 struct alignas(128) CtlSpread {
-  u64 v[CTL_COPIES][16];  // n_changed .. m_front_nh (6), then the lanes that gained (MAX_W)
-  unsigned ticket;
+  u64 v[CTL_COPIES][16];  // n_changed .. m_front_nh (6), the lanes that gained (MAX_W), and at
+                          // SPREAD_CLS the candidates of class sml + (of class mid << 32)
+  u64 qseg[QSEG][16];
+  unsigned ticket[CTL_COPIES][32];
+  unsigned top;
 };
-static_assert(6 + MAX_W <= 16 && CTL_COPIES * 16 <= 256, "CtlSpread layout");
+constexpr int SPREAD_CLS = 6 + MAX_W;
+static_assert(SPREAD_CLS < 16 && CTL_COPIES * 16 <= 256, "CtlSpread layout");
 // A ring of R control blocks is allocated with its CtlSpread behind it and
 // both start a traversal at zero.
 constexpr size_t ctl_ring_bytes(int R) {
@@ -57,7 +77,7 @@ inline CtlSpread *ctl_spread(LevelCtl *ring, int R) {
                                        sizeof(CtlSpread));
 }
 
-enum { Q_TD_S = 0, Q_TD_M = 1, Q_TD_L = 2, Q_BU_S = 3, Q_BU_M = 4, Q_BU_L = 5 };
+enum { Q_TD_S = 0, Q_TD_M = 1, Q_TD_L = 2, Q_BU = 3, NQ = 4 };
 
 // Device-resident plan of a device-driven traversal: the inspector's last
 // workgroup (k_plan_decide with split levels) writes the next level's
@@ -198,8 +218,22 @@ struct EmitSpace {
   const int32_t *deg;  // traversal-space degrees (the edge count of a final window)
 };
 
+// Device graph and the settings its expansions take (pointers: ibfs_graph_s).
+struct GraphDev {
+  const int64_t *beg;
+  const int32_t *adj, *tadj;
+  const int4 *head;  // first 8 traversal-adjacency entries of each vertex: [v] and [V + v]
+  int64_t V;         // traversal vertices
+  int sml, lrg, chunk_shift;
+  HubSplit hsp;
+};
+
+// Entry of `head` past the end of a vertex's list (no id or hub code equals it).
+constexpr int32_t NO_NBR = 0x7fffffff;
+
+// (arrays of queue_entries / chunk_entries entries)
 struct Queues {
-  int32_t *q[6];  // q[Q_TD_L] unused: top-down hubs use `chunks`
+  int32_t *q[NQ];  // q[Q_TD_L] unused: top-down hubs use `chunks`
   int2 *chunks;   // (vertex, chunk index) of top-down large vertices
 };
 
@@ -231,6 +265,7 @@ struct InspectArgs {
   int64_t V;
   Queues q;
   int sml, lrg, chunk_shift;
+  unsigned chunk_extra;  // chunks of a segment beyond one a vertex (chunk_entries)
   const int32_t *hubs;  // hub cache refresh: hs[i] = cur[hubs[i]], i < H
   int64_t H;
   u64 *hs;
@@ -245,10 +280,22 @@ struct InspectArgs {
   int nw;               // waves per workgroup: 4, 8 or 16 (0: 8)
   HubSplit hsplit;      // frontier degrees outside the pulled hubs are counted separately
   CtlSpread *spread;    // the pass's counters before they are folded into ctl
+  int queue_bu;         // host-driven: write the candidate queue (candidates_queued)
   int decide;           // plan mode: the last workgroup also decides the next level
   CtlPost *post;        // host-driven (or null): the control block is posted here
   u64 post_tag;
 };
+
+// Whether the inspection of a level writes the bottom-up candidates to a
+// queue, from the candidates of the level before it (at level 0: every
+// vertex).  Candidates only become fewer within a traversal, so this bounds
+// them.  A bottom-up level over most vertices scans them all instead, which
+// streams their words, heads and flags and spares each inspection a queue
+// entry per vertex and its reservations; below an eighth of the vertices the
+// scan would read more than the queue saves.
+__host__ __device__ inline bool candidates_queued(int L, u64 n_cand_prev, u64 V) {
+  return L > 0 && n_cand_prev * 8 < V;
+}
 
 // The launchers report hipGetLastError() after their launches; a HIP call
 // that failed earlier on the same thread (its result already handled) leaves
@@ -273,27 +320,29 @@ hipError_t launch_admit_dd(int W, const AdmitList *al, const Plan *plan, u64 *ri
                            int64_t V, LevelCtl *ctl_ring, uint8_t *flags, hipStream_t st);
 hipError_t launch_inspect(int W, const InspectArgs &a, hipStream_t st);
 // flags (or null): set for every vertex whose word changes (flag_top_down)
-hipError_t launch_expand_td(int W, const int64_t *beg, const int32_t *adj, const u64 *prev,
-                            u64 *cur, const u64 *lam_prev, Queues q, int64_t ns, int64_t nm,
-                            int64_t nl, int chunk_shift, uint8_t *flags, hipStream_t st);
-// tadj: traversal adjacency (neighbours by descending degree, hub entries
-// encoded as 0x80000000 | hub slot); hs: hub cache mirroring prev.
-hipError_t launch_expand_bu(int W, const int64_t *beg, const int32_t *tadj, const u64 *prev,
-                            const u64 *hs, u64 *cur, uint8_t *flags, const u64 *lam_prev,
-                            Queues q, int64_t ns, int64_t nm, int64_t nl, hipStream_t st);
+hipError_t launch_expand_td(int W, const GraphDev &g, const u64 *prev, u64 *cur,
+                            const LevelCtl *ctl_prev, Queues q, int64_t ns, int64_t nm, int64_t nl,
+                            uint8_t *flags, hipStream_t st);
+// Traversal adjacency: neighbours by descending degree, hub entries encoded
+// as 0x80000000 | hub slot; hs: hub cache mirroring prev.  The n candidates of
+// q, or (n = vertices, queued = 0) every vertex.
+hipError_t launch_expand_bu(int W, const GraphDev &g, const u64 *prev, const u64 *hs, u64 *cur,
+                            uint8_t *flags, const LevelCtl *ctl_prev, Queues q, int64_t n,
+                            int queued, hipStream_t st);
 // Hybrid level, fixed grid (queue lengths read from ctl_prev on the
 // device): the bottom-up candidates OR the hub-cache words of their entries
 // to the pulled hubs, the rest of the top-down frontier pushes; both with
 // atomic ORs.
-hipError_t launch_expand_hy(int W, const int64_t *beg, const int32_t *adj, const int32_t *tadj,
-                            const u64 *prev, const u64 *hs, u64 *cur, const LevelCtl *ctl_prev,
-                            Queues q, int chunk_shift, HubSplit hsplit, int grid, hipStream_t st);
+hipError_t launch_expand_hy(int W, const GraphDev &g, const u64 *prev, const u64 *hs, u64 *cur,
+                            const LevelCtl *ctl_prev, Queues q, int grid, hipStream_t st);
 // Device-driven expansion of plan->level (any direction, or a sparse tail
 // level appending to tl), fixed grid.
-hipError_t launch_expand_dd(int W, const int64_t *beg, const int32_t *adj, const int32_t *tadj,
-                            u64 *ring, uint8_t *flags, int R, int64_t V, const LevelCtl *ctl_ring,
-                            Plan *plan, const u64 *hs, Queues q, int chunk_shift,
-                            HubSplit hsplit, TailLog tl, int grid, hipStream_t st);
+hipError_t launch_expand_dd(int W, const GraphDev &g, u64 *ring, uint8_t *flags, int R,
+                            const LevelCtl *ctl_ring, Plan *plan, const u64 *hs, Queues q,
+                            TailLog tl, int grid, hipStream_t st);
+// head[v], head[V + v] = the first eight entries of v's traversal adjacency.
+hipError_t launch_build_head(const int64_t *beg, const int32_t *tadj, int64_t V, int4 *head,
+                             hipStream_t st);
 // After the emission of a window that ends at a sparse tail's first level T
 // (whose slot holds the final words, so every tail bit was written as
 // T - admit): records [0, n) of level > T write lev - admit into the rows of

@@ -149,10 +149,10 @@ __device__ void plan_decide(Plan *p, const LevelCtl &c, int L) {
 // that advanced (lam of L).  After a bottom-up or a sparse top-down level only
 // the vertices the expander (or the source admission) flagged are diffed
 // (prev is read only for them); after other levels and at level 0 every
-// vertex is.  Flags
-// are cleared as they are read.  It compacts, per degree class, both the top-down
-// frontier of L+1 (changed, degree > 0) and the bottom-up candidates
-// (degree > 0 and missing a lane of lam_prev).  Replaces
+// vertex is.  Flags are cleared as they are read.  It compacts, per degree
+// class, the top-down frontier of L+1 (changed, degree > 0), counts the
+// bottom-up candidates (degree > 0 and missing a lane of lam_prev) and, once
+// they are few (candidates_queued), compacts them too.  Replaces
 // td/sw_frontier_count + insp_scan + td/sw_frontier_gather + extract_depth
 // of inspector.cu:37-500 and scan.cuh:455-904 with a single kernel.
 //
@@ -160,11 +160,16 @@ __device__ void plan_decide(Plan *p, const LevelCtl &c, int L) {
 // lane l of wave w handles vertex (w*VPT + i)*64 + l in round i.  A wave
 // issues all loads of its rounds before any store, classifies in registers,
 // and the waves' class totals meet in LDS, so each tile reserves its queue
-// ranges with three 64-bit atomics (two classes each): same-address device
-// atomics serialize, so their number per level is what this layout keeps
-// small.  Entries go to ballot prefix positions, ascending vertex order
+// ranges with at most two 64-bit atomics (two queues each): same-address
+// device atomics serialize, so their number per level is what this layout
+// keeps small.  Entries go to ballot prefix positions, ascending vertex order
 // within a tile.  Device-driven mode: the level and its slots come from the
 // plan, and the last workgroup picks the next direction.
+//
+// Bound by its streams (88 to 127 MB per pass of R-MAT s22 at 128 lanes, about
+// 30 to 40 us) and, on small graphs, by its chain of dependent accesses
+// (7 us).  Queues and tickets of one counter each: 36 us on average at s22
+// against 32, and 14.6 against 9 us per pass of a 512 x 512 grid.
 __device__ __forceinline__ unsigned lanes_below(u64 m) {
   return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
@@ -172,9 +177,9 @@ __device__ __forceinline__ unsigned lanes_below(u64 m) {
 template <int W, int VPT, int NW>
 __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
   constexpr int IBS = NW * 64;
-  __shared__ unsigned wsum[2][NW][6];   // per-wave class totals, double-buffered by tile parity
-  __shared__ unsigned wbase[2][NW][6];  // per-wave queue bases
-  __shared__ u64 red[NW][6 + W];
+  __shared__ unsigned wsum[2][NW][NQ];   // per-wave queue totals, double-buffered by tile parity
+  __shared__ unsigned wbase[2][NW][NQ];  // per-wave queue bases
+  __shared__ u64 red[NW][7 + W];
   __shared__ u64 fold[CTL_COPIES][16];
   __shared__ LevelCtl fin;
   __shared__ int last_s;
@@ -185,6 +190,10 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
   const u64 *lam_prev = a.lam_prev;
   LevelCtl *ctl = a.ctl, *ctl_zero = a.ctl_zero;
   int full = a.full_diff;
+  bool queue_bu = a.queue_bu != 0;
+  // the hub cache's indexes are level-independent: loaded ahead of the plan's chain
+  const int64_t hub0 = (int64_t)blockIdx.x * IBS + t;
+  int32_t hubv = hub0 < a.H ? a.hubs[hub0] : -1;
   if (a.plan) {
     if (a.plan->done) return;
     const int L = a.plan->level;
@@ -200,6 +209,7 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
     ctl = a.ctl_ring + L % a.R;
     ctl_zero = a.ctl_ring + (L + 1) % a.R;
     lam_prev = L > 0 ? a.ctl_ring[(L - 1) % a.R].lam : a.lanes_all;
+    queue_bu = L > 0 && candidates_queued(L, a.ctl_ring[(L - 1) % a.R].n_cand, (u64)a.V);
   }
   if (blockIdx.x == 0 && ctl_zero && t < (int)(sizeof(LevelCtl) / 8))
     reinterpret_cast<u64 *>(ctl_zero)[t] = 0;
@@ -212,12 +222,7 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
     nand[w] = a.next_and ? a.next_and[w] : ~0ull;
     lamacc[w] = 0;
   }
-  for (int64_t i = (int64_t)blockIdx.x * IBS + t; i < a.H; i += (int64_t)gridDim.x * IBS) {
-    u64 x[W];
-    load_word<W>(cur + (int64_t)a.hubs[i] * W, x);
-    store_word<W>(a.hs + i * W, x);
-  }
-  unsigned n_changed = 0, n_front = 0, n_cand = 0;  // of the wave
+  unsigned n_changed = 0, n_front = 0, n_cs = 0, n_cm = 0, n_cl = 0;  // of the wave
   u64 m_front = 0, m_cand = 0, m_front_nh = 0;      // of the lane
   const HubSplit hsp = a.hsplit;
   const int64_t V = a.V;
@@ -226,11 +231,14 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
   const u64 *__restrict__ curp = cur;
   const u64 *__restrict__ prevp = prev;
   const int32_t *__restrict__ degp = a.deg;
-  // queue lengths as three 64-bit pairs (q[2j] low half, q[2j+1] high half)
-  unsigned long long *qpair = reinterpret_cast<unsigned long long *>(ctl->q);
+  CtlSpread *sp = a.spread;
 
   constexpr int TILE = IBS * VPT;
+  static_assert(TILE <= MAX_TILE, "queue arrays");
   const int64_t ntiles = (V + TILE - 1) / TILE;
+  // segments of the queues: tile k fills segment k % QSEG
+  const unsigned segcap = (unsigned)((ntiles + QSEG - 1) / QSEG) * TILE;
+  const unsigned chunkcap = segcap + a.chunk_extra;
   int par = 0;
   for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x, par ^= 1) {
     const int64_t c0 = tile * TILE + (int64_t)wv * 64 * VPT;
@@ -251,6 +259,9 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
         load_word<W>(curp + v * W, cw[i]);
       }
     }
+    // the workgroup's first share of the hub cache, stored below
+    u64 hubx[W];
+    if (hubv >= 0) load_word<W>(curp + (int64_t)hubv * W, hubx);
     if (prevp) {
 #pragma unroll
       for (int i = 0; i < VPT; ++i)
@@ -258,7 +269,7 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
           load_word<W>(prevp + (c0 + i * 64 + lane) * W, pw[i]);
     }
     uint8_t code[VPT];  // bits 0-1 top-down class, bits 2-3 bottom-up class
-    unsigned tot[6] = {0, 0, 0, 0, 0, 0};  // wave totals (uniform)
+    unsigned tot[NQ] = {0, 0, 0, 0};  // wave totals (uniform)
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int64_t v = c0 + i * 64 + lane;
@@ -304,28 +315,37 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
         n_front += (unsigned)__popcll(m3);
         tot[Q_TD_L] += (unsigned)wave_sum((u64)nck);
       }
-      tot[Q_BU_S] += (unsigned)__popcll(__ballot(bc == 1));
-      tot[Q_BU_M] += (unsigned)__popcll(__ballot(bc == 2));
-      tot[Q_BU_L] += (unsigned)__popcll(__ballot(bc == 3));
+      const unsigned cs1 = (unsigned)__popcll(__ballot(bc == 1));
+      const unsigned cm1 = (unsigned)__popcll(__ballot(bc == 2));
+      const unsigned cl1 = (unsigned)__popcll(__ballot(bc == 3));
+      n_cs += cs1;
+      n_cm += cm1;
+      n_cl += cl1;
+      if (queue_bu) tot[Q_BU] += cs1 + cm1 + cl1;
+    }
+    if (hubv >= 0) {
+      store_word<W>(a.hs + hub0 * W, hubx);
+      hubv = -1;
     }
     n_front += tot[Q_TD_S] + tot[Q_TD_M];
-    n_cand += tot[Q_BU_S] + tot[Q_BU_M] + tot[Q_BU_L];
     if (lane == 0) {
 #pragma unroll
-      for (int k = 0; k < 6; ++k) wsum[par][wv][k] = tot[k];
+      for (int k = 0; k < NQ; ++k) wsum[par][wv][k] = tot[k];
     }
     __syncthreads();
-    // reservation for the tile: thread j < 3 adds classes 2j, 2j+1 in one
+    // reservation for the tile: thread j < 2 adds queues 2j, 2j+1 in one
     // 64-bit atomic and lays out the waves' bases in wave order
-    if (t < 3) {
+    if (t < NQ / 2) {
       unsigned lo = 0, hi = 0;
       for (int w = 0; w < NW; ++w) {
         lo += wsum[par][w][2 * t];
         hi += wsum[par][w][2 * t + 1];
       }
       const unsigned long long add = (unsigned long long)lo | ((unsigned long long)hi << 32);
-      const unsigned long long got = add ? atomicAdd(&qpair[t], add) : 0ull;
-      unsigned blo = (unsigned)got, bhi = (unsigned)(got >> 32);
+      const unsigned seg = (unsigned)(tile % QSEG);
+      const unsigned long long got = add ? atomicAdd(&sp->qseg[seg][t], add) : 0ull;
+      unsigned blo = (unsigned)got + seg * (t == 0 ? segcap : chunkcap);
+      unsigned bhi = (unsigned)(got >> 32) + seg * segcap;
       for (int w = 0; w < NW; ++w) {
         wbase[par][w][2 * t] = blo;
         wbase[par][w][2 * t + 1] = bhi;
@@ -334,9 +354,9 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
       }
     }
     __syncthreads();
-    unsigned base[6];
+    unsigned base[NQ];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) base[k] = wbase[par][wv][k];
+    for (int k = 0; k < NQ; ++k) base[k] = wbase[par][wv][k];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int tc = code[i] & 3, bc = code[i] >> 2;
@@ -356,21 +376,25 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
         }
         base[Q_TD_L] += (unsigned)__shfl((int)inc, 63, 64);
       }
-      m = __ballot(bc == 1);
-      if (bc == 1) a.q.q[Q_BU_S][base[Q_BU_S] + lanes_below(m)] = v;
-      base[Q_BU_S] += (unsigned)__popcll(m);
-      m = __ballot(bc == 2);
-      if (bc == 2) a.q.q[Q_BU_M][base[Q_BU_M] + lanes_below(m)] = v;
-      base[Q_BU_M] += (unsigned)__popcll(m);
-      m = __ballot(bc == 3);
-      if (bc == 3) a.q.q[Q_BU_L][base[Q_BU_L] + lanes_below(m)] = v;
-      base[Q_BU_L] += (unsigned)__popcll(m);
+      if (queue_bu) {
+        m = __ballot(bc != 0);
+        if (bc) a.q.q[Q_BU][base[Q_BU] + lanes_below(m)] = v;
+        base[Q_BU] += (unsigned)__popcll(m);
+      }
     }
+  }
+  // the rest of the hub cache (more hubs than threads; none on the first pass)
+  for (int64_t i = hub0 + (hubv < 0 ? (int64_t)gridDim.x * IBS : 0); i < a.H;
+       i += (int64_t)gridDim.x * IBS) {
+    u64 x[W];
+    load_word<W>(curp + (int64_t)a.hubs[i] * W, x);
+    store_word<W>(a.hs + i * W, x);
   }
 
   // The level's counters: waves, then the workgroup, then one atomic each
   // into the workgroup's copy.
-  u64 vals[6 + W] = {n_changed, n_front, 0, n_cand, 0, 0};
+  const unsigned n_cand = n_cs + n_cm + n_cl;
+  u64 vals[7 + W] = {n_changed, n_front, 0, n_cand, 0, 0};
   if (n_front) {
     vals[2] = wave_sum(m_front);
     vals[5] = wave_sum(m_front_nh);
@@ -378,17 +402,19 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
   if (n_cand) vals[4] = wave_sum(m_cand);
 #pragma unroll
   for (int w = 0; w < W; ++w) vals[6 + w] = n_changed ? wave_or(lamacc[w]) : 0;
+  vals[6 + W] = (u64)n_cs | ((u64)n_cm << 32);
   if (lane == 0) {
 #pragma unroll
-    for (int i = 0; i < 6 + W; ++i) red[wv][i] = vals[i];
+    for (int i = 0; i < 7 + W; ++i) red[wv][i] = vals[i];
   }
   __syncthreads();
-  CtlSpread *sp = a.spread;
-  if (t < 6 + W) {
+  const int copy = blockIdx.x % CTL_COPIES;
+  if (t < 7 + W) {
+    const bool add = t < 6 || t == 6 + W;
     u64 s = 0;
-    for (int w = 0; w < NW; ++w) s = t < 6 ? s + red[w][t] : s | red[w][t];
-    u64 *d = &sp->v[blockIdx.x % CTL_COPIES][t];
-    if (s && t < 6) atomicAdd(d, s);
+    for (int w = 0; w < NW; ++w) s = add ? s + red[w][t] : s | red[w][t];
+    u64 *d = &sp->v[copy][t == 6 + W ? SPREAD_CLS : t];
+    if (s && add) atomicAdd(d, s);
     else if (s) atomicOr(d, s);
   }
   // Measured against one set of counters and a launch of its own that posted
@@ -401,7 +427,12 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
   // on this multi-XCD part.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (t == 0) last_s = atomicAdd(&sp->ticket, 1u) == gridDim.x - 1;
+  if (t == 0) {
+    const unsigned n = gridDim.x, copies = n < CTL_COPIES ? n : CTL_COPIES;
+    const unsigned of_copy = n / CTL_COPIES + ((unsigned)copy < n % CTL_COPIES ? 1 : 0);
+    last_s = atomicAdd(&sp->ticket[copy][0], 1u) == of_copy - 1 &&
+             atomicAdd(&sp->top, 1u) == copies - 1;
+  }
   __syncthreads();
   if (!last_s) return;
   if (t < CTL_COPIES * 16) {
@@ -409,16 +440,43 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
     fold[t >> 4][t & 15] = atomic_read(d);
     __hip_atomic_store(d, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (t == 0) __hip_atomic_store(&sp->ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (t < (int)CTL_WORDS) reinterpret_cast<u64 *>(&fin)[t] = 0;
+  __shared__ u64 segn[QSEG][NQ / 2];
+  if (t < QSEG * NQ / 2) {
+    u64 *d = &sp->qseg[t / (NQ / 2)][t % (NQ / 2)];
+    segn[t / (NQ / 2)][t % (NQ / 2)] = atomic_read(d);
+    __hip_atomic_store(d, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else if (t >= 64 && t < 64 + CTL_COPIES) {
+    __hip_atomic_store(&sp->ticket[t - 64][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else if (t == 128) {
+    __hip_atomic_store(&sp->top, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   __syncthreads();
   if (t < 6 + W) {
     u64 s = 0;
     for (int c = 0; c < CTL_COPIES; ++c) s = t < 6 ? s + fold[c][t] : s | fold[c][t];
     if (t < 6) (&ctl->n_changed)[t] = (&fin.n_changed)[t] = s;
     else ctl->lam[t - 6] = fin.lam[t - 6] = s;
-  } else if (t >= 32 && t < 35) {
-    reinterpret_cast<u64 *>(fin.q)[t - 32] = atomic_read(reinterpret_cast<const u64 *>(ctl->q) + t - 32);
+  } else if (t >= 32 && t < 32 + NQ) {
+    const int c = t - 32;
+    unsigned n = 0;
+    for (int k = 0; k < QSEG; ++k) {
+      ctl->pre[c][k] = fin.pre[c][k] = n;
+      n += (unsigned)(segn[k][c / 2] >> (32 * (c & 1)));
+    }
+    ctl->q[c] = fin.q[c] = n;
+  } else if (t == 48) {
+    ctl->segcap = fin.segcap = segcap;
+    ctl->chunkcap = fin.chunkcap = chunkcap;
+    u64 s = 0, nc = 0;
+    for (int c = 0; c < CTL_COPIES; ++c) {
+      s += fold[c][SPREAD_CLS];
+      nc += fold[c][3];
+    }
+    ctl->cls[0] = fin.cls[0] = (unsigned)s;
+    ctl->cls[1] = fin.cls[1] = (unsigned)(s >> 32);
+    ctl->cls[2] = fin.cls[2] = (unsigned)(nc - (s >> 32) - (s & 0xffffffffull));
+    ctl->bu_queued = fin.bu_queued = queue_bu;
   }
   __syncthreads();
   if (a.post) {  // one wave: the block's words arrive at the host before the tag
@@ -584,6 +642,24 @@ __device__ __forceinline__ void td_push_small(const int64_t *__restrict__ beg,
   }
 }
 
+// Positions of a level's queue entries (LevelCtl::pre).
+struct QIndex {
+  unsigned pre[QSEG];
+  unsigned cap;
+  __device__ __forceinline__ QIndex(const LevelCtl *c, int cls)
+      : cap(cls == Q_TD_L ? c->chunkcap : c->segcap) {
+#pragma unroll
+    for (int s = 0; s < QSEG; ++s) pre[s] = c->pre[cls][s];
+  }
+  __device__ __forceinline__ int64_t operator()(int64_t i) const {
+    unsigned at = (unsigned)i;
+#pragma unroll
+    for (int s = 1; s < QSEG; ++s)
+      if ((unsigned)i >= pre[s]) at = (unsigned)i - pre[s] + (unsigned)s * cap;
+    return at;
+  }
+};
+
 // chunk i of a large top-down vertex: edges [lo, hi)
 __device__ __forceinline__ void td_chunk_range(const int64_t *__restrict__ beg, int2 e, int cs,
                                                int64_t &lo, int64_t &hi) {
@@ -591,11 +667,6 @@ __device__ __forceinline__ void td_chunk_range(const int64_t *__restrict__ beg, 
   const int64_t end = beg[e.x + 1];
   hi = (lo + (1ll << cs)) < end ? (lo + (1ll << cs)) : end;
 }
-
-// neighbours gathered per step by one thread's bottom-up candidate
-#ifndef IBFS_BU_STEP
-#define IBFS_BU_STEP 4
-#endif
 
 // Result of a bottom-up candidate: x (= x0 | new bits) into cur.  A plain
 // store and a flag for the inspector's flagged diff; a hybrid level ORs the
@@ -618,206 +689,327 @@ __device__ __forceinline__ void bu_commit(u64 *cur, uint8_t *flags, int64_t v, c
 // lam_{L-1}, the only lanes that can still be new) in traversal-adjacency
 // order (descending degree, hubs first) and stops as soon as its word
 // covers lam_{L-1} (bitwise early termination, expander.cu:258-359).
-// One candidate per thread, IBFS_BU_STEP neighbours per step.
 // MODE 0: bottom-up level.  MODE 1 (hybrid level): only the prefix of hub
 // entries with slot < cut is read (from the hub cache).  MODE 2 (split
 // level): the whole list, for the dense lanes in lam.  In modes 1 and 2 new
 // bits go in with atomic ORs (frontier vertices push into the same words
 // concurrently) and nothing is flagged.
+//
+// A workgroup takes 256 vertices, one per thread.  Each reads its first eight
+// entries from the head array, which is in vertex order: where vertices are
+// consecutive, words and heads stream, and a vertex that is covered by then
+// (most are, in a dense level) touches neither its offsets nor its list.  The
+// others go on by degree: below sml one vertex per thread, four entries per
+// step; up to lrg one vertex per wave; above, one per workgroup.
 __device__ __forceinline__ bool pulled(int32_t a, int cut) {
   return a < 0 && (a & 0x7fffffff) < cut;
 }
 
-template <int W, int MODE = 0>
-__device__ __forceinline__ void bu_thread(const int64_t *__restrict__ beg,
-                                          const int32_t *__restrict__ tadj, const Gather &gs,
-                                          u64 *cur, uint8_t *flags,
-                                          const u64 (&lam)[W], int64_t v, int cut = 0) {
+// ORs four entries into x; false once the list or the pulled prefix has
+// ended or x covers lam.  own: the vertex's word, read in place of an entry
+// that is not taken (its bits are in x already, or on their way there).
+template <int W, int MODE>
+__device__ __forceinline__ bool bu_four(const Gather &gs, const int32_t (&a)[4], const u64 *own,
+                                        const u64 (&lam)[W], int cut, u64 (&x)[W]) {
+  u64 s[4][W];
+  bool end = false;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const bool ok = MODE == 1 ? pulled(a[r], cut) : a[r] != NO_NBR;
+    const u64 *p = a[r] < 0 ? gs.hs + (int64_t)(a[r] & 0x7fffffff) * W : gs.prev + (int64_t)a[r] * W;
+    load_word<W>(ok ? p : own, s[r]);
+    end |= !ok;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int w = 0; w < W; ++w) x[w] |= s[r][w] & lam[w];
+  return !end && !covers<W>(x, lam);
+}
+
+constexpr int BU_BIG = 16;  // vertices of the workgroup class staged at a time
+
+template <int W>
+struct BuShared {
+  int64_t j[BU_BIG], e[BU_BIG];  // entries left of each
+  u64 x[BU_BIG][W];              // its word
+  u64 part[2][BS / 64][W];       // waves' partial ORs, by step parity
+  int stop[2][BS / 64];          // a wave met the end of the pulled prefix
+  int n;
+};
+
+__device__ __forceinline__ u64 lane_of(u64 x, int l) {
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)x, l);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(x >> 32), l);
+  return (u64)lo | ((u64)hi << 32);
+}
+
+// N entries per lane of [r, e), STRIDE apart from r + i, ORed into acc;
+// returns whether one of them lies past the pulled prefix (MODE 1).
+template <int W, int MODE, int N>
+__device__ __forceinline__ bool bu_gather(const int32_t *__restrict__ tadj, const Gather &gs,
+                                          int64_t r, int64_t e, int i, int stride, int cut,
+                                          u64 (&acc)[W]) {
+  int32_t a[N];
+  bool past = false;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const int64_t j = r + i + (int64_t)k * stride;
+    a[k] = j < e ? tadj[j] : NO_NBR;
+  }
+  u64 y[N][W];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) y[k][w] = 0;
+    if (MODE == 1) {
+      past |= a[k] != NO_NBR && !pulled(a[k], cut);
+      if (pulled(a[k], cut)) load_nbr<W>(gs, a[k], y[k]);
+    } else if (a[k] != NO_NBR) {
+      load_nbr<W>(gs, a[k], y[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+#pragma unroll
+    for (int w = 0; w < W; ++w) acc[w] |= y[k][w];
+  return past;
+}
+
+// The whole workgroup calls it, each thread with its vertex v (-1: none).
+// What bounds it: random 16- to 64-byte reads of neighbour words (L2 misses),
+// and for a graph that does not fill the chip the chain of the slowest wave.
+// R-MAT s22, 128 lanes, against one queue per degree class with 4, 64 or 256
+// list entries at a time: a group's dense level 290 -> 140 us, bottom-up of
+// 1,024 sources 5.0 -> 4.1 ms; batched 1M Chung-Lu 2.32 -> 1.90 ms.
+template <int W, int MODE>
+__device__ __forceinline__ void bu_tile(const GraphDev &g, const Gather &gs, u64 *cur,
+                                        uint8_t *flags, const u64 (&lam)[W], int64_t v,
+                                        BuShared<W> &sh) {
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int cut = g.hsp.cut;
+  const int32_t *__restrict__ tadj = g.tadj;
   u64 x[W], x0[W];
-  load_word<W>(cur + v * W, x);
 #pragma unroll
-  for (int w = 0; w < W; ++w) x0[w] = x[w];
-  if (covers<W>(x, lam)) return;
-  int64_t j = beg[v];
-  const int64_t e = beg[v + 1];
-  while (j < e) {
-    int32_t an[IBFS_BU_STEP];
-    an[0] = tadj[j];
+  for (int w = 0; w < W; ++w) x[w] = 0;
+  int64_t j = 0, e = 0;
+  int64_t deg = 0;
+  bool pend = false;
+  const u64 *own = cur + v * W;
+  if (v >= 0) {
+    const int4 h = g.head[v];
+    load_word<W>(own, x);
 #pragma unroll
-    for (int r = 1; r < IBFS_BU_STEP; ++r) an[r] = (j + r < e) ? tadj[j + r] : an[0];
-    u64 sn[IBFS_BU_STEP][W];
-    bool nonhub = false;
-#pragma unroll
-    for (int r = 0; r < IBFS_BU_STEP; ++r) {
-      if (MODE == 1 && !pulled(an[r], cut)) {
-        nonhub = true;
-#pragma unroll
-        for (int w = 0; w < W; ++w) sn[r][w] = 0;
-      } else {
-        load_nbr<W>(gs, an[r], sn[r]);
+    for (int w = 0; w < W; ++w) x0[w] = x[w];
+    if (!covers<W>(x, lam)) {
+      const int32_t a[4] = {h.x, h.y, h.z, h.w};
+      pend = bu_four<W, MODE>(gs, a, own, lam, cut, x);
+      if (pend) {
+        const int4 h1 = g.head[g.V + v];
+        const int32_t a1[4] = {h1.x, h1.y, h1.z, h1.w};
+        pend = bu_four<W, MODE>(gs, a1, own, lam, cut, x);
+      }
+      if (pend) {
+        j = g.beg[v];
+        e = g.beg[v + 1];
+        deg = e - j;
+        j += 8;
+        pend = j < e;
       }
     }
-#pragma unroll
-    for (int r = 0; r < IBFS_BU_STEP; ++r)
-#pragma unroll
-      for (int w = 0; w < W; ++w) x[w] |= sn[r][w] & lam[w];
-    j += IBFS_BU_STEP;
-    if (covers<W>(x, lam) || nonhub) break;  // pulled prefix ended
-  }
-  bu_commit<W, MODE != 0>(cur, flags, v, x, x0);
-}
-
-// One candidate per wave: 64 neighbours per step, wave OR-reduction.
-template <int W, int MODE = 0>
-__device__ __forceinline__ void bu_wave(const int64_t *__restrict__ beg,
-                                        const int32_t *__restrict__ tadj, const Gather &gs,
-                                        u64 *cur, uint8_t *flags,
-                                        const u64 (&lam)[W], int64_t v, int lane, int cut = 0) {
-  u64 x[W], x0[W];
-  load_word<W>(cur + v * W, x);
-#pragma unroll
-  for (int w = 0; w < W; ++w) x0[w] = x[w];
-  if (covers<W>(x, lam)) return;
-  const int64_t s = beg[v], e = beg[v + 1];
-  for (int64_t r = s; r < e; r += 64) {
-    const int64_t j = r + lane;
-    u64 y[W];
-#pragma unroll
-    for (int w = 0; w < W; ++w) y[w] = 0;
-    bool nonhub = false;
-    if (j < e) {
-      const int32_t a = tadj[j];
-      if (MODE == 1 && !pulled(a, cut)) nonhub = true;
-      else load_nbr<W>(gs, a, y);
-    }
-#pragma unroll
-    for (int w = 0; w < W; ++w) x[w] |= wave_or(y[w] & lam[w]);
-    if (covers<W>(x, lam)) break;
-    if (MODE == 1 && __ballot(nonhub)) break;  // pulled prefix ended
-  }
-  if (lane == 0) bu_commit<W, MODE != 0>(cur, flags, v, x, x0);
-}
-
-// One candidate per workgroup: 256 neighbours per step, the four wave
-// partials combined through LDS.  Must be called by the whole workgroup.
-// nh: four ints of LDS (pulled prefix ended, per wave; used by MODE 1).
-template <int W, int MODE = 0>
-__device__ __forceinline__ void bu_block(const int64_t *__restrict__ beg,
-                                         const int32_t *__restrict__ tadj, const Gather &gs,
-                                         u64 *cur, uint8_t *flags,
-                                         const u64 (&lam)[W], int64_t v, u64 (*part)[W],
-                                         int *nh, int cut = 0) {
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  u64 x[W], x0[W];
-  if (MODE != 0) {
-    // One read of the candidate's word for the whole workgroup: in a hybrid
-    // or split level pushes from other workgroups can change it between the waves'
-    // own reads, and every wave must take the same covers/stop branches
-    // around the barriers below.
-    if (t == 0) {
-      load_word<W>(cur + v * W, x);
-#pragma unroll
-      for (int w = 0; w < W; ++w) part[0][w] = x[w];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < W; ++w) x[w] = part[0][w];
-    __syncthreads();
   } else {
-    load_word<W>(cur + v * W, x);
-  }
 #pragma unroll
-  for (int w = 0; w < W; ++w) x0[w] = x[w];
-  if (covers<W>(x, lam)) return;
-  const int64_t s = beg[v], e = beg[v + 1];
-  for (int64_t r = s; r < e; r += BS) {
-    const int64_t j = r + t;
+    for (int w = 0; w < W; ++w) x0[w] = 0;
+  }
+  // thread class, unless so few lanes of the wave are left that taking them
+  // one at a time is the shorter chain
+  bool small = pend && deg < g.sml;
+  if (__popcll(__ballot(small)) > 4) {
+    while (small) {
+      struct __attribute__((packed, aligned(4))) Four { int32_t a[4]; };
+      const Four f = *reinterpret_cast<const Four *>(tadj + j);  // readable past the last list
+      int32_t a[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a[r] = j + r < e ? f.a[r] : NO_NBR;
+      j += 4;
+      small = bu_four<W, MODE>(gs, a, own, lam, cut, x) && j < e;
+      pend = small;
+    }
+  }
+  // wave class
+  const bool big = pend && deg > g.lrg;
+  u64 m = __ballot(pend && !big);
+  while (m) {
+    const int b = __builtin_ctzll(m);
+    m &= m - 1;
+    const int64_t eb = (int64_t)lane_of((u64)e, b);
     u64 y[W];
 #pragma unroll
-    for (int w = 0; w < W; ++w) y[w] = 0;
-    bool nonhub = false;
-    if (j < e) {
-      const int32_t a = tadj[j];
-      if (MODE == 1 && !pulled(a, cut)) nonhub = true;
-      else load_nbr<W>(gs, a, y);
+    for (int w = 0; w < W; ++w) y[w] = lane_of(x[w], b);
+    for (int64_t r = (int64_t)lane_of((u64)j, b); r < eb; r += 128) {
+      u64 acc[W];
+#pragma unroll
+      for (int w = 0; w < W; ++w) acc[w] = 0;
+      const bool past = bu_gather<W, MODE, 2>(tadj, gs, r, eb, lane, 64, cut, acc);
+#pragma unroll
+      for (int w = 0; w < W; ++w) y[w] |= wave_or(acc[w] & lam[w]);
+      if (covers<W>(y, lam)) break;
+      if (MODE == 1 && __ballot(past)) break;  // pulled prefix ended
     }
+    if (lane == b) {
 #pragma unroll
-    for (int w = 0; w < W; ++w) y[w] = wave_or(y[w] & lam[w]);
-    const bool wnh = MODE == 1 && __ballot(nonhub) != 0;
-    if (lane == 0) {
-#pragma unroll
-      for (int w = 0; w < W; ++w) part[wv][w] = y[w];
-      if (MODE == 1) nh[wv] = wnh;
+      for (int w = 0; w < W; ++w) x[w] = y[w];
     }
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < W; ++w) x[w] |= part[0][w] | part[1][w] | part[2][w] | part[3][w];
-    const bool stop = MODE == 1 && (nh[0] | nh[1] | nh[2] | nh[3]);
-    __syncthreads();
-    if (covers<W>(x, lam) || stop) break;
   }
-  if (t == 0) bu_commit<W, MODE != 0>(cur, flags, v, x, x0);
+  // workgroup class: BU_BIG vertices at a time through LDS, 1,024 entries
+  // per step (a vertex of 160,000 neighbours is one workgroup's chain)
+  if (__syncthreads_or(big)) {
+    if (t == 0) sh.n = 0;
+    __syncthreads();
+    const int at = big ? atomicAdd(&sh.n, 1) : -1;
+    __syncthreads();
+    const int n = sh.n;
+    for (int i0 = 0; i0 < n; i0 += BU_BIG) {
+      const bool mine = big && at >= i0 && at < i0 + BU_BIG;
+      if (mine) {
+        sh.j[at - i0] = j;
+        sh.e[at - i0] = e;
+#pragma unroll
+        for (int w = 0; w < W; ++w) sh.x[at - i0][w] = x[w];
+      }
+      __syncthreads();
+      int par = 0;
+      for (int i = 0; i < BU_BIG && i0 + i < n; ++i) {
+        const int64_t eb = sh.e[i];
+        u64 y[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) y[w] = sh.x[i][w];
+        for (int64_t r = sh.j[i]; r < eb; r += 4 * BS, par ^= 1) {
+          u64 acc[W];
+#pragma unroll
+          for (int w = 0; w < W; ++w) acc[w] = 0;
+          const bool past = bu_gather<W, MODE, 4>(tadj, gs, r, eb, t, BS, cut, acc);
+#pragma unroll
+          for (int w = 0; w < W; ++w) acc[w] = wave_or(acc[w] & lam[w]);
+          const int wpast = MODE == 1 && __ballot(past) != 0;
+          if (lane == 0) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) sh.part[par][wv][w] = acc[w];
+            sh.stop[par][wv] = wpast;
+          }
+          // one barrier per step: the other parity is written next, and a
+          // wave reaches that step's barrier only after reading this one
+          __syncthreads();
+          int stop = 0;
+#pragma unroll
+          for (int k = 0; k < BS / 64; ++k) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) y[w] |= sh.part[par][k][w];
+            stop |= sh.stop[par][k];
+          }
+          if (covers<W>(y, lam) || stop) {
+            par ^= 1;
+            break;
+          }
+        }
+        if (t == 0) {  // every wave has read x[i] before the step's barrier, or alike now
+#pragma unroll
+          for (int w = 0; w < W; ++w) sh.x[i][w] |= y[w];
+        }
+      }
+      __syncthreads();
+      if (mine) {
+#pragma unroll
+        for (int w = 0; w < W; ++w) x[w] = sh.x[at - i0][w];
+      }
+      __syncthreads();
+    }
+  }
+  if (v >= 0) bu_commit<W, MODE != 0>(cur, flags, v, x, x0);
+}
+
+// vertices per wave of bu_level
+__host__ __device__ inline int bu_per_wave(int64_t n) {
+  int pw = 64;
+  while (pw > 8 && n < (int64_t)4 * pw * 2048) pw /= 2;
+  return pw;
+}
+
+// Every candidate (the n of the queue, or every vertex), grid-strided in tiles
+// of 4 waves.  A wave takes 64 vertices, or only 32, 16 or 8 where that keeps
+// the number of workgroups near 2,048 (8 per CU): a wave works off its
+// vertices of the wave class one after another, and with few vertices that
+// chain, not the chip, is the level's time.
+template <int W, int MODE>
+__device__ __forceinline__ void bu_level(const GraphDev &g, const Gather &gs, u64 *cur,
+                                         uint8_t *flags, const u64 (&lam)[W],
+                                         const LevelCtl *ctl, const int32_t *__restrict__ queue,
+                                         int64_t n, BuShared<W> &sh) {
+  const QIndex qi(ctl, Q_BU);
+  const int pw = bu_per_wave(n), lane = threadIdx.x & 63;
+  const int64_t tile = 4 * pw;
+  for (int64_t i0 = blockIdx.x * tile; i0 < n; i0 += gridDim.x * tile) {
+    const int64_t i = i0 + (threadIdx.x >> 6) * pw + lane;
+    const bool on = lane < pw && i < n;
+    bu_tile<W, MODE>(g, gs, cur, flags, lam, on ? (queue ? queue[qi(i)] : i) : -1, sh);
+  }
+}
+
+__global__ void k_build_head(const int64_t *__restrict__ beg, const int32_t *__restrict__ tadj,
+                             int64_t V, int4 *__restrict__ head) {
+  for (int64_t i = (int64_t)blockIdx.x * BS + threadIdx.x; i < 2 * V; i += (int64_t)gridDim.x * BS) {
+    const int64_t v = i < V ? i : i - V, j = beg[v] + (i < V ? 0 : 4), e = beg[v + 1];
+    head[i] = make_int4(j < e ? tadj[j] : NO_NBR, j + 1 < e ? tadj[j + 1] : NO_NBR,
+                        j + 2 < e ? tadj[j + 2] : NO_NBR, j + 3 < e ? tadj[j + 3] : NO_NBR);
+  }
 }
 
 // Host-driven top-down: workgroups [0, nbs) take small vertices one per
 // thread, [nbs, nbs+nbm) mid vertices one per wave, the rest one chunk of
 // 2^chunk_shift edges of a large vertex per workgroup.
 template <int W>
-__global__ __launch_bounds__(BS) void k_expand_td(const int64_t *__restrict__ beg,
-                                                  const int32_t *__restrict__ adj,
-                                                  const u64 *__restrict__ prev, u64 *cur,
-                                                  const u64 *__restrict__ lam_prev, Queues q,
-                                                  int64_t ns, int64_t nm, int64_t nl, int64_t nbs,
-                                                  int64_t nbm, int cs, uint8_t *flags) {
+__global__ __launch_bounds__(BS) void k_expand_td(GraphDev g, const u64 *__restrict__ prev,
+                                                  u64 *cur, const LevelCtl *__restrict__ ctl,
+                                                  Queues q, int64_t ns, int64_t nm, int64_t nl,
+                                                  int64_t nbs, int64_t nbm, uint8_t *flags) {
+  const int64_t *__restrict__ beg = g.beg;
+  const int32_t *__restrict__ adj = g.adj;
+  const int cs = g.chunk_shift;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int64_t b = blockIdx.x;
   u64 lam[W];
 #pragma unroll
-  for (int w = 0; w < W; ++w) lam[w] = lam_prev[w];
+  for (int w = 0; w < W; ++w) lam[w] = ctl->lam[w];
   if (b < nbs) {
     const int64_t i = b * BS + t;
     if (i >= ns) return;
-    td_push_small<W>(beg, adj, prev, cur, lam, q.q[Q_TD_S][i], nullptr, flags);
+    const int32_t u = q.q[Q_TD_S][QIndex(ctl, Q_TD_S)(i)];
+    td_push_small<W>(beg, adj, prev, cur, lam, u, nullptr, flags);
   } else if (b < nbs + nbm) {
     const int64_t i = (b - nbs) * 4 + wv;
     if (i >= nm) return;
-    const int32_t u = q.q[Q_TD_M][i];
+    const int32_t u = q.q[Q_TD_M][QIndex(ctl, Q_TD_M)(i)];
     td_push<W>(beg, adj, prev, cur, lam, u, beg[u] + lane, beg[u + 1], 64, nullptr, flags);
   } else {
     const int64_t i = b - nbs - nbm;
     if (i >= nl) return;
-    const int2 e = q.chunks[i];
+    const int2 e = q.chunks[QIndex(ctl, Q_TD_L)(i)];
     int64_t lo, hi;
     td_chunk_range(beg, e, cs, lo, hi);
     td_push<W>(beg, adj, prev, cur, lam, e.x, lo + t, hi, BS, nullptr, flags);
   }
 }
 
-// Host-driven bottom-up, same workgroup ranges as k_expand_td.
+// Host-driven bottom-up: the n candidates of the queue, or every vertex.
 template <int W>
-__global__ __launch_bounds__(BS) void k_expand_bu(const int64_t *__restrict__ beg,
-                                                  const int32_t *__restrict__ tadj, Gather gs,
-                                                  u64 *__restrict__ cur, uint8_t *flags,
-                                                  const u64 *__restrict__ lam_prev, Queues q,
-                                                  int64_t ns, int64_t nm, int64_t nl, int64_t nbs,
-                                                  int64_t nbm) {
-  __shared__ u64 part[4][W];
-  __shared__ int nh[4];
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int64_t b = blockIdx.x;
+__global__ __launch_bounds__(BS) void k_expand_bu(GraphDev g, Gather gs, u64 *cur, uint8_t *flags,
+                                                  const LevelCtl *__restrict__ ctl,
+                                                  const int32_t *queue, int64_t n) {
+  __shared__ BuShared<W> sh;
   u64 lam[W];
 #pragma unroll
-  for (int w = 0; w < W; ++w) lam[w] = lam_prev[w];
-  if (b < nbs) {
-    const int64_t i = b * BS + t;
-    if (i < ns) bu_thread<W>(beg, tadj, gs, cur, flags, lam, q.q[Q_BU_S][i]);
-  } else if (b < nbs + nbm) {
-    const int64_t i = (b - nbs) * 4 + wv;
-    if (i < nm) bu_wave<W>(beg, tadj, gs, cur, flags, lam, q.q[Q_BU_M][i], lane);
-  } else {
-    const int64_t i = b - nbs - nbm;
-    if (i < nl) bu_block<W>(beg, tadj, gs, cur, flags, lam, q.q[Q_BU_L][i], part, nh);
-  }
+  for (int w = 0; w < W; ++w) lam[w] = ctl->lam[w];
+  bu_level<W, 0>(g, gs, cur, flags, lam, ctl, queue, n, sh);
 }
 
 // Hybrid level from the queues of ctl (the control block of the level
@@ -827,34 +1019,32 @@ __global__ __launch_bounds__(BS) void k_expand_bu(const int64_t *__restrict__ be
 // neighbour v through that prefix of v's traversal-adjacency list; a
 // neighbour that is no candidate already holds every lane u can bring.
 template <int W>
-__device__ __forceinline__ void expand_hybrid(const int64_t *__restrict__ beg,
-                                              const int32_t *__restrict__ adj,
-                                              const int32_t *__restrict__ tadj, const Gather &gs,
-                                              u64 *cur, const u64 (&lam)[W],
-                                              const LevelCtl *ctl, const Queues &q, int cs,
-                                              HubSplit hsp, u64 (*part)[W], int *nh) {
+__device__ __forceinline__ void expand_hybrid(const GraphDev &g, const Gather &gs, u64 *cur,
+                                              const u64 (&lam)[W], const LevelCtl *ctl,
+                                              const Queues &q, BuShared<W> &sh) {
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int64_t G = gridDim.x;
-  const int64_t bs = ctl->q[Q_BU_S], bm = ctl->q[Q_BU_M], bl = ctl->q[Q_BU_L];
-  for (int64_t i = (int64_t)blockIdx.x * BS + t; i < bs; i += G * BS)
-    bu_thread<W, 1>(beg, tadj, gs, cur, nullptr, lam, q.q[Q_BU_S][i], hsp.cut);
-  for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < bm; i += G * 4)
-    bu_wave<W, 1>(beg, tadj, gs, cur, nullptr, lam, q.q[Q_BU_M][i], lane, hsp.cut);
-  for (int64_t i = blockIdx.x; i < bl; i += G)
-    bu_block<W, 1>(beg, tadj, gs, cur, nullptr, lam, q.q[Q_BU_L][i], part, nh, hsp.cut);
+  const int64_t *__restrict__ beg = g.beg;
+  const int32_t *__restrict__ adj = g.adj;
+  const int cs = g.chunk_shift;
+  const HubSplit hsp = g.hsp;
+  const bool queued = ctl->bu_queued != 0;
+  bu_level<W, 1>(g, gs, cur, nullptr, lam, ctl, queued ? q.q[Q_BU] : nullptr,
+                 queued ? (int64_t)ctl->q[Q_BU] : g.V, sh);
+  const QIndex is(ctl, Q_TD_S), im(ctl, Q_TD_M), il(ctl, Q_TD_L);
   const int64_t ts = ctl->q[Q_TD_S], tm = ctl->q[Q_TD_M], tl = ctl->q[Q_TD_L];
   for (int64_t i = (int64_t)blockIdx.x * BS + t; i < ts; i += G * BS) {
-    const int32_t u = q.q[Q_TD_S][i];
+    const int32_t u = q.q[Q_TD_S][is(i)];
     if (!is_hub(hsp, u, (int)(beg[u + 1] - beg[u])))
       td_push_small<W>(beg, adj, gs.prev, cur, lam, u);
   }
   for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < tm; i += G * 4) {
-    const int32_t u = q.q[Q_TD_M][i];
+    const int32_t u = q.q[Q_TD_M][im(i)];
     const int64_t b0 = beg[u], b1 = beg[u + 1];
     if (!is_hub(hsp, u, (int)(b1 - b0))) td_push<W>(beg, adj, gs.prev, cur, lam, u, b0 + lane, b1, 64);
   }
   for (int64_t i = blockIdx.x; i < tl; i += G) {
-    const int2 e = q.chunks[i];
+    const int2 e = q.chunks[il(i)];
     if (is_hub(hsp, e.x, (int)(beg[e.x + 1] - beg[e.x]))) continue;
     int64_t lo, hi;
     td_chunk_range(beg, e, cs, lo, hi);
@@ -864,17 +1054,13 @@ __device__ __forceinline__ void expand_hybrid(const int64_t *__restrict__ beg,
 
 // Host-driven hybrid level (queue lengths read on the device from ctl).
 template <int W>
-__global__ __launch_bounds__(BS) void k_expand_hy(const int64_t *__restrict__ beg,
-                                                  const int32_t *__restrict__ adj,
-                                                  const int32_t *__restrict__ tadj, Gather gs,
-                                                  u64 *cur, const LevelCtl *__restrict__ ctl,
-                                                  Queues q, int cs, HubSplit hsp) {
-  __shared__ u64 part[4][W];
-  __shared__ int nh[4];
+__global__ __launch_bounds__(BS) void k_expand_hy(GraphDev g, Gather gs, u64 *cur,
+                                                  const LevelCtl *__restrict__ ctl, Queues q) {
+  __shared__ BuShared<W> sh;
   u64 lam[W];
 #pragma unroll
   for (int w = 0; w < W; ++w) lam[w] = ctl->lam[w];
-  expand_hybrid<W>(beg, adj, tadj, gs, cur, lam, ctl, q, cs, hsp, part, nh);
+  expand_hybrid<W>(g, gs, cur, lam, ctl, q, sh);
 }
 
 // Sparse tail level L >= T = plan->tail_start: the frontier items push their
@@ -975,6 +1161,7 @@ __device__ void tail_level(const int64_t *__restrict__ beg, const int32_t *__res
   if (L == T) {
     const LevelCtl *c = ctl_ring + (T - 1) % R;
     const int64_t ns = c->q[Q_TD_S], nm = c->q[Q_TD_M], nl = c->q[Q_TD_L];
+    const QIndex is(c, Q_TD_S), im(c, Q_TD_M), il(c, Q_TD_L);
     const u64 *s1 = ring + (int64_t)((T - 1) % R) * slot;
     const u64 *s2 = ring + (int64_t)((T - 2) % R) * slot;
     auto bits = [&](int32_t u, u64(&p)[W]) {
@@ -985,7 +1172,7 @@ __device__ void tail_level(const int64_t *__restrict__ beg, const int32_t *__res
       for (int w = 0; w < W; ++w) p[w] &= ~o[w];
     };
     for (int64_t i = tid; i < ns; i += nthreads) {
-      const int32_t u = q.q[Q_TD_S][i];
+      const int32_t u = q.q[Q_TD_S][is(i)];
       u64 p[W];
       bits(u, p);
       tail_thread<W>(adj, cum, plan, tl, cap, L, p, beg[u], beg[u + 1]);
@@ -994,11 +1181,11 @@ __device__ void tail_level(const int64_t *__restrict__ beg, const int32_t *__res
       int32_t u;
       int64_t lo, hi;
       if (i < nm) {
-        u = q.q[Q_TD_M][i];
+        u = q.q[Q_TD_M][im(i)];
         lo = beg[u];
         hi = beg[u + 1];
       } else {
-        const int2 e = q.chunks[i - nm];
+        const int2 e = q.chunks[il(i - nm)];
         u = e.x;
         td_chunk_range(beg, e, cs, lo, hi);
       }
@@ -1031,16 +1218,16 @@ __device__ void tail_level(const int64_t *__restrict__ beg, const int32_t *__res
 // the class queues of the direction the inspector chose, or over the
 // frontier of a sparse tail level.
 template <int W>
-__global__ __launch_bounds__(BS) void k_expand_dd(const int64_t *__restrict__ beg,
-                                                  const int32_t *__restrict__ adj,
-                                                  const int32_t *__restrict__ tadj, u64 *ring,
-                                                  uint8_t *flags, int R, int64_t V,
+__global__ __launch_bounds__(BS) void k_expand_dd(GraphDev g, u64 *ring, uint8_t *flags, int R,
                                                   const LevelCtl *__restrict__ ctl_ring,
                                                   const Plan *__restrict__ plan,
-                                                  const u64 *__restrict__ hs, Queues q, int cs,
-                                                  HubSplit hsp, TailLog tl) {
-  __shared__ u64 part[4][W];
-  __shared__ int nh[4];
+                                                  const u64 *__restrict__ hs, Queues q,
+                                                  TailLog tl) {
+  __shared__ BuShared<W> sh;
+  const int64_t *__restrict__ beg = g.beg;
+  const int32_t *__restrict__ adj = g.adj;
+  const int64_t V = g.V;
+  const int cs = g.chunk_shift;
   if (plan->done || plan->level < 1) return;
   if (plan->tail_start) {
     tail_level<W>(beg, adj, ring, R, V, ctl_ring, plan, q, cs, tl);
@@ -1056,24 +1243,28 @@ __global__ __launch_bounds__(BS) void k_expand_dd(const int64_t *__restrict__ be
   u64 lam[W];
 #pragma unroll
   for (int w = 0; w < W; ++w) lam[w] = c->lam[w];
+  const bool queued = c->bu_queued != 0;
+  const int32_t *buq = queued ? q.q[Q_BU] : nullptr;
+  const int64_t nbu = queued ? (int64_t)c->q[Q_BU] : V;
   if (dir == 0) {
+    const QIndex is(c, Q_TD_S), im(c, Q_TD_M), il(c, Q_TD_L);
     uint8_t *tf = plan->td_flag ? flags : nullptr;
     const int64_t ns = c->q[Q_TD_S], nm = c->q[Q_TD_M], nl = c->q[Q_TD_L];
     for (int64_t i = (int64_t)blockIdx.x * BS + t; i < ns; i += G * BS)
-      td_push_small<W>(beg, adj, prev, cur, lam, q.q[Q_TD_S][i], nullptr, tf);
+      td_push_small<W>(beg, adj, prev, cur, lam, q.q[Q_TD_S][is(i)], nullptr, tf);
     for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nm; i += G * 4) {
-      const int32_t u = q.q[Q_TD_M][i];
+      const int32_t u = q.q[Q_TD_M][im(i)];
       td_push<W>(beg, adj, prev, cur, lam, u, beg[u] + lane, beg[u + 1], 64, nullptr, tf);
     }
     for (int64_t i = blockIdx.x; i < nl; i += G) {
-      const int2 e = q.chunks[i];
+      const int2 e = q.chunks[il(i)];
       int64_t lo, hi;
       td_chunk_range(beg, e, cs, lo, hi);
       td_push<W>(beg, adj, prev, cur, lam, e.x, lo + t, hi, BS, nullptr, tf);
     }
   } else if (dir == 2) {
     const Gather gs{prev, hs};
-    expand_hybrid<W>(beg, adj, tadj, gs, cur, lam, c, q, cs, hsp, part, nh);
+    expand_hybrid<W>(g, gs, cur, lam, c, q, sh);
   } else if (dir == 3) {
     // split level: the dense lanes pull over whole lists, the sparse lanes
     // push the bits their frontier vertices gained at L-1
@@ -1085,35 +1276,24 @@ __global__ __launch_bounds__(BS) void k_expand_dd(const int64_t *__restrict__ be
       ld[w] = lam[w] & plan->split[w];
       ls[w] = lam[w] & ~plan->split[w];
     }
-    const int64_t bs = c->q[Q_BU_S], bm = c->q[Q_BU_M], bl = c->q[Q_BU_L];
-    for (int64_t i = (int64_t)blockIdx.x * BS + t; i < bs; i += G * BS)
-      bu_thread<W, 2>(beg, tadj, gs, cur, nullptr, ld, q.q[Q_BU_S][i]);
-    for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < bm; i += G * 4)
-      bu_wave<W, 2>(beg, tadj, gs, cur, nullptr, ld, q.q[Q_BU_M][i], lane);
-    for (int64_t i = blockIdx.x; i < bl; i += G)
-      bu_block<W, 2>(beg, tadj, gs, cur, nullptr, ld, q.q[Q_BU_L][i], part, nh);
+    bu_level<W, 2>(g, gs, cur, nullptr, ld, c, buq, nbu, sh);
+    const QIndex is(c, Q_TD_S), im(c, Q_TD_M), il(c, Q_TD_L);
     const int64_t ns = c->q[Q_TD_S], nm = c->q[Q_TD_M], nl = c->q[Q_TD_L];
     for (int64_t i = (int64_t)blockIdx.x * BS + t; i < ns; i += G * BS)
-      td_push_small<W, true>(beg, adj, prev, cur, ls, q.q[Q_TD_S][i], pp);
+      td_push_small<W, true>(beg, adj, prev, cur, ls, q.q[Q_TD_S][is(i)], pp);
     for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nm; i += G * 4) {
-      const int32_t u = q.q[Q_TD_M][i];
+      const int32_t u = q.q[Q_TD_M][im(i)];
       td_push<W, true>(beg, adj, prev, cur, ls, u, beg[u] + lane, beg[u + 1], 64, pp);
     }
     for (int64_t i = blockIdx.x; i < nl; i += G) {
-      const int2 e = q.chunks[i];
+      const int2 e = q.chunks[il(i)];
       int64_t lo, hi;
       td_chunk_range(beg, e, cs, lo, hi);
       td_push<W, true>(beg, adj, prev, cur, ls, e.x, lo + t, hi, BS, pp);
     }
   } else {
-    const int64_t ns = c->q[Q_BU_S], nm = c->q[Q_BU_M], nl = c->q[Q_BU_L];
     const Gather gs{prev, hs};
-    for (int64_t i = (int64_t)blockIdx.x * BS + t; i < ns; i += G * BS)
-      bu_thread<W>(beg, tadj, gs, cur, flags, lam, q.q[Q_BU_S][i]);
-    for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nm; i += G * 4)
-      bu_wave<W>(beg, tadj, gs, cur, flags, lam, q.q[Q_BU_M][i], lane);
-    for (int64_t i = blockIdx.x; i < nl; i += G)
-      bu_block<W>(beg, tadj, gs, cur, flags, lam, q.q[Q_BU_L][i], part, nh);
+    bu_level<W, 0>(g, gs, cur, flags, lam, c, buq, nbu, sh);
   }
 }
 
@@ -1314,41 +1494,45 @@ hipError_t launch_inspect(int W, const InspectArgs &a, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_expand_td(int W, const int64_t *beg, const int32_t *adj, const u64 *prev,
-                            u64 *cur, const u64 *lam_prev, Queues q, int64_t ns, int64_t nm,
-                            int64_t nl, int chunk_shift, uint8_t *flags, hipStream_t st) {
+hipError_t launch_expand_td(int W, const GraphDev &g, const u64 *prev, u64 *cur,
+                            const LevelCtl *ctl_prev, Queues q, int64_t ns, int64_t nm, int64_t nl,
+                            uint8_t *flags, hipStream_t st) {
   const int64_t nbs = (ns + BS - 1) / BS, nbm = (nm + 3) / 4;
   const int64_t nb = nbs + nbm + nl;
   if (nb == 0) return hipSuccess;
   if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
-  dim3 g((unsigned)nb), blk(BS);
-  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_td<WW>, g, blk, 0, st, beg, adj, prev, cur,
-                                        lam_prev, q, ns, nm, nl, nbs, nbm, chunk_shift, flags));
+  dim3 gr((unsigned)nb), blk(BS);
+  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_td<WW>, gr, blk, 0, st, g, prev, cur, ctl_prev, q,
+                                        ns, nm, nl, nbs, nbm, flags));
   return hipGetLastError();
 }
 
-hipError_t launch_expand_bu(int W, const int64_t *beg, const int32_t *tadj, const u64 *prev,
-                            const u64 *hs, u64 *cur, uint8_t *flags, const u64 *lam_prev,
-                            Queues q, int64_t ns, int64_t nm, int64_t nl, hipStream_t st) {
+hipError_t launch_expand_bu(int W, const GraphDev &g, const u64 *prev, const u64 *hs, u64 *cur,
+                            uint8_t *flags, const LevelCtl *ctl_prev, Queues q, int64_t n,
+                            int queued, hipStream_t st) {
   const Gather gs{prev, hs};
-  const int64_t nbs = (ns + BS - 1) / BS, nbm = (nm + 3) / 4;
-  const int64_t nb = nbs + nbm + nl;
-  if (nb == 0) return hipSuccess;
-  if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
-  dim3 g((unsigned)nb), blk(BS);
-  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_bu<WW>, g, blk, 0, st, beg, tadj, gs, cur,
-                                        flags, lam_prev, q, ns, nm, nl, nbs, nbm));
+  if (n <= 0) return hipSuccess;
+  dim3 gr(grid_for(n, 4 * bu_per_wave(n), 0x7fffffff)), blk(BS);
+  const int32_t *queue = queued ? q.q[Q_BU] : nullptr;
+  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_bu<WW>, gr, blk, 0, st, g, gs, cur, flags,
+                                        ctl_prev, queue, n));
   return hipGetLastError();
 }
 
-hipError_t launch_expand_dd(int W, const int64_t *beg, const int32_t *adj, const int32_t *tadj,
-                            u64 *ring, uint8_t *flags, int R, int64_t V, const LevelCtl *ctl_ring,
-                            Plan *plan, const u64 *hs, Queues q, int chunk_shift,
-                            HubSplit hsplit, TailLog tl, int grid, hipStream_t st) {
-  dim3 g(grid > 0 ? grid : 1), blk(BS);
-  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_dd<WW>, g, blk, 0, st, beg, adj, tadj, ring,
-                                        flags, R, V, ctl_ring, plan, hs, q, chunk_shift, hsplit,
-                                        tl));
+hipError_t launch_expand_dd(int W, const GraphDev &g, u64 *ring, uint8_t *flags, int R,
+                            const LevelCtl *ctl_ring, Plan *plan, const u64 *hs, Queues q,
+                            TailLog tl, int grid, hipStream_t st) {
+  dim3 gr(grid > 0 ? grid : 1), blk(BS);
+  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_dd<WW>, gr, blk, 0, st, g, ring, flags, R,
+                                        ctl_ring, plan, hs, q, tl));
+  return hipGetLastError();
+}
+
+hipError_t launch_build_head(const int64_t *beg, const int32_t *tadj, int64_t V, int4 *head,
+                             hipStream_t st) {
+  if (V <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_build_head, dim3(grid_for(2 * V, BS, 65536)), dim3(BS), 0, st, beg, tadj, V,
+                     head);
   return hipGetLastError();
 }
 
@@ -1362,13 +1546,11 @@ hipError_t launch_tail_patch(int W, TailLog tl, int64_t n, int T, const int32_t 
   return hipGetLastError();
 }
 
-hipError_t launch_expand_hy(int W, const int64_t *beg, const int32_t *adj, const int32_t *tadj,
-                            const u64 *prev, const u64 *hs, u64 *cur, const LevelCtl *ctl_prev,
-                            Queues q, int chunk_shift, HubSplit hsplit, int grid, hipStream_t st) {
-  dim3 g(grid > 0 ? grid : 1), blk(BS);
+hipError_t launch_expand_hy(int W, const GraphDev &g, const u64 *prev, const u64 *hs, u64 *cur,
+                            const LevelCtl *ctl_prev, Queues q, int grid, hipStream_t st) {
+  dim3 gr(grid > 0 ? grid : 1), blk(BS);
   const Gather gs{prev, hs};
-  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_hy<WW>, g, blk, 0, st, beg, adj, tadj, gs, cur,
-                                        ctl_prev, q, chunk_shift, hsplit));
+  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_hy<WW>, gr, blk, 0, st, g, gs, cur, ctl_prev, q));
   return hipGetLastError();
 }
 

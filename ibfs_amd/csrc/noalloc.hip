@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "common.h"
+#include "graph_dev.h"
 #include "kernels.h"
 
 using namespace ibfs;
@@ -39,9 +40,9 @@ constexpr size_t SZ_RING = size_t(NA_R) * NA_VT * NA_W * sizeof(u64);
 constexpr size_t OFF_CTL = OFF_RING + up256(SZ_RING);
 constexpr size_t SZ_CTL = ctl_ring_bytes(NA_R);
 constexpr size_t OFF_Q = OFF_CTL + up256(SZ_CTL);
-constexpr size_t SZ_Q1 = up256(size_t(NA_VT) * sizeof(int32_t));
-constexpr size_t OFF_CHUNKS = OFF_Q + 5 * SZ_Q1;
-constexpr size_t SZ_CHUNKS = (size_t(NA_VT) + (size_t(NA_E) >> NA_MIN_CHUNK_SHIFT) + 2) * sizeof(int2);
+constexpr size_t SZ_Q1 = up256(queue_entries(NA_VT) * sizeof(int32_t));
+constexpr size_t OFF_CHUNKS = OFF_Q + (NQ - 1) * SZ_Q1;
+constexpr size_t SZ_CHUNKS = chunk_entries(NA_VT, NA_E, NA_MIN_CHUNK_SHIFT) * sizeof(int2);
 constexpr size_t OFF_HS = OFF_CHUNKS + up256(SZ_CHUNKS);
 constexpr size_t SZ_HS = size_t(NA_H) * NA_W * sizeof(u64);
 constexpr size_t OFF_FLAGS = OFF_HS + up256(SZ_HS);
@@ -167,11 +168,10 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   const int W = k <= 64 ? 1 : 2;
   const int R = NA_R;
   const int64_t V = g->V, Vt = g->Vt;
-  const int cs = __builtin_ctz((unsigned)cfg.td_chunk);
   u64 *ring = reinterpret_cast<u64 *>(base + OFF_RING);
   LevelCtl *ctl = reinterpret_cast<LevelCtl *>(base + OFF_CTL);
   Queues q{};
-  for (int i = 0, j = 0; i < 6; ++i)
+  for (int i = 0, j = 0; i < NQ; ++i)
     if (i != Q_TD_L) q.q[i] = reinterpret_cast<int32_t *>(base + OFF_Q + (size_t)(j++) * SZ_Q1);
   q.chunks = reinterpret_cast<int2 *>(base + OFF_CHUNKS);
   u64 *hs = reinterpret_cast<u64 *>(base + OFF_HS);
@@ -181,7 +181,7 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   Plan *plan = reinterpret_cast<Plan *>(base + OFF_PLAN);
   u64 *count = reinterpret_cast<u64 *>(base + OFF_COUNT);
   const HubCut hc = hub_cut(g, cfg.hybrid_hubs);
-  const HubSplit hsp{hc.deg, hc.tie, hc.cut};
+  const GraphDev gd = graph_dev(g, cfg, hc);
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       cus <= 0)
@@ -213,7 +213,8 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   a.q = q;
   a.sml = cfg.sml_shed;
   a.lrg = cfg.lrg_shed;
-  a.chunk_shift = cs;
+  a.chunk_shift = gd.chunk_shift;
+  a.chunk_extra = (unsigned)(g->E >> gd.chunk_shift) + 1;
   a.hubs = g->d_hubs;
   a.H = g->H;
   a.hs = hs;
@@ -225,7 +226,7 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   a.flags = flags;
   a.vpt = cfg.inspect_vpt;
   a.nw = cfg.wg_size / 64;
-  a.hsplit = hsp;
+  a.hsplit = gd.hsp;
   a.spread = ctl_spread(ctl, R);
   a.decide = 1;
   NA_TRY(launch_inspect(W, a, st));
@@ -242,8 +243,7 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
       B = std::min(8, R - 1 - (level - lo));
     }
     for (int i = 0; i < B; ++i) {
-      NA_TRY(launch_expand_dd(W, g->d_beg, g->d_adj, g->d_tadj, ring, flags, R, Vt, ctl, plan, hs,
-                              q, cs, hsp, TailLog{}, grid, st));
+      NA_TRY(launch_expand_dd(W, gd, ring, flags, R, ctl, plan, hs, q, TailLog{}, grid, st));
       NA_TRY(launch_inspect(W, a, st));
     }
     if (int rc = wait_null_stream()) return rc;

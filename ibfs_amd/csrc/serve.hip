@@ -38,6 +38,7 @@
 #include <vector>
 
 #include "common.h"
+#include "graph_dev.h"
 #include "kernels.h"
 
 using namespace ibfs;
@@ -205,7 +206,7 @@ void release_ctx(SCtx &c) {
   dfree(c.ring);
   dfree(c.ctl);
   hfree(c.h_ctl);
-  for (int i = 0; i < 6; ++i) dfree(c.q.q[i]);
+  for (int i = 0; i < NQ; ++i) dfree(c.q.q[i]);
   dfree(c.q.chunks);
   dfree(c.hs);
   dfree(c.flags);
@@ -231,6 +232,7 @@ InspectArgs plan_args(const ibfs_server_s *s, const SCtx &c) {
   a.sml = s->cfg.sml_shed;
   a.lrg = s->cfg.lrg_shed;
   a.chunk_shift = s->chunk_shift;
+  a.chunk_extra = (unsigned)(s->g->E >> s->chunk_shift) + 1;
   a.hubs = s->g->d_hubs;
   a.H = s->g->H;
   a.hs = c.hs;
@@ -242,7 +244,7 @@ InspectArgs plan_args(const ibfs_server_s *s, const SCtx &c) {
   a.flags = c.flags;
   a.vpt = s->cfg.inspect_vpt;
   a.nw = s->cfg.wg_size / 64;
-  a.hsplit = HubSplit{s->hc.deg, s->hc.tie, s->hc.cut};
+  a.hsplit = hub_split(s->hc);
   a.spread = ctl_spread(c.ctl, s->R);
   a.decide = split_hubs(s->g, s->hc, s->cfg) == 0;
   return a;
@@ -269,9 +271,9 @@ int alloc_ctx(ibfs_server_s *s, SCtx &c) {
   A((void **)&c.ring, (size_t)s->R * (size_t)V * (size_t)s->W * sizeof(u64));
   A((void **)&c.ctl, ctl_ring_bytes(s->R));
   H((void **)&c.h_ctl, sizeof(LevelCtl));
-  for (int i = 0; i < 6; ++i)
-    if (i != Q_TD_L) A((void **)&c.q.q[i], sizeof(int32_t) * (size_t)V);
-  A((void **)&c.q.chunks, sizeof(int2) * ((size_t)V + (size_t)(s->g->E >> s->chunk_shift) + 2));
+  for (int i = 0; i < NQ; ++i)
+    if (i != Q_TD_L) A((void **)&c.q.q[i], sizeof(int32_t) * queue_entries((size_t)V));
+  A((void **)&c.q.chunks, sizeof(int2) * chunk_entries((size_t)V, (size_t)s->g->E, s->chunk_shift));
   A((void **)&c.hs, sizeof(u64) * (size_t)s->W * (size_t)std::max<int64_t>(s->g->H, 1));
   A((void **)&c.flags, sizeof(u64) * (size_t)((V + 7) / 8));
   A((void **)&c.d_mask, sizeof(u64) * mask_words(s));
@@ -306,10 +308,8 @@ int alloc_ctx(ibfs_server_s *s, SCtx &c) {
       HIP_CHK(hipStreamBeginCapture(c.st, hipStreamCaptureModeThreadLocal));
       hipError_t e1 = hipSuccess, e2 = hipSuccess;
       for (int r = 0; r < reps && e1 == hipSuccess && e2 == hipSuccess; ++r) {
-        e1 = launch_expand_dd(Wc, s->g->d_beg, s->g->d_adj, s->g->d_tadj, c.ring, c.flags, s->R,
-                              s->g->Vt, c.ctl, c.d_plan, c.hs, c.q, s->chunk_shift,
-                              HubSplit{s->hc.deg, s->hc.tie, s->hc.cut}, TailLog{}, s->grid,
-                              c.st);
+        e1 = launch_expand_dd(Wc, graph_dev(s->g, s->cfg, s->hc), c.ring, c.flags, s->R, c.ctl,
+                              c.d_plan, c.hs, c.q, TailLog{}, s->grid, c.st);
         e2 = inspect_decide(s, c, Wc);
       }
       hipGraph_t &gr = pass == 0 ? c.graph[i] : c.graph_burst[i];
@@ -379,7 +379,7 @@ int admit(ibfs_server_s *s, SCtx &c, int L, u64 *A, int *n_adm) {
 
 // Inspection of level L (masks in staging slot I) + control-block copy + event.
 int inspect_level(ibfs_server_s *s, SCtx &c, int L, const u64 *filter, const u64 *keep,
-                  const u64 *nand, int full_diff) {
+                  const u64 *nand, int full_diff, int queue_bu) {
   const int W = c.W;
   u64 *h = c.h_mask + 2 * emit_words(s);
   u64 *d = c.d_mask + 2 * emit_words(s);
@@ -404,15 +404,17 @@ int inspect_level(ibfs_server_s *s, SCtx &c, int L, const u64 *filter, const u64
   a.sml = s->cfg.sml_shed;
   a.lrg = s->cfg.lrg_shed;
   a.chunk_shift = s->chunk_shift;
+  a.chunk_extra = (unsigned)(s->g->E >> s->chunk_shift) + 1;
   a.hubs = s->g->d_hubs;
   a.H = s->g->H;
   a.hs = c.hs;
   a.flags = c.flags;
   a.vpt = s->cfg.inspect_vpt;
   a.nw = s->cfg.wg_size / 64;
-  a.hsplit = HubSplit{s->hc.deg, s->hc.tie, s->hc.cut};
+  a.hsplit = hub_split(s->hc);
   a.spread = ctl_spread(c.ctl, s->R);
   a.full_diff = full_diff;
+  a.queue_bu = queue_bu;
   HIP_CHK(launch_inspect(W, a, c.st));
   HIP_CHK(hipMemcpyAsync(c.h_ctl, c.ctl + L % s->R, sizeof(LevelCtl), hipMemcpyDeviceToHost, c.st));
   HIP_CHK(hipEventRecord(c.ev, c.st));
@@ -439,7 +441,7 @@ int start_ctx(ibfs_server_s *s, SCtx &c) {
   int rc = admit(s, c, 0, A.data(), &n);
   if (rc) return rc;
   c.running = true;
-  return inspect_level(s, c, 0, A.data(), keep.data(), nand.data(), 1);
+  return inspect_level(s, c, 0, A.data(), keep.data(), nand.data(), 1, 0);
 }
 
 int decide(const ibfs_server_s *s, int Ln, const LevelCtl &lc, int dir_prev, u64 nf_prev) {
@@ -525,18 +527,18 @@ int process_level(ibfs_server_s *s, SCtx &c) {
   // 2. expansion of L+1
   const int Ln = L + 1;
   const int dir = decide(s, Ln, lc, c.dir_prev, c.nf_prev);
-  const u64 *lamp = reinterpret_cast<const u64 *>(c.ctl + L % s->R);
+  const LevelCtl *cp = c.ctl + L % s->R;
+  const GraphDev gd = graph_dev(s->g, s->cfg, s->hc);
   if (dir == 0)
-    HIP_CHK(launch_expand_td(W, s->g->d_beg, s->g->d_adj, slot(s, c, L), slot(s, c, Ln), lamp,
-                             c.q, lc.q[Q_TD_S], lc.q[Q_TD_M], lc.q[Q_TD_L], s->chunk_shift,
-                             nullptr, c.st));
+    HIP_CHK(launch_expand_td(W, gd, slot(s, c, L), slot(s, c, Ln), cp, c.q, lc.q[Q_TD_S],
+                             lc.q[Q_TD_M], lc.q[Q_TD_L], nullptr, c.st));
   else if (dir == 2)
-    HIP_CHK(launch_expand_hy(W, s->g->d_beg, s->g->d_adj, s->g->d_tadj, slot(s, c, L), c.hs,
-                             slot(s, c, Ln), c.ctl + L % s->R, c.q, s->chunk_shift,
-                             HubSplit{s->hc.deg, s->hc.tie, s->hc.cut}, s->grid, c.st));
+    HIP_CHK(launch_expand_hy(W, gd, slot(s, c, L), c.hs, slot(s, c, Ln), cp, c.q,
+                             s->grid, c.st));
   else
-    HIP_CHK(launch_expand_bu(W, s->g->d_beg, s->g->d_tadj, slot(s, c, L), c.hs, slot(s, c, Ln),
-                             c.flags, lamp, c.q, lc.q[Q_BU_S], lc.q[Q_BU_M], lc.q[Q_BU_L], c.st));
+    HIP_CHK(launch_expand_bu(W, gd, slot(s, c, L), c.hs, slot(s, c, Ln), c.flags, cp, c.q,
+                             lc.bu_queued ? (int64_t)lc.q[Q_BU] : s->g->Vt, (int)lc.bu_queued,
+                             c.st));
   c.dir_prev = dir;
   c.nf_prev = lc.n_front;
   // 3. snapshots older than every unemitted lane's admission are no longer
@@ -578,7 +580,8 @@ int process_level(ibfs_server_s *s, SCtx &c) {
     nand[w] = ~finmask[w];
   }
   // 5. inspection of Ln (clears the lanes freed at L in slot Ln+1)
-  return inspect_level(s, c, Ln, filter.data(), keep.data(), nand.data(), dir != 1 ? 1 : 0);
+  return inspect_level(s, c, Ln, filter.data(), keep.data(), nand.data(), dir != 1 ? 1 : 0,
+                       candidates_queued(Ln, lc.n_cand, (u64)s->g->Vt));
 }
 
 // Waiting sources take the clean lanes of a running cohort at level L
@@ -656,10 +659,8 @@ int cohort_burst(ibfs_server_s *s, SCtx &c, bool locked) {
       if (fresh > 0)
         HIP_CHK(hipMemcpyAsync(c.d_lanes, c.h_lanes, sizeof(LaneOut) * (size_t)c.K,
                                hipMemcpyHostToDevice, c.st));
-      const HubSplit hsp{s->hc.deg, s->hc.tie, s->hc.cut};
-      HIP_CHK(launch_expand_dd(c.W, s->g->d_beg, s->g->d_adj, s->g->d_tadj, c.ring, c.flags, s->R,
-                               s->g->Vt, c.ctl, c.d_plan, c.hs, c.q, s->chunk_shift, hsp,
-                               TailLog{}, s->grid, c.st));
+      HIP_CHK(launch_expand_dd(c.W, graph_dev(s->g, s->cfg, s->hc), c.ring, c.flags, s->R, c.ctl,
+                               c.d_plan, c.hs, c.q, TailLog{}, s->grid, c.st));
       HIP_CHK(launch_admit_dd(c.W, c.d_al, c.d_plan, c.ring, s->R, s->g->Vt, c.ctl, c.flags, c.st));
       HIP_CHK(inspect_decide(s, c, c.W));
     } else {

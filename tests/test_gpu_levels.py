@@ -1,0 +1,84 @@
+"""Level kernels at the edges of their tiles and steps: list lengths around
+the head array, the gather steps and the degree classes, vertex counts around
+the inspector's tiles and the bottom-up tiles, every lane width, against the
+oracle.  Needs an MI355X."""
+import sys
+
+import numpy as np
+import pytest
+
+import ibfs_amd
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, file=sys.stderr, flush=True)
+
+
+def _symmetric(V, a, b):
+    keep = a != b
+    key = np.unique(np.concatenate([a[keep] * V + b[keep], b[keep] * V + a[keep]]))
+    beg = np.concatenate([[0], np.cumsum(np.bincount(key // V, minlength=V))]).astype(np.int64)
+    return beg, (key % V).astype(np.int32)
+
+
+def _degrees_graph(V, seed):
+    """A path over the first half of the vertices, and one vertex per listed
+    degree d joined to d vertices of the path, three apart from its start."""
+    half = V // 2
+    a, b = [np.arange(half - 1)], [np.arange(1, half)]
+    degrees = [1, 2, 3, 4, 5, 7, 8, 9, 11, 12, 13, 63, 64, 65, 71, 72, 73, 135, 136, 137, 511, 512,
+               513, 520, 521, 1031, 1032, 1033, 2048, 2049, 4200]
+    rng = np.random.default_rng(seed)
+    for i, d in enumerate(x for x in degrees for _ in range(3)):
+        if d < half and half + i < V:
+            a.append(np.full(d, half + i))
+            b.append(rng.choice(half, size=d, replace=False))
+    return _symmetric(V, np.concatenate(a), np.concatenate(b))
+
+
+@pytest.mark.parametrize("V", [64, 513, 9000, 70_001])
+@pytest.mark.parametrize("hubs", [None, 0, 16])
+def test_list_lengths_around_the_gather_steps(V, hubs):
+    """Lists of 1 to 4,200 neighbours (lengths around 4, 8, 12, 64 + 8, 128 + 8,
+    512 + 8 and 1,024 + 8), with and without a hub cache, under the bottom-up,
+    the hybrid and the alpha/beta policy, classes by default and with every
+    vertex above degree 9 in the workgroup class."""
+    beg, adj = _degrees_graph(V, seed=V)
+    g = ibfs_amd.DeviceGraph(ibfs_amd.HostCsr.from_arrays(beg, adj), hub_count=hubs)
+    src = np.random.default_rng(1).integers(0, V, size=130).astype(np.int32)
+    want = oracle.bfs_many(beg, adj, src, threads=8)
+    for lanes in (64, 128, 256, 512):
+        for pol in (ibfs_amd.POLICY_BU_ONLY, ibfs_amd.POLICY_HYBRID, ibfs_amd.POLICY_ALPHA_BETA):
+            for cls in ({}, dict(sml_shed=5, lrg_shed=9)):
+                say(f"[gpu] lists V={V} hubs={hubs} lanes={lanes} policy={pol} {cls}")
+                e = ibfs_amd.Engine(g, lane_bits=lanes, policy=pol, hybrid_hubs=40, **cls)
+                np.testing.assert_array_equal(e.run_groups(src), want)
+                e.close()
+
+
+@pytest.mark.parametrize("V", [1, 2, 255, 256, 257, 511, 512, 513, 4095, 4097, 8 * 2048 + 1,
+                               9 * 2048 - 1, 65_537, 300_001])
+def test_vertex_counts_around_the_tiles(V):
+    """Ring graphs with chords: every vertex count around the inspector's tiles
+    and queue segments, frontiers in every segment, candidates queued and
+    scanned, engine and batched form; depths and traversed edges."""
+    say(f"[gpu] tiles V={V}")
+    v = np.arange(V)
+    beg, adj = _symmetric(V, np.concatenate([v, v]), np.concatenate([(v + 1) % V, (v * 7 + 3) % V]))
+    g = ibfs_amd.DeviceGraph(ibfs_amd.HostCsr.from_arrays(beg, adj))
+    src = np.random.default_rng(V).integers(0, V, size=40).astype(np.int32)
+    want = oracle.bfs_many(beg, adj, src, threads=8)
+    edges = sum(oracle.traversed_edges(beg, d) for d in want)
+    for opts in (dict(), dict(policy=ibfs_amd.POLICY_BU_ONLY), dict(wg_size=256, inspect_vpt=1),
+                 dict(wg_size=1024, inspect_vpt=8, policy=ibfs_amd.POLICY_BU_ONLY)):
+        for lanes in (64, 256):
+            e = ibfs_amd.Engine(g, lane_bits=lanes, **opts)
+            np.testing.assert_array_equal(e.traversal(src), want)
+            assert e.last_stats.traversed_edges == edges
+            e.close()
+    b = ibfs_amd.Batch(g, lane_bits=128, contexts=2, burst=4)
+    np.testing.assert_array_equal(b.run(src), want)
+    b.close()
