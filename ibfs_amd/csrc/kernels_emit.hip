@@ -438,79 +438,147 @@ __global__ __launch_bounds__(BS) void k_emit_wide(const u64 *__restrict__ ring, 
 // Closeness reduction over the snapshot window [b, e]: per lane k, the sum
 // over vertices of depth_k(v) and the number of vertices reached, for the
 // vertices whose bit arrived in the window, without writing depth arrays.
-// With the per-vertex bit-sliced counters c_j (depth = sum_j 2^j c_j), the
-// sum over a wave's 64 vertices is sum_j 2^j popcount(ballot(c_j bit k)),
-// so each lane costs NS+1 ballots per 64 vertices.  Lane k of the window is
-// a first window (off_k <= 0: every set bit counts, depth = count) or a
-// continuation (off_k = b - admit > 0: bits set at e but not at b count,
-// depth = off_k + count).  Wave partials meet in LDS, one atomic per lane
-// and workgroup.
-template <int W, int NS>
-__global__ __launch_bounds__(BS) void k_close(const u64 *__restrict__ ring, int R, EmitSpace sp,
-                                              int b, int e, const LaneOut *__restrict__ lanes,
-                                              const u64 *__restrict__ level_masks,
-                                              const u64 *__restrict__ sel, int k_lanes,
-                                              unsigned long long *__restrict__ sum_out,
-                                              unsigned long long *__restrict__ reach_out) {
-  __shared__ int32_t s_off[MAX_LANES];
-  __shared__ u64 red[2][4][MAX_LANES];
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  for (int i = t; i < MAX_LANES; i += BS) s_off[i] = (i < k_lanes) ? b - lanes[i].admit : 0;
-  __syncthreads();
-  u64 selw[W], cont[W];
+// The first window of a run starts at level 0 (every set bit counts, depth =
+// levels of the window at which the lane is admitted and the bit absent).  A
+// later one continues it for the lanes admitted by its base b, which the
+// window before counted up to b: bits set at e but not at b count, depth =
+// b - admit + that count.
+//
+// The lanes are counted side by side: a thread takes one status word (64
+// lanes) of every stride-th vertex and adds, per level, the word of counted
+// bits still absent there into bit-sliced counters (plane j holds bit j of 64
+// sums): a carry-save tree takes eight levels at a time into planes 0 to 2 and
+// ripples one carry into the rest.  Threads of a wave with the same word add
+// their planes in a butterfly, lane k reads off the sum of lane k, and a
+// workgroup adds once per lane to the outputs.  Bound by reading the window's
+// snapshots (consecutive 8-byte words); one ballot per lane, counter bit and
+// 64 vertices instead took 415 us of a 256-lane group on R-MAT s18, most of
+// its time.
+constexpr int CLOSE_BS = 512;
+constexpr int CLOSE_ITEMS = 64;  // words per thread between reductions: plane counts below
+constexpr int CLOSE_SP = 20;     // sums: 64 x 255 levels (14 bits) x 64 threads
+constexpr int CLOSE_RP = 13;     // reach: 64 (7 bits) x 64 threads
+
+__device__ __forceinline__ void csa(u64 &hi, u64 &lo, u64 a, u64 b) {
+  const u64 u = lo ^ a;
+  hi = (lo & a) | (u & b);
+  lo = u ^ b;
+}
+
+// Adds the planes of the lane STEP away; P planes hold the widest sum.
+template <int P>
+__device__ __forceinline__ void planes_add_lane(u64 (&x)[P], int step) {
+  u64 carry = 0;
 #pragma unroll
-  for (int w = 0; w < W; ++w) {
-    selw[w] = sel[w];
-    cont[w] = 0;
-    for (int bit = 0; bit < 64 && w * 64 + bit < k_lanes; ++bit)
-      if (s_off[w * 64 + bit] > 0) cont[w] |= 1ull << bit;
+  for (int j = 0; j < P; ++j) {
+    const u64 y = __shfl_xor(x[j], step, 64);
+    const u64 u = x[j] ^ y, c = (x[j] & y) | (u & carry);
+    x[j] = u ^ carry;
+    carry = c;
   }
-  u64 acc_sum[W], acc_reach[W];
+}
+
+// Number of lane `lane` in the planes of thread `from`.
+template <int P>
+__device__ __forceinline__ unsigned planes_read(const u64 (&x)[P], int from, int lane) {
+  unsigned v = 0;
 #pragma unroll
-  for (int w = 0; w < W; ++w) acc_sum[w] = acc_reach[w] = 0;
-  // reduced over traversal ids: an isolated vertex contributes nothing
-  const int64_t nblk = (sp.Vt + BS - 1) / BS;
-  for (int64_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
-    const int64_t v = blk * BS + t;
-    u64 c[NS][W], fin[W], bs[W], M[W];
-    if (v < sp.Vt) emit_count<W, NS>(ring, R, sp.Vt, b, e, v, level_masks, c, fin, bs);
-    else emit_zero<W, NS>(c, fin, bs);
+  for (int j = 0; j < P; ++j) {
+    const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)x[j], from);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(x[j] >> 32), from);
+    v |= (((lane < 32 ? lo : hi) >> (lane & 31)) & 1u) << j;
+  }
+  return v;
+}
+
+template <int W>
+__global__ __launch_bounds__(CLOSE_BS) void k_close(const u64 *__restrict__ ring, int R,
+                                                    int64_t Vt, int b, int e,
+                                                    const LaneOut *__restrict__ lanes,
+                                                    const u64 *__restrict__ level_masks,
+                                                    const u64 *__restrict__ sel, int k_lanes,
+                                                    unsigned long long *__restrict__ sum_out,
+                                                    unsigned long long *__restrict__ reach_out) {
+  __shared__ u64 s_lm[256 * W];
+  __shared__ u64 s_cont[W];
+  __shared__ unsigned s_sum[W * 64], s_reach[W * 64];
+  const int t = threadIdx.x, lane = t & 63;
+  if (t < W) s_cont[t] = 0;
+  for (int i = t; i < (e - b) * W; i += CLOSE_BS) s_lm[i] = level_masks[i];
+  for (int i = t; i < W * 64; i += CLOSE_BS) s_sum[i] = s_reach[i] = 0;
+  __syncthreads();
+  for (int i = t; i < k_lanes; i += CLOSE_BS)
+    if (b > 0 && b >= lanes[i].admit) atomicOr(&s_cont[i >> 6], 1ull << (i & 63));
+  __syncthreads();
+  const int w = t % W;  // the stride is a multiple of W
+  const u64 cont = s_cont[w], selw = sel[w];
+  const int64_t slot = Vt * W, n = slot, stride = (int64_t)gridDim.x * CLOSE_BS;
+  // consecutive words of the reduced vertices (an isolated one adds nothing)
+  for (int64_t i0 = (int64_t)blockIdx.x * CLOSE_BS; i0 < n; i0 += CLOSE_ITEMS * stride) {
+    u64 S[CLOSE_SP], Q[CLOSE_RP];
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      M[w] = fin[w] & ~(bs[w] & cont[w]) & selw[w];
+    for (int j = 0; j < CLOSE_SP; ++j) S[j] = 0;
 #pragma unroll
-      for (int j = 0; j < NS; ++j) c[j][w] &= M[w];
-    }
+    for (int j = 0; j < CLOSE_RP; ++j) Q[j] = 0;
+    for (int r = 0; r < CLOSE_ITEMS; ++r) {
+      const int64_t i = i0 + r * stride + t;
+      if (i0 + r * stride >= n) break;
+      if (i >= n) continue;
+      const u64 fin = ring[(int64_t)(e % R) * slot + i];
+      u64 m = 0;
+      for (int L0 = b; L0 < e || L0 == b; L0 += 8) {
+        u64 x[8];
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      if (!wave_or(M[w])) continue;  // uniform: no counted bit in this word
-      for (int bit = 0; bit < 64; ++bit) {
-        const int k = w * 64 + bit;
-        if (k >= k_lanes) break;
-        const u64 pm = __popcll(__ballot((M[w] >> bit) & 1ull));
-        if (!pm) continue;
-        u64 s = 0;
+        for (int k = 0; k < 8; ++k)
+          x[k] = L0 + k < e ? ring[(int64_t)((L0 + k) % R) * slot + i] : ~0ull;
+        // a window of one snapshot: its base is the final word
+        if (L0 == b) m = fin & selw & ~((b < e ? x[0] : fin) & cont);
 #pragma unroll
-        for (int j = 0; j < NS; ++j) s += (u64)__popcll(__ballot((c[j][w] >> bit) & 1ull)) << j;
-        if (lane == bit) {
-          acc_reach[w] += pm;
-          acc_sum[w] += s + (u64)(s_off[k] > 0 ? s_off[k] : 0) * pm;
+        for (int k = 0; k < 8; ++k)
+          x[k] = L0 + k < e ? m & ~x[k] & s_lm[(L0 + k - b) * W + w] : 0ull;
+        u64 ta, tb, fa, fb, c;
+        csa(ta, S[0], x[0], x[1]);
+        csa(tb, S[0], x[2], x[3]);
+        csa(fa, S[1], ta, tb);
+        csa(ta, S[0], x[4], x[5]);
+        csa(tb, S[0], x[6], x[7]);
+        csa(fb, S[1], ta, tb);
+        csa(c, S[2], fa, fb);
+#pragma unroll
+        for (int j = 3; j < 14; ++j) {
+          const u64 d = S[j] & c;
+          S[j] ^= c;
+          c = d;
         }
+      }
+#pragma unroll
+      for (int j = 0; j < 7; ++j) {
+        const u64 d = Q[j] & m;
+        Q[j] ^= m;
+        m = d;
+      }
+    }
+    for (int step = W; step < 64; step *= 2) {
+      planes_add_lane(S, step);
+      planes_add_lane(Q, step);
+    }
+    // thread `ww` of the wave holds the totals of word ww
+#pragma unroll
+    for (int ww = 0; ww < W; ++ww) {
+      const unsigned s = planes_read(S, ww, lane), q = planes_read(Q, ww, lane);
+      if (q) {
+        atomicAdd(&s_sum[ww * 64 + lane], s);
+        atomicAdd(&s_reach[ww * 64 + lane], q);
       }
     }
   }
-#pragma unroll
-  for (int w = 0; w < W; ++w) {
-    red[0][wv][w * 64 + lane] = acc_sum[w];
-    red[1][wv][w * 64 + lane] = acc_reach[w];
-  }
   __syncthreads();
-  for (int i = t; i < k_lanes; i += BS) {
-    const u64 s = red[0][0][i] + red[0][1][i] + red[0][2][i] + red[0][3][i];
-    const u64 r = red[1][0][i] + red[1][1][i] + red[1][2][i] + red[1][3][i];
-    if (r) {
-      atomicAdd(&sum_out[i], s);
-      atomicAdd(&reach_out[i], r);
+  for (int i = t; i < k_lanes; i += CLOSE_BS) {
+    const u64 q = s_reach[i];
+    if (q) {
+      const int off = b - lanes[i].admit;
+      atomicAdd(&sum_out[i], (u64)s_sum[i] + (off > 0 ? (u64)off * q : 0ull));
+      atomicAdd(&reach_out[i], q);
     }
   }
 }
@@ -680,16 +748,11 @@ template <int W>
 static hipError_t close_w(const u64 *ring, int R, EmitSpace sp, int b, int e, const LaneOut *lanes,
                           const u64 *masks, const u64 *sel, int k, u64 *sum, u64 *reach,
                           hipStream_t st) {
-  const int span = e - b + 1;
-  dim3 g(grid_for(sp.Vt, BS * 8, 256)), blk(BS);
-  if (span < 16)
-    hipLaunchKernelGGL((k_close<W, 4>), g, blk, 0, st, ring, R, sp, b, e, lanes, masks, sel, k, sum, reach);
-  else if (span < 64)
-    hipLaunchKernelGGL((k_close<W, 6>), g, blk, 0, st, ring, R, sp, b, e, lanes, masks, sel, k, sum, reach);
-  else if (span < 256)
-    hipLaunchKernelGGL((k_close<W, 8>), g, blk, 0, st, ring, R, sp, b, e, lanes, masks, sel, k, sum, reach);
-  else
-    return hipErrorInvalidValue;
+  if (e - b + 1 >= 256) return hipErrorInvalidValue;
+  // a workgroup sums in 32 bits: 255 levels of a 256th of the vertices fit
+  dim3 g(grid_for(sp.Vt * W, CLOSE_BS * 4, 256)), blk(CLOSE_BS);
+  hipLaunchKernelGGL(k_close<W>, g, blk, 0, st, ring, R, sp.Vt, b, e, lanes, masks, sel, k, sum,
+                     reach);
   return hipGetLastError();
 }
 

@@ -82,3 +82,28 @@ def test_vertex_counts_around_the_tiles(V):
     b = ibfs_amd.Batch(g, lane_bits=128, contexts=2, burst=4)
     np.testing.assert_array_equal(b.run(src), want)
     b.close()
+
+
+@pytest.mark.parametrize("V", [1, 2, 3, 9, 10, 18, 65, 300, 2100])
+@pytest.mark.parametrize("ring", [4, 9, 10, 32, 255])
+def test_closeness_windows(V, ring):
+    """Closeness on paths (an extra isolated vertex beside them): windows of
+    one snapshot, of 8 and 9, of many, continued windows, lanes started
+    later, at every width; sums and reach against closed forms."""
+    say(f"[gpu] closeness path V={V} ring={ring}")
+    v = np.arange(V - 1)
+    beg, adj = _symmetric(V + 1, v, v + 1)
+    g = ibfs_amd.DeviceGraph(ibfs_amd.HostCsr.from_arrays(beg, adj))
+    src = np.arange(min(V + 1, 700), dtype=np.int32)
+    if V > 1:
+        src[-1] = V  # the isolated vertex
+    s = src.astype(np.int64)
+    want_sum = np.where(s < V, s * (s + 1) // 2 + (V - 1 - s) * (V - s) // 2, 0)
+    want_reach = np.where(s < V, V, 1)
+    for lanes in (64, 128, 256, 512):
+        for opts in ({}, dict(phase_offsets=2, tail_div=0)):
+            b = ibfs_amd.Batch(g, lane_bits=lanes, contexts=2, burst=4, ring_levels=ring, **opts)
+            dsum, reach = b.closeness(src)
+            np.testing.assert_array_equal(reach, want_reach)
+            np.testing.assert_array_equal(dsum, want_sum)
+            b.close()
