@@ -571,48 +571,23 @@ __device__ __forceinline__ bool td_bits(const u64 *__restrict__ prev, const u64 
   return !NEW || any != 0;
 }
 
+// Edges [j0, j1) of u, every stride-th: four neighbours per step, their
+// entries and words loaded before any atomic, so a step costs one chain of
+// dependent accesses for four neighbours.  An entry past the end reads u's own
+// word, which holds every bit u pushes.
 template <int W, bool NEW = false>
-__device__ __forceinline__ void td_push(const int64_t *__restrict__ beg,
-                                        const int32_t *__restrict__ adj,
+__device__ __forceinline__ void td_push(const int32_t *__restrict__ adj,
                                         const u64 *__restrict__ prev, u64 *cur,
                                         const u64 (&lam)[W], int32_t u, int64_t j0, int64_t j1,
                                         int stride, const u64 *pp = nullptr,
                                         uint8_t *flags = nullptr) {
   u64 p[W];
   if (!td_bits<W, NEW>(prev, pp, lam, u, p)) return;
-  for (int64_t j = j0; j < j1; j += stride) {
-    const int64_t v = adj[j];
-    u64 c[W];
-    load_word<W>(cur + v * W, c);
-    bool ch = false;
-#pragma unroll
-    for (int w = 0; w < W; ++w)
-      if (p[w] & ~c[w]) {
-        atomicOr(&cur[v * W + w], p[w]);
-        ch = true;
-      }
-    if (flags && ch) flags[v] = 1;
-  }
-}
-
-// One thread per small frontier vertex: four neighbours per step, their
-// adjacency entries and words loaded before any atomic, so four dependent
-// load chains are in flight instead of one.
-template <int W, bool NEW = false>
-__device__ __forceinline__ void td_push_small(const int64_t *__restrict__ beg,
-                                              const int32_t *__restrict__ adj,
-                                              const u64 *__restrict__ prev, u64 *cur,
-                                              const u64 (&lam)[W], int32_t u,
-                                              const u64 *pp = nullptr, uint8_t *flags = nullptr) {
-  u64 p[W];
-  if (!td_bits<W, NEW>(prev, pp, lam, u, p)) return;
-  int64_t j = beg[u];
-  const int64_t e = beg[u + 1];
-  for (; j + 4 <= e; j += 4) {
+  for (int64_t j = j0; j < j1; j += 4 * stride) {
     int64_t v[4];
     u64 c[4][W];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = adj[j + r];
+    for (int r = 0; r < 4; ++r) v[r] = j + r * stride < j1 ? adj[j + r * stride] : u;
 #pragma unroll
     for (int r = 0; r < 4; ++r) load_word<W>(cur + v[r] * W, c[r]);
 #pragma unroll
@@ -627,20 +602,16 @@ __device__ __forceinline__ void td_push_small(const int64_t *__restrict__ beg,
       if (flags && ch) flags[v[r]] = 1;
     }
   }
-  for (; j < e; ++j) {
-    const int64_t v = adj[j];
-    u64 c[W];
-    load_word<W>(cur + v * W, c);
-    bool ch = false;
-#pragma unroll
-    for (int w = 0; w < W; ++w)
-      if (p[w] & ~c[w]) {
-        atomicOr(&cur[v * W + w], p[w]);
-        ch = true;
-      }
-    if (flags && ch) flags[v] = 1;
-  }
 }
+
+// Lanes per vertex of the small class (degree below sml): a list of up to 64
+// neighbours is one step.  One thread per vertex walked it in up to 16 steps
+// of dependent accesses, which was the time of a sparse level; the wider
+// classes took one neighbour per lane and step.  Top-down of one s16 group
+// 37 -> 16 us (4 lanes: 19), of 1,024 s22 sources 1.05 -> 0.92 ms, of a dense
+// level on 300K Chung-Lu vertices 9% less; bound there by the random reads of
+// the targets' words.
+constexpr int TD_SMALL = 16;
 
 // Positions of a level's queue entries (LevelCtl::pre).
 struct QIndex {
@@ -981,22 +952,22 @@ __global__ __launch_bounds__(BS) void k_expand_td(GraphDev g, const u64 *__restr
 #pragma unroll
   for (int w = 0; w < W; ++w) lam[w] = ctl->lam[w];
   if (b < nbs) {
-    const int64_t i = b * BS + t;
+    const int64_t i = (b * BS + t) / TD_SMALL;
     if (i >= ns) return;
     const int32_t u = q.q[Q_TD_S][QIndex(ctl, Q_TD_S)(i)];
-    td_push_small<W>(beg, adj, prev, cur, lam, u, nullptr, flags);
+    td_push<W>(adj, prev, cur, lam, u, beg[u] + t % TD_SMALL, beg[u + 1], TD_SMALL, nullptr, flags);
   } else if (b < nbs + nbm) {
     const int64_t i = (b - nbs) * 4 + wv;
     if (i >= nm) return;
     const int32_t u = q.q[Q_TD_M][QIndex(ctl, Q_TD_M)(i)];
-    td_push<W>(beg, adj, prev, cur, lam, u, beg[u] + lane, beg[u + 1], 64, nullptr, flags);
+    td_push<W>(adj, prev, cur, lam, u, beg[u] + lane, beg[u + 1], 64, nullptr, flags);
   } else {
     const int64_t i = b - nbs - nbm;
     if (i >= nl) return;
     const int2 e = q.chunks[QIndex(ctl, Q_TD_L)(i)];
     int64_t lo, hi;
     td_chunk_range(beg, e, cs, lo, hi);
-    td_push<W>(beg, adj, prev, cur, lam, e.x, lo + t, hi, BS, nullptr, flags);
+    td_push<W>(adj, prev, cur, lam, e.x, lo + t, hi, BS, nullptr, flags);
   }
 }
 
@@ -1033,22 +1004,23 @@ __device__ __forceinline__ void expand_hybrid(const GraphDev &g, const Gather &g
                  queued ? (int64_t)ctl->q[Q_BU] : g.V, sh);
   const QIndex is(ctl, Q_TD_S), im(ctl, Q_TD_M), il(ctl, Q_TD_L);
   const int64_t ts = ctl->q[Q_TD_S], tm = ctl->q[Q_TD_M], tl = ctl->q[Q_TD_L];
-  for (int64_t i = (int64_t)blockIdx.x * BS + t; i < ts; i += G * BS) {
+  for (int64_t i = ((int64_t)blockIdx.x * BS + t) / TD_SMALL; i < ts; i += G * (BS / TD_SMALL)) {
     const int32_t u = q.q[Q_TD_S][is(i)];
-    if (!is_hub(hsp, u, (int)(beg[u + 1] - beg[u])))
-      td_push_small<W>(beg, adj, gs.prev, cur, lam, u);
+    const int64_t b0 = beg[u], b1 = beg[u + 1];
+    if (!is_hub(hsp, u, (int)(b1 - b0)))
+      td_push<W>(adj, gs.prev, cur, lam, u, b0 + t % TD_SMALL, b1, TD_SMALL);
   }
   for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < tm; i += G * 4) {
     const int32_t u = q.q[Q_TD_M][im(i)];
     const int64_t b0 = beg[u], b1 = beg[u + 1];
-    if (!is_hub(hsp, u, (int)(b1 - b0))) td_push<W>(beg, adj, gs.prev, cur, lam, u, b0 + lane, b1, 64);
+    if (!is_hub(hsp, u, (int)(b1 - b0))) td_push<W>(adj, gs.prev, cur, lam, u, b0 + lane, b1, 64);
   }
   for (int64_t i = blockIdx.x; i < tl; i += G) {
     const int2 e = q.chunks[il(i)];
     if (is_hub(hsp, e.x, (int)(beg[e.x + 1] - beg[e.x]))) continue;
     int64_t lo, hi;
     td_chunk_range(beg, e, cs, lo, hi);
-    td_push<W>(beg, adj, gs.prev, cur, lam, e.x, lo + t, hi, BS);
+    td_push<W>(adj, gs.prev, cur, lam, e.x, lo + t, hi, BS);
   }
 }
 
@@ -1250,17 +1222,19 @@ __global__ __launch_bounds__(BS) void k_expand_dd(GraphDev g, u64 *ring, uint8_t
     const QIndex is(c, Q_TD_S), im(c, Q_TD_M), il(c, Q_TD_L);
     uint8_t *tf = plan->td_flag ? flags : nullptr;
     const int64_t ns = c->q[Q_TD_S], nm = c->q[Q_TD_M], nl = c->q[Q_TD_L];
-    for (int64_t i = (int64_t)blockIdx.x * BS + t; i < ns; i += G * BS)
-      td_push_small<W>(beg, adj, prev, cur, lam, q.q[Q_TD_S][is(i)], nullptr, tf);
+    for (int64_t i = ((int64_t)blockIdx.x * BS + t) / TD_SMALL; i < ns; i += G * (BS / TD_SMALL)) {
+      const int32_t u = q.q[Q_TD_S][is(i)];
+      td_push<W>(adj, prev, cur, lam, u, beg[u] + t % TD_SMALL, beg[u + 1], TD_SMALL, nullptr, tf);
+    }
     for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nm; i += G * 4) {
       const int32_t u = q.q[Q_TD_M][im(i)];
-      td_push<W>(beg, adj, prev, cur, lam, u, beg[u] + lane, beg[u + 1], 64, nullptr, tf);
+      td_push<W>(adj, prev, cur, lam, u, beg[u] + lane, beg[u + 1], 64, nullptr, tf);
     }
     for (int64_t i = blockIdx.x; i < nl; i += G) {
       const int2 e = q.chunks[il(i)];
       int64_t lo, hi;
       td_chunk_range(beg, e, cs, lo, hi);
-      td_push<W>(beg, adj, prev, cur, lam, e.x, lo + t, hi, BS, nullptr, tf);
+      td_push<W>(adj, prev, cur, lam, e.x, lo + t, hi, BS, nullptr, tf);
     }
   } else if (dir == 2) {
     const Gather gs{prev, hs};
@@ -1279,17 +1253,19 @@ __global__ __launch_bounds__(BS) void k_expand_dd(GraphDev g, u64 *ring, uint8_t
     bu_level<W, 2>(g, gs, cur, nullptr, ld, c, buq, nbu, sh);
     const QIndex is(c, Q_TD_S), im(c, Q_TD_M), il(c, Q_TD_L);
     const int64_t ns = c->q[Q_TD_S], nm = c->q[Q_TD_M], nl = c->q[Q_TD_L];
-    for (int64_t i = (int64_t)blockIdx.x * BS + t; i < ns; i += G * BS)
-      td_push_small<W, true>(beg, adj, prev, cur, ls, q.q[Q_TD_S][is(i)], pp);
+    for (int64_t i = ((int64_t)blockIdx.x * BS + t) / TD_SMALL; i < ns; i += G * (BS / TD_SMALL)) {
+      const int32_t u = q.q[Q_TD_S][is(i)];
+      td_push<W, true>(adj, prev, cur, ls, u, beg[u] + t % TD_SMALL, beg[u + 1], TD_SMALL, pp);
+    }
     for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nm; i += G * 4) {
       const int32_t u = q.q[Q_TD_M][im(i)];
-      td_push<W, true>(beg, adj, prev, cur, ls, u, beg[u] + lane, beg[u + 1], 64, pp);
+      td_push<W, true>(adj, prev, cur, ls, u, beg[u] + lane, beg[u + 1], 64, pp);
     }
     for (int64_t i = blockIdx.x; i < nl; i += G) {
       const int2 e = q.chunks[il(i)];
       int64_t lo, hi;
       td_chunk_range(beg, e, cs, lo, hi);
-      td_push<W, true>(beg, adj, prev, cur, ls, e.x, lo + t, hi, BS, pp);
+      td_push<W, true>(adj, prev, cur, ls, e.x, lo + t, hi, BS, pp);
     }
   } else {
     const Gather gs{prev, hs};
@@ -1497,7 +1473,7 @@ hipError_t launch_inspect(int W, const InspectArgs &a, hipStream_t st) {
 hipError_t launch_expand_td(int W, const GraphDev &g, const u64 *prev, u64 *cur,
                             const LevelCtl *ctl_prev, Queues q, int64_t ns, int64_t nm, int64_t nl,
                             uint8_t *flags, hipStream_t st) {
-  const int64_t nbs = (ns + BS - 1) / BS, nbm = (nm + 3) / 4;
+  const int64_t nbs = (ns * TD_SMALL + BS - 1) / BS, nbm = (nm + 3) / 4;
   const int64_t nb = nbs + nbm + nl;
   if (nb == 0) return hipSuccess;
   if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
