@@ -60,6 +60,7 @@ struct Ctx {
   int state = IDLE;
   int64_t g0 = 0;
   int k = 0;
+  int iso = 0;  // some source of the group is isolated
   int base = 0;
   int level = 0;  // level the device will expand next (host view)
   int32_t *out_host = nullptr;    // host-placed output (rows of the caller's order)
@@ -180,7 +181,7 @@ hipError_t window_out(ibfs_batch_s *b, Ctx &c, int lo, int hi, u64 *edges = null
     return launch_close(b->W, c.ring, b->R, sp, lo, hi, c.d_lanes, c.d_masks + 2 * b->W,
                         c.d_masks + b->W, c.k, b->d_sum + c.g0, b->d_reach + c.g0, c.st);
   return launch_emit(b->W, b->cfg.emit_mode, 0, c.ring, b->R, sp, lo, hi, c.d_lanes,
-                     c.d_masks + 2 * b->W, c.d_masks + b->W, c.k, edges, c.st);
+                     c.d_masks + 2 * b->W, c.d_masks + b->W, c.k, edges, c.iso, c.st);
 }
 
 InspectArgs dd_inspect_args(const ibfs_batch_s *b, const Ctx &c) {
@@ -317,7 +318,9 @@ int start_group(ibfs_batch_s *b, Ctx &c, const int32_t *src, int64_t g0, int k, 
   c.a_max = 0;
   for (int i = 0; i < k; ++i) c.a_max = std::max(c.a_max, c.start[(size_t)i]);
   std::memset(c.h_masks, 0, sizeof(u64) * masks_words(b));
+  c.iso = 0;
   for (int i = 0; i < k; ++i) {
+    c.iso |= b->g->h_cid[src[g0 + i]] < 0;
     const int a = c.start[(size_t)i];
     if (a == 0) c.h_masks[i >> 6] |= 1ull << (i & 63);  // lanes of level 0
     c.h_masks[W + (i >> 6)] |= 1ull << (i & 63);         // every lane of the group

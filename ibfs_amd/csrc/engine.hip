@@ -30,29 +30,29 @@ struct ibfs_engine_s {
   // traversal, the narrowest power of two that holds its sources (at most
   // Wmax = lane_bits / 64, which sizes the buffers)
   int K = 128, W = 2, Wmax = 2, R = 32, chunk_shift = 12;
-  int hy_grid = 8192;  // workgroups of a hybrid expansion
+  int hy_grid = 8192, next_grid = 8192;  // workgroups of a hybrid level, of one enqueued ahead
   HubCut hc;           // hubs a hybrid level pulls through
   hipStream_t st = nullptr;
   hipEvent_t ev_wait = nullptr;  // recorded after each host copy the loop waits for
   u64 *ring = nullptr;
   LevelCtl *d_ctl = nullptr;
-  LevelCtl *h_ctl = nullptr;  // pinned
-  CtlPost *post = nullptr;    // coherent pinned: control blocks posted by the inspector
+  // coherent pinned: control blocks posted by the inspector (level l into
+  // entry l % POSTS with tag post_seq base + l), the end of a group
+  CtlPost *post = nullptr;
+  GroupPost *post_end = nullptr;
   u64 post_seq = 0;
   Queues q{};
   u64 *d_masks = nullptr;     // [0,W) lanes_all, [W,2W) sel, [2W, 2W+(R+1)W) level masks
-  u64 *h_masks = nullptr;     // pinned mirror
-  int32_t *d_src = nullptr;
-  int32_t *h_src = nullptr;   // pinned, K entries
   LaneOut *d_lanes = nullptr;
-  LaneOut *h_lanes = nullptr; // pinned, K entries
   int32_t *d_out = nullptr;   // staging for host-placed output
   size_t d_out_cap = 0;
-  u64 *d_count = nullptr;
-  u64 *h_count = nullptr;
+  u64 *d_count = nullptr;     // edges, start clock; work model at [2], [3]
+  u64 *h_count = nullptr;     // work model, pinned
+  double clock_khz = 1e5;     // of the device clock in d_count and post_end
   u64 *hs = nullptr;          // hub cache, H * W words
   uint8_t *flags = nullptr;   // changed-at-this-level byte per traversal vertex
   int emit_vec4 = 0;          // every lane output of this traversal is 16-byte aligned
+  int iso = 0;                // some source of this traversal is isolated
   std::vector<ibfs_level_info> log;
   std::vector<hipEvent_t> ev;  // event pool
   size_t ev_used = 0;
@@ -65,13 +65,20 @@ struct ibfs_engine_s {
 
 namespace {
 
+constexpr int POSTS = 8;  // > levels enqueued ahead
+// Levels enqueued ahead of the host, and the largest S_L (64-bit words) for
+// it.  Waiting for the host costs 5 to 8 us a level; a fixed grid instead of
+// one sized by the queues costs more once levels are long.  128 lanes, enqueued
+// ahead against not: R-MAT s18 303 / 344 us, s20 (1.3M words) 666 / 676, s21
+// (2.5M) 1,296 / 1,238, s22 1,993 / 1,923.
+constexpr int AHEAD = 2;
+constexpr int64_t AHEAD_WORDS = (int64_t)1 << 21;
+
 size_t masks_words(const ibfs_engine_s *e) { return (size_t)(2 + (e->R + 1)) * e->W; }
 
 // Waits for the work enqueued so far by polling an event recorded behind it
-// (the end of a group: its edge count and timing events).  A blocking wait's
-// wake-up costs tens of microseconds, and an event query reads one completion
-// signal where a stream query takes the stream's lock.  The level loop waits
-// on posted control blocks instead (wait_post).
+// (an earlier call's work after a failure; a group's levels and end are waited
+// for on their posts).
 // Past the wait limit (ibfs_set_wait_timeout) it fails with IBFS_ERR_STATE.
 int poll_stream(hipStream_t st, hipEvent_t ev) {
   const hipError_t r = hipEventRecord(ev, st);
@@ -87,13 +94,12 @@ int poll_stream(hipStream_t st, hipEvent_t ev) {
   }
 }
 
-// Waits for the control block posted with tag seq (a spin on the tag; every
-// 1,024 reads the stream is queried, so an error, or an idle stream without
-// the tag, ends the wait with an error), then copies it to e->h_ctl.
-int wait_post(ibfs_engine_s *e, u64 seq) {
+// Waits until *tag is seq (a spin; every 1,024 reads the stream is queried, so
+// an error, or an idle stream without the tag, ends the wait with an error).
+int wait_post(ibfs_engine_s *e, const u64 *tag, u64 seq) {
   WaitClock clk;
   for (unsigned i = 1;; ++i) {
-    if (__atomic_load_n(&e->post->tag, __ATOMIC_ACQUIRE) == seq) break;
+    if (__atomic_load_n(tag, __ATOMIC_ACQUIRE) == seq) return IBFS_OK;
     if ((i & 1023) == 0) {
       const hipError_t q = hipStreamQuery(e->st);
       if (q == hipErrorNotReady) {
@@ -103,12 +109,10 @@ int wait_post(ibfs_engine_s *e, u64 seq) {
         continue;
       }
       if (q != hipSuccess) return fail(IBFS_ERR_HIP, "stream error: %s", hipGetErrorString(q));
-      if (__atomic_load_n(&e->post->tag, __ATOMIC_ACQUIRE) == seq) break;
+      if (__atomic_load_n(tag, __ATOMIC_ACQUIRE) == seq) return IBFS_OK;
       return fail(IBFS_ERR_STATE, "control block post did not arrive");
     }
   }
-  std::memcpy(e->h_ctl, &e->post->c, sizeof(LevelCtl));
-  return IBFS_OK;
 }
 
 // Elapsed time between two events the device has passed.  A posted control
@@ -186,16 +190,12 @@ void engine_release(ibfs_engine_s *e) {
   if (e->st) (void)hipStreamSynchronize(e->st);
   dfree(e->ring);
   dfree(e->d_ctl);
-  hfree(e->h_ctl);
   hfree(e->post);
+  hfree(e->post_end);
   for (int i = 0; i < NQ; ++i) dfree(e->q.q[i]);
   dfree(e->q.chunks);
   dfree(e->d_masks);
-  hfree(e->h_masks);
-  dfree(e->d_src);
-  hfree(e->h_src);
   dfree(e->d_lanes);
-  hfree(e->h_lanes);
   dfree(e->d_out);
   dfree(e->d_count);
   hfree(e->h_count);
@@ -225,30 +225,22 @@ int64_t isolated_sources(const ibfs_graph_s *g, const int32_t *src, int k) {
   return (int64_t)(std::unique(iso.begin(), iso.end()) - iso.begin());
 }
 
-// direction of level L (0 top-down, 1 bottom-up, 2 hybrid) from the
-// counters of L-1
-int decide(const ibfs_engine_s *e, int L, const LevelCtl &c, int dir_prev, u64 nf_prev) {
+// Arguments of the inspection of level L (the pass also refreshes the hub
+// cache from S_L for the next bottom-up level).  With `on` 1 it decides level
+// L+1 into its control block and posts that with tag `tag` (Decide::on).
+InspectArgs inspect_args(ibfs_engine_s *e, int L, int on, u64 tag) {
   const ibfs_config &k = e->cfg;
-  return choose_direction(k.policy, k.sw_level, k.alpha, k.beta, k.hybrid_gamma, e->hc.rho_q10,
-                          (u64)e->g->V, L, dir_prev, nf_prev, c.n_front, c.m_front, c.m_cand,
-                          c.m_front_nh);
-}
-
-// Host-driven inspector arguments (the pass also refreshes the hub cache
-// from cur for the next bottom-up level); it posts its control block with the
-// next tag (wait_post).
-InspectArgs inspect_args(ibfs_engine_s *e, const u64 *prev, const u64 *cur, u64 *next,
-                         const u64 *lam_prev, LevelCtl *ctl, LevelCtl *ctl_zero, int full_diff,
-                         int queue_bu) {
   InspectArgs a{};
-  a.queue_bu = queue_bu;
-  a.full_diff = full_diff;
-  a.prev = prev;
-  a.cur = cur;
-  a.next = next;
-  a.lam_prev = lam_prev;
-  a.ctl = ctl;
-  a.ctl_zero = ctl_zero;
+  a.full_diff = 1;  // of level 0; later levels derive it
+  a.prev = L > 0 ? slot(e, L - 1) : nullptr;
+  a.cur = slot(e, L);
+  a.next = slot(e, L + 1);
+  a.ctl = &e->d_ctl[L % e->R];
+  a.ctl_zero = &e->d_ctl[(L + 1) % e->R];
+  a.ctl_prev = L > 0 ? &e->d_ctl[(L - 1) % e->R] : nullptr;
+  a.lam_prev = L > 0 ? a.ctl_prev->lam : e->d_masks;
+  a.dec = Decide{on, L, k.policy, k.sw_level, k.alpha, k.beta, k.hybrid_gamma, e->hc.rho_q10,
+                 (u64)e->g->V};
   a.deg = e->g->d_deg;
   a.V = e->g->Vt;
   a.q = e->q;
@@ -263,13 +255,15 @@ InspectArgs inspect_args(ibfs_engine_s *e, const u64 *prev, const u64 *cur, u64 
   a.vpt = e->cfg.inspect_vpt;
   a.nw = e->cfg.wg_size / 64;
   a.hsplit = hub_split(e->hc);
-  a.spread = ctl_spread(e->d_ctl, e->R);
-  a.post = e->post;
-  a.post_tag = ++e->post_seq;
+  a.spread = ctl_spread(e->d_ctl, e->R) + (on == 2 ? L & 1 : 0);
+  if (on == 1) {
+    a.post = &e->post[L % POSTS];
+    a.post_tag = tag;
+  }
   return a;
 }
 
-// Emits the window [b, en] for the lanes in e->h_lanes (already on device).
+// Emits the window [b, en] for the group's lanes.
 // edges (final window only, or null): the pass also adds the TEPS numerator.
 int emit_window(ibfs_engine_s *e, int b, int en, int k, ibfs_stats *stats, u64 *edges) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -279,7 +273,7 @@ int emit_window(ibfs_engine_s *e, int b, int en, int k, ibfs_stats *stats, u64 *
   }
   HIP_TRY(launch_emit(e->W, e->cfg.emit_mode, e->emit_vec4, e->ring, e->R, emit_space(e->g), b,
                       en, e->d_lanes, e->d_masks + 2 * e->W, e->d_masks + e->W, k, edges,
-                      e->st));
+                      e->iso, e->st));
   if (e->cfg.kernel_timing) {
     e1 = next_event(e);
     HIP_TRY(hipEventRecord(e1, e->st));
@@ -290,6 +284,15 @@ int emit_window(ibfs_engine_s *e, int b, int en, int k, ibfs_stats *stats, u64 *
 }
 
 // One group of k sources (lanes 0..k-1), depths into dout (device, k*V).
+//
+// The host enqueues `ahead` levels beyond the last one whose control block it
+// has read: expansions take their direction on the device from the counters
+// of the level before, and once a level has changed nothing the kernels of
+// later ones return at once.  The device then does not wait for the host
+// between levels, and the levels enqueued too many cost about 5 us each at the
+// end.  ahead 0 (kernel events, work model, and graphs whose levels are long:
+// AHEAD_WORDS) launches the direction's own kernel, sized by the counters that
+// the host has read.
 int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_stats *stats) {
   ibfs_graph_s *g = e->g;
   const int64_t V = g->V, Vt = g->Vt;
@@ -302,48 +305,65 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
   e->emit_ev.clear();
   e->log.clear();
   clear_hip_error();
+  const bool timing = e->cfg.kernel_timing != 0;
+  const bool small = Vt * W <= AHEAD_WORDS;
+  const int ahead = (timing || e->cfg.work_model || !small) ? 0 : AHEAD;
 
-  // lanes, masks, sources (pinned staging -> device)
-  std::memset(e->h_masks, 0, sizeof(u64) * masks_words(e));
+  SourceList sl;
+  sl.k = k;
+  e->iso = 0;
   for (int i = 0; i < k; ++i) {
-    e->h_masks[i >> 6] |= 1ull << (i & 63);
-    e->h_src[i] = g->h_cid[src[i]];
-    e->h_lanes[i].out = dout + (size_t)i * (size_t)V;
-    e->h_lanes[i].admit = 0;
-    e->h_lanes[i].src = src[i];
+    sl.src[i] = src[i];
+    e->iso |= g->h_cid[src[i]] < 0;
   }
   e->emit_vec4 = (V % 4 == 0) && ((uintptr_t)dout % 16 == 0);
-  for (int w = 0; w < W; ++w) e->h_masks[W + w] = e->h_masks[w];
-  for (size_t i = 0; i < (size_t)(e->R + 1) * W; ++i) e->h_masks[2 * W + i] = ~0ull;
-  HIP_TRY(hipMemcpyAsync(e->d_masks, e->h_masks, sizeof(u64) * masks_words(e),
-                         hipMemcpyHostToDevice, e->st));
-  HIP_TRY(hipMemcpyAsync(e->d_src, e->h_src, sizeof(int32_t) * k, hipMemcpyHostToDevice, e->st));
-  HIP_TRY(hipMemcpyAsync(e->d_lanes, e->h_lanes, sizeof(LaneOut) * k, hipMemcpyHostToDevice,
-                         e->st));
-
-  const bool timing = e->cfg.kernel_timing != 0;
-  hipEvent_t t_begin = next_event(e);
-  HIP_TRY(hipEventRecord(t_begin, e->st));
-
   // level 0: S_0 = source bits; inspection builds the level-1 queues
-  HIP_TRY(launch_zero3_u64(slot(e, 0), Vt * W, reinterpret_cast<u64 *>(e->flags), (Vt + 7) / 8,
-                           reinterpret_cast<u64 *>(e->d_ctl), (int64_t)(ctl_ring_bytes(e->R) / 8), e->st));
-  HIP_TRY(launch_init_sources(W, e->d_src, k, 0, slot(e, 0), e->flags, e->st));
-  hipEvent_t ti0 = nullptr, ti1 = nullptr;
-  if (timing) { ti0 = next_event(e); HIP_TRY(hipEventRecord(ti0, e->st)); }
-  HIP_TRY(launch_inspect(W, inspect_args(e, nullptr, slot(e, 0), slot(e, 1), e->d_masks,
-                                         &e->d_ctl[0], &e->d_ctl[1 % e->R], 1, 0),
-                         e->st));
-  if (timing) { ti1 = next_event(e); HIP_TRY(hipEventRecord(ti1, e->st)); }
-  {
-    const int rc = wait_post(e, e->post_seq);
-    if (rc) return rc;
-  }
-  auto record = [&](int L, int dir, const LevelCtl &c, float exp_ms, float insp_ms) {
+  HIP_TRY(launch_group_start(W, sl, g->d_cid, dout, V, Vt, slot(e, 0), e->flags,
+                             reinterpret_cast<u64 *>(e->d_ctl), (int64_t)(ctl_ring_bytes(e->R) / 8),
+                             e->d_lanes, e->d_masks, e->R, e->d_count, e->st));
+  const u64 seq0 = e->post_seq + 1;  // tag of level 0
+
+  // events of the level in flight (timing only)
+  hipEvent_t x0 = nullptr, x1 = nullptr, y0 = nullptr, y1 = nullptr;
+  auto mark = [&](hipEvent_t *x) -> hipError_t {
+    *x = next_event(e);
+    return hipEventRecord(*x, e->st);
+  };
+  auto inspect = [&](int L) -> hipError_t {
+    e->post_seq = seq0 + (u64)L;
+    return launch_inspect(W, inspect_args(e, L, ahead ? 2 : 1, e->post_seq), e->st);
+  };
+  if (timing) HIP_TRY(mark(&y0));
+  HIP_TRY(inspect(0));
+  if (timing) HIP_TRY(mark(&y1));
+
+  int known = -1, dir = -1;  // last level whose block was read, and its direction
+  LevelCtl c{};              // that block
+  // Reads the control block of level known+1: counters, level log.
+  auto learn = [&]() -> int {
+    const int l = known + 1;
+    const CtlPost *p = &e->post[l % POSTS];
+    if (int rc = wait_post(e, &p->tag, seq0 + (u64)l)) return rc;
+    if (l > 0) dir = c.next_dir;
+    std::memcpy(&c, &p->c, sizeof c);
+    known = l;
+    float ems = 0, ims = 0;
+    if (timing) {
+      if (l > 0) HIP_TRY(elapsed_ms(&ems, x0, x1));
+      HIP_TRY(elapsed_ms(&ims, y0, y1));
+    }
+    if (stats) {
+      stats->n_inspect_launches++;
+      stats->inspect_ms += ims;
+      if (l > 0) {
+        (dir == 0 ? stats->n_td_launches : dir == 2 ? stats->n_hy_launches : stats->n_bu_launches)++;
+        (dir == 0 ? stats->expand_td_ms : dir == 2 ? stats->expand_hy_ms : stats->expand_bu_ms) += ems;
+      }
+    }
     ibfs_level_info li{};
-    li.level = L;
-    li.direction = dir;
-    li.n_changed = (int64_t)c.n_changed;
+    li.level = l;
+    li.direction = l > 0 ? dir : -1;
+    li.n_changed = (int64_t)c.n_changed + (l == 0 ? isolated_sources(g, src, k) : 0);
     li.n_frontier = (int64_t)c.n_front;
     li.m_frontier = (int64_t)c.m_front;
     li.n_unvisited = (int64_t)c.n_cand;
@@ -352,169 +372,100 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
       li.q_td[i] = c.q[i];
       li.q_bu[i] = c.cls[i];
     }
-    li.expand_ms = exp_ms;
-    li.inspect_ms = insp_ms;
+    li.expand_ms = ems;
+    li.inspect_ms = ims;
     li.m_frontier_nonhub = (int64_t)c.m_front_nh;
+    if (e->cfg.work_model && dir == 1) {
+      li.bu_work = (int64_t)e->h_count[0];
+      li.bu_prefix = (int64_t)e->h_count[1];
+    }
     e->log.push_back(li);
-  };
-  float insp0 = 0;
-  if (timing) {
-    HIP_TRY(elapsed_ms(&insp0, ti0, ti1));
-    if (stats) stats->inspect_ms += insp0;
-  }
-  if (stats) stats->n_inspect_launches++;
-  {
-    LevelCtl c0 = *e->h_ctl;
-    c0.n_changed += (u64)isolated_sources(g, src, k);
-    record(0, -1, c0, 0.f, insp0);
-  }
-
-  // A level's event timings and log entry are settled after the next level's
-  // kernels are enqueued, so the host does that bookkeeping while they run
-  // instead of between the control-block wait and the next launch.
-  struct Pending {
-    bool on = false;
-    int L = 0, dir = 0;
-    hipEvent_t x0 = nullptr, x1 = nullptr, y0 = nullptr, y1 = nullptr;
-    LevelCtl c{};
-    int64_t bu_work = 0, bu_prefix = 0;
-  } pend;
-  auto settle = [&]() -> int {
-    if (!pend.on) return IBFS_OK;
-    pend.on = false;
-    float ems = 0, ims = 0;
-    if (timing) {
-      HIP_TRY(elapsed_ms(&ems, pend.x0, pend.x1));
-      HIP_TRY(elapsed_ms(&ims, pend.y0, pend.y1));
-      if (stats) {
-        (pend.dir == 0 ? stats->expand_td_ms
-                       : pend.dir == 2 ? stats->expand_hy_ms : stats->expand_bu_ms) += ems;
-        stats->inspect_ms += ims;
-      }
-    }
-    record(pend.L, pend.dir, pend.c, ems, ims);
-    if (e->cfg.work_model && pend.dir == 1) {
-      e->log.back().bu_work = pend.bu_work;
-      e->log.back().bu_prefix = pend.bu_prefix;
-    }
     return IBFS_OK;
   };
 
-  int base = 0, last = 0, dir_prev = -1;
-  u64 nf_prev = ~0ull;
+  int base = 0;
   for (int L = 1;; ++L) {
-    const LevelCtl c = *e->h_ctl;  // counters of level L-1
-    if (c.n_changed == 0) {        // only possible at L == 1 with no sources
-      last = L - 1;
-      break;
-    }
+    auto learn_to = [&](int l) -> int {
+      while (known < l && !(known >= 0 && c.n_changed == 0))
+        if (int rc = learn()) return rc;
+      return IBFS_OK;
+    };
+    if (int rc = learn_to(L - 1 - ahead)) return rc;
+    if (known >= 0 && c.n_changed == 0) break;
     if (L > 1 << 20) return fail(IBFS_ERR_STATE, "level limit exceeded");
-    const int dir = decide(e, L, c, dir_prev, nf_prev);
-    const bool tdf = dir == 0 && flag_top_down(c.m_front, (u64)g->V);
-    // lam of level L-1 is the first member of its control block
     const LevelCtl *cp = e->d_ctl + (L - 1) % e->R;
-    const u64 *lamp = cp->lam;
-    hipEvent_t x0 = nullptr, x1 = nullptr, y1 = nullptr;
-    if (timing) { x0 = next_event(e); HIP_TRY(hipEventRecord(x0, e->st)); }
-    if (dir == 0) {
+    if (timing) HIP_TRY(mark(&x0));
+    if (ahead) {
+      CtlSpread *sp = ctl_spread(e->d_ctl, e->R);
+      NextArgs n;
+      n.dec = inspect_args(e, L - 1, 2, 0).dec;
+      n.spread = sp + ((L - 1) & 1);
+      n.spread_old = sp + (L & 1);
+      n.ctl = e->d_ctl + (L - 1) % e->R;
+      n.ctl_prev = L > 1 ? e->d_ctl + (L - 2) % e->R : nullptr;
+      n.post = &e->post[(L - 1) % POSTS];
+      n.post_tag = seq0 + (u64)(L - 1);
+      HIP_TRY(launch_expand_next(W, gd, slot(e, L - 1), slot(e, L), e->hs, e->flags, n, e->q,
+                                 e->next_grid, e->st));
+    } else if (c.next_dir == 0) {
       HIP_TRY(launch_expand_td(W, gd, slot(e, L - 1), slot(e, L), cp, e->q, c.q[Q_TD_S],
-                               c.q[Q_TD_M], c.q[Q_TD_L], tdf ? e->flags : nullptr, e->st));
-      if (stats) stats->n_td_launches++;
-    } else if (dir == 2) {
-      HIP_TRY(launch_expand_hy(W, gd, slot(e, L - 1), e->hs, slot(e, L),
-                               cp, e->q, e->hy_grid, e->st));
-      if (stats) stats->n_hy_launches++;
+                               c.q[Q_TD_M], c.q[Q_TD_L], c.next_flag ? e->flags : nullptr, e->st));
+    } else if (c.next_dir == 2) {
+      HIP_TRY(launch_expand_hy(W, gd, slot(e, L - 1), e->hs, slot(e, L), cp, e->q, e->hy_grid,
+                               e->st));
     } else {
       if (e->cfg.work_model) {  // instrumentation: exact early-termination prefixes
-        HIP_TRY(hipMemsetAsync(e->d_count + 1, 0, 2 * sizeof(u64), e->st));
-        HIP_TRY(launch_bu_model(W, g->d_beg, g->d_tadj, slot(e, L - 1), e->hs, lamp, Vt,
-                                e->d_count + 1, e->st));
-        HIP_TRY(hipMemcpyAsync(e->h_count + 1, e->d_count + 1, 2 * sizeof(u64),
-                               hipMemcpyDeviceToHost, e->st));
+        HIP_TRY(hipMemsetAsync(e->d_count + 2, 0, 2 * sizeof(u64), e->st));
+        HIP_TRY(launch_bu_model(W, g->d_beg, g->d_tadj, slot(e, L - 1), e->hs, cp->lam, Vt,
+                                e->d_count + 2, e->st));
+        HIP_TRY(hipMemcpyAsync(e->h_count, e->d_count + 2, 2 * sizeof(u64), hipMemcpyDeviceToHost,
+                               e->st));
         if (timing) HIP_TRY(hipEventRecord(x0, e->st));
       }
       HIP_TRY(launch_expand_bu(W, gd, slot(e, L - 1), e->hs, slot(e, L), e->flags, cp, e->q,
                                c.bu_queued ? (int64_t)c.q[Q_BU] : Vt, (int)c.bu_queued, e->st));
-      if (stats) stats->n_bu_launches++;
     }
-    if (timing) { x1 = next_event(e); HIP_TRY(hipEventRecord(x1, e->st)); }
+    if (timing) HIP_TRY(mark(&x1));
     // the inspection's start event is the expansion's end event unless a
     // window flush runs in between
-    hipEvent_t y0 = x1;
+    y0 = x1;
     if ((L + 1) - base >= e->R) {  // the next copy would overwrite S_base
-      int rc = emit_window(e, base, L, k, stats, nullptr);
+      // a level that is known to run (a no-op for ahead 0)
+      int rc = learn_to(L - 1);
+      if (rc) return rc;
+      if (c.n_changed == 0) break;
+      rc = emit_window(e, base, L, k, stats, nullptr);
       if (rc) return rc;
       if (stats) stats->emit_windows++;
       base = L;
-      if (timing) { y0 = next_event(e); HIP_TRY(hipEventRecord(y0, e->st)); }
+      if (timing) HIP_TRY(mark(&y0));
     }
-    HIP_TRY(launch_inspect(W, inspect_args(e, slot(e, L - 1), slot(e, L), slot(e, L + 1), lamp,
-                                           &e->d_ctl[L % e->R], &e->d_ctl[(L + 1) % e->R],
-                                           (dir == 1 || tdf) ? 0 : 1,
-                                           candidates_queued(L, c.n_cand, (u64)Vt)),
-                           e->st));
-    if (timing) { y1 = next_event(e); HIP_TRY(hipEventRecord(y1, e->st)); }
-    {
-      const int rc = settle();  // level L-1, while level L runs
-      if (rc) return rc;
-    }
-    {
-      const int rc = wait_post(e, e->post_seq);
-      if (rc) return rc;
-    }
-    if (stats) stats->n_inspect_launches++;
-    pend.on = true;
-    pend.L = L;
-    pend.dir = dir;
-    pend.x0 = x0;
-    pend.x1 = x1;
-    pend.y0 = y0;
-    pend.y1 = y1;
-    pend.c = *e->h_ctl;
-    pend.bu_work = (int64_t)e->h_count[1];
-    pend.bu_prefix = (int64_t)e->h_count[2];
-    dir_prev = dir;
-    nf_prev = c.n_front;
-    if (pend.c.n_changed == 0) {
-      last = L - 1;
-      break;
-    }
+    HIP_TRY(inspect(L));
+    if (timing) HIP_TRY(mark(&y1));
   }
-  {
-    const int rc = settle();
-    if (rc) return rc;
-  }
+  const int last = known > 0 ? known - 1 : 0;
   // the final window also counts the TEPS numerator (over S_last, which its
   // pass reads anyway)
-  bool counted = false;
   if (last >= base) {
-    if (stats) HIP_TRY(hipMemsetAsync(e->d_count, 0, sizeof(u64), e->st));
     int rc = emit_window(e, base, last, k, stats, stats ? e->d_count : nullptr);
     if (rc) return rc;
     if (stats) stats->emit_windows++;
-    counted = stats != nullptr;
+  } else if (stats) {  // no final window (the last flush ended at last + 1)
+    HIP_TRY(launch_count_edges(W, slot(e, last), g->d_deg, Vt, e->d_masks, e->d_count, e->st));
   }
-  // one wait for the group: its end event, the edge count and its copy
-  hipEvent_t t_end = next_event(e);
-  HIP_TRY(hipEventRecord(t_end, e->st));
+  // one wait for the group, on its end
+  const u64 end = ++e->post_seq;
+  HIP_TRY(launch_group_end(e->d_count, e->post_end, end, e->st));
+  if (int rc = wait_post(e, &e->post_end->tag, end)) return rc;
   if (stats) {
-    if (!counted) {  // no final window (the last flush ended at last + 1)
-      HIP_TRY(hipMemsetAsync(e->d_count, 0, sizeof(u64), e->st));
-      HIP_TRY(launch_count_edges(W, slot(e, last), g->d_deg, Vt, e->d_masks, e->d_count, e->st));
-    }
-    HIP_TRY(hipMemcpyAsync(e->h_count, e->d_count, sizeof(u64), hipMemcpyDeviceToHost, e->st));
-  }
-  if (int rc = poll_stream(e->st, e->ev_wait)) return rc;
-  if (stats) {
-    float ms = 0;
-    HIP_TRY(elapsed_ms(&ms, t_begin, t_end));
-    stats->total_ms += ms;
+    stats->total_ms += (double)(e->post_end->t1 - e->post_end->t0) / e->clock_khz;
     for (const auto &x : e->emit_ev) {
+      float ms = 0;
       HIP_TRY(elapsed_ms(&ms, x.first, x.second));
       stats->emit_ms += ms;
     }
     stats->levels = std::max(stats->levels, last + 1);
-    stats->traversed_edges += (int64_t)*e->h_count;
+    stats->traversed_edges += (int64_t)e->post_end->edges;
   }
   return IBFS_OK;
 }
@@ -923,6 +874,14 @@ int ibfs_engine_create(ibfs_graph_t g, const ibfs_config *cfg_in, ibfs_engine_t 
             hipSuccess || cus <= 0)
       cus = 256;
     e->hy_grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 32;
+    // each of its workgroups folds the level's counters, so no more than start
+    // together: 512 x 512 grid 24.3 us per level at 1,024 workgroups, 25.5 at
+    // 2,048, 27.6 at 512, 34.8 at 8,192
+    e->next_grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 4;
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g->device) == hipSuccess &&
+        khz > 0)
+      e->clock_khz = khz;
   }
   e->hc = hub_cut(g, cfg.hybrid_hubs);
   const int64_t Vt = std::max<int64_t>(g->Vt, 1);
@@ -942,18 +901,15 @@ int ibfs_engine_create(ibfs_graph_t g, const ibfs_config *cfg_in, ibfs_engine_t 
   };
   A((void **)&e->ring, (size_t)R * slot_bytes);
   A((void **)&e->d_ctl, ctl_ring_bytes(R));
-  H((void **)&e->h_ctl, sizeof(LevelCtl));
-  if (err == hipSuccess) err = hipHostMalloc((void **)&e->post, sizeof(CtlPost), hipHostMallocCoherent);
-  if (err == hipSuccess) std::memset(e->post, 0, sizeof(CtlPost));
+  if (err == hipSuccess) err = hipHostMalloc((void **)&e->post, POSTS * sizeof(CtlPost), hipHostMallocCoherent);
+  if (err == hipSuccess) std::memset(e->post, 0, POSTS * sizeof(CtlPost));
+  if (err == hipSuccess) err = hipHostMalloc((void **)&e->post_end, sizeof(GroupPost), hipHostMallocCoherent);
+  if (err == hipSuccess) std::memset(e->post_end, 0, sizeof(GroupPost));
   for (int i = 0; i < NQ; ++i)
     if (i != Q_TD_L) A((void **)&e->q.q[i], sizeof(int32_t) * queue_entries((size_t)Vt));
   A((void **)&e->q.chunks, sizeof(int2) * chunk_entries((size_t)Vt, (size_t)g->E, e->chunk_shift));
   A((void **)&e->d_masks, sizeof(u64) * masks_words(e));
-  H((void **)&e->h_masks, sizeof(u64) * masks_words(e));
-  A((void **)&e->d_src, sizeof(int32_t) * (size_t)e->K);
-  H((void **)&e->h_src, sizeof(int32_t) * (size_t)e->K);
   A((void **)&e->d_lanes, sizeof(LaneOut) * (size_t)e->K);
-  H((void **)&e->h_lanes, sizeof(LaneOut) * (size_t)e->K);
   A((void **)&e->hs, sizeof(u64) * (size_t)e->W * (size_t)std::max<int64_t>(g->H, 1));
   A((void **)&e->flags, sizeof(u64) * (size_t)((Vt + 7) / 8));
   A((void **)&e->d_count, 4 * sizeof(u64));

@@ -34,7 +34,11 @@ struct alignas(64) LevelCtl {
   // Queue entry i of class c is at segment s (pre[c][s] <= i, the last such s),
   // position s * cap + i - pre[c][s], cap = chunkcap for td lrg, else segcap.
   unsigned int segcap, chunkcap;
-  unsigned int pad[10];
+  // Decision for the level after this one (Decide): its direction, -1 once a
+  // level changed nothing; whether a top-down level flags its changes.
+  int next_dir;
+  unsigned int next_flag;
+  unsigned int pad[8];
   unsigned int pre[4][QSEG];
 };
 static_assert(sizeof(LevelCtl) == 320, "LevelCtl layout");
@@ -67,14 +71,14 @@ struct alignas(128) CtlSpread {
 };
 constexpr int SPREAD_CLS = 6 + MAX_W;
 static_assert(SPREAD_CLS < 16 && CTL_COPIES * 16 <= 256, "CtlSpread layout");
-// A ring of R control blocks is allocated with its CtlSpread behind it and
-// both start a traversal at zero.
+// A ring of R control blocks is allocated with two CtlSpread behind it (the
+// second for levels enqueued ahead, which alternate) and all start a
+// traversal at zero.
 constexpr size_t ctl_ring_bytes(int R) {
-  return ((sizeof(LevelCtl) * (size_t)R + 127) & ~(size_t)127) + sizeof(CtlSpread);
+  return ((sizeof(LevelCtl) * (size_t)R + 127) & ~(size_t)127) + 2 * sizeof(CtlSpread);
 }
 inline CtlSpread *ctl_spread(LevelCtl *ring, int R) {
-  return reinterpret_cast<CtlSpread *>(reinterpret_cast<char *>(ring) + ctl_ring_bytes(R) -
-                                       sizeof(CtlSpread));
+  return reinterpret_cast<CtlSpread *>(reinterpret_cast<char *>(ring) + ctl_ring_bytes(R)) - 2;
 }
 
 enum { Q_TD_S = 0, Q_TD_M = 1, Q_TD_L = 2, Q_BU = 3, NQ = 4 };
@@ -245,6 +249,18 @@ struct CtlPost {
   u64 tag;
 };
 
+// Direction settings of a host-enqueued run (InspectArgs::dec).  on 1: the
+// inspector's last workgroup folds the counters, decides the next level into
+// the control block and posts that.  on 2 (levels enqueued ahead of the host):
+// the counters stay in the spread, and the expansion of the next level folds
+// them, decides and posts (launch_expand_next), off the inspector's chain.
+struct Decide {
+  int on;
+  int level;  // level being inspected
+  int policy, sw_level, alpha, beta, gamma, rho;
+  u64 V;
+};
+
 // Arguments of one inspector pass.  Host-driven: prev/cur/next/lam_prev/ctl
 // given explicitly and plan == nullptr.  Device-driven: plan != nullptr and
 // the level, snapshot slots and control blocks are derived from plan->level.
@@ -282,6 +298,8 @@ struct InspectArgs {
   CtlSpread *spread;    // the pass's counters before they are folded into ctl
   int queue_bu;         // host-driven: write the candidate queue (candidates_queued)
   int decide;           // plan mode: the last workgroup also decides the next level
+  Decide dec;           // (with ctl_prev, the control block of the level before, or null)
+  const LevelCtl *ctl_prev;
   CtlPost *post;        // host-driven (or null): the control block is posted here
   u64 post_tag;
 };
@@ -308,6 +326,26 @@ hipError_t launch_fill_u64(u64 *p, int64_t n, u64 value, hipStream_t st);
 hipError_t launch_zero3_u64(u64 *p0, int64_t n0, u64 *p1, int64_t n1, u64 *p2, int64_t n2,
                             hipStream_t st);
 hipError_t launch_fill_i32(int32_t *p, int64_t n, int32_t value, hipStream_t st);
+// One launch that prepares a group of sl.k sources (original ids), lane i =
+// source i from level 0: S0 with their bits and the flags, both otherwise zero
+// (Vt vertices), the control ring (ctl_words 64-bit words) zero, lane table
+// (row i of dout), masks ([0,W) and [W,2W) the group's lanes, then R+1 level
+// masks of all ones), counters[0] (edges) zero and counters[1] the device clock.
+struct SourceList {
+  int32_t src[MAX_LANES];
+  int32_t k;
+};
+hipError_t launch_group_start(int W, const SourceList &sl, const int32_t *cid, int32_t *dout,
+                              int64_t V, int64_t Vt, u64 *S0, uint8_t *flags, u64 *ctl,
+                              int64_t ctl_words, LaneOut *lanes, u64 *masks, int R, u64 *counters,
+                              hipStream_t st);
+// End of a group, posted like a control block: the counters of
+// launch_group_start and the device clock.
+struct GroupPost {
+  u64 edges, t0, t1;
+  u64 tag;
+};
+hipError_t launch_group_end(const u64 *counters, GroupPost *post, u64 tag, hipStream_t st);
 // S0[src[i]] |= bit lane0+i, i < k (src in traversal ids; -1 entries skipped).
 hipError_t launch_init_sources(int W, const int32_t *src, int k, int lane0, u64 *S0,
                                uint8_t *flags, hipStream_t st);
@@ -335,6 +373,22 @@ hipError_t launch_expand_bu(int W, const GraphDev &g, const u64 *prev, const u64
 // atomic ORs.
 hipError_t launch_expand_hy(int W, const GraphDev &g, const u64 *prev, const u64 *hs, u64 *cur,
                             const LevelCtl *ctl_prev, Queues q, int grid, hipStream_t st);
+// Expansion after an inspection with Decide::on 2, fixed grid: folds that
+// level's counters into ctl, decides this level's direction (nothing is done
+// once the traversal has ended), posts ctl, and zeroes spread_old for the
+// inspection that follows.
+struct NextArgs {
+  Decide dec;               // of the inspected level
+  const CtlSpread *spread;  // its counters
+  CtlSpread *spread_old;    // those of the level before it, folded already
+  LevelCtl *ctl;            // its control block
+  const LevelCtl *ctl_prev; // that of the level before it (null at level 0)
+  CtlPost *post;
+  u64 post_tag;
+};
+hipError_t launch_expand_next(int W, const GraphDev &g, const u64 *prev, u64 *cur, const u64 *hs,
+                              uint8_t *flags, const NextArgs &n, Queues q, int grid,
+                              hipStream_t st);
 // Device-driven expansion of plan->level (any direction, or a sparse tail
 // level appending to tl), fixed grid.
 hipError_t launch_expand_dd(int W, const GraphDev &g, u64 *ring, uint8_t *flags, int R,
@@ -366,9 +420,10 @@ hipError_t launch_plan_decide(Plan *plan, const LevelCtl *ctl_ring, int R, const
 // 256 vertices, 16-byte stores (1-KB pieces of each lane's row).
 // edges_out (final window only, or null): += sum over v of deg(v) * |S_e[v] &
 // sel|, the TEPS numerator of the selected lanes, counted during the pass.
+// iso 0: no selected lane's source is isolated.
 hipError_t launch_emit(int W, int mode, int vec4, const u64 *ring, int R, EmitSpace sp, int b,
                        int e, const LaneOut *lanes, const u64 *level_masks, const u64 *sel,
-                       int k_lanes, u64 *edges_out, hipStream_t st);
+                       int k_lanes, u64 *edges_out, int iso, hipStream_t st);
 // Closeness reduction of the window [b, e]: sum_out[k] += sum of depths and
 // reach_out[k] += vertices reached, over the bits of lane k that arrived in
 // the window (lane table and masks as for launch_emit).  Isolated sources

@@ -679,7 +679,7 @@ __global__ void k_groupby_sortkey(const int32_t *__restrict__ key, int64_t n,
 template <int W, int NS>
 static void emit_ns(int mode, int vec4, const u64 *ring, int R, EmitSpace sp, int b, int e,
                     const LaneOut *lanes, const u64 *masks, const u64 *sel, int k, u64 *edges_out,
-                    hipStream_t st) {
+                    int iso, hipStream_t st) {
   if (mode == 1) {
     dim3 g(grid_for(sp.V, BS, 4096)), blk(BS);
     hipLaunchKernelGGL((k_emit_tiled<W, NS>), g, blk, 0, st, ring, R, sp, b, e, lanes, masks, sel,
@@ -698,7 +698,7 @@ static void emit_ns(int mode, int vec4, const u64 *ring, int R, EmitSpace sp, in
     dim3 g(grid_for(sp.V, BS, IBFS_EMIT_GRID_CAP)), blk(BS);
     hipLaunchKernelGGL((k_emit<W, NS>), g, blk, 0, st, ring, R, sp, b, e, lanes, masks, sel, k,
                        mode == 2 ? 1 : 0, edges_out);
-    if (NS == 4)  // depth 0 at isolated sources after the fast path's -1
+    if (NS == 4 && iso)  // depth 0 at isolated sources after the fast path's -1
       hipLaunchKernelGGL(k_emit_iso_sources, dim3((k + BS - 1) / BS), dim3(BS), 0, st, lanes, sel,
                          sp.cid, b, k);
   }
@@ -707,25 +707,25 @@ static void emit_ns(int mode, int vec4, const u64 *ring, int R, EmitSpace sp, in
 template <int W>
 static hipError_t emit_w(int mode, int vec4, const u64 *ring, int R, EmitSpace sp, int b, int e,
                          const LaneOut *lanes, const u64 *masks, const u64 *sel, int k,
-                         u64 *edges_out, hipStream_t st) {
+                         u64 *edges_out, int iso, hipStream_t st) {
   const int span = e - b + 1;
-  if (span < 16) emit_ns<W, 4>(mode, vec4, ring, R, sp, b, e, lanes, masks, sel, k, edges_out, st);
-  else if (span < 64) emit_ns<W, 6>(mode, vec4, ring, R, sp, b, e, lanes, masks, sel, k, edges_out, st);
-  else if (span < 256) emit_ns<W, 8>(mode, vec4, ring, R, sp, b, e, lanes, masks, sel, k, edges_out, st);
+  if (span < 16) emit_ns<W, 4>(mode, vec4, ring, R, sp, b, e, lanes, masks, sel, k, edges_out, iso, st);
+  else if (span < 64) emit_ns<W, 6>(mode, vec4, ring, R, sp, b, e, lanes, masks, sel, k, edges_out, iso, st);
+  else if (span < 256) emit_ns<W, 8>(mode, vec4, ring, R, sp, b, e, lanes, masks, sel, k, edges_out, iso, st);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
 hipError_t launch_emit(int W, int mode, int vec4, const u64 *ring, int R, EmitSpace sp, int b,
                        int e, const LaneOut *lanes, const u64 *level_masks, const u64 *sel,
-                       int k_lanes, u64 *edges_out, hipStream_t st) {
+                       int k_lanes, u64 *edges_out, int iso, hipStream_t st) {
   if (sp.V <= 0 || e < b) return hipSuccess;
   if (edges_out && !sp.deg) return hipErrorInvalidValue;
   switch (W) {
-    case 1: return emit_w<1>(mode, vec4, ring, R, sp, b, e, lanes, level_masks, sel, k_lanes, edges_out, st);
-    case 2: return emit_w<2>(mode, vec4, ring, R, sp, b, e, lanes, level_masks, sel, k_lanes, edges_out, st);
-    case 4: return emit_w<4>(mode, vec4, ring, R, sp, b, e, lanes, level_masks, sel, k_lanes, edges_out, st);
-    case 8: return emit_w<8>(mode, vec4, ring, R, sp, b, e, lanes, level_masks, sel, k_lanes, edges_out, st);
+    case 1: return emit_w<1>(mode, vec4, ring, R, sp, b, e, lanes, level_masks, sel, k_lanes, edges_out, iso, st);
+    case 2: return emit_w<2>(mode, vec4, ring, R, sp, b, e, lanes, level_masks, sel, k_lanes, edges_out, iso, st);
+    case 4: return emit_w<4>(mode, vec4, ring, R, sp, b, e, lanes, level_masks, sel, k_lanes, edges_out, iso, st);
+    case 8: return emit_w<8>(mode, vec4, ring, R, sp, b, e, lanes, level_masks, sel, k_lanes, edges_out, iso, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -31,6 +31,63 @@ __global__ void k_fill_i32(int32_t *p, int64_t n, int32_t value) {
     p[i] = value;
 }
 
+// Group start (launch_group_start): a workgroup zeroes the words and flags of
+// its share of the vertices and sets there the bits of the sources that fall
+// into it, so one launch replaces three copies and two fills.  Bound by
+// writing S_0 (9 us at R-MAT s22, 128 lanes).
+template <int W>
+__global__ __launch_bounds__(BS) void k_group_start(SourceList sl, const int32_t *__restrict__ cid,
+                                                    int32_t *dout, int64_t V, int64_t Vt, u64 *S0,
+                                                    uint8_t *flags, u64 *ctl, int64_t ctl_words,
+                                                    LaneOut *lanes, u64 *masks, int R,
+                                                    u64 *counters) {
+  const int t = threadIdx.x;
+  // shares of a multiple of 16 vertices: whole 64-bit words of flags
+  const int64_t share = ((Vt + gridDim.x - 1) / gridDim.x + 15) & ~(int64_t)15;
+  const int64_t v0 = blockIdx.x * share, v1 = v0 + share < Vt ? v0 + share : Vt;
+  for (int64_t i = v0 * W + t; i < v1 * W; i += BS) S0[i] = 0;
+  u64 *f = reinterpret_cast<u64 *>(flags);  // padded to whole words
+  for (int64_t i = v0 / 8 + t; i < (v1 + 7) / 8; i += BS) f[i] = 0;
+  if (blockIdx.x == 0) {
+    if (t == 0) {
+      counters[0] = 0;
+      counters[1] = (u64)wall_clock64();
+    }
+    for (int64_t i = t; i < ctl_words; i += BS) ctl[i] = 0;
+    for (int i = t; i < (2 + R + 1) * W; i += BS) {
+      u64 m = ~0ull;
+      if (i < 2 * W) {
+        const int n = sl.k - (i % W) * 64;
+        m = n >= 64 ? ~0ull : (n <= 0 ? 0ull : (1ull << n) - 1);
+      }
+      masks[i] = m;
+    }
+    for (int i = t; i < sl.k; i += BS) {
+      lanes[i].out = dout + (int64_t)i * V;
+      lanes[i].admit = 0;
+      lanes[i].src = sl.src[i];
+    }
+  }
+  __syncthreads();
+  for (int i = t; i < sl.k; i += BS) {
+    const int32_t v = cid[sl.src[i]];
+    if (v >= v0 && v < v1) {  // (an isolated source has no word)
+      atomicOr(&S0[(int64_t)v * W + (i >> 6)], 1ull << (i & 63));
+      flags[v] = 1;
+    }
+  }
+}
+
+__global__ void k_group_end(const u64 *counters, GroupPost *post, u64 tag) {
+  const int t = threadIdx.x;
+  if (t < 3)
+    __hip_atomic_store(&(&post->edges)[t],
+                       t == 2 ? (u64)wall_clock64() : atomic_read(&counters[t]),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (t == 0) __hip_atomic_store(&post->tag, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Lane init: lane lane0+i gets bit of src[i] (a traversal id).  OR, so
 // duplicate sources keep their bit.  src[i] < 0 is an isolated source: it
 // has no status word and its depth array is -1 except 0 at the source (the
@@ -210,6 +267,15 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
     ctl_zero = a.ctl_ring + (L + 1) % a.R;
     lam_prev = L > 0 ? a.ctl_ring[(L - 1) % a.R].lam : a.lanes_all;
     queue_bu = L > 0 && candidates_queued(L, a.ctl_ring[(L - 1) % a.R].n_cand, (u64)a.V);
+  }
+  if (a.dec.on) {
+    const LevelCtl *cp = a.ctl_prev;
+    if (cp) {
+      const int dir = cp->next_dir;
+      if (dir < 0) return;  // ended before this level (its counters stay zero)
+      full = !(dir == 1 || (dir == 0 && cp->next_flag));
+      queue_bu = candidates_queued(a.dec.level, cp->n_cand, (u64)a.V);
+    }
   }
   if (blockIdx.x == 0 && ctl_zero && t < (int)(sizeof(LevelCtl) / 8))
     reinterpret_cast<u64 *>(ctl_zero)[t] = 0;
@@ -417,6 +483,14 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
     if (s && add) atomicAdd(d, s);
     else if (s) atomicOr(d, s);
   }
+  if (a.dec.on == 2) {  // the next expansion folds
+    if (blockIdx.x == 0 && t == 0) {
+      ctl->segcap = segcap;
+      ctl->chunkcap = chunkcap;
+      ctl->bu_queued = queue_bu;
+    }
+    return;
+  }
   // Measured against one set of counters and a launch of its own that posted
   // or decided: 512 x 512 grid, 128 lanes, 35.1 -> 31.0 us per level; R-MAT
   // s18 closeness 310 -> 291 ms; R-MAT s22, 8 groups of 128, 15.0 -> 14.6 ms.
@@ -479,6 +553,17 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
     ctl->bu_queued = fin.bu_queued = queue_bu;
   }
   __syncthreads();
+  if (a.dec.on && t == 0) {
+    const Decide &d = a.dec;
+    const LevelCtl *cp = a.ctl_prev;
+    int dir = -1;
+    if (fin.n_changed)
+      dir = choose_direction(d.policy, d.sw_level, d.alpha, d.beta, d.gamma, d.rho, d.V,
+                             d.level + 1, cp ? cp->next_dir : -1, cp ? cp->n_front : ~0ull,
+                             fin.n_front, fin.m_front, fin.m_cand, fin.m_front_nh);
+    ctl->next_dir = fin.next_dir = dir;
+    ctl->next_flag = fin.next_flag = dir == 0 && flag_top_down(fin.m_front, d.V);
+  }
   if (a.post) {  // one wave: the block's words arrive at the host before the tag
     if (t < (int)CTL_WORDS)
       __hip_atomic_store(&reinterpret_cast<u64 *>(&a.post->c)[t], reinterpret_cast<u64 *>(&fin)[t],
@@ -1186,9 +1271,131 @@ __device__ void tail_level(const int64_t *__restrict__ beg, const int32_t *__res
   }
 }
 
-// Device-driven expansion of level plan->level: a fixed grid strides over
-// the class queues of the direction the inspector chose, or over the
-// frontier of a sparse tail level.
+// One level in direction dir (0 top-down, tf: flags of what it changes or
+// null; 1 bottom-up; 2 hybrid): a fixed grid strides over the queues, or the
+// vertices, that the inspection of the level before left in c.
+template <int W>
+__device__ __forceinline__ void expand_level(const GraphDev &g, const u64 *prev, u64 *cur,
+                                             const u64 *hs, uint8_t *flags, uint8_t *tf,
+                                             const LevelCtl *__restrict__ c, const Queues &q,
+                                             int dir, BuShared<W> &sh) {
+  const int64_t *__restrict__ beg = g.beg;
+  const int32_t *__restrict__ adj = g.adj;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int64_t G = gridDim.x;
+  u64 lam[W];
+#pragma unroll
+  for (int w = 0; w < W; ++w) lam[w] = c->lam[w];
+  if (dir == 0) {
+    const QIndex is(c, Q_TD_S), im(c, Q_TD_M), il(c, Q_TD_L);
+    const int64_t ns = c->q[Q_TD_S], nm = c->q[Q_TD_M], nl = c->q[Q_TD_L];
+    for (int64_t i = ((int64_t)blockIdx.x * BS + t) / TD_SMALL; i < ns; i += G * (BS / TD_SMALL)) {
+      const int32_t u = q.q[Q_TD_S][is(i)];
+      td_push<W>(adj, prev, cur, lam, u, beg[u] + t % TD_SMALL, beg[u + 1], TD_SMALL, nullptr, tf);
+    }
+    for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nm; i += G * 4) {
+      const int32_t u = q.q[Q_TD_M][im(i)];
+      td_push<W>(adj, prev, cur, lam, u, beg[u] + lane, beg[u + 1], 64, nullptr, tf);
+    }
+    for (int64_t i = blockIdx.x; i < nl; i += G) {
+      const int2 e = q.chunks[il(i)];
+      int64_t lo, hi;
+      td_chunk_range(beg, e, g.chunk_shift, lo, hi);
+      td_push<W>(adj, prev, cur, lam, e.x, lo + t, hi, BS, nullptr, tf);
+    }
+  } else if (dir == 2) {
+    const Gather gs{prev, hs};
+    expand_hybrid<W>(g, gs, cur, lam, c, q, sh);
+  } else {
+    const Gather gs{prev, hs};
+    const bool queued = c->bu_queued != 0;
+    bu_level<W, 0>(g, gs, cur, flags, lam, c, queued ? q.q[Q_BU] : nullptr,
+                   queued ? (int64_t)c->q[Q_BU] : g.V, sh);
+  }
+}
+
+// Levels enqueued ahead of the host: every workgroup folds the inspection's
+// counters for itself (16 cache lines) and comes to the same decision; the
+// first writes it to the control block and to the host.  The inspection ends
+// without a ticket, a fold and a wait for the host's memory, 3 us of its 11 on
+// a 512 x 512 grid.
+template <int W>
+__global__ __launch_bounds__(BS) void k_expand_next(GraphDev g, const u64 *prev, u64 *cur,
+                                                    const u64 *hs, uint8_t *flags, NextArgs n,
+                                                    Queues q) {
+  __shared__ BuShared<W> sh;
+  __shared__ u64 fold[CTL_COPIES][16];
+  __shared__ u64 segn[QSEG][NQ / 2];
+  __shared__ LevelCtl c;
+  const int t = threadIdx.x;
+  static_assert(CTL_COPIES * 16 == BS, "one counter per thread");
+  const int dir_prev = n.ctl_prev ? n.ctl_prev->next_dir : -1;
+  const u64 nf_prev = n.ctl_prev ? n.ctl_prev->n_front : ~0ull;
+  fold[t >> 4][t & 15] = n.spread->v[t >> 4][t & 15];
+  if (t < QSEG * NQ / 2) segn[t / (NQ / 2)][t % (NQ / 2)] = n.spread->qseg[t / (NQ / 2)][t % (NQ / 2)];
+  if (t < (int)CTL_WORDS) reinterpret_cast<u64 *>(&c)[t] = 0;
+  __syncthreads();
+  if (t < 6 + W) {
+    u64 s = 0;
+#pragma unroll
+    for (int k = 0; k < CTL_COPIES; ++k) s = t < 6 ? s + fold[k][t] : s | fold[k][t];
+    if (t < 6) (&c.n_changed)[t] = s;
+    else c.lam[t - 6] = s;
+  } else if (t >= 64 && t < 64 + NQ) {
+    const int k = t - 64;
+    unsigned m = 0;
+#pragma unroll
+    for (int i = 0; i < QSEG; ++i) {
+      c.pre[k][i] = m;
+      m += (unsigned)(segn[i][k / 2] >> (32 * (k & 1)));
+    }
+    c.q[k] = m;
+  } else if (t == 128) {
+    u64 s = 0, nc = 0;
+#pragma unroll
+    for (int k = 0; k < CTL_COPIES; ++k) {
+      s += fold[k][SPREAD_CLS];
+      nc += fold[k][3];
+    }
+    c.cls[0] = (unsigned)s;
+    c.cls[1] = (unsigned)(s >> 32);
+    c.cls[2] = (unsigned)(nc - (s >> 32) - (s & 0xffffffffull));
+  } else if (t == 192) {
+    c.segcap = n.ctl->segcap;
+    c.chunkcap = n.ctl->chunkcap;
+    c.bu_queued = n.ctl->bu_queued;
+  }
+  __syncthreads();
+  if (t == 0) {
+    const Decide &d = n.dec;
+    int dir = -1;
+    if (c.n_changed)
+      dir = choose_direction(d.policy, d.sw_level, d.alpha, d.beta, d.gamma, d.rho, d.V,
+                             d.level + 1, dir_prev, nf_prev, c.n_front, c.m_front, c.m_cand,
+                             c.m_front_nh);
+    c.next_dir = dir;
+    c.next_flag = dir == 0 && flag_top_down(c.m_front, d.V);
+  }
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    u64 *old = reinterpret_cast<u64 *>(n.spread_old);
+    for (int i = t; i < (int)(sizeof(CtlSpread) / 8); i += BS) old[i] = 0;
+    if (t < (int)CTL_WORDS) {
+      const u64 x = reinterpret_cast<const u64 *>(&c)[t];
+      reinterpret_cast<u64 *>(n.ctl)[t] = x;
+      __hip_atomic_store(&reinterpret_cast<u64 *>(&n.post->c)[t], x, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (t == 0)
+        __hip_atomic_store(&n.post->tag, n.post_tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+  if (c.next_dir < 0) return;
+  expand_level<W>(g, prev, cur, hs, flags, c.next_flag ? flags : nullptr, &c, q, c.next_dir, sh);
+}
+
+// Device-driven expansion of level plan->level, or of the frontier of a
+// sparse tail level.
 template <int W>
 __global__ __launch_bounds__(BS) void k_expand_dd(GraphDev g, u64 *ring, uint8_t *flags, int R,
                                                   const LevelCtl *__restrict__ ctl_ring,
@@ -1210,66 +1417,41 @@ __global__ __launch_bounds__(BS) void k_expand_dd(GraphDev g, u64 *ring, uint8_t
   const int64_t slot = V * W;
   const u64 *prev = ring + (int64_t)((L - 1) % R) * slot;
   u64 *cur = ring + (int64_t)(L % R) * slot;
+  if (dir != 3) {
+    expand_level<W>(g, prev, cur, hs, flags, plan->td_flag ? flags : nullptr, c, q, dir, sh);
+    return;
+  }
+  // split level: the dense lanes pull over whole lists, the sparse lanes
+  // push the bits their frontier vertices gained at L-1
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int64_t G = gridDim.x;
-  u64 lam[W];
+  const Gather gs{prev, hs};
+  const u64 *pp = L >= 2 ? ring + (int64_t)((L - 2) % R) * slot : nullptr;
+  u64 ld[W], ls[W];
 #pragma unroll
-  for (int w = 0; w < W; ++w) lam[w] = c->lam[w];
+  for (int w = 0; w < W; ++w) {
+    const u64 lw = c->lam[w];
+    ld[w] = lw & plan->split[w];
+    ls[w] = lw & ~plan->split[w];
+  }
   const bool queued = c->bu_queued != 0;
-  const int32_t *buq = queued ? q.q[Q_BU] : nullptr;
-  const int64_t nbu = queued ? (int64_t)c->q[Q_BU] : V;
-  if (dir == 0) {
-    const QIndex is(c, Q_TD_S), im(c, Q_TD_M), il(c, Q_TD_L);
-    uint8_t *tf = plan->td_flag ? flags : nullptr;
-    const int64_t ns = c->q[Q_TD_S], nm = c->q[Q_TD_M], nl = c->q[Q_TD_L];
-    for (int64_t i = ((int64_t)blockIdx.x * BS + t) / TD_SMALL; i < ns; i += G * (BS / TD_SMALL)) {
-      const int32_t u = q.q[Q_TD_S][is(i)];
-      td_push<W>(adj, prev, cur, lam, u, beg[u] + t % TD_SMALL, beg[u + 1], TD_SMALL, nullptr, tf);
-    }
-    for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nm; i += G * 4) {
-      const int32_t u = q.q[Q_TD_M][im(i)];
-      td_push<W>(adj, prev, cur, lam, u, beg[u] + lane, beg[u + 1], 64, nullptr, tf);
-    }
-    for (int64_t i = blockIdx.x; i < nl; i += G) {
-      const int2 e = q.chunks[il(i)];
-      int64_t lo, hi;
-      td_chunk_range(beg, e, cs, lo, hi);
-      td_push<W>(adj, prev, cur, lam, e.x, lo + t, hi, BS, nullptr, tf);
-    }
-  } else if (dir == 2) {
-    const Gather gs{prev, hs};
-    expand_hybrid<W>(g, gs, cur, lam, c, q, sh);
-  } else if (dir == 3) {
-    // split level: the dense lanes pull over whole lists, the sparse lanes
-    // push the bits their frontier vertices gained at L-1
-    const Gather gs{prev, hs};
-    const u64 *pp = L >= 2 ? ring + (int64_t)((L - 2) % R) * slot : nullptr;
-    u64 ld[W], ls[W];
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      ld[w] = lam[w] & plan->split[w];
-      ls[w] = lam[w] & ~plan->split[w];
-    }
-    bu_level<W, 2>(g, gs, cur, nullptr, ld, c, buq, nbu, sh);
-    const QIndex is(c, Q_TD_S), im(c, Q_TD_M), il(c, Q_TD_L);
-    const int64_t ns = c->q[Q_TD_S], nm = c->q[Q_TD_M], nl = c->q[Q_TD_L];
-    for (int64_t i = ((int64_t)blockIdx.x * BS + t) / TD_SMALL; i < ns; i += G * (BS / TD_SMALL)) {
-      const int32_t u = q.q[Q_TD_S][is(i)];
-      td_push<W, true>(adj, prev, cur, ls, u, beg[u] + t % TD_SMALL, beg[u + 1], TD_SMALL, pp);
-    }
-    for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nm; i += G * 4) {
-      const int32_t u = q.q[Q_TD_M][im(i)];
-      td_push<W, true>(adj, prev, cur, ls, u, beg[u] + lane, beg[u + 1], 64, pp);
-    }
-    for (int64_t i = blockIdx.x; i < nl; i += G) {
-      const int2 e = q.chunks[il(i)];
-      int64_t lo, hi;
-      td_chunk_range(beg, e, cs, lo, hi);
-      td_push<W, true>(adj, prev, cur, ls, e.x, lo + t, hi, BS, pp);
-    }
-  } else {
-    const Gather gs{prev, hs};
-    bu_level<W, 0>(g, gs, cur, flags, lam, c, buq, nbu, sh);
+  bu_level<W, 2>(g, gs, cur, nullptr, ld, c, queued ? q.q[Q_BU] : nullptr,
+                 queued ? (int64_t)c->q[Q_BU] : V, sh);
+  const QIndex is(c, Q_TD_S), im(c, Q_TD_M), il(c, Q_TD_L);
+  const int64_t ns = c->q[Q_TD_S], nm = c->q[Q_TD_M], nl = c->q[Q_TD_L];
+  for (int64_t i = ((int64_t)blockIdx.x * BS + t) / TD_SMALL; i < ns; i += G * (BS / TD_SMALL)) {
+    const int32_t u = q.q[Q_TD_S][is(i)];
+    td_push<W, true>(adj, prev, cur, ls, u, beg[u] + t % TD_SMALL, beg[u + 1], TD_SMALL, pp);
+  }
+  for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nm; i += G * 4) {
+    const int32_t u = q.q[Q_TD_M][im(i)];
+    td_push<W, true>(adj, prev, cur, ls, u, beg[u] + lane, beg[u + 1], 64, pp);
+  }
+  for (int64_t i = blockIdx.x; i < nl; i += G) {
+    const int2 e = q.chunks[il(i)];
+    int64_t lo, hi;
+    td_chunk_range(beg, e, cs, lo, hi);
+    td_push<W, true>(adj, prev, cur, ls, e.x, lo + t, hi, BS, pp);
   }
 }
 
@@ -1388,6 +1570,21 @@ hipError_t launch_fill_i32(int32_t *p, int64_t n, int32_t value, hipStream_t st)
   return hipGetLastError();
 }
 
+hipError_t launch_group_start(int W, const SourceList &sl, const int32_t *cid, int32_t *dout,
+                              int64_t V, int64_t Vt, u64 *S0, uint8_t *flags, u64 *ctl,
+                              int64_t ctl_words, LaneOut *lanes, u64 *masks, int R, u64 *counters,
+                              hipStream_t st) {
+  dim3 g(grid_for(Vt * W, BS * 8, 8192)), blk(BS);
+  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_group_start<WW>, g, blk, 0, st, sl, cid, dout, V, Vt, S0,
+                                        flags, ctl, ctl_words, lanes, masks, R, counters));
+  return hipGetLastError();
+}
+
+hipError_t launch_group_end(const u64 *counters, GroupPost *post, u64 tag, hipStream_t st) {
+  hipLaunchKernelGGL(k_group_end, dim3(1), dim3(64), 0, st, counters, post, tag);
+  return hipGetLastError();
+}
+
 hipError_t launch_init_sources(int W, const int32_t *src, int k, int lane0, u64 *S0,
                                uint8_t *flags, hipStream_t st) {
   if (k <= 0) return hipSuccess;
@@ -1492,6 +1689,15 @@ hipError_t launch_expand_bu(int W, const GraphDev &g, const u64 *prev, const u64
   const int32_t *queue = queued ? q.q[Q_BU] : nullptr;
   IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_bu<WW>, gr, blk, 0, st, g, gs, cur, flags,
                                         ctl_prev, queue, n));
+  return hipGetLastError();
+}
+
+hipError_t launch_expand_next(int W, const GraphDev &g, const u64 *prev, u64 *cur, const u64 *hs,
+                              uint8_t *flags, const NextArgs &n, Queues q, int grid,
+                              hipStream_t st) {
+  dim3 gr(grid > 0 ? grid : 1), blk(BS);
+  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_expand_next<WW>, gr, blk, 0, st, g, prev, cur, hs, flags,
+                                        n, q));
   return hipGetLastError();
 }
 

@@ -61,45 +61,16 @@ static_assert(NA_BYTES == IBFS_NOALLOC_SCRATCH_BYTES, "scratch size in ibfs.h");
 // hipGetSymbolAddress (scratch_ptr below).
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
 
-struct SourceList {  // sources of the group, passed by value to the set-up kernel
-  int32_t src[NA_K];
-  int32_t k;
-};
-
 struct PlanInit {
   int policy, sw_level, alpha, beta, gamma, rho;
   u64 V;
 };
 
-// Set-up of one traversal (slot 0, flags and control blocks already zero):
-// lane table, masks, source bits of S_0, plan.  One workgroup.
-template <int W>
-__global__ void k_noalloc_setup(SourceList sl, const int32_t *__restrict__ cid, int32_t *dout,
-                                int64_t V, u64 *S0, uint8_t *flags, LaneOut *lanes, u64 *masks,
-                                int R, Plan *plan, PlanInit pi) {
+// Plan of one traversal before its level 0.  One wave.
+__global__ void k_noalloc_plan(Plan *plan, PlanInit pi) {
   const int t = threadIdx.x;
   for (int i = t; i < (int)(sizeof(Plan) / 4); i += blockDim.x)
     reinterpret_cast<uint32_t *>(plan)[i] = 0;
-  for (int i = t; i < (2 + R + 1) * W; i += blockDim.x) {
-    u64 m = ~0ull;  // level masks: every lane admitted at level 0
-    if (i < 2 * W) {
-      const int w = i % W, lo = w * 64;
-      const int n = sl.k - lo;
-      m = n >= 64 ? ~0ull : (n <= 0 ? 0ull : (1ull << n) - 1);
-    }
-    masks[i] = m;
-  }
-  if (t < sl.k) {
-    const int32_t s = sl.src[t];
-    lanes[t].out = dout + (int64_t)t * V;
-    lanes[t].admit = 0;
-    lanes[t].src = s;
-    const int32_t v = cid[s];
-    if (v >= 0) {
-      atomicOr(&S0[(int64_t)v * W + (t >> 6)], 1ull << (t & 63));
-      flags[v] = 1;
-    }
-  }
   __syncthreads();
   if (t == 0) {
     plan->policy = pi.policy;
@@ -190,21 +161,19 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   hipStream_t st = nullptr;  // the null stream: nothing to create
 
   // the previous call's contents stay in the array: clear what starts at zero
-  NA_TRY(launch_fill_u64(ring, Vt * W, 0ull, st));  // slot 0
-  NA_TRY(launch_fill_u64(reinterpret_cast<u64 *>(flags), (Vt + 7) / 8, 0ull, st));
-  NA_TRY(launch_fill_u64(reinterpret_cast<u64 *>(ctl), (int64_t)(ctl_ring_bytes(R) / 8), 0ull, st));
-  NA_TRY(launch_fill_u64(count, 1, 0ull, st));
-  SourceList sl{};
-  for (int i = 0; i < k; ++i) sl.src[i] = src[i];
+  SourceList sl;
   sl.k = k;
+  int iso = 0;
+  for (int i = 0; i < k; ++i) {
+    sl.src[i] = src[i];
+    iso |= g->h_cid[src[i]] < 0;
+  }
+  NA_TRY(launch_group_start(W, sl, g->d_cid, dout, V, Vt, ring, flags,
+                            reinterpret_cast<u64 *>(ctl), (int64_t)(ctl_ring_bytes(R) / 8), lanes,
+                            masks, R, count, st));
   const PlanInit pi{cfg.policy, cfg.sw_level, cfg.alpha, cfg.beta, cfg.hybrid_gamma, hc.rho_q10,
                     (u64)V};
-  if (W == 1)
-    hipLaunchKernelGGL(k_noalloc_setup<1>, dim3(1), dim3(NA_K), 0, st, sl, g->d_cid, dout, V,
-                       ring, flags, lanes, masks, R, plan, pi);
-  else
-    hipLaunchKernelGGL(k_noalloc_setup<2>, dim3(1), dim3(NA_K), 0, st, sl, g->d_cid, dout, V,
-                       ring, flags, lanes, masks, R, plan, pi);
+  hipLaunchKernelGGL(k_noalloc_plan, dim3(1), dim3(64), 0, st, plan, pi);
   NA_TRY(hipGetLastError());
 
   InspectArgs a{};
@@ -238,7 +207,7 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
     int B = std::min(8, R - 1 - (level - lo));
     if (B < 1) {  // the next levels would overwrite S_lo: emit [lo, level-1]
       NA_TRY(launch_emit(W, cfg.emit_mode, vec4, ring, R, sp, lo, level - 1, lanes, masks + 2 * W,
-                         masks + W, k, nullptr, st));
+                         masks + W, k, nullptr, iso, st));
       lo = level - 1;
       B = std::min(8, R - 1 - (level - lo));
     }
@@ -252,7 +221,7 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
     if (ph.done) {
       if (ph.last >= lo)
         NA_TRY(launch_emit(W, cfg.emit_mode, vec4, ring, R, sp, lo, ph.last, lanes, masks + 2 * W,
-                           masks + W, k, edges ? count : nullptr, st));
+                           masks + W, k, edges ? count : nullptr, iso, st));
       else if (edges)  // no final window: count over S_last
         NA_TRY(launch_count_edges(W, ring + (int64_t)(ph.last % R) * Vt * W, g->d_deg, Vt, masks,
                                   count, st));
