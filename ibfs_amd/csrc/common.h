@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -133,6 +134,16 @@ struct ibfs_graph_s {
   // hub_entries[i] = traversal-adjacency entries that point to slots < i
   std::vector<int32_t> h_hub_deg, h_hub_id;
   std::vector<int64_t> h_hub_entries;
+  // workspace of small GroupBy calls (made by the first, freed with the
+  // graph); the mutex serialises calls of several threads
+  struct {
+    std::mutex mu;
+    void *st = nullptr;           // hipStream_t
+    void *post = nullptr;         // GroupbyPost, coherent pinned
+    unsigned long long *comp = nullptr, *ticket = nullptr;
+    unsigned long long seq = 0;
+    bool unsettled = false;       // a call failed with work possibly enqueued
+  } gb;
 };
 
 // Pull cut of hybrid levels at the top r hubs (r <= 0 or r > H: all H hubs):

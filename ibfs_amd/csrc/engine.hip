@@ -96,21 +96,21 @@ int poll_stream(hipStream_t st, hipEvent_t ev) {
 
 // Waits until *tag is seq (a spin; every 1,024 reads the stream is queried, so
 // an error, or an idle stream without the tag, ends the wait with an error).
-int wait_post(ibfs_engine_s *e, const u64 *tag, u64 seq) {
+int wait_tag(hipStream_t st, const u64 *tag, u64 seq, const char *what) {
   WaitClock clk;
   for (unsigned i = 1;; ++i) {
     if (__atomic_load_n(tag, __ATOMIC_ACQUIRE) == seq) return IBFS_OK;
     if ((i & 1023) == 0) {
-      const hipError_t q = hipStreamQuery(e->st);
+      const hipError_t q = hipStreamQuery(st);
       if (q == hipErrorNotReady) {
         if (clk.expired())
-          return fail(IBFS_ERR_STATE, "level did not finish within the wait limit (%.1f s)",
+          return fail(IBFS_ERR_STATE, "%s did not finish within the wait limit (%.1f s)", what,
                       wait_timeout_s());
         continue;
       }
       if (q != hipSuccess) return fail(IBFS_ERR_HIP, "stream error: %s", hipGetErrorString(q));
       if (__atomic_load_n(tag, __ATOMIC_ACQUIRE) == seq) return IBFS_OK;
-      return fail(IBFS_ERR_STATE, "control block post did not arrive");
+      return fail(IBFS_ERR_STATE, "%s: post did not arrive", what);
     }
   }
 }
@@ -343,7 +343,7 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
   auto learn = [&]() -> int {
     const int l = known + 1;
     const CtlPost *p = &e->post[l % POSTS];
-    if (int rc = wait_post(e, &p->tag, seq0 + (u64)l)) return rc;
+    if (int rc = wait_tag(e->st, &p->tag, seq0 + (u64)l, "level")) return rc;
     if (l > 0) dir = c.next_dir;
     std::memcpy(&c, &p->c, sizeof c);
     known = l;
@@ -456,7 +456,7 @@ int traverse(ibfs_engine_s *e, const int32_t *src, int k, int32_t *dout, ibfs_st
   // one wait for the group, on its end
   const u64 end = ++e->post_seq;
   HIP_TRY(launch_group_end(e->d_count, e->post_end, end, e->st));
-  if (int rc = wait_post(e, &e->post_end->tag, end)) return rc;
+  if (int rc = wait_tag(e->st, &e->post_end->tag, end, "group")) return rc;
   if (stats) {
     stats->total_ms += (double)(e->post_end->t1 - e->post_end->t0) / e->clock_khz;
     for (const auto &x : e->emit_ev) {
@@ -801,6 +801,12 @@ int ibfs_graph_hub_entries(ibfs_graph_t g, int64_t top, int64_t *entries) {
 int ibfs_graph_destroy(ibfs_graph_t g) {
   if (!g) return IBFS_OK;
   (void)hipSetDevice(g->device);
+  if (g->gb.st) {
+    (void)hipStreamSynchronize((hipStream_t)g->gb.st);
+    (void)hipStreamDestroy((hipStream_t)g->gb.st);
+    (void)hipHostFree(g->gb.post);
+    (void)hipFree(g->gb.comp);
+  }
   dfree(g->d_beg);
   dfree(g->d_adj);
   dfree(g->d_tadj);
@@ -813,6 +819,54 @@ int ibfs_graph_destroy(ibfs_graph_t g) {
   return IBFS_OK;
 }
 
+}  // extern "C"
+
+// GroupBy through the graph's own workspace (n <= GROUPBY_SMALL).
+static int groupby_small(ibfs_graph_s *g, const int32_t *src, int n, int32_t *out) {
+  auto &w = g->gb;
+  std::lock_guard<std::mutex> lk(w.mu);
+  if (!w.st) {
+    hipStream_t st = nullptr;
+    void *post = nullptr;
+    u64 *comp = nullptr;
+    hipError_t err = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+    if (err == hipSuccess) err = hipHostMalloc(&post, sizeof(GroupbyPost), hipHostMallocCoherent);
+    if (err == hipSuccess) err = hipMalloc((void **)&comp, sizeof(u64) * (GROUPBY_SMALL + 1));
+    if (err == hipSuccess) err = launch_fill_u64(comp + GROUPBY_SMALL, 1, 0ull, st);
+    if (err != hipSuccess) {
+      if (comp) (void)hipFree(comp);
+      if (post) (void)hipHostFree(post);
+      if (st) (void)hipStreamDestroy(st);
+      return fail(err == hipErrorOutOfMemory ? IBFS_ERR_NOMEM : IBFS_ERR_HIP,
+                  "groupby workspace: %s", hipGetErrorString(err));
+    }
+    std::memset(post, 0, sizeof(GroupbyPost));
+    w.st = st;
+    w.post = post;
+    w.comp = comp;
+    w.ticket = comp + GROUPBY_SMALL;
+  }
+  hipStream_t st = (hipStream_t)w.st;
+  if (w.unsettled) {  // an earlier call's kernel may still read the sources
+    HIP_TRY(hipStreamSynchronize(st));
+    w.unsettled = false;
+  }
+  auto *post = static_cast<GroupbyPost *>(w.post);
+  std::memcpy(post->src, src, sizeof(int32_t) * (size_t)n);
+  const u64 tag = ++w.seq;
+  clear_hip_error();
+  HIP_TRY(launch_groupby_small(g->d_beg, g->d_adj, g->d_deg, g->d_cid, n, post, w.comp,
+                               reinterpret_cast<unsigned *>(w.ticket), tag, st));
+  if (int rc = wait_tag(st, &post->tag, tag, "groupby")) {
+    w.unsettled = true;
+    return rc;
+  }
+  std::memcpy(out, post->out, sizeof(int32_t) * (size_t)n);
+  return IBFS_OK;
+}
+
+extern "C" {
+
 int ibfs_groupby(ibfs_graph_t g, const int32_t *src, int64_t n, int32_t *out) {
   if (!g || (n > 0 && (!src || !out)) || n < 0) return fail(IBFS_ERR_ARG, "ibfs_groupby: bad arguments");
   if (n == 0) return IBFS_OK;
@@ -821,6 +875,7 @@ int ibfs_groupby(ibfs_graph_t g, const int32_t *src, int64_t n, int32_t *out) {
       return fail(IBFS_ERR_ARG, "source %lld = %d out of range", (long long)i, src[i]);
   int rc = check_device(g->device);
   if (rc) return rc;
+  if (n <= GROUPBY_SMALL) return groupby_small(g, src, (int)n, out);
   int32_t *d = nullptr;
   void *ws = nullptr;
   const size_t wsb = groupby_workspace_bytes(n);

@@ -447,6 +447,18 @@ hipError_t launch_two_hop(const int64_t *beg, const int32_t *adj, const int32_t 
 // radix sort (O(n)).  src holds original ids (cid maps them to the traversal
 // CSR); keys are traversal ids, whose order is the original order.  ws: device
 // workspace of groupby_workspace_bytes(n) bytes.
+// Up to GROUPBY_SMALL sources in one launch that reads them from, and posts the
+// order to, coherent pinned host memory.  comp: device workspace of as many
+// words; ticket: a zero word, zero again afterwards.
+constexpr int GROUPBY_SMALL = 4096;
+struct GroupbyPost {
+  int32_t src[GROUPBY_SMALL];
+  int32_t out[GROUPBY_SMALL];
+  u64 tag;
+};
+hipError_t launch_groupby_small(const int64_t *beg, const int32_t *adj, const int32_t *deg,
+                                const int32_t *cid, int n, GroupbyPost *post, u64 *comp,
+                                unsigned *ticket, u64 tag, hipStream_t st);
 size_t groupby_workspace_bytes(int64_t n);
 hipError_t launch_groupby(const int64_t *beg, const int32_t *adj, const int32_t *deg,
                           const int32_t *cid, const int32_t *src, int64_t n, int32_t *key,

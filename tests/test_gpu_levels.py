@@ -107,3 +107,34 @@ def test_closeness_windows(V, ring):
             np.testing.assert_array_equal(reach, want_reach)
             np.testing.assert_array_equal(dsum, want_sum)
             b.close()
+
+
+def test_groupby_sizes_and_threads():
+    """GroupBy around the steps of its sort and its small/large limit, sources
+    with repeats and isolated ones, and four threads on one graph at once."""
+    import threading
+    h = ibfs_amd.HostCsr.rmat(15, 16, seed=5)
+    beg, adj = h.arrays()
+    g = ibfs_amd.DeviceGraph(h)
+    rng = np.random.default_rng(3)
+    for n in (1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 1000, 1024, 1025, 2049, 4095, 4096, 4097):
+        say(f"[gpu] groupby n={n}")
+        src = rng.integers(0, h.vert_count, size=n).astype(np.int32)
+        np.testing.assert_array_equal(g.groupby(src), oracle.groupby(beg, adj, src))
+    lists = [rng.integers(0, h.vert_count, size=700 + i).astype(np.int32) for i in range(4)]
+    got = [[] for _ in lists]
+
+    def work(i):
+        for _ in range(20):
+            got[i].append(g.groupby(lists[i]))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    for src, outs in zip(lists, got):
+        want = oracle.groupby(beg, adj, src)
+        assert len(outs) == 20
+        for o in outs:
+            np.testing.assert_array_equal(o, want)
