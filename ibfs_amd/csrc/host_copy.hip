@@ -11,6 +11,7 @@
 #include "host_copy.h"
 
 #include <algorithm>
+#include <atomic>
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
@@ -24,26 +25,52 @@ namespace ibfs {
 namespace {
 
 constexpr size_t kChunk = size_t(64) << 20;
+// A copy moves in parts of a quarter of it, at least 4 MiB and at most a chunk:
+// the first part's DMA and the last part's copy-out overlap nothing, so a copy
+// of one or two chunks in parts of a whole chunk is not pipelined at all
+// (67 MB with its traversal 2.6 ms, in quarters 1.9 ms).
+constexpr size_t kMinPart = size_t(4) << 20;
 constexpr int kThreads = 8;
 // copies below this size keep the runtime's path (no pipeline to fill)
 constexpr size_t kDirect = size_t(4) << 20;
 
-// Host threads that copy one buffer in kThreads slices; copy() returns when
-// every slice is done.  The threads live as long as the process.
+// Host threads that copy the parts of one transfer, each thread its slice of
+// every part.  They are woken once per transfer and then spin for the next part
+// (a wake-up of eight sleeping threads costs about as much as copying 8 MB);
+// between transfers they sleep.  They live as long as the process.
 class CopyPool {
  public:
+  struct Part {
+    char *dst;
+    const char *src;
+    size_t bytes;
+    std::atomic<int> left{kThreads};
+  };
+
   CopyPool() {
     for (int k = 0; k < kThreads; ++k) th_.emplace_back([this, k] { run(k); });
   }
 
-  void copy(void *dst, const void *src, size_t bytes) {
-    std::unique_lock<std::mutex> lk(mu_);
-    dst_ = static_cast<char *>(dst);
-    src_ = static_cast<const char *>(src);
-    bytes_ = bytes;
+  // Starts a transfer of n parts; part j is copied once ready(j + 1) was called.
+  void begin(Part *parts, int n) {
+    std::lock_guard<std::mutex> lk(mu_);
+    parts_ = parts;
+    n_ = n;
+    ready_.store(0, std::memory_order_relaxed);
     left_ = kThreads;
     ++gen_;
     go_.notify_all();
+  }
+  void ready(int n) { ready_.store(n, std::memory_order_release); }
+  void wait_part(int j) {
+    for (unsigned i = 1; parts_[j].left.load(std::memory_order_acquire) > 0; ++i)
+      if ((i & 255) == 0) std::this_thread::yield();
+  }
+  // Ends the transfer (parts not yet ready are dropped): no thread touches
+  // the parts afterwards.
+  void end() {
+    ready_.store(-1, std::memory_order_release);
+    std::unique_lock<std::mutex> lk(mu_);
     done_.wait(lk, [this] { return left_ == 0; });
   }
 
@@ -51,19 +78,28 @@ class CopyPool {
   void run(int k) {
     uint64_t seen = 0;
     for (;;) {
-      char *d;
-      const char *s;
-      size_t b;
+      Part *p;
+      int n;
       {
         std::unique_lock<std::mutex> lk(mu_);
         go_.wait(lk, [&] { return gen_ != seen; });
         seen = gen_;
-        d = dst_;
-        s = src_;
-        b = bytes_;
+        p = parts_;
+        n = n_;
       }
-      const size_t lo = b * (size_t)k / kThreads, hi = b * (size_t)(k + 1) / kThreads;
-      if (hi > lo) std::memcpy(d + lo, s + lo, hi - lo);
+      for (int j = 0; j < n; ++j) {
+        int r = 0;
+        for (unsigned i = 1;; ++i) {
+          r = ready_.load(std::memory_order_acquire);
+          if (r > j || r < 0) break;
+          if ((i & 255) == 0) std::this_thread::yield();
+        }
+        if (r < 0) break;
+        const size_t b = p[j].bytes;
+        const size_t lo = b * (size_t)k / kThreads, hi = b * (size_t)(k + 1) / kThreads;
+        if (hi > lo) std::memcpy(p[j].dst + lo, p[j].src + lo, hi - lo);
+        p[j].left.fetch_sub(1, std::memory_order_release);
+      }
       std::lock_guard<std::mutex> lk(mu_);
       if (--left_ == 0) done_.notify_one();
     }
@@ -72,9 +108,9 @@ class CopyPool {
   std::vector<std::thread> th_;
   std::mutex mu_;
   std::condition_variable go_, done_;
-  char *dst_ = nullptr;
-  const char *src_ = nullptr;
-  size_t bytes_ = 0;
+  Part *parts_ = nullptr;
+  int n_ = 0;
+  std::atomic<int> ready_{0};
   int left_ = 0;
   uint64_t gen_ = 0;
 };
@@ -143,41 +179,51 @@ int copy_to_host(const D2HPiece *pieces, size_t n, hipStream_t st) {
       return copy_direct(pieces, n, st);  // no threads: the runtime's path
     }
   }
-  // the pieces cut into chunk-sized parts, copied in order
+  // the pieces cut into parts, copied in order
   std::vector<D2HPiece> q;
+  const size_t part =
+      std::min(kChunk, std::max(kMinPart, (total / 4 + 4095) & ~(size_t)4095));
   for (size_t i = 0; i < n; ++i)
-    for (size_t off = 0; off < pieces[i].bytes; off += kChunk)
+    for (size_t off = 0; off < pieces[i].bytes; off += part)
       q.push_back({static_cast<char *>(pieces[i].dst) + off,
                    static_cast<const char *>(pieces[i].src) + off,
-                   std::min(kChunk, pieces[i].bytes - off)});
+                   std::min(part, pieces[i].bytes - off)});
   hipEvent_t ev[2] = {nullptr, nullptr};
   hipError_t e = hipEventCreateWithFlags(&ev[0], hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[1], hipEventDisableTiming);
   int rc = e == hipSuccess ? IBFS_OK
                            : fail(IBFS_ERR_HIP, "copy to host: %s", hipGetErrorString(e));
-  // part j goes to chunk j & 1; that chunk's previous part (j - 2) was copied
-  // out before part j - 1 was waited for, so the DMA never overwrites data
+  // part j goes to chunk j & 1; that chunk's previous part (j - 2) has been
+  // copied out before its DMA is issued, so the DMA never overwrites data
   // still being read
+  std::vector<CopyPool::Part> parts(q.size());
+  for (size_t j = 0; j < q.size(); ++j) {
+    parts[j].dst = static_cast<char *>(q[j].dst);
+    parts[j].src = s.pin + (j & 1) * kChunk;
+    parts[j].bytes = q[j].bytes;
+  }
+  s.pool->begin(parts.data(), (int)q.size());
   size_t issued = 0;
-  for (size_t j = 0; rc == IBFS_OK && j < q.size(); ++j) {
-    char *slot = s.pin + (j & 1) * kChunk;
-    e = hipMemcpyAsync(slot, q[j].src, q[j].bytes, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipEventRecord(ev[j & 1], st);
-    if (e != hipSuccess) {
-      rc = fail(IBFS_ERR_HIP, "copy to host: %s", hipGetErrorString(e));
-      break;
+  for (size_t j = 0; rc == IBFS_OK && j <= q.size(); ++j) {
+    if (j < q.size()) {
+      if (j >= 2) s.pool->wait_part((int)j - 2);
+      e = hipMemcpyAsync(s.pin + (j & 1) * kChunk, q[j].src, q[j].bytes, hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipEventRecord(ev[j & 1], st);
+      if (e != hipSuccess) {
+        rc = fail(IBFS_ERR_HIP, "copy to host: %s", hipGetErrorString(e));
+        break;
+      }
+      issued = j + 1;
     }
-    issued = j + 1;
     if (j >= 1) {
       rc = wait_event(ev[(j - 1) & 1]);
-      if (rc == IBFS_OK) s.pool->copy(q[j - 1].dst, s.pin + ((j - 1) & 1) * kChunk, q[j - 1].bytes);
+      if (rc == IBFS_OK) s.pool->ready((int)j);
     }
   }
-  if (rc == IBFS_OK) {
-    const size_t last = q.size() - 1;
-    rc = wait_event(ev[last & 1]);
-    if (rc == IBFS_OK) s.pool->copy(q[last].dst, s.pin + (last & 1) * kChunk, q[last].bytes);
-  } else if (issued > 0) {
+  if (rc == IBFS_OK)
+    for (size_t j = q.size() < 2 ? 0 : q.size() - 2; j < q.size(); ++j) s.pool->wait_part((int)j);
+  s.pool->end();
+  if (rc != IBFS_OK && issued > 0) {
     // An error part-way (a failed copy or a wait past the limit): DMA already
     // issued may still write the chunks, and waiting for it could outlast the
     // limit.  The chunks are abandoned, never freed, and the next pipelined

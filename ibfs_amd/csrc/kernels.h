@@ -383,7 +383,7 @@ struct NextArgs {
   CtlSpread *spread_old;    // those of the level before it, folded already
   LevelCtl *ctl;            // its control block
   const LevelCtl *ctl_prev; // that of the level before it (null at level 0)
-  CtlPost *post;
+  CtlPost *post;            // (or null)
   u64 post_tag;
 };
 hipError_t launch_expand_next(int W, const GraphDev &g, const u64 *prev, u64 *cur, const u64 *hs,

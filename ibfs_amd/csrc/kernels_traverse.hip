@@ -1383,11 +1383,13 @@ __global__ __launch_bounds__(BS) void k_expand_next(GraphDev g, const u64 *prev,
     if (t < (int)CTL_WORDS) {
       const u64 x = reinterpret_cast<const u64 *>(&c)[t];
       reinterpret_cast<u64 *>(n.ctl)[t] = x;
-      __hip_atomic_store(&reinterpret_cast<u64 *>(&n.post->c)[t], x, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_SYSTEM);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (t == 0)
-        __hip_atomic_store(&n.post->tag, n.post_tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      if (n.post) {
+        __hip_atomic_store(&reinterpret_cast<u64 *>(&n.post->c)[t], x, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (t == 0)
+          __hip_atomic_store(&n.post->tag, n.post_tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
     }
   }
   if (c.next_dir < 0) return;

@@ -1,9 +1,8 @@
 // Allocation-free traversal: one group of up to 128 sources with every
 // scratch buffer (status snapshots, queues, control blocks, hub cache,
-// changed flags, lane table, masks, plan, edge counter) in one file-scope
-// device array, and the device-driven level loop (captured-level kernels
-// launched directly on the null stream, direction decided on the device,
-// the host reading only the plan's head between bursts).  For callers that
+// changed flags, lane table, masks, edge counter) in one file-scope device
+// array, and levels enqueued eight at a time on the null stream (direction
+// decided on the device, the host reading the control blocks in between).  For callers that
 // cannot allocate: code under HIP graph capture, tight serving loops,
 // harnesses that forbid allocation.
 #include <hip/hip_runtime.h>
@@ -29,7 +28,8 @@ constexpr int NA_K = 64 * NA_W;
 constexpr int64_t NA_VT = int64_t(1) << 18;
 constexpr int64_t NA_E = int64_t(1) << 24;
 constexpr int64_t NA_H = 131072;
-constexpr int NA_R = 8;
+constexpr int NA_R = 8;       // at the vertex limit and 128 lanes; smaller graphs keep more
+constexpr int NA_RMAX = 32;
 constexpr int NA_MIN_CHUNK_SHIFT = 11;
 
 constexpr size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -38,7 +38,7 @@ constexpr size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 constexpr size_t OFF_RING = 0;
 constexpr size_t SZ_RING = size_t(NA_R) * NA_VT * NA_W * sizeof(u64);
 constexpr size_t OFF_CTL = OFF_RING + up256(SZ_RING);
-constexpr size_t SZ_CTL = ctl_ring_bytes(NA_R);
+constexpr size_t SZ_CTL = ctl_ring_bytes(NA_RMAX);
 constexpr size_t OFF_Q = OFF_CTL + up256(SZ_CTL);
 constexpr size_t SZ_Q1 = up256(queue_entries(NA_VT) * sizeof(int32_t));
 constexpr size_t OFF_CHUNKS = OFF_Q + (NQ - 1) * SZ_Q1;
@@ -48,11 +48,10 @@ constexpr size_t SZ_HS = size_t(NA_H) * NA_W * sizeof(u64);
 constexpr size_t OFF_FLAGS = OFF_HS + up256(SZ_HS);
 constexpr size_t SZ_FLAGS = size_t(NA_VT);
 constexpr size_t OFF_MASKS = OFF_FLAGS + up256(SZ_FLAGS);
-constexpr size_t SZ_MASKS = size_t(2 + NA_R + 1) * NA_W * sizeof(u64);
+constexpr size_t SZ_MASKS = size_t(2 + NA_RMAX + 1) * NA_W * sizeof(u64);
 constexpr size_t OFF_LANES = OFF_MASKS + up256(SZ_MASKS);
 constexpr size_t SZ_LANES = size_t(NA_K) * sizeof(LaneOut);
-constexpr size_t OFF_PLAN = OFF_LANES + up256(SZ_LANES);
-constexpr size_t OFF_COUNT = OFF_PLAN + up256(sizeof(Plan));
+constexpr size_t OFF_COUNT = OFF_LANES + up256(SZ_LANES);
 constexpr size_t NA_BYTES = OFF_COUNT + 256;
 static_assert(NA_BYTES == IBFS_NOALLOC_SCRATCH_BYTES, "scratch size in ibfs.h");
 
@@ -60,31 +59,6 @@ static_assert(NA_BYTES == IBFS_NOALLOC_SCRATCH_BYTES, "scratch size in ibfs.h");
 // device address: host code uses only the per-device address from
 // hipGetSymbolAddress (scratch_ptr below).
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
-
-struct PlanInit {
-  int policy, sw_level, alpha, beta, gamma, rho;
-  u64 V;
-};
-
-// Plan of one traversal before its level 0.  One wave.
-__global__ void k_noalloc_plan(Plan *plan, PlanInit pi) {
-  const int t = threadIdx.x;
-  for (int i = t; i < (int)(sizeof(Plan) / 4); i += blockDim.x)
-    reinterpret_cast<uint32_t *>(plan)[i] = 0;
-  __syncthreads();
-  if (t == 0) {
-    plan->policy = pi.policy;
-    plan->sw_level = pi.sw_level;
-    plan->alpha = pi.alpha;
-    plan->beta = pi.beta;
-    plan->gamma = pi.gamma;
-    plan->rho = pi.rho;
-    plan->split_cov = 0;
-    plan->nf_prev = ~0ull;
-    plan->V = pi.V;
-    plan->dir = -1;
-  }
-}
 
 std::mutex g_mu;  // one traversal at a time per process (the array is shared)
 std::vector<unsigned char *> g_ptr;  // per device: the array's device address
@@ -126,10 +100,6 @@ int wait_null_stream() {
   }
 }
 
-struct PlanHead {  // the first members of Plan
-  int level, dir, done, last;
-};
-
 int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int32_t *dout,
         int64_t *edges) {
   int dev = 0;
@@ -137,8 +107,9 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   unsigned char *base = nullptr;
   if (int rc = scratch_ptr(dev, &base)) return rc;
   const int W = k <= 64 ? 1 : 2;
-  const int R = NA_R;
   const int64_t V = g->V, Vt = g->Vt;
+  const int R = (int)std::min<int64_t>(
+      NA_RMAX, (int64_t)(SZ_RING / sizeof(u64)) / std::max<int64_t>(Vt * W, 1));
   u64 *ring = reinterpret_cast<u64 *>(base + OFF_RING);
   LevelCtl *ctl = reinterpret_cast<LevelCtl *>(base + OFF_CTL);
   Queues q{};
@@ -149,7 +120,6 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   uint8_t *flags = base + OFF_FLAGS;
   u64 *masks = reinterpret_cast<u64 *>(base + OFF_MASKS);
   LaneOut *lanes = reinterpret_cast<LaneOut *>(base + OFF_LANES);
-  Plan *plan = reinterpret_cast<Plan *>(base + OFF_PLAN);
   u64 *count = reinterpret_cast<u64 *>(base + OFF_COUNT);
   const HubCut hc = hub_cut(g, cfg.hybrid_hubs);
   const GraphDev gd = graph_dev(g, cfg, hc);
@@ -157,7 +127,7 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       cus <= 0)
     cus = 256;
-  const int grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 32;
+  const int grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 4;  // as the engine's levels enqueued ahead
   hipStream_t st = nullptr;  // the null stream: nothing to create
 
   // the previous call's contents stay in the array: clear what starts at zero
@@ -171,38 +141,54 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
   NA_TRY(launch_group_start(W, sl, g->d_cid, dout, V, Vt, ring, flags,
                             reinterpret_cast<u64 *>(ctl), (int64_t)(ctl_ring_bytes(R) / 8), lanes,
                             masks, R, count, st));
-  const PlanInit pi{cfg.policy, cfg.sw_level, cfg.alpha, cfg.beta, cfg.hybrid_gamma, hc.rho_q10,
-                    (u64)V};
-  hipLaunchKernelGGL(k_noalloc_plan, dim3(1), dim3(64), 0, st, plan, pi);
-  NA_TRY(hipGetLastError());
-
-  InspectArgs a{};
-  a.deg = g->d_deg;
-  a.V = Vt;
-  a.q = q;
-  a.sml = cfg.sml_shed;
-  a.lrg = cfg.lrg_shed;
-  a.chunk_shift = gd.chunk_shift;
-  a.chunk_extra = (unsigned)(g->E >> gd.chunk_shift) + 1;
-  a.hubs = g->d_hubs;
-  a.H = g->H;
-  a.hs = hs;
-  a.plan = plan;
-  a.ring = ring;
-  a.R = R;
-  a.ctl_ring = ctl;
-  a.lanes_all = masks;
-  a.flags = flags;
-  a.vpt = cfg.inspect_vpt;
-  a.nw = cfg.wg_size / 64;
-  a.hsplit = gd.hsp;
-  a.spread = ctl_spread(ctl, R);
-  a.decide = 1;
-  NA_TRY(launch_inspect(W, a, st));
+  CtlSpread *spread = ctl_spread(ctl, R);
+  auto dec = [&](int L) {
+    return Decide{2, L, cfg.policy, cfg.sw_level, cfg.alpha, cfg.beta, cfg.hybrid_gamma, hc.rho_q10,
+                  (u64)V};
+  };
+  auto slot = [&](int L) { return ring + (int64_t)(L % R) * Vt * W; };
+  auto inspect = [&](int L) {
+    InspectArgs a{};
+    a.full_diff = 1;
+    a.prev = L > 0 ? slot(L - 1) : nullptr;
+    a.cur = slot(L);
+    a.next = slot(L + 1);
+    a.ctl = ctl + L % R;
+    a.ctl_zero = ctl + (L + 1) % R;
+    a.ctl_prev = L > 0 ? ctl + (L - 1) % R : nullptr;
+    a.lam_prev = L > 0 ? a.ctl_prev->lam : masks;
+    a.dec = dec(L);
+    a.deg = g->d_deg;
+    a.V = Vt;
+    a.q = q;
+    a.sml = cfg.sml_shed;
+    a.lrg = cfg.lrg_shed;
+    a.chunk_shift = gd.chunk_shift;
+    a.chunk_extra = (unsigned)(g->E >> gd.chunk_shift) + 1;
+    a.hubs = g->d_hubs;
+    a.H = g->H;
+    a.hs = hs;
+    a.flags = flags;
+    a.vpt = cfg.inspect_vpt;
+    a.nw = cfg.wg_size / 64;
+    a.hsplit = gd.hsp;
+    a.spread = spread + (L & 1);
+    return launch_inspect(W, a, st);
+  };
+  auto expand = [&](int L) {
+    NextArgs n{};
+    n.dec = dec(L - 1);
+    n.spread = spread + ((L - 1) & 1);
+    n.spread_old = spread + (L & 1);
+    n.ctl = ctl + (L - 1) % R;
+    n.ctl_prev = L > 1 ? ctl + (L - 2) % R : nullptr;
+    return launch_expand_next(W, gd, slot(L - 1), slot(L), hs, flags, n, q, grid, st);
+  };
+  NA_TRY(inspect(0));
 
   const EmitSpace sp{g->d_cid, V, Vt, g->d_deg};
   const int vec4 = (V % 4 == 0) && ((uintptr_t)dout % 16 == 0);
-  int level = 1, lo = 0;
+  int level = 1, lo = 0;  // next level to enqueue, base of the emission window
   for (;;) {
     int B = std::min(8, R - 1 - (level - lo));
     if (B < 1) {  // the next levels would overwrite S_lo: emit [lo, level-1]
@@ -211,20 +197,24 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
       lo = level - 1;
       B = std::min(8, R - 1 - (level - lo));
     }
-    for (int i = 0; i < B; ++i) {
-      NA_TRY(launch_expand_dd(W, gd, ring, flags, R, ctl, plan, hs, q, TailLog{}, grid, st));
-      NA_TRY(launch_inspect(W, a, st));
+    for (int i = 0; i < B; ++i, ++level) {
+      NA_TRY(expand(level));
+      NA_TRY(inspect(level));
     }
     if (int rc = wait_null_stream()) return rc;
-    PlanHead ph{};
-    NA_TRY(hipMemcpy(&ph, plan, sizeof ph, hipMemcpyDeviceToHost));
-    if (ph.done) {
-      if (ph.last >= lo)
-        NA_TRY(launch_emit(W, cfg.emit_mode, vec4, ring, R, sp, lo, ph.last, lanes, masks + 2 * W,
+    // the expansion of level-1 folded the counters of level-2: whether a level
+    // up to that one changed nothing, and the first that did
+    LevelCtl h[NA_RMAX];
+    NA_TRY(hipMemcpy(h, ctl, sizeof(LevelCtl) * (size_t)R, hipMemcpyDeviceToHost));
+    if (h[(level - 2) % R].next_dir < 0) {
+      int end = level - 2;
+      while (end > 0 && end > level - 1 - B && h[(end - 1) % R].next_dir < 0) --end;
+      const int last = end > 0 ? end - 1 : 0;
+      if (last >= lo)
+        NA_TRY(launch_emit(W, cfg.emit_mode, vec4, ring, R, sp, lo, last, lanes, masks + 2 * W,
                            masks + W, k, edges ? count : nullptr, iso, st));
       else if (edges)  // no final window: count over S_last
-        NA_TRY(launch_count_edges(W, ring + (int64_t)(ph.last % R) * Vt * W, g->d_deg, Vt, masks,
-                                  count, st));
+        NA_TRY(launch_count_edges(W, slot(last), g->d_deg, Vt, masks, count, st));
       if (int rc = wait_null_stream()) return rc;
       if (edges) {
         u64 c = 0;
@@ -234,8 +224,7 @@ int run(ibfs_graph_s *g, const ibfs_config &cfg, const int32_t *src, int k, int3
       }
       return IBFS_OK;
     }
-    if (ph.level > Vt + 2) return fail(IBFS_ERR_STATE, "traversal exceeded V+2 levels");
-    level = ph.level;
+    if (level > Vt + 2 + B) return fail(IBFS_ERR_STATE, "traversal exceeded V+2 levels");
   }
 }
 

@@ -138,3 +138,26 @@ def test_groupby_sizes_and_threads():
         assert len(outs) == 20
         for o in outs:
             np.testing.assert_array_equal(o, want)
+
+
+@pytest.mark.parametrize("rows,cols,n", [(512, 512, 70), (40, 300, 128), (1, 50, 1)])
+def test_noalloc_levels_enqueued_in_bursts(rows, cols, n):
+    """Grids through the allocation-free call: at the vertex limit its ring
+    holds 8 snapshots and is flushed over a hundred times, smaller graphs keep
+    up to 32; traversals that end anywhere in a burst of eight levels."""
+    say(f"[gpu] noalloc grid {rows}x{cols}")
+    v = np.arange(rows * cols).reshape(rows, cols)
+    beg, adj = _symmetric(rows * cols, np.concatenate([v[:, :-1].ravel(), v[:-1].ravel()]),
+                          np.concatenate([v[:, 1:].ravel(), v[1:].ravel()]))
+    g = ibfs_amd.DeviceGraph(ibfs_amd.HostCsr.from_arrays(beg, adj))
+    out = ibfs_amd.DeviceBuffer(4 * n * rows * cols)
+    src = np.random.default_rng(rows).integers(0, rows * cols, size=n).astype(np.int32)
+    want = oracle.bfs_many(beg, adj, src, threads=8)
+    edges = g.traversal_noalloc(src, out)
+    np.testing.assert_array_equal(out.to_host().reshape(n, -1), want)
+    assert edges == sum(oracle.traversed_edges(beg, d) for d in want)
+    for k in range(1, min(cols, 20)):  # one source ever closer to the end
+        s = np.array([rows * cols - k], dtype=np.int32)
+        g.traversal_noalloc(s, out)
+        np.testing.assert_array_equal(out.to_host(count=rows * cols),
+                                      oracle.bfs_many(beg, adj, s, threads=1)[0])
