@@ -110,6 +110,22 @@ __device__ __forceinline__ int32_t lane_depth(const u64 (&c)[NS][W], const u64 (
   return (set && !at_base) ? off + cnt : SKIP;
 }
 
+// From four counter planes of 32 lanes and their final word: depth + 1, and 0
+// where the bit never arrived, as nibbles: nibble q of n[m] is lane 4q + m.
+// One shift and one and-or serve eight lanes of a plane; four extracts per
+// lane take three times the instructions.
+__device__ __forceinline__ void depth_nibbles(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
+                                              uint32_t f, uint32_t (&n)[4]) {
+  const uint32_t p[4] = {~c0 & f, (c1 ^ c0) & f, (c2 ^ (c1 & c0)) & f, (c3 ^ (c2 & c1 & c0)) & f};
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    n[m] = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      n[m] |= (j >= m ? p[j] << (j - m) : p[j] >> (m - j)) & (0x11111111u << j);
+  }
+}
+
 // Stores of one vertex's depths when every selected lane is in its first
 // window and the window has fewer than 16 levels (4 counter bits): the lane
 // loop is unrolled over 32-bit halves of the words, so each bit position is
@@ -133,21 +149,19 @@ __device__ __forceinline__ void emit_first4(const u64 (&c)[4][W], const u64 (&fi
       const uint32_t c0 = (uint32_t)(c[0][w] >> (32 * h)), c1 = (uint32_t)(c[1][w] >> (32 * h));
       const uint32_t c2 = (uint32_t)(c[2][w] >> (32 * h)), c3 = (uint32_t)(c[3][w] >> (32 * h));
       const uint32_t f = (uint32_t)(fin[w] >> (32 * h));
+      uint32_t n[4];
+      depth_nibbles(c0, c1, c2, c3, f, n);
 #pragma unroll
       for (int g = 0; g < 32; g += 8) {
         int32_t *o[8];
-        int32_t d[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = s_out[w * 64 + h * 32 + g + i];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int bt = g + i;
-          o[i] = s_out[w * 64 + h * 32 + bt];
-          const uint32_t cnt = ((c0 >> bt) & 1u) | (((c1 >> bt) & 1u) << 1) |
-                               (((c2 >> bt) & 1u) << 2) | (((c3 >> bt) & 1u) << 3);
-          d[i] = (int32_t)(cnt | (((f >> bt) & 1u) - 1u));
+          const int32_t d = (int32_t)((n[bt & 3] >> (4 * (bt >> 2))) & 15u) - 1;
+          if (o[i]) put_depth(o[i], v, d, nt);
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (o[i]) put_depth(o[i], v, d[i], nt);
       }
     }
   }
@@ -173,8 +187,13 @@ __global__ __launch_bounds__(BS) void k_emit(const u64 *__restrict__ ring, int R
     cont |= on && s_off[i] > 0;
   }
   const bool fast = NS == 4 && !__syncthreads_or(cont);
-  for (int64_t v = (int64_t)blockIdx.x * BS + threadIdx.x; v < sp.V;
-       v += (int64_t)gridDim.x * BS) {
+  // Workgroups go to the 8 XCDs in turn: XCD x takes the x-th eighth of the
+  // vertices, so neighbouring 1-KB pieces of a row, which share a cache line
+  // where the row is not aligned, are written through one L2 and leave it whole.
+  const int64_t per = ((sp.V + BS - 1) / BS + 7) / 8;
+  for (int64_t i = blockIdx.x; i < 8 * per; i += gridDim.x) {
+    const int64_t v = ((i & 7) * per + (i >> 3)) * BS + threadIdx.x;
+    if (v >= sp.V) continue;
     const int32_t ci = sp.cid[v];
     const bool iso = ci < 0;
     u64 c[NS][W], fin[W], bs[W];
@@ -312,7 +331,8 @@ __global__ __launch_bounds__(BS) void k_emit_tiled(const u64 *__restrict__ ring,
 // per-vertex state is NS+2 words of those four vertices and every store
 // instruction writes 16 bytes per thread: one lane's 256 depths as a single
 // 1-KB contiguous piece of its row (k_emit writes 256-byte pieces, one
-// vertex per thread).  The waves of a workgroup take consecutive (chunk,
+// vertex per thread).  Where every lane is in its first window of fewer than
+// 16 levels, depths come from nibbles as in k_emit.  The waves of a workgroup take consecutive (chunk,
 // word) units, so the words of one vertex are read by neighbouring waves
 // from the same lines.  A lane row that is not 16-byte aligned, a chunk
 // that ends past V, and a piece holding an entry a continuation window must
@@ -342,19 +362,24 @@ __global__ __launch_bounds__(BS) void k_emit_wide(const u64 *__restrict__ ring, 
   __shared__ int32_t s_src[MAX_LANES];
   __shared__ u64 red[BS / 64];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  for (int i = t; i < k_lanes; i += BS) {
-    const bool on = (sel[i >> 6] >> (i & 63)) & 1ull;
+  int cont = 0;  // some selected lane continues an earlier window
+  for (int i = t; i < W * 64; i += BS) {  // null past the group
+    const bool on = i < k_lanes && ((sel[i >> 6] >> (i & 63)) & 1ull);
     s_out[i] = on ? lanes[i].out : nullptr;
-    s_off[i] = b - lanes[i].admit;
-    s_src[i] = lanes[i].src;
+    s_off[i] = on ? b - lanes[i].admit : 0;
+    s_src[i] = on ? lanes[i].src : -1;
+    cont |= on && s_off[i] > 0;
   }
-  __syncthreads();
+  const bool fast = NS == 4 && !__syncthreads_or(cont);
   const int64_t V = sp.V, slot = sp.Vt * W;
   const bool v4 = (V & 3) == 0;
+  // XCD shares as in k_emit, by workgroups of four units
   const int64_t units = ((V + 255) >> 8) * W;
+  const int64_t per = ((units + BS / 64 - 1) / (BS / 64) + 7) / 8;
   u64 acc = 0;
-  for (int64_t u = (int64_t)blockIdx.x * (BS / 64) + wv; u < units;
-       u += (int64_t)gridDim.x * (BS / 64)) {
+  for (int64_t g = blockIdx.x; g < 8 * per; g += gridDim.x) {
+    const int64_t u = ((g & 7) * per + (g >> 3)) * (BS / 64) + wv;
+    if (u >= units) continue;
     const int64_t chunk = u / W;
     const int w = (int)(u % W);
     const int64_t v0 = chunk * 256 + 4 * lane;
@@ -369,27 +394,30 @@ __global__ __launch_bounds__(BS) void k_emit_wide(const u64 *__restrict__ ring, 
       for (int j = 0; j < NS; ++j) c[j][i] = 0;
     }
     const u64 *Sw = ring + w;
+    constexpr int NB = 4;  // levels loaded before any of them is counted
+    for (int L0 = b; L0 <= e; L0 += NB) {
+      u64 x[NB][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (ci[i] >= 0) {
-        fin[i] = Sw[(int64_t)(e % R) * slot + (int64_t)ci[i] * W];
-        bs[i] = Sw[(int64_t)(b % R) * slot + (int64_t)ci[i] * W];
+      for (int k = 0; k < NB; ++k) {
+        const u64 *S = Sw + (int64_t)((L0 + k) % R) * slot;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[k][i] = ci[i] >= 0 && L0 + k <= e ? S[(int64_t)ci[i] * W] : ~0ull;
       }
-    }
-    for (int L = b; L <= e; ++L) {
-      const u64 lm = level_masks[(int64_t)(L - b) * W + w];
-      const u64 *S = Sw + (int64_t)(L % R) * slot;
-      u64 x[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = ci[i] >= 0 ? S[(int64_t)ci[i] * W] : ~0ull;
+      for (int k = 0; k < NB; ++k) {
+        if (L0 + k > e) break;
+        const u64 lm = level_masks[(int64_t)(L0 + k - b) * W + w];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        u64 carry = ~x[i] & lm;
+        for (int i = 0; i < 4; ++i) {
+          if (L0 + k == b) bs[i] = ci[i] >= 0 ? x[k][i] : 0;
+          if (L0 + k == e) fin[i] = ci[i] >= 0 ? x[k][i] : 0;
+          u64 carry = ~x[k][i] & lm;
 #pragma unroll
-        for (int j = 0; j < NS; ++j) {
-          const u64 nc = c[j][i] & carry;
-          c[j][i] ^= carry;
-          carry = nc;
+          for (int j = 0; j < NS; ++j) {
+            const u64 nc = c[j][i] & carry;
+            c[j][i] ^= carry;
+            carry = nc;
+          }
         }
       }
     }
@@ -397,6 +425,45 @@ __global__ __launch_bounds__(BS) void k_emit_wide(const u64 *__restrict__ ring, 
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (ci[i] >= 0) acc += (u64)__popcll(fin[i] & sel[w]) * (u64)sp.deg[ci[i]];
+    }
+    if constexpr (NS == 4) {
+      if (fast) {
+        typedef int v4u __attribute__((ext_vector_type(4), aligned(4)));
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // as in emit_first4
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          uint32_t n[4][4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            depth_nibbles((uint32_t)(c[0][i] >> (32 * h)), (uint32_t)(c[1][i] >> (32 * h)),
+                          (uint32_t)(c[2][i] >> (32 * h)), (uint32_t)(c[3][i] >> (32 * h)),
+                          (uint32_t)(fin[i] >> (32 * h)), n[i]);
+#pragma unroll
+          for (int q = 0; q < 32; q += 8) {
+            int32_t *o[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o[i] = s_out[w * 64 + h * 32 + q + i];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+              if (!o[r]) continue;
+              const int bt = q + r;
+              v4u x;
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                x[i] = (int32_t)((n[i][bt & 3] >> (4 * (bt >> 2))) & 15u) - 1;
+              gint32 *at = (gint32 *)o[r] + v0;
+              if (v0 + 3 < V) {
+                *(__attribute__((address_space(1))) v4u *)at = x;
+              } else {
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                  if (v0 + i < V) at[i] = x[i];
+              }
+            }
+          }
+        }
+        continue;
+      }
     }
     for (int bit = 0; bit < 64; ++bit) {
       const int k = w * 64 + bit;
@@ -742,6 +809,17 @@ __global__ void k_groupby_sortkey(const int32_t *__restrict__ key, int64_t n,
 #define IBFS_EMIT_GRID_CAP 65536
 #endif
 
+// Whether mode 0 takes the wide-store kernel.  Rows that do not start on cache
+// lines (V % 32): a 256-byte piece of a wave then covers three lines instead
+// of two, a 1-KB piece nine instead of eight (1,000,003 vertices, 512 rows: 256
+// lanes 0.57 -> 0.54 ms, 128 lanes 0.474 -> 0.463).  One status word: few
+// stores per vertex repay its reads (R-MAT s22, 512 rows: 2.13 -> 1.94 ms).
+// Otherwise one vertex per thread reads each word once (256 lanes 1.94 ms
+// against 2.01; 512 lanes 1.98 against 2.40, and not taken there at all).
+static bool emit_wide_is_faster(int W, int NS, int64_t V) {
+  return NS == 4 && (W == 1 || (W <= 4 && V % 32 != 0));
+}
+
 template <int W, int NS>
 static void emit_ns(int mode, int vec4, const u64 *ring, int R, EmitSpace sp, int b, int e,
                     const LaneOut *lanes, const u64 *masks, const u64 *sel, int k, u64 *edges_out,
@@ -755,13 +833,17 @@ static void emit_ns(int mode, int vec4, const u64 *ring, int R, EmitSpace sp, in
       hipLaunchKernelGGL(k_count_edges<W>, gc, blk, 0, st, ring + (int64_t)(e % R) * sp.Vt * W,
                          sp.deg, sp.Vt, sel, edges_out);
     }
-  } else if (mode == 3) {
+  } else if (mode == 3 || (mode == 0 && emit_wide_is_faster(W, NS, sp.V))) {
     const int64_t units = ((sp.V + 255) >> 8) * W;
-    dim3 g(grid_for(units, BS / 64, IBFS_EMIT_GRID_CAP)), blk(BS);
+    dim3 g(8 * grid_for(units, 8 * BS / 64, IBFS_EMIT_GRID_CAP / 8)), blk(BS);
     hipLaunchKernelGGL((k_emit_wide<W, NS>), g, blk, 0, st, ring, R, sp, b, e, lanes, masks, sel,
                        k, edges_out);
+    if (NS == 4 && iso)  // as below
+      hipLaunchKernelGGL(k_emit_iso_sources, dim3((k + BS - 1) / BS), dim3(BS), 0, st, lanes, sel,
+                         sp.cid, b, k);
   } else {
-    dim3 g(grid_for(sp.V, BS, IBFS_EMIT_GRID_CAP)), blk(BS);
+    // a multiple of 8: a workgroup's pieces stay in its XCD's share
+    dim3 g(8 * grid_for(sp.V, 8 * BS, IBFS_EMIT_GRID_CAP / 8)), blk(BS);
     hipLaunchKernelGGL((k_emit<W, NS>), g, blk, 0, st, ring, R, sp, b, e, lanes, masks, sel, k,
                        mode == 2 ? 1 : 0, edges_out);
     if (NS == 4 && iso)  // depth 0 at isolated sources after the fast path's -1

@@ -70,7 +70,7 @@ typedef struct ibfs_config {
   int32_t work_model;  /* 1: measure each bottom-up level's early-termination
                           prefix into the level log (instrumentation)        */
   int32_t emit_mode;   /* depth emission: 0 one vertex per thread, 4-byte
-                          stores; 1 LDS-tiled; 2 as 0 with non-temporal
+                          stores, or as 3 where that is faster; 1 LDS-tiled; 2 as 0 with non-temporal
                           stores; 3 one status word of 256 vertices per wave,
                           1-KB pieces of each lane's row per store           */
   int32_t dd_grid;     /* workgroups of the device-driven expander (0: auto)  */
