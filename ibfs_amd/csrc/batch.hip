@@ -515,9 +515,13 @@ int ibfs_batch_create(ibfs_graph_t g, const ibfs_config *cfg_in, int32_t context
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device) != hipSuccess ||
       cus <= 0)
     cus = 256;
-  // 32 workgroups per CU: a fixed grid strides over the queues, and fewer
-  // workgroups leave too few gathers in flight (measured on R-MAT s22)
-  b->grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 32;
+  // Four workgroups per CU, about what is resident together: a fixed grid strides
+  // over the queues, and every workgroup beyond that costs a launch and a look at
+  // the level's counters also where the level is nearly empty.  1,024 workgroups
+  // against 8,192: closeness of 4,096 sources on R-MAT s16 2.47 ms, 2.87, on s18
+  // 3.76, 4.19, on a power-law graph of 1M vertices 8.9, 9.5; depths of 1,024
+  // sources on s22 8.36, 8.49; closeness on a 1,024 x 1,024 grid 230, 250.
+  b->grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 4;
   b->hc = hub_cut(b->g, cfg.hybrid_hubs);
   b->ctx.resize(contexts);
   hipError_t err = hipMalloc((void **)&b->d_edges, sizeof(u64));

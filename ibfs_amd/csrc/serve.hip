@@ -921,7 +921,7 @@ int ibfs_server_create(ibfs_graph_t g, const ibfs_config *cfg_in, int64_t status
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device) != hipSuccess ||
       cus <= 0)
     cus = 256;
-  s->grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 32;
+  s->grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 4;  // as in a batch, for the same reason
   s->hc = hub_cut(s->g, cfg.hybrid_hubs);
   {  // two-hop size of every vertex, for cohort composition
     const int64_t V = g->V;
