@@ -86,6 +86,15 @@ __device__ __forceinline__ u64 wave_or(u64 x) {
   return lane63(x);
 }
 
+// Over a row of 16 lanes, in all of them.
+__device__ __forceinline__ u64 row_or(u64 x) {
+  x |= dpp_or_zero<0x121, 0xf>(x);  // row_ror:1
+  x |= dpp_or_zero<0x122, 0xf>(x);
+  x |= dpp_or_zero<0x124, 0xf>(x);
+  x |= dpp_or_zero<0x128, 0xf>(x);
+  return x;
+}
+
 __device__ __forceinline__ u64 wave_sum(u64 x) {
   x += dpp_or_zero<0x111, 0xf>(x);
   x += dpp_or_zero<0x112, 0xf>(x);

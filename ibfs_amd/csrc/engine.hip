@@ -500,9 +500,9 @@ int ibfs_config_default(ibfs_config *cfg) {
   if (!cfg) return fail(IBFS_ERR_ARG, "null config");
   std::memset(cfg, 0, sizeof *cfg);
   cfg->lane_bits = 128;
-  // wave64: a vertex with fewer than 64 edges would leave lanes of its wave
-  // idle, so it takes the one-thread class (the reference's 32 matches a
-  // 32-wide warp); measured 3% faster on R-MAT s22
+  // wave64: a top-down vertex with fewer than 64 edges would leave lanes of its
+  // wave idle, so it takes a row of 16 lanes (the reference's 32 matches a
+  // 32-wide warp)
   cfg->sml_shed = 64;
   cfg->lrg_shed = 512;
   cfg->policy = IBFS_POLICY_ALPHA_BETA;
@@ -724,8 +724,7 @@ int ibfs_graph_create_ex(const int64_t *beg, int64_t V, const int32_t *adj, int6
   const size_t vtb = sizeof(int32_t) * (size_t)std::max<int64_t>(Vt, 1);
   hipError_t err = hipMalloc((void **)&g->d_beg, sizeof(int64_t) * (size_t)(Vt + 1));
   if (err == hipSuccess) err = hipMalloc((void **)&g->d_adj, eb);
-  // bottom-up reads four entries at a time, so up to three past the last list
-  if (err == hipSuccess) err = hipMalloc((void **)&g->d_tadj, eb + 4 * sizeof(int32_t));
+  if (err == hipSuccess) err = hipMalloc((void **)&g->d_tadj, eb);
   if (err == hipSuccess) err = hipMalloc((void **)&g->d_head, sizeof(int4) * 2 * (size_t)std::max<int64_t>(Vt, 1));
   if (err == hipSuccess) err = hipMalloc((void **)&g->d_deg, vtb);
   if (err == hipSuccess) err = hipMalloc((void **)&g->d_hubs, sizeof(int32_t) * (size_t)std::max<int64_t>(H, 1));

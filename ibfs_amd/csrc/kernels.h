@@ -228,7 +228,7 @@ struct GraphDev {
   const int32_t *adj, *tadj;
   const int4 *head;  // first 8 traversal-adjacency entries of each vertex: [v] and [V + v]
   int64_t V;         // traversal vertices
-  int sml, lrg, chunk_shift;
+  int lrg, chunk_shift;
   HubSplit hsp;
 };
 

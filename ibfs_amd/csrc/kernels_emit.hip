@@ -332,11 +332,11 @@ __global__ __launch_bounds__(BS) void k_emit_tiled(const u64 *__restrict__ ring,
 // instruction writes 16 bytes per thread: one lane's 256 depths as a single
 // 1-KB contiguous piece of its row (k_emit writes 256-byte pieces, one
 // vertex per thread).  Where every lane is in its first window of fewer than
-// 16 levels, depths come from nibbles as in k_emit.  The waves of a workgroup take consecutive (chunk,
-// word) units, so the words of one vertex are read by neighbouring waves
-// from the same lines.  A lane row that is not 16-byte aligned, a chunk
-// that ends past V, and a piece holding an entry a continuation window must
-// not touch fall back to 4-byte stores.
+// 16 levels, depths come from nibbles as in k_emit.  The waves of a workgroup
+// take consecutive (chunk, word) units, so the words of one vertex are read by
+// neighbouring waves from the same lines.  A lane row that is not 16-byte
+// aligned, a chunk that ends past V, and a piece holding an entry a
+// continuation window must not touch fall back to 4-byte stores.
 template <int NS>
 __device__ __forceinline__ int32_t lane_depth4(const u64 (&c)[NS][4], const u64 (&fin)[4],
                                                const u64 (&bs)[4], int i, int bit, int off,

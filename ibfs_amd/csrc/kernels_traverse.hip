@@ -755,8 +755,8 @@ __device__ __forceinline__ void bu_commit(u64 *cur, uint8_t *flags, int64_t v, c
 // entries from the head array, which is in vertex order: where vertices are
 // consecutive, words and heads stream, and a vertex that is covered by then
 // (most are, in a dense level) touches neither its offsets nor its list.  The
-// others go on by degree: below sml one vertex per thread, four entries per
-// step; up to lrg one vertex per wave; above, one per workgroup.
+// others go on by degree: up to lrg one vertex per row of 16 lanes, above, one
+// per workgroup.
 __device__ __forceinline__ bool pulled(int32_t a, int cut) {
   return a < 0 && (a & 0x7fffffff) < cut;
 }
@@ -783,6 +783,7 @@ __device__ __forceinline__ bool bu_four(const Gather &gs, const int32_t (&a)[4],
   return !end && !covers<W>(x, lam);
 }
 
+constexpr int BU_ROW = 4;   // entries per lane and step of the row class
 constexpr int BU_BIG = 16;  // vertices of the workgroup class staged at a time
 
 template <int W>
@@ -794,25 +795,23 @@ struct BuShared {
   int n;
 };
 
-__device__ __forceinline__ u64 lane_of(u64 x, int l) {
-  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)x, l);
-  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(x >> 32), l);
-  return (u64)lo | ((u64)hi << 32);
-}
-
-// N entries per lane of [r, e), STRIDE apart from r + i, ORed into acc;
-// returns whether one of them lies past the pulled prefix (MODE 1).
-template <int W, int MODE, int N>
-__device__ __forceinline__ bool bu_gather(const int32_t *__restrict__ tadj, const Gather &gs,
-                                          int64_t r, int64_t e, int i, int stride, int cut,
-                                          u64 (&acc)[W]) {
-  int32_t a[N];
-  bool past = false;
+// N entries per lane of [r, e), stride apart from r + i.
+template <int N>
+__device__ __forceinline__ void bu_entries(const int32_t *__restrict__ tadj, int64_t r, int64_t e,
+                                           int i, int stride, int32_t (&a)[N]) {
 #pragma unroll
   for (int k = 0; k < N; ++k) {
     const int64_t j = r + i + (int64_t)k * stride;
     a[k] = j < e ? tadj[j] : NO_NBR;
   }
+}
+
+// ORs N entries' words into acc; returns whether one of the entries lies
+// past the pulled prefix (MODE 1).
+template <int W, int MODE, int N>
+__device__ __forceinline__ bool bu_gather(const Gather &gs, const int32_t (&a)[N], int cut,
+                                          u64 (&acc)[W]) {
+  bool past = false;
   u64 y[N][W];
 #pragma unroll
   for (int k = 0; k < N; ++k) {
@@ -838,6 +837,14 @@ __device__ __forceinline__ bool bu_gather(const int32_t *__restrict__ tadj, cons
 // R-MAT s22, 128 lanes, against one queue per degree class with 4, 64 or 256
 // list entries at a time: a group's dense level 290 -> 140 us, bottom-up of
 // 1,024 sources 5.0 -> 4.1 ms; batched 1M Chung-Lu 2.32 -> 1.90 ms.
+// Rows of 16 lanes against one vertex per thread below 64 neighbours and one
+// per wave above: a row reads its list in lines where a thread reads 16 bytes,
+// a wave has four lists in flight where it had one, and an average list fills
+// it.  s22 at 256 lanes, first two dense levels 295 + 270 -> 269 + 245 us;
+// closeness of 4,096 sources on s18 3.76 -> 3.60 ms, with 512 lanes
+// 3.51 -> 3.24, on a power-law graph of 1M vertices 8.9 -> 8.6.  Slower or
+// alike: 2, 3 or 6 entries per lane for 4, the next four vertices' entries
+// loaded ahead, the first hubs' words in LDS.
 template <int W, int MODE>
 __device__ __forceinline__ void bu_tile(const GraphDev &g, const Gather &gs, u64 *cur,
                                         uint8_t *flags, const u64 (&lam)[W], int64_t v,
@@ -877,44 +884,43 @@ __device__ __forceinline__ void bu_tile(const GraphDev &g, const Gather &gs, u64
 #pragma unroll
     for (int w = 0; w < W; ++w) x0[w] = 0;
   }
-  // thread class, unless so few lanes of the wave are left that taking them
-  // one at a time is the shorter chain
-  bool small = pend && deg < g.sml;
-  if (__popcll(__ballot(small)) > 4) {
-    while (small) {
-      struct __attribute__((packed, aligned(4))) Four { int32_t a[4]; };
-      const Four f = *reinterpret_cast<const Four *>(tadj + j);  // readable past the last list
-      int32_t a[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) a[r] = j + r < e ? f.a[r] : NO_NBR;
-      j += 4;
-      small = bu_four<W, MODE>(gs, a, own, lam, cut, x) && j < e;
-      pend = small;
-    }
-  }
-  // wave class
+  // row class: four vertices at a time, one per row of 16 lanes
   const bool big = pend && deg > g.lrg;
   u64 m = __ballot(pend && !big);
   while (m) {
-    const int b = __builtin_ctzll(m);
-    m &= m - 1;
-    const int64_t eb = (int64_t)lane_of((u64)e, b);
+    int from = -1, back = -1;  // the lane this row works for, the row that works for this lane
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (m) {
+        const int b = __builtin_ctzll(m);
+        m &= m - 1;
+        if (lane >> 4 == k) from = b;
+        if (lane == b) back = 16 * k;
+      }
+    }
+    int64_t r = __shfl(j, from & 63, 64);
+    const int64_t er = __shfl(e, from & 63, 64);
     u64 y[W];
 #pragma unroll
-    for (int w = 0; w < W; ++w) y[w] = lane_of(x[w], b);
-    for (int64_t r = (int64_t)lane_of((u64)j, b); r < eb; r += 128) {
+    for (int w = 0; w < W; ++w) y[w] = __shfl(x[w], from & 63, 64);
+    bool more = from >= 0;
+    while (more) {
+      int32_t a[BU_ROW];
+      bu_entries<BU_ROW>(tadj, r, er, lane & 15, 16, a);
       u64 acc[W];
 #pragma unroll
       for (int w = 0; w < W; ++w) acc[w] = 0;
-      const bool past = bu_gather<W, MODE, 2>(tadj, gs, r, eb, lane, 64, cut, acc);
+      const bool past = bu_gather<W, MODE, BU_ROW>(gs, a, cut, acc);
 #pragma unroll
-      for (int w = 0; w < W; ++w) y[w] |= wave_or(acc[w] & lam[w]);
-      if (covers<W>(y, lam)) break;
-      if (MODE == 1 && __ballot(past)) break;  // pulled prefix ended
+      for (int w = 0; w < W; ++w) y[w] |= row_or(acc[w] & lam[w]);
+      r += 16 * BU_ROW;
+      more = r < er && !covers<W>(y, lam);
+      if (MODE == 1 && ((__ballot(past) >> (lane & 48)) & 0xffff)) more = false;
     }
-    if (lane == b) {
 #pragma unroll
-      for (int w = 0; w < W; ++w) x[w] = y[w];
+    for (int w = 0; w < W; ++w) {
+      const u64 z = __shfl(y[w], back & 63, 64);
+      if (back >= 0) x[w] = z;
     }
   }
   // workgroup class: BU_BIG vertices at a time through LDS, 1,024 entries
@@ -944,7 +950,9 @@ __device__ __forceinline__ void bu_tile(const GraphDev &g, const Gather &gs, u64
           u64 acc[W];
 #pragma unroll
           for (int w = 0; w < W; ++w) acc[w] = 0;
-          const bool past = bu_gather<W, MODE, 4>(tadj, gs, r, eb, t, BS, cut, acc);
+          int32_t a[4];
+          bu_entries<4>(tadj, r, eb, t, BS, a);
+          const bool past = bu_gather<W, MODE, 4>(gs, a, cut, acc);
 #pragma unroll
           for (int w = 0; w < W; ++w) acc[w] = wave_or(acc[w] & lam[w]);
           const int wpast = MODE == 1 && __ballot(past) != 0;
@@ -994,8 +1002,8 @@ __host__ __device__ inline int bu_per_wave(int64_t n) {
 // Every candidate (the n of the queue, or every vertex), grid-strided in tiles
 // of 4 waves.  A wave takes 64 vertices, or only 32, 16 or 8 where that keeps
 // the number of workgroups near 2,048 (8 per CU): a wave works off its
-// vertices of the wave class one after another, and with few vertices that
-// chain, not the chip, is the level's time.
+// vertices of the row class four by four, and with few vertices that chain, not
+// the chip, is the level's time.
 template <int W, int MODE>
 __device__ __forceinline__ void bu_level(const GraphDev &g, const Gather &gs, u64 *cur,
                                          uint8_t *flags, const u64 (&lam)[W],

@@ -53,10 +53,10 @@ typedef struct ibfs_server_s *ibfs_server_t;
 /* Engine configuration.  Defaults (ibfs_config_default): 128 lanes
  * (concurrent-count, readme.md:27), lrg_shed=512 as the reference
  * (main.cu:56-57), sml_shed=64 where the reference has 32 (main.cu:56): the
- * thread/wave class boundary follows the 64-wide wavefront. */
+ * boundary of top-down classes follows the 64-wide wavefront. */
 typedef struct ibfs_config {
   int32_t lane_bits;   /* 64, 128, 256 or 512 source lanes per status word     */
-  int32_t sml_shed;    /* degree < sml_shed        -> thread class             */
+  int32_t sml_shed;    /* degree < sml_shed        -> 16 lanes, top-down       */
   int32_t lrg_shed;    /* degree > lrg_shed        -> workgroup class          */
   int32_t policy;      /* IBFS_POLICY_*                                        */
   int32_t sw_level;    /* last top-down level for IBFS_POLICY_FIXED (argv[4])   */
