@@ -40,14 +40,13 @@ struct Ctx {
   Queues q{};
   u64 *hs = nullptr;
   uint8_t *flags = nullptr;  // changed-at-this-level byte per traversal vertex
-  // a group's set-up data (level masks, sources, lane table, plan) lives in
-  // one pinned block and one device block of the same layout, so a group
-  // starts with one copy; the pointers below point into them
+  // a group's set-up data (level masks, lane table, plan) lives in one pinned
+  // block and one device block of the same layout, so the launch that starts
+  // a group copies it too; the pointers below point into them
   char *d_setup = nullptr, *h_setup = nullptr;
   size_t setup_bytes = 0;
   Plan *d_plan = nullptr, *h_plan = nullptr;
   u64 *d_masks = nullptr, *h_masks = nullptr;  // [0,W) lanes_all, [W,2W) sel, then (R+1)W level masks
-  int32_t *d_src = nullptr, *h_src = nullptr;
   LaneOut *d_lanes = nullptr, *h_lanes = nullptr;
   int32_t *d_stage = nullptr;  // host-placed output staging, K*V
   hipGraph_t graph = nullptr;
@@ -144,7 +143,6 @@ void release_ctx(Ctx &c) {
   hfree(c.h_setup);
   c.d_plan = c.h_plan = nullptr;
   c.d_masks = c.h_masks = nullptr;
-  c.d_src = c.h_src = nullptr;
   c.d_lanes = c.h_lanes = nullptr;
   dfree(c.d_stage);
   dfree(c.d_al);
@@ -237,10 +235,9 @@ int alloc_ctx(ibfs_batch_s *b, Ctx &c) {
   A((void **)&c.q.chunks, sizeof(int2) * chunk_entries((size_t)Vq, (size_t)b->g->E, b->chunk_shift));
   A((void **)&c.hs, sizeof(u64) * (size_t)b->W * (size_t)std::max<int64_t>(b->g->H, 1));
   A((void **)&c.flags, sizeof(u64) * (size_t)((Vq + 7) / 8));
-  {  // set-up block: masks, sources, lane table, plan (256-byte aligned parts)
+  {  // set-up block: masks, lane table, plan (256-byte aligned parts)
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t o_src = al(sizeof(u64) * masks_words(b));
-    const size_t o_lanes = o_src + al(sizeof(int32_t) * (size_t)b->K);
+    const size_t o_lanes = al(sizeof(u64) * masks_words(b));
     const size_t o_plan = o_lanes + al(sizeof(LaneOut) * (size_t)b->K);
     c.setup_bytes = o_plan + al(sizeof(Plan));
     A((void **)&c.d_setup, c.setup_bytes);
@@ -248,8 +245,6 @@ int alloc_ctx(ibfs_batch_s *b, Ctx &c) {
     if (err == hipSuccess) {
       c.d_masks = reinterpret_cast<u64 *>(c.d_setup);
       c.h_masks = reinterpret_cast<u64 *>(c.h_setup);
-      c.d_src = reinterpret_cast<int32_t *>(c.d_setup + o_src);
-      c.h_src = reinterpret_cast<int32_t *>(c.h_setup + o_src);
       c.d_lanes = reinterpret_cast<LaneOut *>(c.d_setup + o_lanes);
       c.h_lanes = reinterpret_cast<LaneOut *>(c.h_setup + o_lanes);
       c.d_plan = reinterpret_cast<Plan *>(c.d_setup + o_plan);
@@ -319,13 +314,15 @@ int start_group(ibfs_batch_s *b, Ctx &c, const int32_t *src, int64_t g0, int k, 
   for (int i = 0; i < k; ++i) c.a_max = std::max(c.a_max, c.start[(size_t)i]);
   std::memset(c.h_masks, 0, sizeof(u64) * masks_words(b));
   c.iso = 0;
+  SourceList sl;
+  sl.k = k;
   for (int i = 0; i < k; ++i) {
     c.iso |= b->g->h_cid[src[g0 + i]] < 0;
     const int a = c.start[(size_t)i];
     if (a == 0) c.h_masks[i >> 6] |= 1ull << (i & 63);  // lanes of level 0
     c.h_masks[W + (i >> 6)] |= 1ull << (i & 63);         // every lane of the group
     // lanes starting later are set by the admission of their level
-    c.h_src[i] = a == 0 ? b->g->h_cid[src[g0 + i]] : -1;
+    sl.src[i] = a == 0 ? b->g->h_cid[src[g0 + i]] : -1;
     c.h_lanes[i].out = dev_out ? dev_out + (size_t)rows[i] * (size_t)V
                                : (stage ? stage + (size_t)i * (size_t)V : nullptr);
     c.h_lanes[i].admit = a;
@@ -350,14 +347,14 @@ int start_group(ibfs_batch_s *b, Ctx &c, const int32_t *src, int64_t g0, int k, 
     c.h_plan->tail_cap = c.tail_cap;
     c.h_plan->E = (u64)b->g->E;
   }
-  // masks, sources, lane table and plan in one copy (lane entries past k are
-  // stale and never read: every kernel takes the group's k); then S_0, the
-  // flags and the control blocks zeroed in one launch
-  HIP_TRY(hipMemcpyAsync(c.d_setup, c.h_setup, c.setup_bytes, hipMemcpyHostToDevice, c.st));
-  HIP_TRY(launch_zero3_u64(slot(b, c, 0), b->g->Vt * W, reinterpret_cast<u64 *>(c.flags),
-                           (b->g->Vt + 7) / 8, reinterpret_cast<u64 *>(c.ctl),
-                           (int64_t)(ctl_ring_bytes(b->R) / 8), c.st));
-  HIP_TRY(launch_init_sources(W, c.d_src, k, 0, slot(b, c, 0), c.flags, c.st));
+  // masks, lane table and plan copied (lane entries past k are stale and never
+  // read: every kernel takes the group's k), S_0, the flags and the control
+  // blocks set in one launch
+  HIP_TRY(launch_plan_start(W, sl, b->g->Vt, slot(b, c, 0), c.flags,
+                            reinterpret_cast<u64 *>(c.ctl), (int64_t)(ctl_ring_bytes(b->R) / 8),
+                            reinterpret_cast<const u64 *>(c.h_setup),
+                            reinterpret_cast<u64 *>(c.d_setup), (int64_t)(c.setup_bytes / 8),
+                            c.st));
   HIP_TRY(inspect_decide(b, c));
   c.g0 = g0;
   c.k = k;

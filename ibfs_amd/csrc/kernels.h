@@ -339,6 +339,13 @@ hipError_t launch_group_start(int W, const SourceList &sl, const int32_t *cid, i
                               int64_t V, int64_t Vt, u64 *S0, uint8_t *flags, u64 *ctl,
                               int64_t ctl_words, LaneOut *lanes, u64 *masks, int R, u64 *counters,
                               hipStream_t st);
+// One launch that prepares a device-planned traversal of sl.k sources
+// (traversal ids, -1: none), lane i = source i: S0, flags and control ring as
+// above, and `words` 64-bit words of pinned host memory copied to dev (masks,
+// lane table, plan).
+hipError_t launch_plan_start(int W, const SourceList &sl, int64_t Vt, u64 *S0, uint8_t *flags,
+                             u64 *ctl, int64_t ctl_words, const u64 *host, u64 *dev, int64_t words,
+                             hipStream_t st);
 // End of a group, posted like a control block: the counters of
 // launch_group_start and the device clock.
 struct GroupPost {
@@ -347,8 +354,6 @@ struct GroupPost {
 };
 hipError_t launch_group_end(const u64 *counters, GroupPost *post, u64 tag, hipStream_t st);
 // S0[src[i]] |= bit lane0+i, i < k (src in traversal ids; -1 entries skipped).
-hipError_t launch_init_sources(int W, const int32_t *src, int k, int lane0, u64 *S0,
-                               uint8_t *flags, hipStream_t st);
 // S[src[i]] |= bit lane[i], i < n (traversal ids; -1 entries skipped).
 hipError_t launch_admit(int W, const int32_t *src, const int32_t *lane, int n, u64 *S,
                         uint8_t *flags, hipStream_t st);

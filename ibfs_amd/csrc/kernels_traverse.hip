@@ -78,6 +78,38 @@ __global__ __launch_bounds__(BS) void k_group_start(SourceList sl, const int32_t
   }
 }
 
+// Start of a device-planned traversal (launch_plan_start), shared out like
+// k_group_start, with one word of the set-up block per thread of the first
+// workgroups.  Bound by its launch on small graphs: in place of a copy, a fill
+// and a set-up kernel, 42 -> 10 us from the set-up's first command to the first
+// inspection on R-MAT s16 (closeness of 4,096 sources on s18 3.59 -> 3.51 ms, of
+// 8,192 on s14 3.84 -> 3.76); a server's cohort had three copies more.  The
+// host's memory is read past the caches, which may hold the block of the
+// traversal before.
+template <int W>
+__global__ __launch_bounds__(BS) void k_plan_start(SourceList sl, int64_t Vt, u64 *S0,
+                                                   uint8_t *flags, u64 *ctl, int64_t ctl_words,
+                                                   const u64 *host, u64 *dev, int64_t words) {
+  const int t = threadIdx.x;
+  const int64_t at = (int64_t)blockIdx.x * BS + t, all = (int64_t)gridDim.x * BS;
+  for (int64_t i = at; i < words; i += all)
+    dev[i] = __hip_atomic_load(&host[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  for (int64_t i = at; i < ctl_words; i += all) ctl[i] = 0;
+  const int64_t share = ((Vt + gridDim.x - 1) / gridDim.x + 15) & ~(int64_t)15;
+  const int64_t v0 = blockIdx.x * share, v1 = v0 + share < Vt ? v0 + share : Vt;
+  for (int64_t i = v0 * W + t; i < v1 * W; i += BS) S0[i] = 0;
+  u64 *f = reinterpret_cast<u64 *>(flags);  // padded to whole words
+  for (int64_t i = v0 / 8 + t; i < (v1 + 7) / 8; i += BS) f[i] = 0;
+  __syncthreads();
+  for (int i = t; i < sl.k; i += BS) {
+    const int32_t v = sl.src[i];
+    if (v >= v0 && v < v1) {
+      atomicOr(&S0[(int64_t)v * W + (i >> 6)], 1ull << (i & 63));
+      flags[v] = 1;
+    }
+  }
+}
+
 __global__ void k_group_end(const u64 *counters, GroupPost *post, u64 tag) {
   const int t = threadIdx.x;
   if (t < 3)
@@ -88,20 +120,10 @@ __global__ void k_group_end(const u64 *counters, GroupPost *post, u64 tag) {
   if (t == 0) __hip_atomic_store(&post->tag, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Lane init: lane lane0+i gets bit of src[i] (a traversal id).  OR, so
+// Admission: bit lane[i] set in S[src[i]] (lanes of any position).  OR, so
 // duplicate sources keep their bit.  src[i] < 0 is an isolated source: it
 // has no status word and its depth array is -1 except 0 at the source (the
 // reference stores and skips zero-degree sources, expander.cu:63,70-71).
-template <int W>
-__global__ void k_init_sources(const int32_t *src, int k, int lane0, u64 *S0, uint8_t *flags) {
-  int i = blockIdx.x * BS + threadIdx.x;
-  if (i >= k || src[i] < 0) return;
-  int lane = lane0 + i;
-  atomicOr(&S0[(int64_t)src[i] * W + (lane >> 6)], 1ull << (lane & 63));
-  flags[src[i]] = 1;
-}
-
-// Admission: bit lane[i] set in S[src[i]] (lanes of any position).
 template <int W>
 __global__ void k_admit(const int32_t *src, const int32_t *lane, int n, u64 *S, uint8_t *flags) {
   int i = blockIdx.x * BS + threadIdx.x;
@@ -1590,17 +1612,17 @@ hipError_t launch_group_start(int W, const SourceList &sl, const int32_t *cid, i
   return hipGetLastError();
 }
 
-hipError_t launch_group_end(const u64 *counters, GroupPost *post, u64 tag, hipStream_t st) {
-  hipLaunchKernelGGL(k_group_end, dim3(1), dim3(64), 0, st, counters, post, tag);
+hipError_t launch_plan_start(int W, const SourceList &sl, int64_t Vt, u64 *S0, uint8_t *flags,
+                             u64 *ctl, int64_t ctl_words, const u64 *host, u64 *dev, int64_t words,
+                             hipStream_t st) {
+  dim3 g(std::max(grid_for(Vt * W, BS * 8, 8192), grid_for(words, BS, 64))), blk(BS);
+  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_plan_start<WW>, g, blk, 0, st, sl, Vt, S0, flags, ctl,
+                                        ctl_words, host, dev, words));
   return hipGetLastError();
 }
 
-hipError_t launch_init_sources(int W, const int32_t *src, int k, int lane0, u64 *S0,
-                               uint8_t *flags, hipStream_t st) {
-  if (k <= 0) return hipSuccess;
-  dim3 g(grid_for(k, BS, 1 << 20)), blk(BS);
-  IBFS_DISPATCH_W(W, hipLaunchKernelGGL(k_init_sources<WW>, g, blk, 0, st, src, k, lane0, S0,
-                                        flags));
+hipError_t launch_group_end(const u64 *counters, GroupPost *post, u64 tag, hipStream_t st) {
+  hipLaunchKernelGGL(k_group_end, dim3(1), dim3(64), 0, st, counters, post, tag);
   return hipGetLastError();
 }
 

@@ -96,6 +96,11 @@ struct SCtx {
   uint8_t *flags = nullptr;  // changed-at-this-level byte per traversal vertex
   u64 *d_mask = nullptr, *h_mask = nullptr;
   int32_t *d_adm = nullptr, *h_adm = nullptr;  // [0,K) sources, [K,2K) lanes
+  // a cohort's set-up data (lanes, lane table, plan) lives in one pinned block
+  // and one device block of the same layout, so the launch that starts a
+  // cohort copies it too; h/d_lanes, _plan and _all point into them
+  char *d_setup = nullptr, *h_setup = nullptr;
+  size_t setup_bytes = 0;
   LaneOut *d_lanes = nullptr, *h_lanes = nullptr;
   hipEvent_t ev = nullptr;
   std::vector<Lane> lanes;
@@ -197,10 +202,11 @@ void release_ctx(SCtx &c) {
     c.exec[i] = c.exec_burst[i] = nullptr;
     c.graph[i] = c.graph_burst[i] = nullptr;
   }
-  dfree(c.d_plan);
-  hfree(c.h_plan);
-  dfree(c.d_all);
-  hfree(c.h_all);
+  dfree(c.d_setup);
+  hfree(c.h_setup);
+  c.d_plan = c.h_plan = nullptr;
+  c.d_all = c.h_all = nullptr;
+  c.d_lanes = c.h_lanes = nullptr;
   dfree(c.d_al);
   hfree(c.h_al);
   dfree(c.ring);
@@ -214,8 +220,6 @@ void release_ctx(SCtx &c) {
   hfree(c.h_mask);
   dfree(c.d_adm);
   hfree(c.h_adm);
-  dfree(c.d_lanes);
-  hfree(c.h_lanes);
   if (c.ev) (void)hipEventDestroy(c.ev);
   c.ev = nullptr;
   if (c.st) (void)hipStreamDestroy(c.st);
@@ -280,19 +284,29 @@ int alloc_ctx(ibfs_server_s *s, SCtx &c) {
   H((void **)&c.h_mask, sizeof(u64) * mask_words(s));
   A((void **)&c.d_adm, sizeof(int32_t) * 2 * (size_t)s->K);
   H((void **)&c.h_adm, sizeof(int32_t) * 2 * (size_t)s->K);
-  A((void **)&c.d_lanes, sizeof(LaneOut) * (size_t)s->K);
-  H((void **)&c.h_lanes, sizeof(LaneOut) * (size_t)s->K);
-  A((void **)&c.d_plan, sizeof(Plan));
-  H((void **)&c.h_plan, sizeof(Plan));
-  A((void **)&c.d_all, sizeof(u64) * (size_t)s->W);
-  H((void **)&c.h_all, sizeof(u64) * (size_t)s->W);
+  {  // set-up block: cohort lanes, lane table, plan (256-byte aligned parts)
+    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t o_lanes = al(sizeof(u64) * (size_t)s->W);
+    const size_t o_plan = o_lanes + al(sizeof(LaneOut) * (size_t)s->K);
+    c.setup_bytes = o_plan + al(sizeof(Plan));
+    A((void **)&c.d_setup, c.setup_bytes);
+    H((void **)&c.h_setup, c.setup_bytes);
+    if (err == hipSuccess) {
+      c.d_all = reinterpret_cast<u64 *>(c.d_setup);
+      c.h_all = reinterpret_cast<u64 *>(c.h_setup);
+      c.d_lanes = reinterpret_cast<LaneOut *>(c.d_setup + o_lanes);
+      c.h_lanes = reinterpret_cast<LaneOut *>(c.h_setup + o_lanes);
+      c.d_plan = reinterpret_cast<Plan *>(c.d_setup + o_plan);
+      c.h_plan = reinterpret_cast<Plan *>(c.h_setup + o_plan);
+      std::memset(c.h_setup, 0, c.setup_bytes);
+    }
+  }
   A((void **)&c.d_al, sizeof(AdmitList));
   H((void **)&c.h_al, sizeof(AdmitList));
   if (err == hipSuccess) err = hipEventCreateWithFlags(&c.ev, hipEventDisableTiming);
   if (err != hipSuccess)
     return fail(err == hipErrorOutOfMemory ? IBFS_ERR_NOMEM : IBFS_ERR_HIP,
                 "server context allocation failed: %s", hipGetErrorString(err));
-  std::memset(c.h_lanes, 0, sizeof(LaneOut) * (size_t)s->K);
   c.lanes.assign(s->K, Lane{});
   // one cohort level per width: device-driven expansion, inspection,
   // direction decision (every kernel derives its slot stride from its width)
@@ -718,14 +732,11 @@ int start_cohort(ibfs_server_s *s, SCtx &c) {
   pick_cohort(s, c.K);
   const int W = c.W;
   for (auto &l : c.lanes) l = Lane{};
-  // S_0, the changed flags and the control blocks zeroed in one launch
-  HIP_CHK(launch_zero3_u64(slot(s, c, 0), s->g->Vt * W, reinterpret_cast<u64 *>(c.flags),
-                           (s->g->Vt + 7) / 8, reinterpret_cast<u64 *>(c.ctl),
-                           (int64_t)(ctl_ring_bytes(s->R) / 8), c.st));
   // the cohort's first sources take lanes 0, 1, ...; with phase offsets a
   // lane whose source's two-hop size says it runs ahead of the others starts
   // at a later level (admitted then through the admission list)
   std::memset(c.h_all, 0, sizeof(u64) * W);
+  SourceList sl;
   int n = 0;
   for (int k = 0; k < c.K && !s->pending.empty(); ++k) {
     const PendingSrc p = s->pending.front();
@@ -734,8 +745,7 @@ int start_cohort(ibfs_server_s *s, SCtx &c) {
     c.lanes[k].state = ACTIVE;
     c.lanes[k].qid = p.qid;
     c.lanes[k].admit = 0;
-    c.h_adm[n] = s->g->h_cid[q.src[p.idx]];
-    c.h_adm[s->K + n] = k;
+    sl.src[k] = s->g->h_cid[q.src[p.idx]];
     c.h_lanes[k].out = q.out + (size_t)p.idx * (size_t)s->g->V;
     c.h_lanes[k].admit = 0;
     c.h_lanes[k].src = q.src[p.idx];
@@ -756,24 +766,21 @@ int start_cohort(ibfs_server_s *s, SCtx &c) {
       if (a == 0) continue;
       c.lanes[i].admit = a;
       c.h_lanes[i].admit = a;
-      c.h_adm[i] = -1;  // not set at level 0
+      sl.src[i] = -1;  // not set at level 0
       c.deferred.emplace_back(i, a);
       c.a_max = std::max(c.a_max, a);
     }
   }
   for (int i = 0; i < n; ++i)
     if (c.lanes[i].admit == 0) set_bit(c.h_all, i);
-  if (n > 0) {
-    HIP_CHK(hipMemcpyAsync(c.d_adm, c.h_adm, sizeof(int32_t) * 2 * (size_t)s->K,
-                           hipMemcpyHostToDevice, c.st));
-    HIP_CHK(hipMemcpyAsync(c.d_lanes, c.h_lanes, sizeof(LaneOut) * (size_t)s->K,
-                           hipMemcpyHostToDevice, c.st));
-    HIP_CHK(launch_admit(c.W, c.d_adm, c.d_adm + s->K, n, slot(s, c, 0), c.flags, c.st));
-  }
-  HIP_CHK(hipMemcpyAsync(c.d_all, c.h_all, sizeof(u64) * W, hipMemcpyHostToDevice, c.st));
   plan_init(c.h_plan, s->cfg, s->hc.rho_q10, (u64)s->g->V);
   c.h_plan->hold = c.a_max;
-  HIP_CHK(hipMemcpyAsync(c.d_plan, c.h_plan, sizeof(Plan), hipMemcpyHostToDevice, c.st));
+  sl.k = n;
+  HIP_CHK(launch_plan_start(W, sl, s->g->Vt, slot(s, c, 0), c.flags,
+                            reinterpret_cast<u64 *>(c.ctl), (int64_t)(ctl_ring_bytes(s->R) / 8),
+                            reinterpret_cast<const u64 *>(c.h_setup),
+                            reinterpret_cast<u64 *>(c.d_setup), (int64_t)(c.setup_bytes / 8),
+                            c.st));
   HIP_CHK(inspect_decide(s, c, W));
   c.coh = 1;
   c.dlevel = 1;

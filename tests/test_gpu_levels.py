@@ -161,3 +161,31 @@ def test_noalloc_levels_enqueued_in_bursts(rows, cols, n):
         g.traversal_noalloc(s, out)
         np.testing.assert_array_equal(out.to_host(count=rows * cols),
                                       oracle.bfs_many(beg, adj, s, threads=1)[0])
+
+
+@pytest.mark.parametrize("V,isolated", [(5, 5), (3, 0), (17, 1), (4097, 100), (70_001, 30_000)])
+@pytest.mark.parametrize("lanes", [64, 128, 256, 512])
+def test_planned_traversals_start_over(V, isolated, lanes):
+    """Groups and cohorts of changing size started over and over on the same
+    contexts (set-up block, snapshots, flags and counters of the traversal
+    before), with repeated and isolated sources, on a graph without an edge,
+    below one workgroup's share, and of many shares."""
+    say(f"[gpu] starts V={V} isolated={isolated} lanes={lanes}")
+    n = V - isolated
+    v = np.arange(max(n, 1))
+    beg, adj = _symmetric(V, np.concatenate([v, v]),
+                          np.concatenate([(v + 1) % max(n, 1), (v * 7 + 3) % max(n, 1)]))
+    g = ibfs_amd.DeviceGraph(ibfs_amd.HostCsr.from_arrays(beg, adj))
+    b = ibfs_amd.Batch(g, lane_bits=lanes, contexts=2, burst=3)
+    s = ibfs_amd.Server(g, lane_bits=lanes)
+    for k in (1, lanes + 3, 2 * lanes + 17, 5):
+        src = np.random.default_rng(k).integers(0, V, size=k).astype(np.int32)
+        src[k // 2] = src[0]
+        src[-1] = V - 1
+        want = oracle.bfs_many(beg, adj, src, threads=8)
+        np.testing.assert_array_equal(b.run(src), want)
+        out = ibfs_amd.DeviceBuffer(4 * k * V)
+        s.wait(s.submit(src, out))
+        np.testing.assert_array_equal(out.to_host(np.int32, k * V).reshape(k, V), want)
+    s.close()
+    b.close()
