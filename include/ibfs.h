@@ -299,7 +299,7 @@ int ibfs_engine_level_log(ibfs_engine_t e, ibfs_level_info *out, int32_t cap,
  * buffer of k*V int32, as ibfs_traversal does; *traversed_edges (optional)
  * receives the TEPS numerator.  It calls no allocating routine: every
  * scratch buffer lives in one file-scope device array of
- * IBFS_NOALLOC_SCRATCH_BYTES 43015680that each GPU the library runs on holds until
+ * IBFS_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds until
  * the process ends, and kernels run on the null stream.  Limits, rejected
  * with IBFS_ERR_ARG: at most 262,144 vertices with an edge, 2^24 adjacency
  * entries, 131,072 hubs, td_chunk >= 2048.  Calls on one device share the
