@@ -122,6 +122,11 @@ struct SCtx {
   // graph launches leave ≈8 µs between levels)
   hipGraph_t graph_burst[4] = {};
   hipGraphExec_t exec_burst[4] = {};
+  // burst graphs per host poll: a poll leaves the device idle for 50 to 60 us, a
+  // level past the end costs it 9.  Two where the context's last cohort needed
+  // more than one: a query of one source on R-MAT s14 178 -> 164 us, of 128 on a
+  // power-law graph of 300K vertices 351 -> 341, 32 queries on s20 6.93 -> 6.81 ms.
+  int bursts = 1;
   int W = 0, K = 0;  // current width: words per vertex and lanes (<= the server's)
   int coh = 0;     // 0: host-driven levels, 1: cohort levels on the device, 2: cohort emitting
   int dlevel = 0;  // cohort level the device expands next (host view)
@@ -179,7 +184,7 @@ struct ibfs_server_s {
 };
 
 namespace {
-constexpr int kCohortBurst = 4;  // level graphs per host poll in cohort mode
+constexpr int kCohortBurst = 4;  // levels of a burst graph
 }
 
 namespace {
@@ -628,12 +633,12 @@ void take_pending(ibfs_server_s *s, SCtx &c, int L, int n0, int *n_new) {
 // context's event.  Inside the admission window (levels 1..admit_window of
 // the cohort) one level at a time, each joined by the sources waiting at its
 // boundary: expansion, admission, inspection and decision launched
-// directly; after the window up to kCohortBurst captured level graphs
+// directly; after the window up to one or two bursts of captured level graphs
 // (bounded so that no snapshot of the emission window is overwritten; the
 // window is flushed first when it is full).  locked: the caller holds the
 // server lock.
 int cohort_burst(ibfs_server_s *s, SCtx &c, bool locked) {
-  int B = std::min(kCohortBurst, s->R - 1 - (c.dlevel - c.base));
+  int B = std::min(kCohortBurst * c.bursts, s->R - 1 - (c.dlevel - c.base));
   if (B < 1) {
     std::vector<int> act;
     for (int k = 0; k < c.K; ++k)
@@ -641,7 +646,7 @@ int cohort_burst(ibfs_server_s *s, SCtx &c, bool locked) {
     int rc = emit_lanes(s, c, act, c.base, c.dlevel - 1, 1);
     if (rc) return rc;
     c.base = c.dlevel - 1;
-    B = std::min(kCohortBurst, s->R - 1 - (c.dlevel - c.base));
+    B = std::min(kCohortBurst * c.bursts, s->R - 1 - (c.dlevel - c.base));
   }
   hipGraphExec_t x = c.exec[__builtin_ctz((unsigned)c.W)];
   const int win = s->admit_window;
@@ -680,10 +685,10 @@ int cohort_burst(ibfs_server_s *s, SCtx &c, bool locked) {
     } else {
       HIP_CHK(hipGraphLaunch(x, c.st));
     }
-  } else if (B == kCohortBurst) {
-    HIP_CHK(hipGraphLaunch(c.exec_burst[__builtin_ctz((unsigned)c.W)], c.st));
   } else {
-    for (int i = 0; i < B; ++i) HIP_CHK(hipGraphLaunch(x, c.st));
+    for (; B >= kCohortBurst; B -= kCohortBurst)
+      HIP_CHK(hipGraphLaunch(c.exec_burst[__builtin_ctz((unsigned)c.W)], c.st));
+    for (; B > 0; --B) HIP_CHK(hipGraphLaunch(x, c.st));
   }
   HIP_CHK(hipMemcpyAsync(c.h_plan, c.d_plan, offsetof(Plan, dirlog), hipMemcpyDeviceToHost, c.st));
   HIP_CHK(hipEventRecord(c.ev, c.st));
@@ -796,6 +801,7 @@ int start_cohort(ibfs_server_s *s, SCtx &c) {
 int cohort_step(ibfs_server_s *s, SCtx &c) {
   if (c.coh == 1) {
     if (c.h_plan->done) {
+      c.bursts = c.h_plan->last + 1 > kCohortBurst ? 2 : 1;
       std::vector<int> act;
       for (int k = 0; k < c.K; ++k)
         if (c.lanes[k].state == ACTIVE) act.push_back(k);
