@@ -186,7 +186,9 @@ __global__ __launch_bounds__(BS) void k_emit(const u64 *__restrict__ ring, int R
     s_src[i] = on ? lanes[i].src : -1;
     cont |= on && s_off[i] > 0;
   }
-  const bool fast = NS == 4 && !__syncthreads_or(cont);
+  // the barrier also orders the lane table above, at every NS
+  const int continued = __syncthreads_or(cont);
+  const bool fast = NS == 4 && !continued;
   // Workgroups go to the 8 XCDs in turn: XCD x takes the x-th eighth of the
   // vertices, so neighbouring 1-KB pieces of a row, which share a cache line
   // where the row is not aligned, are written through one L2 and leave it whole.
@@ -370,7 +372,9 @@ __global__ __launch_bounds__(BS) void k_emit_wide(const u64 *__restrict__ ring, 
     s_src[i] = on ? lanes[i].src : -1;
     cont |= on && s_off[i] > 0;
   }
-  const bool fast = NS == 4 && !__syncthreads_or(cont);
+  // the barrier also orders the lane table above, at every NS
+  const int continued = __syncthreads_or(cont);
+  const bool fast = NS == 4 && !continued;
   const int64_t V = sp.V, slot = sp.Vt * W;
   const bool v4 = (V & 3) == 0;
   // XCD shares as in k_emit, by workgroups of four units

@@ -223,3 +223,38 @@ def test_planned_traversals_start_over(V, isolated, lanes):
         np.testing.assert_array_equal(out.to_host(np.int32, k * V).reshape(k, V), want)
     s.close()
     b.close()
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 150), (7, 43), (40, 301), (3, 1200)])
+@pytest.mark.parametrize("mode", [0, 2, 3])
+def test_emission_of_deep_windows(rows, cols, mode):
+    """Paths and grids of 47 to 1,200 levels: emission windows of 16 levels and
+    more (rings of 32 and 64) and of 64 and more (ring of 255), continued ones
+    too, aligned and unaligned rows, a partial second group, in the engine, the
+    batched form, the server and the allocation-free call."""
+    V = rows * cols
+    v = np.arange(V).reshape(rows, cols)
+    beg, adj = _symmetric(V, np.concatenate([v[:, :-1].ravel(), v[:-1].ravel()]),
+                          np.concatenate([v[:, 1:].ravel(), v[1:].ravel()]))
+    g = ibfs_amd.DeviceGraph(ibfs_amd.HostCsr.from_arrays(beg, adj))
+    every = np.random.default_rng(V).integers(0, V, size=515).astype(np.int32)
+    depths = oracle.bfs_many(beg, adj, every, threads=8)
+    for lanes in (64, 128, 256, 512):
+        src, want = every[:lanes + 3], depths[:lanes + 3]
+        for ring in (32, 64, 255):
+            say(f"[gpu] deep windows {rows}x{cols} mode={mode} lanes={lanes} ring={ring}")
+            e = ibfs_amd.Engine(g, lane_bits=lanes, emit_mode=mode, ring_levels=ring)
+            np.testing.assert_array_equal(e.run_groups(src), want)
+            e.close()
+            b = ibfs_amd.Batch(g, lane_bits=lanes, contexts=2, burst=8, emit_mode=mode,
+                               ring_levels=ring)
+            np.testing.assert_array_equal(b.run(src), want)
+            b.close()
+        s = ibfs_amd.Server(g, lane_bits=lanes, emit_mode=mode)
+        out = ibfs_amd.DeviceBuffer(4 * len(src) * V)
+        s.wait(s.submit(src, out))
+        np.testing.assert_array_equal(out.to_host(np.int32, len(src) * V).reshape(-1, V), want)
+        s.close()
+    out = ibfs_amd.DeviceBuffer(4 * 128 * V)
+    g.traversal_noalloc(every[:128], out, ibfs_amd.default_config(emit_mode=mode))
+    np.testing.assert_array_equal(out.to_host().reshape(128, V), depths[:128])
