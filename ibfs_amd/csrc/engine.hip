@@ -849,8 +849,8 @@ static int groupby_small(ibfs_graph_s *g, const int32_t *src, int n, int32_t *ou
     u64 *comp = nullptr;
     hipError_t err = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
     if (err == hipSuccess) err = hipHostMalloc(&post, sizeof(GroupbyPost), hipHostMallocCoherent);
-    if (err == hipSuccess) err = hipMalloc((void **)&comp, sizeof(u64) * (GROUPBY_SMALL + 1));
-    if (err == hipSuccess) err = launch_fill_u64(comp + GROUPBY_SMALL, 1, 0ull, st);
+    if (err == hipSuccess) err = hipMalloc((void **)&comp, sizeof(u64) * (GROUPBY_WORDS + 1));
+    if (err == hipSuccess) err = launch_fill_u64(comp + GROUPBY_WORDS, 1, 0ull, st);
     if (err != hipSuccess) {
       if (comp) (void)hipFree(comp);
       if (post) (void)hipHostFree(post);
@@ -862,7 +862,7 @@ static int groupby_small(ibfs_graph_s *g, const int32_t *src, int n, int32_t *ou
     w.st = st;
     w.post = post;
     w.comp = comp;
-    w.ticket = comp + GROUPBY_SMALL;
+    w.ticket = comp + GROUPBY_WORDS;
   }
   hipStream_t st = (hipStream_t)w.st;
   if (w.unsettled) {  // an earlier call's kernel may still read the sources

@@ -453,9 +453,9 @@ hipError_t launch_two_hop(const int64_t *beg, const int32_t *adj, const int32_t 
 // CSR); keys are traversal ids, whose order is the original order.  ws: device
 // workspace of groupby_workspace_bytes(n) bytes.
 // Up to GROUPBY_SMALL sources in one launch that reads them from, and posts the
-// order to, coherent pinned host memory.  comp: device workspace of as many
-// words; ticket: a zero word, zero again afterwards.
-constexpr int GROUPBY_SMALL = 4096;
+// order to, coherent pinned host memory.  comp: device workspace of
+// GROUPBY_WORDS words (keys, sources); ticket: a zero word, zero again afterwards.
+constexpr int GROUPBY_SMALL = 4096, GROUPBY_WORDS = GROUPBY_SMALL + GROUPBY_SMALL / 2;
 struct GroupbyPost {
   int32_t src[GROUPBY_SMALL];
   int32_t out[GROUPBY_SMALL];

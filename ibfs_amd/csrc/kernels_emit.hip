@@ -734,11 +734,13 @@ __global__ __launch_bounds__(BS) void k_groupby_key(const int64_t *__restrict__ 
 
 // GroupBy of up to GROUPBY_SMALL sources: every wave keys one source, and the
 // last workgroup to finish sorts (key, position) in LDS, bitonic on distinct
-// 64-bit words, which is the stable order.  The keys cross workgroups as
+// 64-bit words, which is the stable order.  Keys and sources cross workgroups as
 // agent-scope stores and loads behind a ticket, the sources and the order
-// cross the bus as system-scope ones.  Bound by its chain: about nine
-// dependent accesses and, for 1,024 sources, 55 steps of the sorting network.
-// 1,024 sources took 52 us with two allocations, two copies and three launches.
+// cross the bus as system-scope ones: the host rewrites the post for the next
+// call, of any graph, without a runtime call that would clear a cache.  Bound
+// by its chain: about nine dependent accesses and, for 1,024 sources, 55 steps
+// of the sorting network.  1,024 sources took 52 us with two allocations, two
+// copies and three launches.
 constexpr int GB_BS = 1024;
 __global__ __launch_bounds__(GB_BS) void k_groupby_small(const int64_t *__restrict__ beg,
                                                          const int32_t *__restrict__ adj,
@@ -750,9 +752,19 @@ __global__ __launch_bounds__(GB_BS) void k_groupby_small(const int64_t *__restri
   __shared__ int32_t s_src[GROUPBY_SMALL];
   __shared__ int last_s;
   const int t = threadIdx.x, lane = t & 63;
-  const int i = blockIdx.x * (GB_BS / 64) + (t >> 6);
+  constexpr int WAVES = GB_BS / 64;
+  const int i0 = blockIdx.x * WAVES, i = i0 + (t >> 6);
+  int32_t *dsrc = reinterpret_cast<int32_t *>(comp + GROUPBY_SMALL);
+  // the workgroup's sources: one request of the host's memory
+  if (t < WAVES && i0 + t < n) {
+    const int32_t s =
+        __hip_atomic_load(&post->src[i0 + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    s_src[t] = s;
+    __hip_atomic_store(&dsrc[i0 + t], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
   if (i < n) {
-    const int32_t h = first_hub(beg, adj, deg, cid, post->src[i], lane);
+    const int32_t h = first_hub(beg, adj, deg, cid, s_src[t >> 6], lane);
     if (lane == 0)
       __hip_atomic_store(&comp[i], (h >= 0 ? (u64)h << 32 : ~0ull << 32) | (unsigned)i,
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -766,7 +778,8 @@ __global__ __launch_bounds__(GB_BS) void k_groupby_small(const int64_t *__restri
   while (N < n) N *= 2;
   for (int k = t; k < N; k += GB_BS) {
     w[k] = k < n ? atomic_read(&comp[k]) : ~0ull;
-    s_src[k] = k < n ? post->src[k] : 0;
+    s_src[k] =
+        k < n ? __hip_atomic_load(&dsrc[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
   }
   if (t == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();

@@ -38,3 +38,17 @@ def test_no_barrier_behind_a_short_circuit(name):
     """A barrier that orders shared memory is reached whatever the operands
     beside it are, compile-time constants among them."""
     assert conditional_barriers(code(name)) == []
+
+
+@pytest.mark.parametrize("name", [n for n in HIP if n.startswith("kernels_")])
+def test_posts_are_read_and_written_past_the_caches(name):
+    """The host rewrites a post (coherent pinned memory) between calls without
+    a runtime call that would clear caches: kernels take and leave its members
+    with system-scope accesses only."""
+    text = code(name)
+    for m in re.finditer(r"\bpost->", text):
+        before = re.split(r"[;{}]", text[:m.start()])[-1]
+        after = re.split(r"[;{}]", text[m.start():])[0]
+        statement = " ".join((before + after).split())
+        assert re.search(r"__hip_atomic_(load|store)\(\s*&[^,]*$", before), statement
+        assert "__HIP_MEMORY_SCOPE_SYSTEM" in after, statement

@@ -258,3 +258,17 @@ def test_emission_of_deep_windows(rows, cols, mode):
     out = ibfs_amd.DeviceBuffer(4 * 128 * V)
     g.traversal_noalloc(every[:128], out, ibfs_amd.default_config(emit_mode=mode))
     np.testing.assert_array_equal(out.to_host().reshape(128, V), depths[:128])
+
+
+def test_groupby_takes_the_sources_of_its_own_call():
+    """Calls of one size with other sources each time, on two graphs in turn
+    and with nothing in between: the block that holds the sources is the same."""
+    say("[gpu] groupby, other sources each call")
+    hosts = [ibfs_amd.HostCsr.rmat(13, 16, seed=s) for s in (1, 2)]
+    graphs = [ibfs_amd.DeviceGraph(h) for h in hosts]
+    rng = np.random.default_rng(0)
+    for n in (1, 16, 700, 4096):
+        lists = [rng.integers(0, 1 << 13, size=n).astype(np.int32) for _ in range(12)]
+        got = [graphs[i % 2].groupby(s) for i, s in enumerate(lists)]
+        for i, s in enumerate(lists):
+            np.testing.assert_array_equal(got[i], oracle.groupby(*hosts[i % 2].arrays(), s))
