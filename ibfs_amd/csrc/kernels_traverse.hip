@@ -588,6 +588,7 @@ __global__ __launch_bounds__(NW * 64) void k_inspect(InspectArgs a) {
     ctl->next_dir = fin.next_dir = dir;
     ctl->next_flag = fin.next_flag = dir == 0 && flag_top_down(fin.m_front, d.V);
   }
+  __syncthreads();  // the decision is in the block that other lanes copy
   if (a.post) {  // one wave: the block's words arrive at the host before the tag
     if (t < (int)CTL_WORDS)
       __hip_atomic_store(&reinterpret_cast<u64 *>(&a.post->c)[t], reinterpret_cast<u64 *>(&fin)[t],

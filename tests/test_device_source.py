@@ -52,3 +52,15 @@ def test_posts_are_read_and_written_past_the_caches(name):
         statement = " ".join((before + after).split())
         assert re.search(r"__hip_atomic_(load|store)\(\s*&[^,]*$", before), statement
         assert "__HIP_MEMORY_SCOPE_SYSTEM" in after, statement
+
+
+def test_a_control_block_is_complete_before_it_is_posted():
+    """One thread decides the next level into the block in LDS; the lanes that
+    copy the block to the host, as other types, do so behind a barrier."""
+    text = code("kernels_traverse.hip")
+    copies = [m.start() for m in
+              re.finditer(r"__hip_atomic_store\(&reinterpret_cast<u64 \*>\(&\w+\.post->c\)", text)]
+    assert len(copies) == 2  # the inspector's last workgroup, the expansion of levels ahead
+    for at in copies:
+        decided = text.rindex("next_flag =", 0, at)
+        assert "__syncthreads();" in text[decided:at]

@@ -272,3 +272,43 @@ def test_groupby_takes_the_sources_of_its_own_call():
         got = [graphs[i % 2].groupby(s) for i, s in enumerate(lists)]
         for i, s in enumerate(lists):
             np.testing.assert_array_equal(got[i], oracle.groupby(*hosts[i % 2].arrays(), s))
+
+
+@pytest.mark.parametrize("opts", [dict(policy=ibfs_amd.POLICY_FIXED, sw_level=1),
+                                  dict(policy=ibfs_amd.POLICY_FIXED, sw_level=3),
+                                  dict(policy=ibfs_amd.POLICY_BU_ONLY),
+                                  dict(hybrid_gamma=0), dict(hybrid_gamma=0, alpha=14, beta=24)])
+def test_posted_directions_follow_the_rule(opts):
+    """The direction of every level is the rule's for the counters posted with
+    it, where the host launches the posted direction's kernel (kernel timing)
+    and where levels are enqueued ahead; both log the same levels."""
+    say(f"[gpu] posted directions {opts}")
+    h = ibfs_amd.HostCsr.rmat(14, 16, seed=6)
+    g = ibfs_amd.DeviceGraph(h)
+    src = h.gen_sources(256, seed=7)
+    want = oracle.bfs_many(*h.arrays(), src, threads=8)
+    cfg = ibfs_amd.default_config(**opts)
+
+    def rule(level, prev, li, li_before):
+        if cfg.policy == ibfs_amd.POLICY_BU_ONLY:
+            return 1
+        if cfg.policy == ibfs_amd.POLICY_FIXED:
+            return 0 if level <= cfg.sw_level else 1
+        if prev != 1:
+            return 1 if li["m_frontier"] * cfg.alpha > li["m_unvisited"] else 0
+        nf = li["n_frontier"]
+        return 0 if nf * cfg.beta < h.vert_count and nf < li_before["n_frontier"] else 1
+
+    logs = []
+    for timing in (1, 0):
+        e = ibfs_amd.Engine(g, lane_bits=128, kernel_timing=timing, **opts)
+        for half, depths in ((src[:128], want[:128]), (src[128:], want[128:])):
+            np.testing.assert_array_equal(e.traversal(half), depths)
+            log = e.level_log()
+            for level in range(1, len(log)):
+                before = log[level - 2] if level > 1 else dict(n_frontier=1 << 62)
+                prev = log[level - 1]["direction"] if level > 1 else -1
+                assert log[level]["direction"] == rule(level, prev, log[level - 1], before), level
+            logs.append([(x["direction"], x["n_changed"], x["n_frontier"], x["n_unvisited"]) for x in log])
+        e.close()
+    assert logs[:2] == logs[2:]
