@@ -101,18 +101,29 @@ class WaitClock {
   unsigned n_ = 0;
 };
 
-// Workspace of small GroupBy calls, one per device: made by the first call,
-// shared by the device's graphs and freed with the last of them.  With one
-// per graph a graph's first call took 150 to 180 us (a stream, pinned memory);
-// now 62 to 93 while another graph has one, and 31 to 58 from the second on.  The mutex serialises calls of several threads.
+// Workspace of one small GroupBy call.
 struct GroupbyWork {
-  std::mutex mu;
   void *st = nullptr;    // hipStream_t
   void *post = nullptr;  // GroupbyPost, coherent pinned
   unsigned long long *comp = nullptr, *ticket = nullptr;
   unsigned long long seq = 0;
-  bool unsettled = false;  // a call failed with work possibly enqueued
+  const void *graph = nullptr;  // of a call that failed with work possibly enqueued
+  GroupbyWork *next = nullptr;
   ~GroupbyWork();
+};
+
+// The workspaces of a device, shared by its graphs and freed with the last of
+// them: a call takes an idle one or makes one, so calls at once, of one graph
+// or of several, do not wait for each other, and keeps it idle for the next (a
+// graph's first call took 150 to 180 us with workspaces of its own, a stream
+// and pinned memory; 62 to 93 with an idle one).  One whose call failed with
+// its kernel possibly enqueued is `late` until the stream has drained.
+struct GroupbyPool {
+  static constexpr int KEEP = 4;  // idle ones kept; late ones past which a call waits
+  std::mutex mu;                  // held for the lists alone
+  GroupbyWork *idle = nullptr, *late = nullptr;
+  int n_idle = 0, n_late = 0;
+  ~GroupbyPool();
 };
 
 }  // namespace ibfs
@@ -149,7 +160,7 @@ struct ibfs_graph_s {
   // hub_entries[i] = traversal-adjacency entries that point to slots < i
   std::vector<int32_t> h_hub_deg, h_hub_id;
   std::vector<int64_t> h_hub_entries;
-  std::shared_ptr<ibfs::GroupbyWork> gb;
+  std::shared_ptr<ibfs::GroupbyPool> gb;
 };
 
 // Pull cut of hybrid levels at the top r hubs (r <= 0 or r > H: all H hubs):

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -479,25 +480,104 @@ int ensure_out(ibfs_engine_s *e, size_t elems) {
   return IBFS_OK;
 }
 
-// The device's GroupBy workspace, empty until a call fills it.
-std::shared_ptr<GroupbyWork> groupby_work(int device) {
+// The device's GroupBy workspaces (null without host memory for them: GroupBy
+// then takes the form of large source sets).
+std::shared_ptr<GroupbyPool> groupby_pool(int device) {
   static std::mutex mu;
-  static std::vector<std::weak_ptr<GroupbyWork>> of;
-  std::lock_guard<std::mutex> lk(mu);
-  if ((size_t)device >= of.size()) of.resize((size_t)device + 1);
-  auto w = of[(size_t)device].lock();
-  if (!w) of[(size_t)device] = w = std::make_shared<GroupbyWork>();
-  return w;
+  static std::vector<std::weak_ptr<GroupbyPool>> of;
+  try {
+    std::lock_guard<std::mutex> lk(mu);
+    if ((size_t)device >= of.size()) of.resize((size_t)device + 1);
+    auto w = of[(size_t)device].lock();
+    if (!w) of[(size_t)device] = w = std::make_shared<GroupbyPool>();
+    return w;
+  } catch (...) {
+    return nullptr;
+  }
+}
+
+// A workspace for one call, in *out.
+int groupby_take(GroupbyPool &p, GroupbyWork **out) {
+  for (WaitClock clk;;) {
+    {
+      std::lock_guard<std::mutex> lk(p.mu);
+      for (GroupbyWork **at = &p.late; *at;) {
+        GroupbyWork *w = *at;
+        if (hipStreamQuery((hipStream_t)w->st) == hipSuccess) {
+          *at = w->next;
+          --p.n_late;
+          w->next = p.idle;
+          p.idle = w;
+          ++p.n_idle;
+        } else {
+          at = &w->next;
+        }
+      }
+      if (p.idle) {
+        *out = p.idle;
+        p.idle = p.idle->next;
+        --p.n_idle;
+        return IBFS_OK;
+      }
+      if (p.n_late < GroupbyPool::KEEP) break;
+    }
+    if (clk.expired())
+      return fail(IBFS_ERR_STATE, "groupby: earlier calls did not finish within the wait limit (%.1f s)",
+                  wait_timeout_s());
+  }
+  GroupbyWork *w = new (std::nothrow) GroupbyWork();
+  if (!w) return fail(IBFS_ERR_NOMEM, "groupby workspace");
+  hipStream_t st = nullptr;
+  hipError_t err = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+  w->st = st;
+  if (err == hipSuccess) err = hipHostMalloc(&w->post, sizeof(GroupbyPost), hipHostMallocCoherent);
+  if (err == hipSuccess) err = hipMalloc((void **)&w->comp, sizeof(u64) * (GROUPBY_WORDS + 1));
+  if (err == hipSuccess) err = launch_fill_u64(w->comp + GROUPBY_WORDS, 1, 0ull, st);
+  if (err != hipSuccess) {
+    delete w;
+    return fail(err == hipErrorOutOfMemory ? IBFS_ERR_NOMEM : IBFS_ERR_HIP,
+                "groupby workspace: %s", hipGetErrorString(err));
+  }
+  std::memset(w->post, 0, sizeof(GroupbyPost));
+  w->ticket = w->comp + GROUPBY_WORDS;
+  *out = w;
+  return IBFS_OK;
+}
+
+// Gives a workspace back; of (or null): the graph that its kernel may still read.
+void groupby_put(GroupbyPool &p, GroupbyWork *w, const void *of) {
+  w->graph = of;
+  {
+    std::lock_guard<std::mutex> lk(p.mu);
+    if (of || p.n_idle < GroupbyPool::KEEP) {
+      GroupbyWork *&list = of ? p.late : p.idle;
+      w->next = list;
+      list = w;
+      ++(of ? p.n_late : p.n_idle);
+      return;
+    }
+  }
+  delete w;  // more calls at once than are kept
 }
 
 }  // namespace
 
 ibfs::GroupbyWork::~GroupbyWork() {
-  if (!st) return;
-  (void)hipStreamSynchronize((hipStream_t)st);
-  (void)hipStreamDestroy((hipStream_t)st);
-  (void)hipHostFree(post);
-  (void)hipFree(comp);
+  if (st) {
+    (void)hipStreamSynchronize((hipStream_t)st);
+    (void)hipStreamDestroy((hipStream_t)st);
+  }
+  if (post) (void)hipHostFree(post);
+  if (comp) (void)hipFree(comp);
+}
+
+ibfs::GroupbyPool::~GroupbyPool() {
+  for (GroupbyWork *list : {idle, late})
+    while (list) {
+      GroupbyWork *w = list;
+      list = w->next;
+      delete w;
+    }
 }
 
 HubCut hub_cut(const ibfs_graph_s *g, int64_t r) {
@@ -776,7 +856,7 @@ int ibfs_graph_create_ex(const int64_t *beg, int64_t V, const int32_t *adj, int6
     return fail(err == hipErrorOutOfMemory ? IBFS_ERR_NOMEM : IBFS_ERR_HIP,
                 "graph upload failed: %s", hipGetErrorString(err));
   }
-  g->gb = groupby_work(device);
+  g->gb = groupby_pool(device);
   *out = g;
   return IBFS_OK;
 }
@@ -820,10 +900,27 @@ int ibfs_graph_hub_entries(ibfs_graph_t g, int64_t top, int64_t *entries) {
 int ibfs_graph_destroy(ibfs_graph_t g) {
   if (!g) return IBFS_OK;
   (void)hipSetDevice(g->device);
-  if (g->gb) {  // an earlier call's kernel may still read the graph
-    std::lock_guard<std::mutex> lk(g->gb->mu);
-    if (g->gb->unsettled) (void)hipStreamSynchronize((hipStream_t)g->gb->st);
-    g->gb->unsettled = false;
+  if (g->gb) {  // a failed call's kernel may still read the graph
+    GroupbyWork *mine = nullptr;
+    {
+      std::lock_guard<std::mutex> lk(g->gb->mu);
+      for (GroupbyWork **at = &g->gb->late; *at;) {
+        GroupbyWork *w = *at;
+        if (w->graph == g) {
+          *at = w->next;
+          --g->gb->n_late;
+          w->next = mine;
+          mine = w;
+        } else {
+          at = &w->next;
+        }
+      }
+    }
+    while (mine) {  // waits for its stream
+      GroupbyWork *w = mine;
+      mine = w->next;
+      delete w;
+    }
   }
   dfree(g->d_beg);
   dfree(g->d_adj);
@@ -839,48 +936,26 @@ int ibfs_graph_destroy(ibfs_graph_t g) {
 
 }  // extern "C"
 
-// GroupBy through the device's workspace (n <= GROUPBY_SMALL).
+// GroupBy through a workspace of the device (n <= GROUPBY_SMALL).
 static int groupby_small(ibfs_graph_s *g, const int32_t *src, int n, int32_t *out) {
-  auto &w = *g->gb;
-  std::lock_guard<std::mutex> lk(w.mu);
-  if (!w.st) {
-    hipStream_t st = nullptr;
-    void *post = nullptr;
-    u64 *comp = nullptr;
-    hipError_t err = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
-    if (err == hipSuccess) err = hipHostMalloc(&post, sizeof(GroupbyPost), hipHostMallocCoherent);
-    if (err == hipSuccess) err = hipMalloc((void **)&comp, sizeof(u64) * (GROUPBY_WORDS + 1));
-    if (err == hipSuccess) err = launch_fill_u64(comp + GROUPBY_WORDS, 1, 0ull, st);
-    if (err != hipSuccess) {
-      if (comp) (void)hipFree(comp);
-      if (post) (void)hipHostFree(post);
-      if (st) (void)hipStreamDestroy(st);
-      return fail(err == hipErrorOutOfMemory ? IBFS_ERR_NOMEM : IBFS_ERR_HIP,
-                  "groupby workspace: %s", hipGetErrorString(err));
-    }
-    std::memset(post, 0, sizeof(GroupbyPost));
-    w.st = st;
-    w.post = post;
-    w.comp = comp;
-    w.ticket = comp + GROUPBY_WORDS;
-  }
-  hipStream_t st = (hipStream_t)w.st;
-  if (w.unsettled) {  // an earlier call's kernel may still read the sources
-    HIP_TRY(hipStreamSynchronize(st));
-    w.unsettled = false;
-  }
-  auto *post = static_cast<GroupbyPost *>(w.post);
+  GroupbyWork *w = nullptr;
+  if (int rc = groupby_take(*g->gb, &w)) return rc;
+  hipStream_t st = (hipStream_t)w->st;
+  auto *post = static_cast<GroupbyPost *>(w->post);
   std::memcpy(post->src, src, sizeof(int32_t) * (size_t)n);
-  const u64 tag = ++w.seq;
+  const u64 tag = ++w->seq;
   clear_hip_error();
-  HIP_TRY(launch_groupby_small(g->d_beg, g->d_adj, g->d_deg, g->d_cid, n, post, w.comp,
-                               reinterpret_cast<unsigned *>(w.ticket), tag, st));
-  if (int rc = wait_tag(st, &post->tag, tag, "groupby")) {
-    w.unsettled = true;
-    return rc;
-  }
-  std::memcpy(out, post->out, sizeof(int32_t) * (size_t)n);
-  return IBFS_OK;
+  const hipError_t err = launch_groupby_small(g->d_beg, g->d_adj, g->d_deg, g->d_cid, n, post,
+                                              w->comp, reinterpret_cast<unsigned *>(w->ticket),
+                                              tag, st);
+  int rc = IBFS_OK;
+  if (err != hipSuccess)
+    rc = fail(IBFS_ERR_HIP, "groupby launch: %s", hipGetErrorString(err));
+  else
+    rc = wait_tag(st, &post->tag, tag, "groupby");
+  if (rc == IBFS_OK) std::memcpy(out, post->out, sizeof(int32_t) * (size_t)n);
+  groupby_put(*g->gb, w, rc == IBFS_OK ? nullptr : g);
+  return rc;
 }
 
 extern "C" {
@@ -893,7 +968,7 @@ int ibfs_groupby(ibfs_graph_t g, const int32_t *src, int64_t n, int32_t *out) {
       return fail(IBFS_ERR_ARG, "source %lld = %d out of range", (long long)i, src[i]);
   int rc = check_device(g->device);
   if (rc) return rc;
-  if (n <= GROUPBY_SMALL) return groupby_small(g, src, (int)n, out);
+  if (n <= GROUPBY_SMALL && g->gb) return groupby_small(g, src, (int)n, out);
   int32_t *d = nullptr;
   void *ws = nullptr;
   const size_t wsb = groupby_workspace_bytes(n);

@@ -312,3 +312,81 @@ def test_posted_directions_follow_the_rule(opts):
             logs.append([(x["direction"], x["n_changed"], x["n_frontier"], x["n_unvisited"]) for x in log])
         e.close()
     assert logs[:2] == logs[2:]
+
+
+def test_groupby_calls_do_not_wait_for_each_other():
+    """Two threads, each with its graph: calls overlap on the device, so both
+    take well under the time that one thread takes for all of them (half of it
+    where they overlap, nearly all of it where a call waits for the other's)."""
+    import threading
+    import time
+    say("[gpu] groupby of two graphs at once")
+    hosts = [ibfs_amd.HostCsr.rmat(14, 16, seed=s) for s in (3, 4)]
+    graphs = [ibfs_amd.DeviceGraph(h) for h in hosts]
+    lists = [np.random.default_rng(s).integers(0, 1 << 14, size=4096).astype(np.int32) for s in (3, 4)]
+
+    def calls(i, out=None):
+        for _ in range(300):
+            got = graphs[i].groupby(lists[i])
+        if out is not None:
+            out[i] = got
+
+    def at_once(out):
+        threads = [threading.Thread(target=calls, args=(i, out)) for i in (0, 1)]
+        t0 = time.perf_counter()
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(timeout=60)
+        return time.perf_counter() - t0
+
+    def in_turn():
+        t0 = time.perf_counter()
+        calls(0)
+        calls(1)
+        return time.perf_counter() - t0
+
+    got = [None, None]
+    at_once(got)
+    for h, src, o in zip(hosts, lists, got):
+        np.testing.assert_array_equal(o, oracle.groupby(*h.arrays(), src))
+    ratio = min(at_once(got) for _ in range(5)) / min(in_turn() for _ in range(5))
+    say(f"[gpu] at once / in turn: {ratio:.2f}")
+    assert ratio < 0.75
+
+
+def test_groupby_past_the_wait_limit():
+    """Calls that give up (the limit set from the host; their kernels end
+    normally) from many threads, then closing their graph, and calls of another
+    graph before and after it: exact, and no call of the other graph fails."""
+    import threading
+    say("[gpu] groupby past the wait limit")
+    h = ibfs_amd.HostCsr.rmat(14, 16, seed=5)
+    src = np.random.default_rng(5).integers(0, 1 << 14, size=4096).astype(np.int32)
+    want = oracle.groupby(*h.arrays(), src)
+    other = ibfs_amd.DeviceGraph(h)
+    for _ in range(3):
+        g = ibfs_amd.DeviceGraph(h)
+        codes = []
+
+        def work():
+            for _ in range(8):
+                try:
+                    np.testing.assert_array_equal(g.groupby(src), want)
+                except ibfs_amd.IbfsError as e:
+                    codes.append(e.code)
+
+        old = ibfs_amd.get_wait_timeout()
+        ibfs_amd.set_wait_timeout(1e-9)
+        try:
+            threads = [threading.Thread(target=work) for _ in range(6)]
+            for t in threads:
+                t.start()
+            for t in threads:
+                t.join(timeout=60)
+        finally:
+            ibfs_amd.set_wait_timeout(old)
+        assert set(codes) <= {ibfs_amd._lib.IBFS_ERR_STATE}
+        np.testing.assert_array_equal(other.groupby(src), want)
+        g.close()
+        np.testing.assert_array_equal(other.groupby(src), want)
