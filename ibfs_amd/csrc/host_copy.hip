@@ -8,15 +8,13 @@
 // engine fills one chunk while eight host threads copy the other out, which
 // measured 55 GB/s into pageable memory (8 and 16 threads alike; 4 threads
 // 46 GB/s).
+#include "copy_pool.h"
 #include "host_copy.h"
 
 #include <algorithm>
-#include <atomic>
-#include <condition_variable>
 #include <cstdint>
 #include <cstring>
 #include <mutex>
-#include <thread>
 #include <vector>
 
 #include "common.h"
@@ -30,90 +28,8 @@ constexpr size_t kChunk = size_t(64) << 20;
 // of one or two chunks in parts of a whole chunk is not pipelined at all
 // (67 MB with its traversal 2.6 ms, in quarters 1.9 ms).
 constexpr size_t kMinPart = size_t(4) << 20;
-constexpr int kThreads = 8;
 // copies below this size keep the runtime's path (no pipeline to fill)
 constexpr size_t kDirect = size_t(4) << 20;
-
-// Host threads that copy the parts of one transfer, each thread its slice of
-// every part.  They are woken once per transfer and then spin for the next part
-// (a wake-up of eight sleeping threads costs about as much as copying 8 MB);
-// between transfers they sleep.  They live as long as the process.
-class CopyPool {
- public:
-  struct Part {
-    char *dst;
-    const char *src;
-    size_t bytes;
-    std::atomic<int> left{kThreads};
-  };
-
-  CopyPool() {
-    for (int k = 0; k < kThreads; ++k) th_.emplace_back([this, k] { run(k); });
-  }
-
-  // Starts a transfer of n parts; part j is copied once ready(j + 1) was called.
-  void begin(Part *parts, int n) {
-    std::lock_guard<std::mutex> lk(mu_);
-    parts_ = parts;
-    n_ = n;
-    ready_.store(0, std::memory_order_relaxed);
-    left_ = kThreads;
-    ++gen_;
-    go_.notify_all();
-  }
-  void ready(int n) { ready_.store(n, std::memory_order_release); }
-  void wait_part(int j) {
-    for (unsigned i = 1; parts_[j].left.load(std::memory_order_acquire) > 0; ++i)
-      if ((i & 255) == 0) std::this_thread::yield();
-  }
-  // Ends the transfer (parts not yet ready are dropped): no thread touches
-  // the parts afterwards.
-  void end() {
-    ready_.store(-1, std::memory_order_release);
-    std::unique_lock<std::mutex> lk(mu_);
-    done_.wait(lk, [this] { return left_ == 0; });
-  }
-
- private:
-  void run(int k) {
-    uint64_t seen = 0;
-    for (;;) {
-      Part *p;
-      int n;
-      {
-        std::unique_lock<std::mutex> lk(mu_);
-        go_.wait(lk, [&] { return gen_ != seen; });
-        seen = gen_;
-        p = parts_;
-        n = n_;
-      }
-      for (int j = 0; j < n; ++j) {
-        int r = 0;
-        for (unsigned i = 1;; ++i) {
-          r = ready_.load(std::memory_order_acquire);
-          if (r > j || r < 0) break;
-          if ((i & 255) == 0) std::this_thread::yield();
-        }
-        if (r < 0) break;
-        const size_t b = p[j].bytes;
-        const size_t lo = b * (size_t)k / kThreads, hi = b * (size_t)(k + 1) / kThreads;
-        if (hi > lo) std::memcpy(p[j].dst + lo, p[j].src + lo, hi - lo);
-        p[j].left.fetch_sub(1, std::memory_order_release);
-      }
-      std::lock_guard<std::mutex> lk(mu_);
-      if (--left_ == 0) done_.notify_one();
-    }
-  }
-
-  std::vector<std::thread> th_;
-  std::mutex mu_;
-  std::condition_variable go_, done_;
-  Part *parts_ = nullptr;
-  int n_ = 0;
-  std::atomic<int> ready_{0};
-  int left_ = 0;
-  uint64_t gen_ = 0;
-};
 
 // The pinned chunks and the pool, made on first use and kept for the
 // process; one pipelined copy at a time.
@@ -202,7 +118,8 @@ int copy_to_host(const D2HPiece *pieces, size_t n, hipStream_t st) {
     parts[j].src = s.pin + (j & 1) * kChunk;
     parts[j].bytes = q[j].bytes;
   }
-  s.pool->begin(parts.data(), (int)q.size());
+  // parts of a whole chunk (from 256 MiB on): a wake-up is little beside a part
+  s.pool->begin(parts.data(), (int)q.size(), part < kChunk);
   size_t issued = 0;
   for (size_t j = 0; rc == IBFS_OK && j <= q.size(); ++j) {
     if (j < q.size()) {
