@@ -96,6 +96,7 @@ struct ibfs_batch_s {
   ibfs_config cfg{};
   int K = 128, W = 2, R = 16, C = 2, burst = 8, chunk_shift = 12, grid = 2048;
   HubCut hc;  // hubs a hybrid level pulls through
+  HeadsUse heads;
   std::vector<Ctx> ctx;
   // grouping order of the current run: order[p] = caller's index of the
   // source at position p (groups are consecutive positions); psrc = sources
@@ -466,6 +467,16 @@ int finish_group(ibfs_batch_s *b, Ctx &c, int last, ibfs_stats *stats) {
   return IBFS_OK;
 }
 
+int alloc_batch(ibfs_batch_s *b) {
+  b->ctx.resize((size_t)b->C);
+  hipError_t err = hipMalloc((void **)&b->d_edges, sizeof(u64));
+  if (err == hipSuccess) err = hipHostMalloc((void **)&b->h_edges, sizeof(u64), hipHostMallocDefault);
+  if (err != hipSuccess) return fail(IBFS_ERR_NOMEM, "batch allocation failed");
+  for (auto &c : b->ctx)
+    if (int rc = alloc_ctx(b, c)) return rc;
+  return IBFS_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -520,21 +531,16 @@ int ibfs_batch_create(ibfs_graph_t g, const ibfs_config *cfg_in, int32_t context
   // sources on s22 8.36, 8.49; closeness on a 1,024 x 1,024 grid 230, 250.
   b->grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 4;
   b->hc = hub_cut(b->g, cfg.hybrid_hubs);
-  b->ctx.resize(contexts);
-  hipError_t err = hipMalloc((void **)&b->d_edges, sizeof(u64));
-  if (err == hipSuccess) err = hipHostMalloc((void **)&b->h_edges, sizeof(u64), hipHostMallocDefault);
-  if (err != hipSuccess) {
+  b->heads.take(g->heads);
+  int rc = alloc_batch(b);
+  if (rc == IBFS_ERR_NOMEM && b->heads.drop()) {
+    release_batch(b);
+    rc = alloc_batch(b);
+  }
+  if (rc) {
     release_batch(b);
     delete b;
-    return fail(IBFS_ERR_NOMEM, "batch allocation failed");
-  }
-  for (auto &c : b->ctx) {
-    int rc = alloc_ctx(b, c);
-    if (rc) {
-      release_batch(b);
-      delete b;
-      return rc;
-    }
+    return rc;
   }
   *out = b;
   return IBFS_OK;

@@ -126,6 +126,32 @@ struct GroupbyPool {
   ~GroupbyPool();
 };
 
+// The first 8 entries of each traversal-adjacency list, 32 bytes per vertex.
+// Bottom-up levels read them faster than the lists, and nothing needs them: a
+// graph is made without where the memory left does not hold them, and a handle
+// whose own buffers do not fit frees them if it is the graph's only one.
+struct GraphHeads {
+  std::mutex mu;
+  int users = 0;         // handles and running calls whose kernels may read d
+  int32_t *d = nullptr;  // 2 x Vt x 4, or null
+};
+
+// A handle's (or call's) use of its graph's heads, from before its first
+// allocation until after its last kernel.
+class HeadsUse {
+ public:
+  HeadsUse() = default;
+  HeadsUse(const HeadsUse &) = delete;
+  ~HeadsUse();
+  void take(const std::shared_ptr<GraphHeads> &h);
+  // Frees the heads if there are any and nobody else uses them (the caller has
+  // no kernel in flight); whether it did.
+  bool drop();
+
+ private:
+  std::shared_ptr<GraphHeads> h_;
+};
+
 }  // namespace ibfs
 
 struct ibfs_hostcsr_s {
@@ -148,7 +174,7 @@ struct ibfs_graph_s {
   int64_t *d_beg = nullptr;   // Vt+1, traversal ids
   int32_t *d_adj = nullptr;   // adjacency in input order (top-down, GroupBy)
   int32_t *d_tadj = nullptr;  // traversal adjacency: by descending degree, hubs encoded
-  int32_t *d_head = nullptr;  // 2 x Vt x 4: the first 8 entries of each traversal-adjacency list
+  std::shared_ptr<ibfs::GraphHeads> heads = std::make_shared<ibfs::GraphHeads>();
   int32_t *d_deg = nullptr;   // Vt
   int32_t *d_hubs = nullptr;  // the H highest-degree vertices
   int32_t *d_cid = nullptr;   // V: original id -> traversal id or -1

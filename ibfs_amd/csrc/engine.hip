@@ -33,6 +33,7 @@ struct ibfs_engine_s {
   int K = 128, W = 2, Wmax = 2, R = 32, chunk_shift = 12;
   int hy_grid = 8192, next_grid = 8192;  // workgroups of a hybrid level, of one enqueued ahead
   HubCut hc;           // hubs a hybrid level pulls through
+  HeadsUse heads;
   hipStream_t st = nullptr;
   hipEvent_t ev_wait = nullptr;  // recorded after each host copy the loop waits for
   u64 *ring = nullptr;
@@ -208,6 +209,36 @@ void engine_release(ibfs_engine_s *e) {
   e->ev_wait = nullptr;
   if (e->st) (void)hipStreamDestroy(e->st);
   e->st = nullptr;
+}
+
+// The engine's stream, event and buffers, for its settings.
+hipError_t engine_alloc(ibfs_engine_s *e) {
+  const ibfs_graph_s *g = e->g;
+  const int64_t Vt = std::max<int64_t>(g->Vt, 1);
+  hipError_t err = hipStreamCreateWithFlags(&e->st, hipStreamNonBlocking);
+  if (err == hipSuccess) err = hipEventCreateWithFlags(&e->ev_wait, hipEventDisableTiming);
+  auto A = [&](void **p, size_t bytes) {
+    if (err == hipSuccess) err = hipMalloc(p, bytes ? bytes : 1);
+  };
+  auto H = [&](void **p, size_t bytes) {
+    if (err == hipSuccess) err = hipHostMalloc(p, bytes ? bytes : 1, hipHostMallocDefault);
+  };
+  A((void **)&e->ring, (size_t)e->R * (size_t)Vt * (size_t)e->W * sizeof(u64));
+  A((void **)&e->d_ctl, ctl_ring_bytes(e->R));
+  if (err == hipSuccess) err = hipHostMalloc((void **)&e->post, POSTS * sizeof(CtlPost), hipHostMallocCoherent);
+  if (err == hipSuccess) std::memset(e->post, 0, POSTS * sizeof(CtlPost));
+  if (err == hipSuccess) err = hipHostMalloc((void **)&e->post_end, sizeof(GroupPost), hipHostMallocCoherent);
+  if (err == hipSuccess) std::memset(e->post_end, 0, sizeof(GroupPost));
+  for (int i = 0; i < NQ; ++i)
+    if (i != Q_TD_L) A((void **)&e->q.q[i], sizeof(int32_t) * queue_entries((size_t)Vt));
+  A((void **)&e->q.chunks, sizeof(int2) * chunk_entries((size_t)Vt, (size_t)g->E, e->chunk_shift));
+  A((void **)&e->d_masks, sizeof(u64) * masks_words(e));
+  A((void **)&e->d_lanes, sizeof(LaneOut) * (size_t)e->K);
+  A((void **)&e->hs, sizeof(u64) * (size_t)e->W * (size_t)std::max<int64_t>(g->H, 1));
+  A((void **)&e->flags, sizeof(u64) * (size_t)((Vt + 7) / 8));
+  A((void **)&e->d_count, 4 * sizeof(u64));
+  H((void **)&e->h_count, 4 * sizeof(u64));
+  return err;
 }
 
 u64 *slot(ibfs_engine_s *e, int L) {
@@ -475,7 +506,10 @@ int ensure_out(ibfs_engine_s *e, size_t elems) {
   if (e->d_out_cap >= elems) return IBFS_OK;
   dfree(e->d_out);
   e->d_out_cap = 0;
-  HIP_TRY(hipMalloc((void **)&e->d_out, elems * sizeof(int32_t)));
+  hipError_t err = hipMalloc((void **)&e->d_out, elems * sizeof(int32_t));
+  if (err == hipErrorOutOfMemory && e->heads.drop())
+    err = hipMalloc((void **)&e->d_out, elems * sizeof(int32_t));
+  HIP_TRY(err);
   e->d_out_cap = elems;
   return IBFS_OK;
 }
@@ -578,6 +612,26 @@ ibfs::GroupbyPool::~GroupbyPool() {
       list = w->next;
       delete w;
     }
+}
+
+ibfs::HeadsUse::~HeadsUse() {
+  if (!h_) return;
+  std::lock_guard<std::mutex> lk(h_->mu);
+  --h_->users;
+}
+
+void ibfs::HeadsUse::take(const std::shared_ptr<GraphHeads> &h) {
+  h_ = h;
+  std::lock_guard<std::mutex> lk(h_->mu);
+  ++h_->users;
+}
+
+bool ibfs::HeadsUse::drop() {
+  std::lock_guard<std::mutex> lk(h_->mu);
+  if (!h_->d || h_->users > 1) return false;
+  dfree(h_->d);
+  clear_hip_error();
+  return true;
 }
 
 HubCut hub_cut(const ibfs_graph_s *g, int64_t r) {
@@ -821,18 +875,32 @@ int ibfs_graph_create_ex(const int64_t *beg, int64_t V, const int32_t *adj, int6
   }
   const size_t eb = sizeof(int32_t) * (size_t)std::max<int64_t>(E, 1);
   const size_t vtb = sizeof(int32_t) * (size_t)std::max<int64_t>(Vt, 1);
-  hipError_t err = hipMalloc((void **)&g->d_beg, sizeof(int64_t) * (size_t)(Vt + 1));
-  if (err == hipSuccess) err = hipMalloc((void **)&g->d_adj, eb);
-  if (err == hipSuccess) err = hipMalloc((void **)&g->d_tadj, eb);
-  if (err == hipSuccess) err = hipMalloc((void **)&g->d_head, sizeof(int4) * 2 * (size_t)std::max<int64_t>(Vt, 1));
-  if (err == hipSuccess) err = hipMalloc((void **)&g->d_deg, vtb);
-  if (err == hipSuccess) err = hipMalloc((void **)&g->d_hubs, sizeof(int32_t) * (size_t)std::max<int64_t>(H, 1));
-  if (err == hipSuccess) err = hipMalloc((void **)&g->d_cid, sizeof(int32_t) * (size_t)V);
-  if (err == hipSuccess) err = hipMalloc((void **)&g->d_vid, vtb);
+  // the heads are made where memory holds them beside the rest
+  int32_t *&head = g->heads->d;
+  hipError_t err = hipSuccess;
+  auto A = [&](void **p, size_t bytes) {
+    if (err != hipSuccess) return;
+    err = hipMalloc(p, bytes);
+    if (err == hipErrorOutOfMemory && head) {
+      dfree(head);
+      err = hipMalloc(p, bytes);
+    }
+  };
+  A((void **)&g->d_beg, sizeof(int64_t) * (size_t)(Vt + 1));
+  A((void **)&g->d_adj, eb);
+  A((void **)&g->d_tadj, eb);
+  if (err == hipSuccess &&
+      hipMalloc((void **)&head, sizeof(int4) * 2 * (size_t)std::max<int64_t>(Vt, 1)) != hipSuccess)
+    head = nullptr;
+  A((void **)&g->d_deg, vtb);
+  A((void **)&g->d_hubs, sizeof(int32_t) * (size_t)std::max<int64_t>(H, 1));
+  A((void **)&g->d_cid, sizeof(int32_t) * (size_t)V);
+  A((void **)&g->d_vid, vtb);
+  clear_hip_error();
   if (err == hipSuccess) err = hipMemcpy(g->d_beg, tbeg.data(), sizeof(int64_t) * (size_t)(Vt + 1), hipMemcpyHostToDevice);
   if (err == hipSuccess && E > 0) err = hipMemcpy(g->d_adj, xadj.data(), sizeof(int32_t) * (size_t)E, hipMemcpyHostToDevice);
   if (err == hipSuccess && E > 0) err = hipMemcpy(g->d_tadj, tadj.data(), sizeof(int32_t) * (size_t)E, hipMemcpyHostToDevice);
-  if (err == hipSuccess) err = launch_build_head(g->d_beg, g->d_tadj, Vt, reinterpret_cast<int4 *>(g->d_head), nullptr);
+  if (err == hipSuccess && head) err = launch_build_head(g->d_beg, g->d_tadj, Vt, reinterpret_cast<int4 *>(head), nullptr);
   if (err == hipSuccess && Vt > 0) err = hipMemcpy(g->d_deg, tdeg.data(), sizeof(int32_t) * (size_t)Vt, hipMemcpyHostToDevice);
   if (err == hipSuccess && H > 0) err = hipMemcpy(g->d_hubs, order.data(), sizeof(int32_t) * (size_t)H, hipMemcpyHostToDevice);
   if (err == hipSuccess) err = hipMemcpy(g->d_cid, cid.data(), sizeof(int32_t) * (size_t)V, hipMemcpyHostToDevice);
@@ -847,7 +915,7 @@ int ibfs_graph_create_ex(const int64_t *beg, int64_t V, const int32_t *adj, int6
     dfree(g->d_beg);
     dfree(g->d_adj);
     dfree(g->d_tadj);
-    dfree(g->d_head);
+    dfree(head);
     dfree(g->d_deg);
     dfree(g->d_hubs);
     dfree(g->d_cid);
@@ -925,7 +993,7 @@ int ibfs_graph_destroy(ibfs_graph_t g) {
   dfree(g->d_beg);
   dfree(g->d_adj);
   dfree(g->d_tadj);
-  dfree(g->d_head);
+  dfree(g->heads->d);
   dfree(g->d_deg);
   dfree(g->d_hubs);
   dfree(g->d_cid);
@@ -1039,29 +1107,12 @@ int ibfs_engine_create(ibfs_graph_t g, const ibfs_config *cfg_in, ibfs_engine_t 
   const size_t budget = (size_t)8 << 30;
   while (R > 4 && (size_t)R * slot_bytes > budget) --R;
   e->R = R;
-  hipError_t err = hipStreamCreateWithFlags(&e->st, hipStreamNonBlocking);
-  if (err == hipSuccess) err = hipEventCreateWithFlags(&e->ev_wait, hipEventDisableTiming);
-  auto A = [&](void **p, size_t bytes) {
-    if (err == hipSuccess) err = hipMalloc(p, bytes ? bytes : 1);
-  };
-  auto H = [&](void **p, size_t bytes) {
-    if (err == hipSuccess) err = hipHostMalloc(p, bytes ? bytes : 1, hipHostMallocDefault);
-  };
-  A((void **)&e->ring, (size_t)R * slot_bytes);
-  A((void **)&e->d_ctl, ctl_ring_bytes(R));
-  if (err == hipSuccess) err = hipHostMalloc((void **)&e->post, POSTS * sizeof(CtlPost), hipHostMallocCoherent);
-  if (err == hipSuccess) std::memset(e->post, 0, POSTS * sizeof(CtlPost));
-  if (err == hipSuccess) err = hipHostMalloc((void **)&e->post_end, sizeof(GroupPost), hipHostMallocCoherent);
-  if (err == hipSuccess) std::memset(e->post_end, 0, sizeof(GroupPost));
-  for (int i = 0; i < NQ; ++i)
-    if (i != Q_TD_L) A((void **)&e->q.q[i], sizeof(int32_t) * queue_entries((size_t)Vt));
-  A((void **)&e->q.chunks, sizeof(int2) * chunk_entries((size_t)Vt, (size_t)g->E, e->chunk_shift));
-  A((void **)&e->d_masks, sizeof(u64) * masks_words(e));
-  A((void **)&e->d_lanes, sizeof(LaneOut) * (size_t)e->K);
-  A((void **)&e->hs, sizeof(u64) * (size_t)e->W * (size_t)std::max<int64_t>(g->H, 1));
-  A((void **)&e->flags, sizeof(u64) * (size_t)((Vt + 7) / 8));
-  A((void **)&e->d_count, 4 * sizeof(u64));
-  H((void **)&e->h_count, 4 * sizeof(u64));
+  e->heads.take(g->heads);
+  hipError_t err = engine_alloc(e);
+  if (err == hipErrorOutOfMemory && e->heads.drop()) {
+    engine_release(e);
+    err = engine_alloc(e);
+  }
   if (err != hipSuccess) {
     engine_release(e);
     delete e;

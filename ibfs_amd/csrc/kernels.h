@@ -226,7 +226,8 @@ struct EmitSpace {
 struct GraphDev {
   const int64_t *beg;
   const int32_t *adj, *tadj;
-  const int4 *head;  // first 8 traversal-adjacency entries of each vertex: [v] and [V + v]
+  const int4 *head;  // first 8 traversal-adjacency entries of each vertex: [v] and [V + v]; or
+                     // null (no memory for them): read from the lists
   int64_t V;         // traversal vertices
   int lrg, chunk_shift;
   HubSplit hsp;

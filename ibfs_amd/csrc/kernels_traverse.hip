@@ -808,6 +808,18 @@ __device__ __forceinline__ bool bu_four(const Gather &gs, const int32_t (&a)[4],
   return !end && !covers<W>(x, lam);
 }
 
+// Entries 4 * part to 4 * part + 3 of v's traversal adjacency.
+__device__ __forceinline__ int4 list_head(const int64_t *__restrict__ beg,
+                                          const int32_t *__restrict__ tadj, int64_t v, int part) {
+  const int64_t j = beg[v] + 4 * part, e = beg[v + 1];
+  return make_int4(j < e ? tadj[j] : NO_NBR, j + 1 < e ? tadj[j + 1] : NO_NBR,
+                   j + 2 < e ? tadj[j + 2] : NO_NBR, j + 3 < e ? tadj[j + 3] : NO_NBR);
+}
+
+__device__ __forceinline__ int4 head_entries(const GraphDev &g, int64_t v, int part) {
+  return g.head ? g.head[part * g.V + v] : list_head(g.beg, g.tadj, v, part);
+}
+
 constexpr int BU_ROW = 4;   // entries per lane and step of the row class
 constexpr int BU_BIG = 16;  // vertices of the workgroup class staged at a time
 
@@ -885,7 +897,7 @@ __device__ __forceinline__ void bu_tile(const GraphDev &g, const Gather &gs, u64
   bool pend = false;
   const u64 *own = cur + v * W;
   if (v >= 0) {
-    const int4 h = g.head[v];
+    const int4 h = head_entries(g, v, 0);
     load_word<W>(own, x);
 #pragma unroll
     for (int w = 0; w < W; ++w) x0[w] = x[w];
@@ -893,7 +905,7 @@ __device__ __forceinline__ void bu_tile(const GraphDev &g, const Gather &gs, u64
       const int32_t a[4] = {h.x, h.y, h.z, h.w};
       pend = bu_four<W, MODE>(gs, a, own, lam, cut, x);
       if (pend) {
-        const int4 h1 = g.head[g.V + v];
+        const int4 h1 = head_entries(g, v, 1);
         const int32_t a1[4] = {h1.x, h1.y, h1.z, h1.w};
         pend = bu_four<W, MODE>(gs, a1, own, lam, cut, x);
       }
@@ -1047,9 +1059,7 @@ __device__ __forceinline__ void bu_level(const GraphDev &g, const Gather &gs, u6
 __global__ void k_build_head(const int64_t *__restrict__ beg, const int32_t *__restrict__ tadj,
                              int64_t V, int4 *__restrict__ head) {
   for (int64_t i = (int64_t)blockIdx.x * BS + threadIdx.x; i < 2 * V; i += (int64_t)gridDim.x * BS) {
-    const int64_t v = i < V ? i : i - V, j = beg[v] + (i < V ? 0 : 4), e = beg[v + 1];
-    head[i] = make_int4(j < e ? tadj[j] : NO_NBR, j + 1 < e ? tadj[j + 1] : NO_NBR,
-                        j + 2 < e ? tadj[j + 2] : NO_NBR, j + 3 < e ? tadj[j + 3] : NO_NBR);
+    head[i] = list_head(beg, tadj, i < V ? i : i - V, i < V ? 0 : 1);
   }
 }
 

@@ -263,6 +263,8 @@ int ibfs_traversal_noalloc(ibfs_graph_t g, const ibfs_config *cfg_in, const int3
   int cur = 0;
   NA_TRY(hipGetDevice(&cur));
   NA_TRY(hipSetDevice(g->device));
+  HeadsUse heads;
+  heads.take(g->heads);
   const int rc = run(g, cfg, src, k, depth_out, traversed_edges);
   (void)hipSetDevice(cur);
   return rc;

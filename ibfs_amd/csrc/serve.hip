@@ -155,6 +155,7 @@ struct ibfs_server_s {
   ibfs_graph_s *g = nullptr;
   ibfs_config cfg{};
   int K = 256, W = 4, R = 32, C = 1, chunk_shift = 12;
+  HeadsUse heads;
   std::vector<SCtx> ctx;
   std::thread worker;
   std::mutex mu;
@@ -888,6 +889,33 @@ void worker_main(ibfs_server_s *s) {
   }
 }
 
+// The server's keys and contexts.
+int alloc_server(ibfs_server_s *s) {
+  const ibfs_graph_s *g = s->g;
+  {  // two-hop size of every vertex, for cohort composition
+    const int64_t V = g->V;
+    std::vector<int32_t> all((size_t)V);
+    std::iota(all.begin(), all.end(), 0);
+    int32_t *d_all = nullptr;
+    u64 *d_key = nullptr;
+    hipError_t err = hipMalloc((void **)&d_all, sizeof(int32_t) * (size_t)std::max<int64_t>(V, 1));
+    if (err == hipSuccess) err = hipMalloc((void **)&d_key, sizeof(u64) * (size_t)std::max<int64_t>(V, 1));
+    if (err == hipSuccess) err = hipMemcpy(d_all, all.data(), sizeof(int32_t) * (size_t)V, hipMemcpyHostToDevice);
+    if (err == hipSuccess) err = launch_two_hop(g->d_beg, g->d_adj, g->d_deg, g->d_cid, d_all, V, d_key, nullptr);
+    if (err == hipSuccess) {
+      s->h_key.resize((size_t)V);
+      err = hipMemcpy(s->h_key.data(), d_key, sizeof(u64) * (size_t)V, hipMemcpyDeviceToHost);
+    }
+    if (d_all) (void)hipFree(d_all);
+    if (d_key) (void)hipFree(d_key);
+    if (err != hipSuccess) return fail(IBFS_ERR_HIP, "server key pass failed: %s", hipGetErrorString(err));
+  }
+  s->ctx.resize((size_t)s->C);
+  for (auto &c : s->ctx)
+    if (int rc = alloc_ctx(s, c)) return rc;
+  return IBFS_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -936,35 +964,17 @@ int ibfs_server_create(ibfs_graph_t g, const ibfs_config *cfg_in, int64_t status
     cus = 256;
   s->grid = cfg.dd_grid > 0 ? cfg.dd_grid : cus * 4;  // as in a batch, for the same reason
   s->hc = hub_cut(s->g, cfg.hybrid_hubs);
-  {  // two-hop size of every vertex, for cohort composition
-    const int64_t V = g->V;
-    std::vector<int32_t> all((size_t)V);
-    std::iota(all.begin(), all.end(), 0);
-    int32_t *d_all = nullptr;
-    u64 *d_key = nullptr;
-    hipError_t err = hipMalloc((void **)&d_all, sizeof(int32_t) * (size_t)std::max<int64_t>(V, 1));
-    if (err == hipSuccess) err = hipMalloc((void **)&d_key, sizeof(u64) * (size_t)std::max<int64_t>(V, 1));
-    if (err == hipSuccess) err = hipMemcpy(d_all, all.data(), sizeof(int32_t) * (size_t)V, hipMemcpyHostToDevice);
-    if (err == hipSuccess) err = launch_two_hop(g->d_beg, g->d_adj, g->d_deg, g->d_cid, d_all, V, d_key, nullptr);
-    if (err == hipSuccess) {
-      s->h_key.resize((size_t)V);
-      err = hipMemcpy(s->h_key.data(), d_key, sizeof(u64) * (size_t)V, hipMemcpyDeviceToHost);
-    }
-    if (d_all) (void)hipFree(d_all);
-    if (d_key) (void)hipFree(d_key);
-    if (err != hipSuccess) {
-      delete s;
-      return fail(IBFS_ERR_HIP, "server key pass failed: %s", hipGetErrorString(err));
-    }
+  s->heads.take(g->heads);
+  int rc = alloc_server(s);
+  if (rc && s->heads.drop()) {
+    for (auto &x : s->ctx) release_ctx(x);
+    s->ctx.clear();
+    rc = alloc_server(s);
   }
-  s->ctx.resize(C);
-  for (auto &c : s->ctx) {
-    int rc = alloc_ctx(s, c);
-    if (rc) {
-      for (auto &x : s->ctx) release_ctx(x);
-      delete s;
-      return rc;
-    }
+  if (rc) {
+    for (auto &x : s->ctx) release_ctx(x);
+    delete s;
+    return rc;
   }
   s->worker = std::thread(worker_main, s);
   *out = s;

@@ -247,8 +247,13 @@ int ibfs_graph_opts_default(ibfs_graph_opts *opts);
  * plus a traversal copy of the adjacency ordered by descending neighbour
  * degree).  The device copy keeps only the vertices with an edge (in or
  * out), renumbered in their original order; isolated vertices get no status
- * words and their depths come from the source list alone.  Replaces the
- * graph upload in the gpu_ibfs constructor (gpu_ibfs.cu:54-116). */
+ * words and their depths come from the source list alone.  Device memory: 16
+ * bytes per vertex with an edge, 4 per vertex, 8 per adjacency entry, 4 per
+ * hub; and, where it fits beside them, 32 per vertex with an edge for the heads
+ * of the lists, which speed bottom-up levels up (without them results are the
+ * same; an engine, batch or server that would not fit beside the heads frees
+ * them if it is the graph's only one).  Replaces the graph upload in the
+ * gpu_ibfs constructor (gpu_ibfs.cu:54-116). */
 int ibfs_graph_create(const int64_t *beg_pos, int64_t vert_count,
                       const int32_t *adj, int64_t edge_count, int device,
                       ibfs_graph_t *out);
