@@ -122,11 +122,12 @@ struct SCtx {
   // graph launches leave ≈8 µs between levels)
   hipGraph_t graph_burst[4] = {};
   hipGraphExec_t exec_burst[4] = {};
-  // burst graphs per host poll: a poll leaves the device idle for 50 to 60 us, a
-  // level past the end costs it 9.  Two where the context's last cohort needed
-  // more than one: a query of one source on R-MAT s14 178 -> 164 us, of 128 on a
-  // power-law graph of 300K vertices 351 -> 341, 32 queries on s20 6.93 -> 6.81 ms.
-  int bursts = 1;
+  // Cohorts in a row that needed more than one burst.  From kDeepRun on a host
+  // poll launches two: a poll leaves the device idle, which costs such a cohort
+  // 13 to 18 us (one source on R-MAT s14 178 -> 165 us, on s18 242 -> 229), but a
+  // cohort of fewer levels then runs four empty ones, which cost it 22 (a star's
+  // one source 110 -> 131), so it should come once in many.
+  int deep = 0;
   int W = 0, K = 0;  // current width: words per vertex and lanes (<= the server's)
   int coh = 0;     // 0: host-driven levels, 1: cohort levels on the device, 2: cohort emitting
   int dlevel = 0;  // cohort level the device expands next (host view)
@@ -186,6 +187,7 @@ struct ibfs_server_s {
 
 namespace {
 constexpr int kCohortBurst = 4;  // levels of a burst graph
+constexpr int kDeepRun = 8;      // SCtx::deep
 }
 
 namespace {
@@ -639,7 +641,8 @@ void take_pending(ibfs_server_s *s, SCtx &c, int L, int n0, int *n_new) {
 // window is flushed first when it is full).  locked: the caller holds the
 // server lock.
 int cohort_burst(ibfs_server_s *s, SCtx &c, bool locked) {
-  int B = std::min(kCohortBurst * c.bursts, s->R - 1 - (c.dlevel - c.base));
+  const int most = c.deep >= kDeepRun ? 2 * kCohortBurst : kCohortBurst;
+  int B = std::min(most, s->R - 1 - (c.dlevel - c.base));
   if (B < 1) {
     std::vector<int> act;
     for (int k = 0; k < c.K; ++k)
@@ -647,7 +650,7 @@ int cohort_burst(ibfs_server_s *s, SCtx &c, bool locked) {
     int rc = emit_lanes(s, c, act, c.base, c.dlevel - 1, 1);
     if (rc) return rc;
     c.base = c.dlevel - 1;
-    B = std::min(kCohortBurst * c.bursts, s->R - 1 - (c.dlevel - c.base));
+    B = std::min(most, s->R - 1 - (c.dlevel - c.base));
   }
   hipGraphExec_t x = c.exec[__builtin_ctz((unsigned)c.W)];
   const int win = s->admit_window;
@@ -802,7 +805,7 @@ int start_cohort(ibfs_server_s *s, SCtx &c) {
 int cohort_step(ibfs_server_s *s, SCtx &c) {
   if (c.coh == 1) {
     if (c.h_plan->done) {
-      c.bursts = c.h_plan->last + 1 > kCohortBurst ? 2 : 1;
+      c.deep = c.h_plan->last + 1 > kCohortBurst ? std::min(c.deep + 1, kDeepRun) : 0;
       std::vector<int> act;
       for (int k = 0; k < c.K; ++k)
         if (c.lanes[k].state == ACTIVE) act.push_back(k);

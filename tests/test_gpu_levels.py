@@ -390,3 +390,33 @@ def test_groupby_past_the_wait_limit():
         np.testing.assert_array_equal(other.groupby(src), want)
         g.close()
         np.testing.assert_array_equal(other.groupby(src), want)
+
+
+def test_server_launches_two_bursts_after_a_run_of_deep_cohorts():
+    """Polls of the host per cohort (four or eight levels each, by the server's
+    counter): a query of 12 levels takes fewer once eight such cohorts came in a
+    row, not before, and one of two levels ends that."""
+    say("[gpu] server bursts")
+    n = 2000  # a star, and a path of 12 behind it
+    a = np.concatenate([np.zeros(n - 1, dtype=np.int64), n + np.arange(11)])
+    b = np.concatenate([np.arange(1, n), n + 1 + np.arange(11)])
+    beg, adj = _symmetric(n + 12, a, b)
+    g = ibfs_amd.DeviceGraph(ibfs_amd.HostCsr.from_arrays(beg, adj))
+    s = ibfs_amd.Server(g, lane_bits=64)
+    out = ibfs_amd.DeviceBuffer(4 * (n + 12))
+    want = {v: oracle.bfs_many(beg, adj, np.array([v], dtype=np.int32), threads=1)[0] for v in (n, 5)}
+
+    def polls(v):
+        before = s.counters()["levels"]
+        q = s.submit(np.array([v], dtype=np.int32), out)
+        s.wait(q)
+        s.release(q)
+        np.testing.assert_array_equal(out.to_host(), want[v])
+        return s.counters()["levels"] - before
+
+    for _ in range(2):
+        assert [polls(n) for _ in range(8)] == [3] * 8  # levels 1 to 12, the last changes nothing
+        assert polls(n) == 2
+        assert polls(5) == 1
+        assert polls(n) == 3 and polls(5) == 1
+    s.close()
