@@ -92,7 +92,6 @@ struct Plan {
                         // 4 sparse tail
   int done;             // 1 once a level produced no change
   int last;             // deepest level with a change (valid when done)
-  unsigned int blocks_done;  // unused (kept for the layout the host copies)
   int policy, sw_level, alpha, beta;
   int gamma;            // hybrid cost factor (1/64 units; 0: never hybrid)
   int rho;              // hub entries per adjacency entry of the graph (1/1024 units)
@@ -109,7 +108,7 @@ struct Plan {
   // inspection and its full-slot copy are skipped.  tail_div 0: never.
   int tail_div;
   int tail_start;       // first sparse level (0: every level so far was dense)
-  int tail_pad[2];
+  int tail_pad;
   u64 tail_cap;         // records the log holds
   u64 tail_lo, tail_hi; // records of level `level`-1: the frontier of `level`
   u64 tail_count;       // records appended (device atomics); > tail_cap: the
@@ -326,7 +325,6 @@ hipError_t launch_fill_u64(u64 *p, int64_t n, u64 value, hipStream_t st);
 // zeros in [p0, p0+n0), [p1, p1+n1) and [p2, p2+n2) (u64 words), one launch
 hipError_t launch_zero3_u64(u64 *p0, int64_t n0, u64 *p1, int64_t n1, u64 *p2, int64_t n2,
                             hipStream_t st);
-hipError_t launch_fill_i32(int32_t *p, int64_t n, int32_t value, hipStream_t st);
 // One launch that prepares a group of sl.k sources (original ids), lane i =
 // source i from level 0: S0 with their bits and the flags, both otherwise zero
 // (Vt vertices), the control ring (ctl_words 64-bit words) zero, lane table

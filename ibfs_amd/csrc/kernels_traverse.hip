@@ -26,11 +26,6 @@ __global__ void k_zero3_u64(u64 *p0, int64_t n0, u64 *p1, int64_t n1, u64 *p2, i
   }
 }
 
-__global__ void k_fill_i32(int32_t *p, int64_t n, int32_t value) {
-  for (int64_t i = (int64_t)blockIdx.x * BS + threadIdx.x; i < n; i += (int64_t)gridDim.x * BS)
-    p[i] = value;
-}
-
 // Group start (launch_group_start): a workgroup zeroes the words and flags of
 // its share of the vertices and sets there the bits of the sources that fall
 // into it, so one launch replaces three copies and two fills.  Bound by
@@ -1606,12 +1601,6 @@ hipError_t launch_zero3_u64(u64 *p0, int64_t n0, u64 *p1, int64_t n1, u64 *p2, i
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_zero3_u64, dim3(grid_for(n, BS * 8, 8192)), dim3(BS), 0, st, p0, n0, p1, n1,
                      p2, n2);
-  return hipGetLastError();
-}
-
-hipError_t launch_fill_i32(int32_t *p, int64_t n, int32_t value, hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(n, BS * 8, 8192)), dim3(BS), 0, st, p, n, value);
   return hipGetLastError();
 }
 
