@@ -518,17 +518,23 @@ __global__ __launch_bounds__(BS) void k_emit_wide(const u64 *__restrict__ ring, 
 // The lanes are counted side by side: a thread takes one status word (64
 // lanes) of every stride-th vertex and adds, per level, the word of counted
 // bits still absent there into bit-sliced counters (plane j holds bit j of 64
-// sums): a carry-save tree takes eight levels at a time into planes 0 to 2 and
-// ripples one carry into the rest.  Threads of a wave with the same word add
-// their planes in a butterfly, lane k reads off the sum of lane k, and a
-// workgroup adds once per lane to the outputs.  Bound by reading the window's
-// snapshots (consecutive 8-byte words); one ballot per lane, counter bit and
-// 64 vertices instead took 415 us of a 256-lane group on R-MAT s18, most of
-// its time.
+// sums): a carry-save tree (that of the Harley-Seal population count) takes
+// eight levels at a time into planes 0 to 2 and ripples one carry into the rest.
+// Threads of a wave with the same word add their planes in a butterfly, lane k
+// reads off the sum of lane k, and a workgroup adds once per lane to the
+// outputs.  Bound by reading the window's snapshots (consecutive 8-byte words);
+// one ballot per lane, counter bit and 64 vertices instead took 415 us of a
+// 256-lane group on R-MAT s18, most of its time.
 constexpr int CLOSE_BS = 512;
 constexpr int CLOSE_ITEMS = 64;  // words per thread between reductions: plane counts below
 constexpr int CLOSE_SP = 20;     // sums: 64 x 255 levels (14 bits) x 64 threads
 constexpr int CLOSE_RP = 13;     // reach: 64 (7 bits) x 64 threads
+// A workgroup sums in 32 bits: at most 254 counted levels (windows under 256) of
+// its share of the vertices, the most where the grid is CLOSE_GRID workgroups.
+constexpr int CLOSE_GRID = 256;
+static_assert((((u64)1 << 31) / CLOSE_GRID + CLOSE_BS) * 254 < (u64)1 << 32, "k_close sums");
+static_assert(CLOSE_ITEMS * 254 * 64 < 1 << CLOSE_SP && CLOSE_ITEMS * 64 < 1 << CLOSE_RP,
+              "k_close planes");
 
 __device__ __forceinline__ void csa(u64 &hi, u64 &lo, u64 a, u64 b) {
   const u64 u = lo ^ a;
@@ -914,8 +920,7 @@ static hipError_t close_w(const u64 *ring, int R, EmitSpace sp, int b, int e, co
                           const u64 *masks, const u64 *sel, int k, u64 *sum, u64 *reach,
                           hipStream_t st) {
   if (e - b + 1 >= 256) return hipErrorInvalidValue;
-  // a workgroup sums in 32 bits: 255 levels of a 256th of the vertices fit
-  dim3 g(grid_for(sp.Vt * W, CLOSE_BS * 4, 256)), blk(CLOSE_BS);
+  dim3 g(grid_for(sp.Vt * W, CLOSE_BS * 4, CLOSE_GRID)), blk(CLOSE_BS);
   hipLaunchKernelGGL(k_close<W>, g, blk, 0, st, ring, R, sp.Vt, b, e, lanes, masks, sel, k, sum,
                      reach);
   return hipGetLastError();
