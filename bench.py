@@ -43,10 +43,10 @@ WORKLOADS = {
 
 # Plain-leg engine settings per workload: inspector workgroup size and the
 # degree classes' thresholds (the reference's gpu_ibfs takes sml_shed and
-# lrg_shed as constructor arguments, gpu_ibfs.cu:36-45).  For R-MAT s22 a sweep
-# of the three on 8 x 128 lanes took 15.12 ms per 1,024 sources with these
-# against 15.43-15.47 ms with the library defaults (512, 64, 512); other
-# workloads keep the defaults.
+# lrg_shed as constructor arguments, gpu_ibfs.cu:36-45).  For R-MAT s22 these came
+# out of a sweep of the three on 8 x 128 lanes, on kernels that have changed
+# since: 1,024 sources now take 12.63 ms with them and 12.59 with the library
+# defaults (512, 64, 512).  Other workloads keep the defaults.
 PLAIN_SETTINGS = {"s22": dict(wg_size=1024, sml_shed=128, lrg_shed=2048)}
 
 

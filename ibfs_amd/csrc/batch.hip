@@ -681,10 +681,10 @@ static int batch_run_impl(ibfs_batch_s *b, const int32_t *src, int64_t n, int32_
             if (stats) stats->n_tail_reruns++;
           } else if (c.h_plan->done) {
             // the group's emission is enqueued; the context's next group can
-            // be enqueued behind it at once (stream order: its set-up copy
-            // and fills start after the emission has read the ring, the lane
-            // table and the tail log), and the final stream synchronisation
-            // waits for the last one
+            // be enqueued behind it at once (stream order: its set-up launch
+            // starts after the emission has read the ring, the lane table and
+            // the tail log), and the final stream synchronisation waits for
+            // the last one
             rc = finish_group(b, c, c.h_plan->last, stats);
             c.state = IDLE;
             ++finished;

@@ -35,7 +35,7 @@ struct ibfs_engine_s {
   HubCut hc;           // hubs a hybrid level pulls through
   HeadsUse heads;
   hipStream_t st = nullptr;
-  hipEvent_t ev_wait = nullptr;  // recorded after each host copy the loop waits for
+  hipEvent_t ev_wait = nullptr;  // behind a failed call's work (poll_stream)
   u64 *ring = nullptr;
   LevelCtl *d_ctl = nullptr;
   // coherent pinned: control blocks posted by the inspector (level l into

@@ -306,11 +306,13 @@ struct InspectArgs {
 
 // Whether the inspection of a level writes the bottom-up candidates to a
 // queue, from the candidates of the level before it (at level 0: every
-// vertex).  Candidates only become fewer within a traversal, so this bounds
-// them.  A bottom-up level over most vertices scans them all instead, which
+// vertex).  A bottom-up level over most vertices scans them all instead, which
 // streams their words, heads and flags and spares each inspection a queue
 // entry per vertex and its reservations; below an eighth of the vertices the
-// scan would read more than the queue saves.
+// scan would read more than the queue saves.  This foresees the queue's length
+// while the lanes are the same, for candidates then only become fewer; where
+// lanes join (phase offsets, admission) nearly every vertex is one again, and
+// that level's queue is long.  A queue holds every vertex (queue_entries).
 __host__ __device__ inline bool candidates_queued(int L, u64 n_cand_prev, u64 V) {
   return L > 0 && n_cand_prev * 8 < V;
 }
@@ -352,7 +354,6 @@ struct GroupPost {
   u64 tag;
 };
 hipError_t launch_group_end(const u64 *counters, GroupPost *post, u64 tag, hipStream_t st);
-// S0[src[i]] |= bit lane0+i, i < k (src in traversal ids; -1 entries skipped).
 // S[src[i]] |= bit lane[i], i < n (traversal ids; -1 entries skipped).
 hipError_t launch_admit(int W, const int32_t *src, const int32_t *lane, int n, u64 *S,
                         uint8_t *flags, hipStream_t st);

@@ -1058,9 +1058,9 @@ __global__ void k_build_head(const int64_t *__restrict__ beg, const int32_t *__r
   }
 }
 
-// Host-driven top-down: workgroups [0, nbs) take small vertices one per
-// thread, [nbs, nbs+nbm) mid vertices one per wave, the rest one chunk of
-// 2^chunk_shift edges of a large vertex per workgroup.
+// Host-driven top-down: workgroups [0, nbs) take small vertices one per row of
+// TD_SMALL lanes, [nbs, nbs+nbm) mid vertices one per wave, the rest one chunk
+// of 2^chunk_shift edges of a large vertex per workgroup.
 template <int W>
 __global__ __launch_bounds__(BS) void k_expand_td(GraphDev g, const u64 *__restrict__ prev,
                                                   u64 *cur, const LevelCtl *__restrict__ ctl,
