@@ -126,7 +126,9 @@ struct SCtx {
   // poll launches two: a poll leaves the device idle, which costs such a cohort
   // 13 to 18 us (one source on R-MAT s14 178 -> 165 us, on s18 242 -> 229), but a
   // cohort of fewer levels then runs four empty ones, which cost it 22 (a star's
-  // one source 110 -> 131), so it should come once in many.
+  // one source 110 -> 131), so deep ones and others in turn get one burst.  Two in
+  // a row are enough: with four or eight, a burst of 32 queries on s20, a few
+  // cohorts on a new server, took 0 to 2% longer.
   int deep = 0;
   int W = 0, K = 0;  // current width: words per vertex and lanes (<= the server's)
   int coh = 0;     // 0: host-driven levels, 1: cohort levels on the device, 2: cohort emitting
@@ -187,7 +189,7 @@ struct ibfs_server_s {
 
 namespace {
 constexpr int kCohortBurst = 4;  // levels of a burst graph
-constexpr int kDeepRun = 8;      // SCtx::deep
+constexpr int kDeepRun = 2;      // SCtx::deep
 }
 
 namespace {

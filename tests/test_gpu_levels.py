@@ -394,7 +394,7 @@ def test_groupby_past_the_wait_limit():
 
 def test_server_launches_two_bursts_after_a_run_of_deep_cohorts():
     """Polls of the host per cohort (four or eight levels each, by the server's
-    counter): a query of 12 levels takes fewer once eight such cohorts came in a
+    counter): a query of 12 levels takes fewer once two such cohorts came in a
     row, not before, and one of two levels ends that."""
     say("[gpu] server bursts")
     n = 2000  # a star, and a path of 12 behind it
@@ -415,7 +415,7 @@ def test_server_launches_two_bursts_after_a_run_of_deep_cohorts():
         return s.counters()["levels"] - before
 
     for _ in range(2):
-        assert [polls(n) for _ in range(8)] == [3] * 8  # levels 1 to 12, the last changes nothing
+        assert [polls(n) for _ in range(2)] == [3] * 2  # levels 1 to 12, the last changes nothing
         assert polls(n) == 2
         assert polls(5) == 1
         assert polls(n) == 3 and polls(5) == 1
